@@ -193,6 +193,18 @@ typedef struct fqehip_sector {
    * (tile FQEHIP_TILE_OZAKI; fqehip_beta_block_digits): when set, the
    * beta-beta GEMM also runs as digit products; NULL keeps it in FP64. */
   const void* hbb_oz;
+  /* Pull form of the complex128 two-body apply (real, complex or
+   * spin-orbital operators): H C = Haa C + C Hbb^T + sum_q E^b_q (sum_p
+   * W[p][q] E^a_p C).  When pull_w is set (with all the fields below) and
+   * fqehip_pull_supported() holds, fqehip_apply takes it; its workspace is
+   * then one complex128 row accumulator (16 lena lenb bytes).  For a complex
+   * operator (complex_op = 1) W, Haa and Hbb are complex128. */
+  const int32_t* dexc_a;   /* alpha de-excitation rows (fqehip_string_tables) */
+  const double* pull_w;    /* [npull][npull] coupling, alpha pair p, beta pair q */
+  const double* haa;       /* fqehip_spin_block of the alpha strings */
+  const double* hbb;       /* fqehip_spin_block of the beta strings */
+  const uint32_t* pull_fwd; /* [npull][lenb] fqehip_pull_table of the beta strings */
+  int npull;               /* pairs of one spin: norb(norb+1)/2 or norb^2 */
 } fqehip_sector;
 
 #define FQEHIP_TILE_ROWS4 4
@@ -263,6 +275,26 @@ int64_t fqehip_beta_block_ld(int64_t lenb);
 int fqehip_beta_block(int npair, int64_t lenb, const int32_t* d_fwd_b,
                       const double* d_a, double* d_hcol, uint16_t* d_hhi,
                       uint16_t* d_hlo, int64_t ldh, void* stream);
+/* Matrix of a two-body operator on the strings of one spin,
+ *   H = sum_pq V[p][q] E_p E_q + sum_q h[q] E_q,
+ * by source string: d_hcol[I][I'] = <I'|H|I> (len x len; complex128 when
+ * complex_op).  V[p][q] is element (p, q) of d_v with lda doubles per row and
+ * h the row d_h (for complex_op both in the real 2 x 2 block form of
+ * fqehip_operator, d_v and d_h at the real part of element (0, 0)); d_fwd the
+ * forward table of the npair pairs.  fqehip_beta_block is the real case with
+ * its bfloat16 split.  (len + npair) * 8 bytes (16 for complex_op) <= 160 KiB;
+ * the same bits on every run. */
+int fqehip_spin_block(int complex_op, int npair, int64_t len,
+                      const int32_t* d_fwd, const double* d_v, int64_t lda,
+                      const double* d_h, double* d_hcol, void* stream);
+/* Target words of the pull form's row kernel, from the forward table d_fwd
+ * ([npair][len], sign*(tgt+1) or 0): 8 (tgt + 1) with the sign in bit 31. */
+int fqehip_pull_table(int npair, int64_t len, const int32_t* d_fwd,
+                      uint32_t* d_tab, void* stream);
+/* Whether fqehip_apply takes the pull form for this sector and operator. */
+int fqehip_pull_supported(int precision, const fqehip_sector* s,
+                          const fqehip_operator* op);
+
 /* Ozaki digits of an FP64 beta-beta block (d_hcol, the hcol output of
  * fqehip_beta_block) for the digit apply's beta-beta GEMM, written to d_hoz
  * (fqehip_beta_block_digits_bytes(lenb) bytes): int8 [5][lenb][ldk]
@@ -315,7 +347,8 @@ int fqehip_apply_slot_reduce(int precision, const fqehip_sector* s,
 
 /* Bytes of workspace for one apply of a sector: the larger of the unfused
  * path (dvec + Y planes) and the fused path (slot rows + row
- * accumulators). */
+ * accumulators); with pull_w set and the sector within the pull form's
+ * limits, its row accumulator alone. */
 int64_t fqehip_apply_workspace_bytes(int precision, const fqehip_sector* s);
 
 /* out = alpha * H C + beta * cin (see fqehip_scatter for acc/partials).

@@ -640,6 +640,16 @@ int launch_slot_reduce(int precision, bool p48, int nslot, int64_t lena,
                        const void* cin, void* out, double* acc,
                        double* partials, hipStream_t st, const int32_t* done);
 
+// Defined in pull.hip.
+bool pull_supported(const fqehip_sector* s);
+int launch_same_spin(const fqehip_sector* s, int complex_op,
+                     const double* coeff, double* rowacc, hipStream_t st,
+                     const int32_t* done);
+int launch_pull_rows(const fqehip_sector* s, int complex_op,
+                     const double* coeff, double* rowacc, double ar, double ai,
+                     double br, double bi, const double* cin, double* out,
+                     double* acc, hipStream_t st, const int32_t* done);
+
 // Declared in gemm_bf16.hip.
 int launch_gemm_bf16x3(int m, int k, const double* a, int64_t ncol,
                        const float* b, float* y, hipStream_t st,
@@ -835,6 +845,12 @@ bool ozaki_split(int precision, const fqehip_sector* s) {
          s->tile == FQEHIP_TILE_OZAKI;
 }
 
+// Whether two-body applies of the sector take the pull form: it carries the
+// form's tables and is within its limits.
+bool pull_sector(int precision, const fqehip_sector* s) {
+  return precision == FQEHIP_C128 && s->pull_w != nullptr && pull_supported(s);
+}
+
 // Workspace of the fused / split paths: slot rows, row accumulators and,
 // for the Ozaki-digit split apply, the beta gather table (lenb x 128
 // words), the row maxima of |C| (lena doubles) and, with hbb_oz, the C
@@ -852,6 +868,11 @@ int64_t fused_workspace_bytes(int precision, const fqehip_sector* s) {
 }
 
 }  // namespace
+
+extern "C" int fqehip_pull_supported(int precision, const fqehip_sector* s,
+                                     const fqehip_operator* op) {
+  return s && op && op->a && !op->h1 && pull_sector(precision, s);
+}
 
 extern "C" int fqehip_fused_supported(int precision, const fqehip_sector* s,
                                       const fqehip_operator* op) {
@@ -876,6 +897,15 @@ int fused_rows(int precision, const fqehip_sector* s, const fqehip_operator* op,
                const void* d_coeff, void* d_workspace, const int32_t* d_done,
                void* stream, bool reuse_tables) {
   if (int rc = check_sector_op(precision, s, op)) return rc;
+  if (fqehip_pull_supported(precision, s, op)) {
+    FQEHIP_CHECK_ARG(d_coeff && d_workspace, "NULL pointer");
+    const double* c = static_cast<const double*>(d_coeff);
+    double* rowacc = static_cast<double*>(d_workspace);
+    int rc = launch_same_spin(s, op->complex_op, c, rowacc, as_stream(stream), d_done);
+    if (rc) return rc;
+    return launch_pull_rows(s, op->complex_op, c, rowacc, 1.0, 0.0, 0.0, 0.0,
+                            nullptr, nullptr, nullptr, as_stream(stream), d_done);
+  }
   FQEHIP_CHECK_ARG(fqehip_fused_supported(precision, s, op),
                    "the fused path does not support this sector/operator");
   FQEHIP_CHECK_ARG(d_coeff && d_workspace, "NULL pointer");
@@ -969,6 +999,11 @@ extern "C" int fqehip_apply_slot_reduce(int precision, const fqehip_sector* s,
                    "beta != 0 needs d_cin");
   const int64_t n = s->lena * s->lenb;
   const char* ws = static_cast<const char*>(d_workspace);
+  if (pull_sector(precision, s))   // no slot rows: the accumulators are H C
+    return launch_slot_reduce(precision, false, 0, s->lena, s->lenb, ws, ws,
+                              alpha_re, alpha_im, beta_re, beta_im, d_cin,
+                              d_out, d_acc, d_norm_partials, as_stream(stream),
+                              d_done);
   const void* rowacc = ws + static_cast<int64_t>(s->nslot) * 2 * n * elem_size(precision);
   // the Ozaki-digit row kernel writes the slot rows in 48 bits per double
   return launch_slot_reduce(precision, ozaki_split(precision, s), s->nslot,
@@ -981,6 +1016,7 @@ extern "C" int64_t fqehip_apply_workspace_bytes(int precision,
                                                const fqehip_sector* s) {
   if (!s) return -1;
   const int64_t n = s->lena * s->lenb;
+  if (pull_sector(precision, s)) return 2 * n * static_cast<int64_t>(sizeof(double));
   const int64_t unfused = static_cast<int64_t>(2 * s->npair + 1) * 2 * n *
                           static_cast<int64_t>(elem_size(precision));
   const int64_t fused = fused_workspace_bytes(precision, s);
@@ -1008,6 +1044,28 @@ int fqehip::apply_reusing_tables(
   FQEHIP_CHECK_ARG(d_workspace != nullptr, "NULL workspace");
   const int64_t n = s->lena * s->lenb;
   char* ws = static_cast<char*>(d_workspace);
+  if (fqehip_pull_supported(precision, s, op)) {
+    FQEHIP_CHECK_ARG((beta_re == 0.0 && beta_im == 0.0) || d_cin,
+                     "beta != 0 needs d_cin");
+    // the epilogue in the row kernel, except in place (other rows still read
+    // d_coeff) and for norm partials (one per 256 elements)
+    if (d_out == d_coeff || d_norm_partials) {
+      int rc = fused_rows(precision, s, op, d_coeff, d_workspace, d_done, stream,
+                          false);
+      if (rc) return rc;
+      return fqehip_apply_slot_reduce(precision, s, d_workspace, alpha_re,
+                                      alpha_im, beta_re, beta_im, d_cin, d_out,
+                                      d_acc, d_norm_partials, d_done, stream);
+    }
+    const double* c = static_cast<const double*>(d_coeff);
+    double* rowacc = static_cast<double*>(d_workspace);
+    hipStream_t st = as_stream(stream);
+    int rc = launch_same_spin(s, op->complex_op, c, rowacc, st, d_done);
+    if (rc) return rc;
+    return launch_pull_rows(s, op->complex_op, c, rowacc, alpha_re, alpha_im,
+                            beta_re, beta_im, static_cast<const double*>(d_cin),
+                            static_cast<double*>(d_out), d_acc, st, d_done);
+  }
   if (fqehip_fused_supported(precision, s, op)) {
     int rc = fused_rows(precision, s, op, d_coeff, d_workspace, d_done, stream,
                         reuse_tables);

@@ -11,7 +11,7 @@
 // makes the same same-spin / opposite-spin split in its lm kernels
 // (src/fqe/lib/fqe_data.c:668-720 and :879-996).
 //
-//   k_beta_block:  Hbb column by column from the beta forward table
+//   k_spin_block:  Hbb column by column from the beta forward table
 //                  (one workgroup per source string, column in LDS);
 //   k_beta_split:  transpose and split into bfloat16 hi + lo, zero-padded
 //                  to ldh x ldh (ldh a multiple of 128);
@@ -43,22 +43,38 @@ __device__ __forceinline__ float from_bf16(__bf16 h) {
 
 __device__ __forceinline__ int32_t iabs(int32_t v) { return v < 0 ? -v : v; }
 
-// Column Ib of Hbb: LDS accumulator of lenb doubles, built in a fixed
+// Column Ib of the block: LDS accumulator of lenb values, built in a fixed
 // order so that every run gives the same bits.  For each q in turn the
 // intermediate string s = E_q Ib is uniform over the workgroup; the
 // off-diagonal pairs p move one electron of s, so they reach distinct
 // targets t != s and are added by one thread each; the diagonal pairs
 // (t = s) and the one-body term of q are summed by wave 0 in a fixed lane
 // order (per-lane strided sums, then an xor butterfly) and added to s.
+// V[p][q] is amat[p * lda + q], the one-body term h1[q]; CPLX: both in the
+// real 2 x 2 block form (real part at [2p][2q], imaginary at [2p + 1][2q]).
+template <bool CPLX>
+struct BlockValue {
+  double re, im;
+};
+template <>
+struct BlockValue<false> {
+  double re;
+};
+
+template <bool CPLX>
 __global__ void __launch_bounds__(kBlockThreads)
-k_beta_block(int npair, int64_t lenb, const int32_t* __restrict__ fwd,
-             const double* __restrict__ amat, double* __restrict__ hcol) {
-  extern __shared__ double col[];
-  double* diag = col + lenb;                  // [npair] diagonal terms of q
+k_spin_block(int npair, int64_t lenb, const int32_t* __restrict__ fwd,
+             const double* __restrict__ amat, int64_t lda,
+             const double* __restrict__ h1, double* __restrict__ hcol) {
+  typedef BlockValue<CPLX> V;
+  constexpr int kW = CPLX ? 2 : 1;            // rows and columns per pair
+  extern __shared__ __align__(16) char block_smem[];
+  V* col = reinterpret_cast<V*>(block_smem);
+  V* diag = col + lenb;                       // [npair] diagonal terms of q
   const int64_t ib = blockIdx.x;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  for (int64_t x = tid; x < lenb; x += kBlockThreads) col[x] = 0.0;
+  for (int64_t x = tid; x < lenb; x += kBlockThreads) col[x] = V{};
   __syncthreads();
   const int K = npair;
   for (int q = 0; q < K; ++q) {
@@ -68,26 +84,43 @@ k_beta_block(int npair, int64_t lenb, const int32_t* __restrict__ fwd,
     const double sf = f > 0 ? 1.0 : -1.0;
     for (int p = tid; p < K; p += kBlockThreads) {
       const int32_t g = fwd[static_cast<int64_t>(p) * lenb + s];
-      double v = 0.0;
+      V v{};
       if (g) {
-        const double c = (g > 0 ? sf : -sf) * amat[static_cast<int64_t>(p) * K + q];
+        const double sg = g > 0 ? sf : -sf;
+        const double* e = amat + static_cast<int64_t>(kW) * p * lda + kW * q;
+        V c{};
+        c.re = sg * e[0];
+        if constexpr (CPLX) c.im = sg * e[lda];
         const int64_t t = iabs(g) - 1;
-        if (t == s) v = c;
-        else col[t] += c;
+        if (t == s) {
+          v = c;
+        } else {
+          col[t].re += c.re;
+          if constexpr (CPLX) col[t].im += c.im;
+        }
       }
       diag[p] = v;
     }
     __syncthreads();
     if (tid < 64) {
-      double v = 0.0;
-      for (int p = lane; p < K; p += 64) v += diag[p];
+      V v{};
+      for (int p = lane; p < K; p += 64) {
+        v.re += diag[p].re;
+        if constexpr (CPLX) v.im += diag[p].im;
+      }
 #pragma unroll
-      for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m);
-      if (lane == 0) col[s] += v + sf * amat[static_cast<int64_t>(npair) * K + q];
+      for (int m = 32; m >= 1; m >>= 1) {
+        v.re += __shfl_xor(v.re, m);
+        if constexpr (CPLX) v.im += __shfl_xor(v.im, m);
+      }
+      if (lane == 0) {
+        col[s].re += v.re + sf * h1[kW * q];
+        if constexpr (CPLX) col[s].im += v.im + sf * h1[lda + kW * q];
+      }
     }
     __syncthreads();
   }
-  double* dst = hcol + ib * lenb;
+  V* dst = reinterpret_cast<V*>(hcol) + ib * lenb;
   for (int64_t x = tid; x < lenb; x += kBlockThreads) dst[x] = col[x];
 }
 
@@ -498,15 +531,42 @@ extern "C" int fqehip_beta_block(int npair, int64_t lenb, const int32_t* d_fwd_b
   FQEHIP_CHECK_ARG(npair == 0 || d_fwd_b, "NULL beta forward table");
   hipStream_t st = as_stream(stream);
   // npair == 0 (no orbitals) leaves the LDS column zero: Hbb = 0
-  k_beta_block<<<static_cast<unsigned>(lenb), kBlockThreads,
-                 (lenb + npair) * sizeof(double), st>>>(npair, lenb, d_fwd_b, d_a,
-                                                        d_hcol);
-  FQEHIP_CHECK_LAUNCH("k_beta_block");
+  k_spin_block<false><<<static_cast<unsigned>(lenb), kBlockThreads,
+                        (lenb + npair) * sizeof(double), st>>>(
+      npair, lenb, d_fwd_b, d_a, npair,
+      d_a + static_cast<int64_t>(npair) * npair, d_hcol);
+  FQEHIP_CHECK_LAUNCH("k_spin_block");
   dim3 grid(static_cast<unsigned>(ldh / 32), static_cast<unsigned>(ldh / 32));
   k_beta_split<<<grid, 256, 0, st>>>(lenb, ldh, d_hcol,
                                       reinterpret_cast<__bf16*>(d_hhi),
                                       reinterpret_cast<__bf16*>(d_hlo));
   FQEHIP_CHECK_LAUNCH("k_beta_split");
+  return FQEHIP_OK;
+}
+
+extern "C" int fqehip_spin_block(int complex_op, int npair, int64_t len,
+                                 const int32_t* d_fwd, const double* d_v,
+                                 int64_t lda, const double* d_h, double* d_hcol,
+                                 void* stream) {
+  clear_error();
+  FQEHIP_CHECK_ARG(complex_op == 0 || complex_op == 1, "complex_op=%d", complex_op);
+  const int64_t w = complex_op ? 2 : 1;
+  FQEHIP_CHECK_ARG(npair >= 0 && len >= 0 && lda >= w * npair,
+                   "npair=%d len=%lld lda=%lld", npair,
+                   static_cast<long long>(len), static_cast<long long>(lda));
+  const size_t lds = static_cast<size_t>(len + npair) * sizeof(double) * w;
+  FQEHIP_CHECK_ARG(lds <= 160 * 1024, "len=%lld exceeds the LDS column of the block",
+                   static_cast<long long>(len));
+  if (len == 0) return FQEHIP_OK;
+  FQEHIP_CHECK_ARG(d_hcol && (npair == 0 || (d_fwd && d_v && d_h)), "NULL pointer");
+  hipStream_t st = as_stream(stream);
+  if (complex_op)
+    k_spin_block<true><<<static_cast<unsigned>(len), kBlockThreads, lds, st>>>(
+        npair, len, d_fwd, d_v, lda, d_h, d_hcol);
+  else
+    k_spin_block<false><<<static_cast<unsigned>(len), kBlockThreads, lds, st>>>(
+        npair, len, d_fwd, d_v, lda, d_h, d_hcol);
+  FQEHIP_CHECK_LAUNCH("k_spin_block");
   return FQEHIP_OK;
 }
 

@@ -1,0 +1,695 @@
+// Pull form of the complex128 two-body apply, without a dvec and without
+// slot rows.
+//
+// Alpha and beta pair operators commute, so for any operator in the dvec
+// form H = sum_pq V[p][q] E_p E_q + sum_q h1'[q] E_q, E_p = E^a_p + E^b_p
+// (reference src/fqe/fqe_data.py:646-683), or with separate spin-orbital
+// blocks (:712-741),
+//
+//   H C = Haa C + C Hbb^T + sum_q E^b_q ( sum_p W[p][q] E^a_p C ),
+//
+// Haa and Hbb the matrices of the operator on the strings of one spin
+// (fqehip_spin_block), W[p][q] = V[p][q] + V[q][p] (alpha pair p, beta pair
+// q) the opposite-spin coupling; the reference's lm kernels make the same
+// three-way split (src/fqe/lib/fqe_data.c:668-720, :879-996).
+//
+//   k_same_spin_f64:  rowacc = Haa C + C Hbb^T, both products accumulated in
+//       the same registers (one pass over K = lena, then over K = lenb);
+//   k_pull_rows_f64:  one workgroup per alpha string ia.  E^a_p C at row ia
+//       is +-C[src_p(ia), :], a whole row of C, so the contraction over p is
+//       a GEMM of W (beta pairs x the live alpha pairs of ia) with rows of
+//       C as they lie in memory, and E^b_q moves its result within row ia,
+//       which is an accumulator row in LDS.
+//
+// Against the split form (beta excitations gathered, alpha excitations
+// scattered to slot rows in HBM): the B operand needs no gather within the
+// row, no sign and no conversion; K is the live alpha pairs (50 of 105 at
+// norb 14) instead of all pairs; and the slot rows, nalpha (norb - nalpha)
+// values of 16 bytes per determinant written and read again, are gone.  The
+// price is the dense Haa C.
+#include <type_traits>
+
+#include "fqehip_common.h"
+#include "rows_common.h"
+
+namespace fqehip {
+namespace {
+
+using namespace rows;
+
+typedef double double4_t __attribute__((ext_vector_type(4)));
+
+constexpr size_t kLdsLimit = 160 * 1024;
+constexpr int64_t kOffLimit = int64_t(1) << 31;   // 32-bit buffer offsets
+
+__device__ __forceinline__ double u2d(uint32_t lo, uint32_t hi) {
+  return __longlong_as_double(static_cast<long long>(
+      static_cast<uint64_t>(lo) | (static_cast<uint64_t>(hi) << 32)));
+}
+
+// v with its sign flipped where bit 31 of sg is set
+__device__ __forceinline__ double with_sign(double v, uint32_t sg) {
+  const uint64_t b = static_cast<uint64_t>(__double_as_longlong(v));
+  return u2d(static_cast<uint32_t>(b), static_cast<uint32_t>(b >> 32) ^ sg);
+}
+
+// auxiliary bits of a buffer load: volatile (the compiler does not move it)
+constexpr int kVolatile = static_cast<int>(0x80000000u);
+
+// ---------------------------------------------------------------------------
+// rowacc = Haa C + C Hbb^T
+// ---------------------------------------------------------------------------
+// Both products accumulate in the same registers: P[ia][k] Q[k][ib] over
+// k < lena with P = Haa, Q = C, then over k < lenb with P = C, Q = Hbb.  A
+// wave owns 16 RA x 16 RB complex outputs, a workgroup of 4 waves (2 x 2)
+// the neighbouring ones.
+//
+// No LDS: every operand is loaded in the layout of v_mfma_f64_16x16x4f64
+// (A: row l%16, k l/16; B: k l/16, column l%16) straight from memory, D k
+// steps ahead in a register ring.  Haa, Hbb (stored by source string) and C
+// as Q are runs of 16 consecutive elements per k; C as P is 64 bytes of 16
+// rows, the other half of the cache line serving the next k step.  An MFMA
+// takes 64 clocks, so a k step of 2 x 2 tiles (8 MFMAs, 512 clocks) needs 3 KB
+// per wave, 24 bytes per clock and CU of the L1's 64 (2 x 4 tiles: 20), and
+// the waves need no barrier and no staging work.  norb 14 7a7b (3.2e11
+// flops): 4.7 ms, 69 TFLOP/s of the 78 that the instruction reaches, with 2 x 4
+// tiles; 5.7 ms with 2 x 2; 5.7 ms with both operands staged through
+// double-buffered LDS tiles of 64 x 64 (6.6 ms with 128 x 64).
+//
+// k past lena or lenb is out of range, hence zero, for H (and masked for C);
+// columns past a row read what follows into outputs that are not stored.
+constexpr int kSpinDepth = 4;              // k steps in flight
+
+__device__ __forceinline__ double load_d(__amdgpu_buffer_rsrc_t r, int off) {
+  const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
+  return u2d(v[0], v[1]);
+}
+
+template <bool CPLX, int RA, int RB>
+__global__ void __launch_bounds__(256, RA * RB > 4 || CPLX ? 2 : 4)
+k_same_spin_f64(int64_t lena, int64_t lenb, const double* __restrict__ ha,
+                const double* __restrict__ hb, const double* __restrict__ coeff,
+                double* __restrict__ out, const int32_t* __restrict__ done,
+                int ta, int tb) {
+  constexpr int D = kSpinDepth;
+  constexpr int kH = CPLX ? 16 : 8;               // bytes per H element
+  if (done && *done) return;
+  const int t = static_cast<int>(xcd_order(blockIdx.x, ta * tb));
+  // groups of 8 tile rows, so neighbouring workgroups share C and H rows
+  const int grp = t / (8 * tb);
+  const int left = ta - grp * 8;
+  const int rows = left < 8 ? left : 8;
+  const int w = t - grp * 8 * tb;
+  const int wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int kq = lane >> 4;
+  const int cl = lane & 15;
+  const int a0 = ((grp * 8 + w % rows) * 2 + (wave >> 1)) * 16 * RA;
+  const int b0 = ((w / rows) * 2 + (wave & 1)) * 16 * RB;
+  const int la = static_cast<int>(lena), lb = static_cast<int>(lenb);
+  if (a0 >= la || b0 >= lb) return;
+  const __amdgpu_buffer_rsrc_t rc = buffer_of(coeff, lena * lenb * 16);
+  const __amdgpu_buffer_rsrc_t rha = buffer_of(ha, lena * lena * kH);
+  const __amdgpu_buffer_rsrc_t rhb = buffer_of(hb, lenb * lenb * kH);
+
+  double4_t are[RA][RB], aim[RA][RB];
+#pragma unroll
+  for (int i = 0; i < RA; ++i)
+#pragma unroll
+    for (int j = 0; j < RB; ++j) {
+      are[i][j] = double4_t{0, 0, 0, 0};
+      aim[i][j] = double4_t{0, 0, 0, 0};
+    }
+  // an operand value of a k step: real and imaginary part (H: real only
+  // unless CPLX)
+  auto load_h = [&](__amdgpu_buffer_rsrc_t r, int off, double& re, double& im) {
+    if constexpr (CPLX) {
+      const double2 v = bload_d2(r, off);
+      re = v.x;
+      im = v.y;
+    } else {
+      re = load_d(r, off);
+    }
+  };
+  {
+    double pr[D][RA], pi[D][RA];
+    double2 q[D][RB];
+    auto load = [&](int s, int d) {
+      const int k = 4 * s + kq;
+#pragma unroll
+      for (int i = 0; i < RA; ++i)
+        load_h(rha, (k * la + a0 + 16 * i + cl) * kH, pr[d][i], pi[d][i]);
+#pragma unroll
+      for (int j = 0; j < RB; ++j)
+        q[d][j] = bload_d2(rc, (k * lb + b0 + 16 * j + cl) * 16);
+    };
+#pragma unroll
+    for (int d = 0; d < D; ++d) load(d, d);
+    const int ns = (la + 3) / 4;
+    for (int s0 = 0; s0 < ns; s0 += D) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+#pragma unroll
+        for (int i = 0; i < RA; ++i)
+#pragma unroll
+          for (int j = 0; j < RB; ++j) {
+            are[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(pr[d][i], q[d][j].x, are[i][j], 0, 0, 0);
+            aim[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(pr[d][i], q[d][j].y, aim[i][j], 0, 0, 0);
+            if constexpr (CPLX) {
+              are[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(-pi[d][i], q[d][j].y, are[i][j], 0, 0, 0);
+              aim[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(pi[d][i], q[d][j].x, aim[i][j], 0, 0, 0);
+            }
+          }
+        load(s0 + d + D, d);
+      }
+    }
+  }
+  {
+    double2 p[D][RA];
+    double qr[D][RB], qi[D][RB];
+    auto load = [&](int s, int d) {
+      const int k = 4 * s + kq;
+#pragma unroll
+      for (int i = 0; i < RA; ++i)
+        p[d][i] = bload_d2(rc, k < lb ? ((a0 + 16 * i + cl) * lb + k) * 16 : -1);
+#pragma unroll
+      for (int j = 0; j < RB; ++j)
+        load_h(rhb, (k * lb + b0 + 16 * j + cl) * kH, qr[d][j], qi[d][j]);
+    };
+#pragma unroll
+    for (int d = 0; d < D; ++d) load(d, d);
+    const int ns = (lb + 3) / 4;
+    for (int s0 = 0; s0 < ns; s0 += D) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+#pragma unroll
+        for (int i = 0; i < RA; ++i)
+#pragma unroll
+          for (int j = 0; j < RB; ++j) {
+            are[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(p[d][i].x, qr[d][j], are[i][j], 0, 0, 0);
+            aim[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(p[d][i].y, qr[d][j], aim[i][j], 0, 0, 0);
+            if constexpr (CPLX) {
+              are[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(-p[d][i].y, qi[d][j], are[i][j], 0, 0, 0);
+              aim[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(p[d][i].x, qi[d][j], aim[i][j], 0, 0, 0);
+            }
+          }
+        load(s0 + d + D, d);
+      }
+    }
+  }
+  // item e of lane l: row l/16 + 4 e, column l%16
+#pragma unroll
+  for (int i = 0; i < RA; ++i)
+#pragma unroll
+    for (int j = 0; j < RB; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int a = a0 + 16 * i + kq + 4 * e;
+        const int b = b0 + 16 * j + cl;
+        if (a < la && b < lb)
+          *reinterpret_cast<double2*>(out + (static_cast<int64_t>(a) * lb + b) * 2) =
+              make_double2(are[i][j][e], aim[i][j][e]);
+      }
+}
+
+template <bool CPLX, int RA, int RB>
+void same_spin(int64_t lena, int64_t lenb, const double* ha, const double* hb,
+               const double* coeff, double* out, hipStream_t st,
+               const int32_t* done) {
+  const int ta = static_cast<int>((lena + 32 * RA - 1) / (32 * RA));
+  const int tb = static_cast<int>((lenb + 32 * RB - 1) / (32 * RB));
+  k_same_spin_f64<CPLX, RA, RB><<<static_cast<unsigned>(ta * tb), 256, 0, st>>>(
+      lena, lenb, ha, hb, coeff, out, done, ta, tb);
+}
+
+// ---------------------------------------------------------------------------
+// Opposite-spin rows
+// ---------------------------------------------------------------------------
+constexpr int kPullMaxK = 64;              // live alpha pairs + folded row
+constexpr int kPullTiles = 7;              // 16-row W tiles per pass
+constexpr int kPullDepth = 4;              // k steps of B in flight
+constexpr int kPullRows = kPullMaxK + 4 * kPullDepth;   // lrow entries
+constexpr uint32_t kPullNoRow = 0x80000000u;   // past the end of C
+
+struct PullArgs {
+  int norb, compressed, nele, nq;          // nq: pairs of one spin
+  int64_t lena, lenb;
+  int ks, pass, copies;                    // k steps, passes, accumulator rows
+  const double* w;                         // [p][q] (complex: interleaved)
+  const int32_t* dexc;                     // [lena][nexc][3]
+  const uint32_t* fwd;                     // [nq][lenb] (fqehip_pull_table)
+  const double* coeff;
+  double* rowacc;
+  // out != NULL: out = alpha (rowacc + row) + beta cin, acc += that value;
+  // else rowacc += row
+  double alpha_re, alpha_im, beta_re, beta_im;
+  const double* cin;
+  double* out;
+  double* acc;
+  const int32_t* done;
+};
+
+size_t pull_lds_bytes(bool cplx, int ks, int64_t lenb, int tiles, int copies) {
+  return static_cast<size_t>(copies) * lenb * 16 +
+         static_cast<size_t>(tiles) * ks * 64 * 8 * (cplx ? 2 : 1) +
+         kPullMaxK * (8 + 4 + 4) + kPullRows * 4 + 8 * 4;
+}
+
+// One alpha string ia per workgroup; G 16-row tiles of W per pass.
+//
+// Set-up: the live alpha pairs of ia are its de-excitation rows to another
+// string (noff = nele (norb - nele) of them: source row of C, pair, sign),
+// plus one folded row, C[ia] itself, whose coefficient is the sum over the
+// occupied orbitals' diagonal pairs.  W restricted to them, with the signs,
+// goes to LDS in MFMA A-operand order ([k step][tile][lane]).
+//
+// Then each wave takes 16-column tiles of the row in turn: the B operand of
+// lane l (k = 4 s + l/16, column l%16) is the 16-byte value C[src_k][col], so
+// the loads are the operand, kPullDepth steps ahead in a ring; each k step
+// feeds G x (re, im) independent MFMAs; and the G x 16 values Z[q][col] are
+// added, with the sign of E^b_q, to the accumulator row at their target
+// column (ds_add_f64, about 10 clocks per wave instruction).
+//
+// Order of the additions: `copies` accumulator rows, wave w adding to row
+// w % copies.  The waves that share one add in turn, tile after tile (`turn`,
+// a counter per row in LDS: the tile whose turn it is), so every accumulator
+// sees the same sequence of additions on every run, and the rows are summed
+// in order at the end.  A wave waits only for waves with earlier tiles, and
+// those for none after them, so every wait ends.
+//
+// norb 14 7a7b: 5.4 ms (2.7e11 flops with the padding, 50 TFLOP/s of 78), against
+// 7.6 + 1.6 ms of the slot-row kernel and its reduction; 4.8 ms without the
+// additions, 5.1 without their order.  norb 12 6a6b: 0.24 against 0.47 + 0.09;
+// complex operator, norb 11 4a6b: 0.14 against 1.23 for the unfused kernels.
+template <bool CPLX, int G>
+__global__ void __launch_bounds__(512, 2) k_pull_rows_f64(PullArgs p) {
+  constexpr int kF = CPLX ? 128 : 64;      // doubles per W fragment
+  extern __shared__ __align__(16) char smem[];
+  if (p.done && *p.done) return;
+  const int tid = threadIdx.x;
+  const int nt = blockDim.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nwave = nt >> 6;
+  const int lane = tid & 63;
+  const int kq = lane >> 4;
+  const int cl = lane & 15;
+  const int lenb = static_cast<int>(p.lenb);
+  const int ks = p.ks;
+  const int64_t ia = xcd_order(blockIdx.x, p.lena);
+  double2* accs = reinterpret_cast<double2*>(smem);    // [copies][lenb]
+  double* wf = reinterpret_cast<double*>(accs + p.copies * lenb);   // [ks][G][kF]
+  double* lsg = wf + G * ks * kF;
+  uint32_t* lrow = reinterpret_cast<uint32_t*>(lsg + kPullMaxK);
+  int32_t* lp = reinterpret_cast<int32_t*>(lrow + kPullRows);
+  int32_t* ldiag = lp + kPullMaxK;
+  int32_t* turns = ldiag + kPullMaxK;              // [8]
+  const int noff = p.nele * (p.norb - p.nele);
+  const int mine = wave % p.copies;
+  // the table's offsets are those of element target + 1
+  char* accum = reinterpret_cast<char*>(accs + mine * lenb) - 16;
+  int32_t* turn = turns + mine;
+
+  for (int x = tid; x < p.copies * lenb; x += nt) accs[x] = make_double2(0.0, 0.0);
+  if (wave == 0) {
+    const int nexc = p.nele * (p.norb - p.nele + 1);
+    int32_t src = -1, ij = 0, sg = 0;
+    if (lane < nexc) {
+      const int32_t* e = p.dexc + (ia * nexc + lane) * 3;
+      src = e[0];
+      ij = e[1];
+      sg = e[2];
+    }
+    const bool diag = lane < nexc && src == ia;
+    const bool off = lane < nexc && src != ia;
+    const uint64_t mo = __ballot(off), md = __ballot(diag);
+    const uint64_t below = (1ull << lane) - 1ull;
+    const int i = ij / p.norb, j = ij % p.norb;
+    const int pair = p.compressed ? comp_pair(i, j) : ij;
+    if (off) {
+      const int pos = __popcll(mo & below);
+      lrow[pos] = static_cast<uint32_t>(src) * static_cast<uint32_t>(lenb) * 16u;
+      lp[pos] = pair;
+      lsg[pos] = static_cast<double>(sg);
+    }
+    if (diag) ldiag[__popcll(md & below)] = pair;
+    if (lane >= noff)
+      lrow[lane] = lane == noff
+                       ? static_cast<uint32_t>(ia) * static_cast<uint32_t>(lenb) * 16u
+                       : kPullNoRow;
+    if (lane < kPullRows - kPullMaxK) lrow[kPullMaxK + lane] = kPullNoRow;
+  }
+  __syncthreads();
+
+  const __amdgpu_buffer_rsrc_t rc = buffer_of(p.coeff, p.lena * p.lenb * 16);
+  const __amdgpu_buffer_rsrc_t rf = buffer_of(p.fwd, static_cast<int64_t>(p.nq) * lenb * 4);
+  const __amdgpu_buffer_rsrc_t rw =
+      buffer_of(p.w, static_cast<int64_t>(p.nq) * p.nq * (CPLX ? 16 : 8));
+  const int ntile = (lenb + 15) >> 4;
+
+  for (int ps = 0; ps < p.pass; ++ps) {
+    const int q0 = 16 * G * ps;
+    // elements of rows past the live ones, of pairs past the last and of the
+    // folded row (next loop) are out of range and read zero
+#pragma unroll 4
+    for (int f = wave; f < G * ks; f += nwave) {
+      const int q = q0 + 16 * (f % G) + cl;
+      const int k = 4 * (f / G) + kq;
+      const int off = k < noff && q < p.nq ? (lp[k] * p.nq + q) * (CPLX ? 16 : 8) : -1;
+      const double sg = k < noff ? lsg[k] : 0.0;
+      if (CPLX) {
+        const double2 v = bload_d2(rw, off);
+        wf[f * kF + lane] = sg * v.x;
+        wf[f * kF + 64 + lane] = sg * v.y;
+      } else {
+        wf[f * kF + lane] = sg * load_d(rw, off);
+      }
+    }
+    __syncthreads();
+    for (int t = wave; t < G; t += nwave) {
+      const int q = q0 + 16 * t + cl;
+      double vr = 0.0, vi = 0.0;
+      for (int d = kq; d < p.nele; d += 4) {
+        const int off = q < p.nq ? (ldiag[d] * p.nq + q) * (CPLX ? 16 : 8) : -1;
+        if (CPLX) {
+          const double2 v = bload_d2(rw, off);
+          vr += v.x;
+          vi += v.y;
+        } else {
+          vr += load_d(rw, off);
+        }
+      }
+      vr += __shfl_xor(vr, 16);
+      vr += __shfl_xor(vr, 32);
+      double* fold = wf + ((noff >> 2) * G + t) * kF + 16 * (noff & 3) + cl;
+      if (kq == 0) fold[0] = vr;
+      if (CPLX) {
+        vi += __shfl_xor(vi, 16);
+        vi += __shfl_xor(vi, 32);
+        if (kq == 0) fold[64] = vi;
+      }
+    }
+    if (tid < p.copies) turns[tid] = tid;
+    __syncthreads();
+
+    u32x4 ring[kPullDepth];
+    // k step s of a tile; rows past the live ones and columns past the row
+    // are out of range and read zero
+    auto load_b = [&](int s, uint32_t o) {
+      const uint32_t r = lrow[4 * s + kq];
+      return __builtin_amdgcn_raw_buffer_load_b128(
+          rc, static_cast<int>(r | o) < 0 ? -1 : static_cast<int>(r + o), 0, 0);
+    };
+    auto column = [&](int tile) {
+      const int jb = tile * 16 + cl;
+      return jb < lenb ? static_cast<uint32_t>(jb) * 16u : kPullNoRow;
+    };
+    if (wave < ntile) {
+#pragma unroll
+      for (int j = 0; j < kPullDepth; ++j) ring[j] = load_b(j, column(wave));
+    }
+    for (int tile = wave; tile < ntile; tile += nwave) {
+      const int jb = tile * 16 + cl;
+      const uint32_t o = column(tile);
+      // target words, volatile so that the loads stay ahead of the products
+      uint32_t fv[G][4];
+#pragma unroll
+      for (int t = 0; t < G; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int q = q0 + 16 * t + kq + 4 * e;
+          fv[t][e] = __builtin_amdgcn_raw_buffer_load_b32(
+              rf, (q < p.nq && jb < lenb) ? (q * lenb + jb) * 4 : -1, 0, kVolatile);
+        }
+      double4_t zr[G], zi[G];
+#pragma unroll
+      for (int t = 0; t < G; ++t) {
+        zr[t] = double4_t{0, 0, 0, 0};
+        zi[t] = double4_t{0, 0, 0, 0};
+      }
+      // A of step s + 1 is read while step s multiplies
+      double ar[2][G], ai[2][G];
+      auto load_a = [&](int s, double (&r)[G], double (&im)[G]) {
+        const double* f = wf + (s < ks ? s : 0) * (G * kF) + lane;
+#pragma unroll
+        for (int t = 0; t < G; ++t) {
+          r[t] = f[t * kF];
+          if (CPLX) im[t] = f[t * kF + 64];
+        }
+      };
+      auto step = [&](u32x4 bv, const double (&r)[G], const double (&im)[G]) {
+        const double br = u2d(bv[0], bv[1]);
+        const double bi = u2d(bv[2], bv[3]);
+#pragma unroll
+        for (int t = 0; t < G; ++t) {
+          zr[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(r[t], br, zr[t], 0, 0, 0);
+          zi[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(r[t], bi, zi[t], 0, 0, 0);
+        }
+        if (CPLX) {
+#pragma unroll
+          for (int t = 0; t < G; ++t) {
+            zr[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(-im[t], bi, zr[t], 0, 0, 0);
+            zi[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(im[t], br, zi[t], 0, 0, 0);
+          }
+        }
+      };
+      load_a(0, ar[0], ai[0]);
+      int s0 = 0;
+      for (; s0 + kPullDepth <= ks; s0 += kPullDepth) {
+#pragma unroll
+        for (int j = 0; j < kPullDepth; ++j) {
+          load_a(s0 + j + 1, ar[(j + 1) & 1], ai[(j + 1) & 1]);
+          step(ring[j], ar[j & 1], ai[j & 1]);
+          ring[j] = load_b(s0 + j + kPullDepth, o);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < kPullDepth - 1; ++j)
+        if (s0 + j < ks) {
+          load_a(s0 + j + 1, ar[(j + 1) & 1], ai[(j + 1) & 1]);
+          step(ring[j], ar[j & 1], ai[j & 1]);
+        }
+      // the next tile's first steps are in flight during the additions
+      if (tile + nwave < ntile) {
+#pragma unroll
+        for (int j = 0; j < kPullDepth; ++j) ring[j] = load_b(j, column(tile + nwave));
+      }
+      // the rows' adders ahead of the waves that multiply
+      __builtin_amdgcn_s_setprio(2);
+      if (p.copies < nwave)
+        while (__builtin_amdgcn_readfirstlane(__hip_atomic_load(
+                   turn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) != tile)
+          __builtin_amdgcn_s_sleep(1);
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int t = 0; t < G; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t f = fv[t][e];
+          if (f) {
+            double* to = reinterpret_cast<double*>(accum + (f << 1));
+            const uint32_t sg = f & 0x80000000u;
+            __hip_atomic_fetch_add(to, with_sign(zr[t][e], sg), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+            __hip_atomic_fetch_add(to + 1, with_sign(zi[t][e], sg), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+          }
+        }
+      if (p.copies < nwave) {
+        // this tile's additions are done before the next one's begin
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (lane == 0)
+          __hip_atomic_store(turn, tile + p.copies, __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
+      __builtin_amdgcn_s_setprio(0);
+    }
+    __syncthreads();
+  }
+  double2* racc = reinterpret_cast<double2*>(p.rowacc) + ia * p.lenb;
+  for (int x = tid; x < lenb; x += nt) {
+    const double2 r = racc[x];
+    double re = r.x, im = r.y;
+    for (int c = 0; c < p.copies; ++c) {
+      const double2 v = accs[c * lenb + x];
+      re += v.x;
+      im += v.y;
+    }
+    if (!p.out) {
+      racc[x] = make_double2(re, im);
+      continue;
+    }
+    const int64_t idx = ia * p.lenb + x;
+    double vr = p.alpha_re * re - p.alpha_im * im;
+    double vi = p.alpha_re * im + p.alpha_im * re;
+    if (p.beta_re != 0.0 || p.beta_im != 0.0) {
+      const double2 c = reinterpret_cast<const double2*>(p.cin)[idx];
+      vr += p.beta_re * c.x - p.beta_im * c.y;
+      vi += p.beta_re * c.y + p.beta_im * c.x;
+    }
+    reinterpret_cast<double2*>(p.out)[idx] = make_double2(vr, vi);
+    if (p.acc) {
+      p.acc[2 * idx] += vr;
+      p.acc[2 * idx + 1] += vi;
+    }
+  }
+}
+
+// Target words of the row kernel from a forward table: 8 (target + 1), bit 31
+// the sign; 0 where the excitation vanishes.  (word << 1) is the byte offset
+// of accumulator target + 1.
+__global__ void __launch_bounds__(256)
+k_pull_table(int64_t n, const int32_t* __restrict__ fwd, uint32_t* __restrict__ tab) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= n) return;
+  const int32_t f = fwd[i];
+  tab[i] = static_cast<uint32_t>(iabs(f)) << 3 | (f < 0 ? 0x80000000u : 0u);
+}
+
+// How a sector runs: W tiles per pass, waves, accumulator rows.
+struct PullPlan {
+  int ks, tiles, pass, copies, threads;
+  size_t lds;
+};
+
+// False if not even one W tile fits beside one accumulator row.
+bool pull_plan(bool cplx, int noff, int64_t lenb, int nq, PullPlan* pl) {
+  const int ks = (noff + 1 + 3) / 4;
+  const int nqt = (nq + 15) / 16;
+  int g = nqt < kPullTiles ? nqt : kPullTiles;
+  while (g > 0 && pull_lds_bytes(cplx, ks, lenb, g, 1) > kLdsLimit) --g;
+  if (g <= 0) return false;
+  pl->ks = ks;
+  pl->pass = (nqt + g - 1) / g;
+  pl->tiles = (nqt + pl->pass - 1) / pl->pass;
+  // two 4-wave workgroups per CU while their LDS fits, else one of 8 waves;
+  // as many accumulator rows as the rest of that LDS holds
+  const bool two = pull_lds_bytes(cplx, ks, lenb, pl->tiles, 1) <= kLdsLimit / 2;
+  const size_t limit = two ? kLdsLimit / 2 : kLdsLimit;
+  pl->threads = two ? 256 : 512;
+  pl->copies = 1;
+  while (2 * pl->copies * 64 <= pl->threads &&
+         pull_lds_bytes(cplx, ks, lenb, pl->tiles, 2 * pl->copies) <= limit)
+    pl->copies *= 2;
+  pl->lds = pull_lds_bytes(cplx, ks, lenb, pl->tiles, pl->copies);
+  return true;
+}
+
+template <bool CPLX>
+int launch_rows(const PullPlan& pl, const PullArgs& p, hipStream_t st) {
+  const unsigned grid = static_cast<unsigned>(p.lena);
+  switch (pl.tiles) {
+#define FQEHIP_PULL_CASE(N)                                            \
+  case N:                                                              \
+    k_pull_rows_f64<CPLX, N><<<grid, pl.threads, pl.lds, st>>>(p);     \
+    break;
+    FQEHIP_PULL_CASE(1)
+    FQEHIP_PULL_CASE(2)
+    FQEHIP_PULL_CASE(3)
+    FQEHIP_PULL_CASE(4)
+    FQEHIP_PULL_CASE(5)
+    FQEHIP_PULL_CASE(6)
+    FQEHIP_PULL_CASE(7)
+#undef FQEHIP_PULL_CASE
+    default:
+      set_error("k_pull_rows_f64: %d tiles", pl.tiles);
+      return FQEHIP_ERR_INVALID;
+  }
+  FQEHIP_CHECK_LAUNCH("k_pull_rows_f64");
+  return FQEHIP_OK;
+}
+
+}  // namespace
+
+// The limits are those of a complex operator (the narrower ones), so that
+// the answer is the sector's alone.
+bool pull_supported(const fqehip_sector* s) {
+  if (!s->pull_w || !s->haa || !s->hbb || !s->dexc_a || !s->pull_fwd) return false;
+  const int noff = s->nalpha * (s->norb - s->nalpha);
+  PullPlan pl;
+  return s->npull > 0 && s->lena > 0 && s->lenb > 0 &&
+         s->nalpha * (s->norb - s->nalpha + 1) <= 64 && noff < kPullMaxK &&
+         s->lena * s->lenb * 16 < kOffLimit && s->lena * s->lena * 16 < kOffLimit &&
+         s->lenb * s->lenb * 16 < kOffLimit &&
+         static_cast<int64_t>(s->npull) * s->lenb * 4 < kOffLimit &&
+         pull_plan(true, noff, s->lenb, s->npull, &pl);
+}
+
+// rowacc = Haa C + C Hbb^T (complex128, 16 lena lenb bytes).
+int launch_same_spin(const fqehip_sector* s, int complex_op,
+                     const double* coeff, double* rowacc, hipStream_t st,
+                     const int32_t* done) {
+  // tiles of 64 x 128 (64 x 64 complex operators) once they give every CU two
+  // workgroups; 32 x 64 from half a workgroup per CU on (norb 12 6a6b, 435 of
+  // them: 0.126 ms, 0.149 with 64 x 64, 0.164 with 32 x 32); else 32 x 32
+  const int64_t l = s->lena, m = s->lenb;
+  const bool large = (l + 63) / 64 * ((m + (complex_op ? 63 : 127)) / (complex_op ? 64 : 128)) >= 512;
+  const bool mid = !large && (l + 63) / 64 * ((m + 63) / 64) >= 100;
+  if (complex_op) {
+    if (large) same_spin<true, 2, 2>(l, m, s->haa, s->hbb, coeff, rowacc, st, done);
+    else if (mid) same_spin<true, 1, 2>(l, m, s->haa, s->hbb, coeff, rowacc, st, done);
+    else same_spin<true, 1, 1>(l, m, s->haa, s->hbb, coeff, rowacc, st, done);
+  } else {
+    if (large) same_spin<false, 2, 4>(l, m, s->haa, s->hbb, coeff, rowacc, st, done);
+    else if (mid) same_spin<false, 1, 2>(l, m, s->haa, s->hbb, coeff, rowacc, st, done);
+    else same_spin<false, 1, 1>(l, m, s->haa, s->hbb, coeff, rowacc, st, done);
+  }
+  FQEHIP_CHECK_LAUNCH("k_same_spin_f64");
+  return FQEHIP_OK;
+}
+
+// The opposite-spin rows on top of rowacc; with out set also the epilogue
+// out = alpha (H C) + beta cin, acc += out (out must not alias coeff: other
+// workgroups still read it).
+int launch_pull_rows(const fqehip_sector* s, int complex_op,
+                     const double* coeff, double* rowacc, double ar, double ai,
+                     double br, double bi, const double* cin, double* out,
+                     double* acc, hipStream_t st, const int32_t* done) {
+  PullPlan pl;
+  if (!pull_plan(complex_op != 0, s->nalpha * (s->norb - s->nalpha), s->lenb,
+                 s->npull, &pl)) {
+    set_error("k_pull_rows_f64: lenb=%lld does not fit in LDS",
+              static_cast<long long>(s->lenb));
+    return FQEHIP_ERR_INVALID;
+  }
+  PullArgs p{};
+  p.norb = s->norb;
+  p.compressed = s->npull == s->norb * (s->norb + 1) / 2 ? 1 : 0;
+  p.nele = s->nalpha;
+  p.nq = s->npull;
+  p.lena = s->lena;
+  p.lenb = s->lenb;
+  p.ks = pl.ks;
+  p.pass = pl.pass;
+  p.copies = pl.copies;
+  p.w = s->pull_w;
+  p.dexc = s->dexc_a;
+  p.fwd = s->pull_fwd;
+  p.coeff = coeff;
+  p.rowacc = rowacc;
+  p.alpha_re = ar;
+  p.alpha_im = ai;
+  p.beta_re = br;
+  p.beta_im = bi;
+  p.cin = cin;
+  p.out = out;
+  p.acc = acc;
+  p.done = done;
+  return complex_op ? launch_rows<true>(pl, p, st) : launch_rows<false>(pl, p, st);
+}
+
+}  // namespace fqehip
+
+using namespace fqehip;
+
+extern "C" int fqehip_pull_table(int npair, int64_t len, const int32_t* d_fwd,
+                                 uint32_t* d_tab, void* stream) {
+  clear_error();
+  FQEHIP_CHECK_ARG(npair >= 0 && len >= 0 && len < (1 << 27), "npair=%d len=%lld",
+                   npair, static_cast<long long>(len));
+  const int64_t n = npair * len;
+  if (n == 0) return FQEHIP_OK;
+  FQEHIP_CHECK_ARG(d_fwd && d_tab, "NULL pointer");
+  k_pull_table<<<blocks_for(n, 256), 256, 0, as_stream(stream)>>>(n, d_fwd, d_tab);
+  FQEHIP_CHECK_LAUNCH("k_pull_table");
+  return FQEHIP_OK;
+}

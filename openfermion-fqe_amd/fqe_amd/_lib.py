@@ -42,7 +42,9 @@ class Sector(ctypes.Structure):
                 ("fwd_a", c_void_p), ("fwd_b", c_void_p),
                 ("slot_a", c_void_p), ("nslot", c_int),
                 ("hbb_hi", c_void_p), ("hbb_lo", c_void_p), ("ldh", c_int64),
-                ("tile", c_int), ("hbb_f64", c_void_p), ("hbb_oz", c_void_p)]
+                ("tile", c_int), ("hbb_f64", c_void_p), ("hbb_oz", c_void_p),
+                ("dexc_a", c_void_p), ("pull_w", c_void_p), ("haa", c_void_p),
+                ("hbb", c_void_p), ("pull_fwd", c_void_p), ("npull", c_int)]
 
 
 class Operator(ctypes.Structure):
@@ -98,6 +100,12 @@ _SIGNATURES = {
                                          c_void_p]),
     "fqehip_apply_workspace_bytes": (c_int64, [c_int, POINTER(Sector)]),
     "fqehip_beta_block_ld": (c_int64, [c_int64]),
+    "fqehip_spin_block": (c_int, [c_int, c_int, c_int64, c_void_p, c_void_p,
+                                  c_int64, c_void_p, c_void_p, c_void_p]),
+    "fqehip_pull_table": (c_int, [c_int, c_int64, c_void_p, c_void_p,
+                                  c_void_p]),
+    "fqehip_pull_supported": (c_int, [c_int, POINTER(Sector),
+                                      POINTER(Operator)]),
     "fqehip_batch_create": (c_int, [c_int, c_int, POINTER(BatchItem), c_double,
                                     c_int, c_int, c_int, c_void_p,
                                     POINTER(c_void_p)]),

@@ -43,6 +43,10 @@ class PreparedOperator:
                       norb * (norb + 1) // 2 if compressed else norb * norb)
         # A[p][q] == A[q][p] exactly (p, q < npair): the split apply applies
         self.pair_symmetric = False
+        # opposite-spin coupling W[p][q] = V[p][q] + V[q][p] (device, alpha
+        # pair p, beta pair q) of a two-body operator: the pull form
+        self.coupling: Optional[torch.Tensor] = None
+        self._pull = {}
         self._hbb = {}
         self._hoz = {}
 
@@ -88,6 +92,52 @@ class PreparedOperator:
                       _lib.ptr(hoz), _lib.stream_ptr())
             self._hoz[key] = hoz
         return self._hoz[key]
+
+    def _spin_block(self, tables, alpha: bool) -> torch.Tensor:
+        """Matrix of this two-body operator on the strings of one spin, by
+        source string (fqehip_spin_block)."""
+        n, npull = tables.length, self.coupling.shape[0]
+        w = 2 if self.complex_op else 1
+        lda = self.a.shape[1]
+        # spin-orbital operators: the beta block of A follows the alpha one
+        first = w * npull if self.spin and not alpha else 0
+        fwd, _ = tables.fused_tables(self.compressed)
+        out = torch.empty((n, n), device=self.a.device,
+                          dtype=torch.complex128 if self.complex_op else
+                          torch.float64)
+        _lib.call("fqehip_spin_block", int(self.complex_op), npull, n,
+                  _lib.ptr(fwd), _lib.ptr(self.a[first:, first:]), lda,
+                  _lib.ptr(self.a[w * self.npair:, first:]), _lib.ptr(out),
+                  _lib.stream_ptr())
+        return out
+
+    def pull_tables(self, graph):
+        """(W, Haa, Hbb, beta target words, alpha de-excitation rows) of
+        the pull form on the sector of ``graph``, cached per (nalpha, nbeta,
+        device); None where the form does not apply (one-body operators,
+        sectors past its limits)."""
+        na, nb, norb = graph.nalpha(), graph.nbeta(), graph.norb()
+        if (self.coupling is None or na * (norb - na + 1) > 64
+                or norb == 0):
+            return None
+        width = 16 if self.complex_op else 8
+        if ((max(graph.lena(), graph.lenb()) + self.coupling.shape[0]) * width
+                > 160 * 1024):
+            return None
+        key = (na, nb, self.a.device.index)
+        if key not in self._pull:
+            ta, tb = graph.tables(True), graph.tables(False)
+            blocks = []
+            for nele, tab, alpha in ((na, ta, True), (nb, tb, False)):
+                # restricted operators: one matrix per electron count
+                side = ("side", alpha if self.spin else None, nele,
+                        self.a.device.index)
+                if side not in self._pull:
+                    self._pull[side] = self._spin_block(tab, alpha)
+                blocks.append(self._pull[side])
+            self._pull[key] = (self.coupling, blocks[0], blocks[1],
+                               tb.pull_table(self.compressed), ta.dexc)
+        return self._pull[key]
 
     def c_struct(self) -> _lib.Operator:
         return _lib.Operator(int(self.complex_op), _lib.ptr(self.a),
@@ -142,13 +192,28 @@ def prepare_operator(tensors: Sequence[numpy.ndarray], norb: int,
     h1row = h1p.reshape(-1)[rows]
     full = numpy.vstack([vm, h1row[None, :]])  # (npair+1) x npair, complex
     a = _real_block_form(full, complex_op)
-    dev_a = torch.from_numpy(numpy.ascontiguousarray(a, dtype=numpy.float64)
-                             ).to(device)
+    dev_a, coupling = _upload(a, vm + vm.T, complex_op, device)
     prepared = PreparedOperator(norb, compressed, complex_op, dev_a, None)
+    prepared.coupling = coupling
     if not complex_op:
         sq = a[:-1, :]
         prepared.pair_symmetric = bool(numpy.array_equal(sq, sq.T))
     return prepared
+
+
+def _upload(a: numpy.ndarray, w: numpy.ndarray, complex_op: bool,
+            device: torch.device) -> Tuple[torch.Tensor, torch.Tensor]:
+    """The GEMM matrix and the coupling (real unless complex_op) on the
+    device, in one transfer."""
+    dtype = numpy.complex128 if complex_op else numpy.float64
+    w = numpy.ascontiguousarray(w if complex_op else w.real, dtype=dtype)
+    flat = numpy.concatenate([numpy.asarray(a, dtype=numpy.float64).ravel(),
+                              w.view(numpy.float64).ravel()])
+    dev = torch.from_numpy(flat).to(device)
+    dev_w = dev[a.size:]
+    if complex_op:
+        dev_w = torch.view_as_complex(dev_w.reshape(-1, 2))
+    return dev[:a.size].reshape(a.shape), dev_w.reshape(w.shape)
 
 
 def _real_block_form(full: numpy.ndarray, complex_op: bool) -> numpy.ndarray:
@@ -217,10 +282,13 @@ def prepare_spin_operator(tensors: Sequence[numpy.ndarray], norb: int,
                                h1p[n:, n:].reshape(-1)])
     full = numpy.vstack([vm, h1row[None, :]])
     complex_op = bool(numpy.any(full.imag))
-    a = _real_block_form(full, complex_op)
-    dev_a = torch.from_numpy(numpy.ascontiguousarray(a, dtype=numpy.float64)
-                             ).to(device)
-    return PreparedOperator(norb, False, complex_op, dev_a, None, spin=True)
+    w = vm[:npair, npair:] + vm[npair:, :npair].T
+    dev_a, coupling = _upload(_real_block_form(full, complex_op), w,
+                              complex_op, device)
+    prepared = PreparedOperator(norb, False, complex_op, dev_a, None,
+                                spin=True)
+    prepared.coupling = coupling
+    return prepared
 
 
 def precision_of(dtype: torch.dtype) -> int:
@@ -238,7 +306,9 @@ def sector_struct(graph, op: PreparedOperator,
     element keeps the tables referenced.  For a pair-symmetric operator the
     beta-beta block is attached (split apply): its bfloat16 hi/lo split for
     complex64 (``settings.split``), its FP64 columns for complex128
-    (``settings.split_fp64``)."""
+    (``settings.split_fp64``).  Two-body operators in complex128 get the
+    tables of the pull form, unless the digit engine or another kernel is
+    asked for (``settings.contraction``, ``split_tile_fp64``)."""
     if op.spin:
         ta = graph.tables(True).spin_pair_table(True)
         tb = graph.tables(False).spin_pair_table(False)
@@ -259,10 +329,18 @@ def sector_struct(graph, op: PreparedOperator,
     # shared-D-tile variant), at most 64 live pair rows (norb^2/4 + 1)
     kmax = 112 if (settings.contraction == "fp64" and
                    settings.split_tile_fp64 == _lib.TILE_SPLIT_F64_DTILE) else 128
+    pull = None
+    if (settings.fused and settings.split_fp64 and op.h1 is None
+            and settings.split_tile_fp64 is None and precision == _lib.C128
+            and settings.contraction == "fp64"):
+        pull = op.pull_tables(graph)
     if (fwa is not None and settings.split_fp64 and precision == _lib.C128
             and op.npair + 1 <= kmax and graph.norb() ** 2 // 4 + 1 <= 64):
-        blk = op.beta_block(graph)
-        hbb64 = blk[4] if blk else None
+        if pull is not None and op.pair_symmetric:
+            hbb64 = pull[2]          # the same matrix
+        else:
+            blk = op.beta_block(graph)
+            hbb64 = blk[4] if blk else None
     s = _lib.Sector(graph.norb(), graph.nalpha(), graph.nbeta(), op.npair,
                     graph.lena(), graph.lenb(), _lib.ptr(ta), _lib.ptr(tb),
                     _lib.ptr(fwa), _lib.ptr(fwb), _lib.ptr(sla), nslot,
@@ -283,9 +361,14 @@ def sector_struct(graph, op: PreparedOperator,
                     keep.append(hoz)
                     s.hbb_oz = _lib.ptr(hoz)
         elif settings.contraction == "fp64":
-            s.tile = int(settings.split_tile_fp64)
+            s.tile = int(settings.split_tile_fp64 or 0)
         else:
             raise ValueError(f"settings.contraction={settings.contraction!r}")
+    if pull is not None:
+        keep += pull
+        s.pull_w, s.haa, s.hbb, s.pull_fwd, s.dexc_a = (
+            _lib.ptr(t) if t.numel() else None for t in pull)
+        s.npull = op.coupling.shape[0]
     return s, tuple(keep)
 
 
@@ -306,7 +389,7 @@ def workspace(sector: _lib.Sector, precision: int,
             ldk = (sector.lenb + 63) // 64 * 64
             fused += 6 * 2 * sector.lena * ldk + 8 * sector.lena
     need = max((2 * sector.npair + 1) * 2 * n * elem, fused)
-    if nbytes != need:
+    if nbytes != need and not (sector.pull_w and nbytes == 16 * n):
         raise _lib.FqeHipError(f"workspace size {nbytes} != {need}")
     nbytes = max(nbytes, 16 * sector.lena * sector.lenb, 16)
     return torch.empty(nbytes, dtype=torch.uint8, device=device)
@@ -320,8 +403,11 @@ def needs_panels(sector: _lib.Sector, op: PreparedOperator,
         return False
     import ctypes
     opc = op.c_struct()
-    if _lib.lib().fqehip_fused_supported(precision, ctypes.byref(sector),
-                                         ctypes.byref(opc)):
+    if (_lib.lib().fqehip_pull_supported(precision, ctypes.byref(sector),
+                                         ctypes.byref(opc))
+            or _lib.lib().fqehip_fused_supported(precision,
+                                                 ctypes.byref(sector),
+                                                 ctypes.byref(opc))):
         return False
     n = sector.lena * sector.lenb
     return (2 * sector.npair + 1) * 2 * n * 8 > settings.max_workspace_bytes

@@ -88,6 +88,19 @@ class SpinTables:
             self._ptab[key] = (fwd, slot)
         return self._ptab[key]
 
+    def pull_table(self, compressed: bool) -> torch.Tensor:
+        """Target words of the pull form (fqehip_pull_table), int32
+        [npair][length]."""
+        key = ("pull", bool(compressed))
+        if key not in self._ptab:
+            fwd, _ = self.fused_tables(compressed)
+            tab = torch.empty_like(fwd)
+            if fwd.numel():
+                _lib.call("fqehip_pull_table", fwd.shape[0], self.length,
+                          _lib.ptr(fwd), _lib.ptr(tab), _lib.stream_ptr())
+            self._ptab[key] = tab
+        return self._ptab[key]
+
     def map_lengths(self) -> numpy.ndarray:
         n, k = self.norb, self.nele
         off = comb(n - 2, k - 1) if n >= 2 and k >= 1 else 0

@@ -38,10 +38,14 @@ split_fp64 = True
 # diagonal row); 16 = MFMAs over all npair + 1 pair rows.
 split_tile = 0
 
-# Kernel of the complex128 split row pass: 0 = column-owned waves (the D'
-# values of a wave's columns gathered into its MFMA registers, A' in LDS);
-# 32 = the kernel with a shared, double-buffered D tile.
-split_tile_fp64 = 0
+# Kernel of complex128 two-body applies (with split_fp64): None = the pull
+# form (alpha rows of C contracted with the opposite-spin coupling, beta
+# excitations accumulated within the row), for real, complex and
+# spin-orbital operators; a number = the split row pass of real
+# pair-symmetric operators, 0 with column-owned waves (the D' values of a
+# wave's columns gathered into its MFMA registers, A' in LDS), 32 with a
+# shared, double-buffered D tile, other operators on the unfused kernels.
+split_tile_fp64 = None
 
 # Arithmetic of the complex128 split row pass: "fp64" (FP64 matrix cores)
 # or "ozaki" (exact int8 digit products, FP64 assembly).

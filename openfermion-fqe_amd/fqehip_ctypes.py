@@ -44,7 +44,9 @@ class Sector(ctypes.Structure):
                 ("fwd_a", c_void_p), ("fwd_b", c_void_p),
                 ("slot_a", c_void_p), ("nslot", c_int),
                 ("hbb_hi", c_void_p), ("hbb_lo", c_void_p), ("ldh", c_int64),
-                ("tile", c_int), ("hbb_f64", c_void_p), ("hbb_oz", c_void_p)]
+                ("tile", c_int), ("hbb_f64", c_void_p), ("hbb_oz", c_void_p),
+                ("dexc_a", c_void_p), ("pull_w", c_void_p), ("haa", c_void_p),
+                ("hbb", c_void_p), ("pull_fwd", c_void_p), ("npull", c_int)]
 
 
 class Operator(ctypes.Structure):

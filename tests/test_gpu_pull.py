@@ -1,0 +1,139 @@
+"""The pull form of the complex128 apply (k_same_spin_f64 and
+k_pull_rows_f64), on the GPU, against the oracle where it is small enough
+and against the slot-row and unfused kernels elsewhere.
+
+Sizes: one to several 16-column tiles with remainders, one and several
+passes over the W tiles (npair 3 to 196), one and several accumulator rows,
+4- and 8-wave workgroups, no off-diagonal alpha pair (empty or full alpha
+shell).  Tolerance 1e-12 normwise, as for every FP64 kernel here (sums of at
+most a few thousand products of random signs, each rounded to 1.1e-16).
+"""
+
+import copy
+
+import numpy
+import pytest
+
+from oracle import fqe_oracle as fo
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-12
+
+
+@pytest.fixture(scope="module")
+def fqe():
+    import torch
+    assert torch.cuda.is_available()
+    import fqe_amd
+    return fqe_amd
+
+
+def rel(a, b):
+    return numpy.linalg.norm(a - b) / numpy.linalg.norm(b)
+
+
+def tensors(kind, norb, rng):
+    h1, h2 = fo.synthetic_hamiltonian(norb, norb, rng)
+    if kind == "real":
+        return h1, h2
+    if kind == "nonsymmetric":
+        return (h1 + 0.1 * rng.normal(size=h1.shape),
+                h2 + 0.02 * rng.normal(size=h2.shape))
+    if kind == "complex":
+        return (h1 + 0.1j * rng.normal(size=h1.shape),
+                h2 + 0.02j * rng.normal(size=h2.shape))
+    m = 2 * norb
+    h1 = rng.normal(size=(m, m)) + 1j * rng.normal(size=(m, m))
+    h2 = rng.normal(size=(m,) * 4) + 1j * rng.normal(size=(m,) * 4)
+    return (h1.real, h2.real) if kind == "spin" else (h1, h2)
+
+
+def sector(fqe, na, nb, norb, seed):
+    rng = numpy.random.default_rng(seed)
+    g = fo.OracleGraph(na, nb, norb)
+    d = fqe.FqeData(na, nb, norb, dtype=numpy.complex128)
+    c = fo.synthetic_coeff(g.lena, g.lenb, rng)
+    d.coeff = c
+    return d, c, g, rng
+
+
+def prepared(fqe, kind, h, norb):
+    from fqe_amd import _lib, engine
+    make = (engine.prepare_spin_operator if kind.startswith("spin") else
+            engine.prepare_operator)
+    return make(h, norb, _lib.device())
+
+
+def takes_pull(d, op):
+    import ctypes
+    from fqe_amd import _lib, engine
+    s, keep = engine.sector_struct(d.get_fcigraph(), op, _lib.C128)
+    return bool(_lib.lib().fqehip_pull_supported(
+        _lib.C128, ctypes.byref(s), ctypes.byref(op.c_struct())))
+
+
+@pytest.mark.parametrize("kind", ["real", "nonsymmetric", "complex", "spin",
+                                  "spin_complex"])
+@pytest.mark.parametrize("na,nb,norb", [(1, 1, 2), (1, 2, 3), (2, 1, 5),
+                                        (3, 3, 6), (6, 2, 6), (2, 6, 7),
+                                        (5, 3, 7), (4, 3, 8), (3, 7, 9)])
+def test_pull_matches_oracle(fqe, kind, na, nb, norb):
+    print(f"pull {kind} {na} {nb} {norb}", flush=True)
+    d, c, g, rng = sector(fqe, na, nb, norb, 31 * norb + 7 * na + nb)
+    h = tensors(kind, norb, rng)
+    op = prepared(fqe, kind, h, norb)
+    assert takes_pull(d, op)
+    ref = (fo.apply_spin12(c, h[0], h[1], g) if kind.startswith("spin") else
+           fo.apply_12(c, h[0], h[1], g))
+    outs = []
+    for _ in range(2):
+        e = copy.deepcopy(d)
+        e.apply_inplace_scaled(h, op=op)
+        outs.append(e.coeff)
+    assert rel(outs[0], ref) < TOL
+    assert numpy.array_equal(outs[0], outs[1])
+    # the separate epilogue (in place, with accumulation and norm) and the
+    # one in the row kernel
+    from fqe_amd import engine
+    import torch
+    x = d.device_coeff().clone()
+    acc = torch.zeros_like(x)
+    n = engine.norm_partials_count(x.numel())
+    part = torch.zeros(max(n, 1), dtype=torch.float64, device=x.device)
+    engine.apply_sector(d.get_fcigraph(), x, op, x, alpha=0.5 - 2j,
+                        acc=torch.view_as_real(acc), partials=part)
+    want = (0.5 - 2j) * ref
+    assert rel(x.cpu().numpy(), want) < TOL
+    assert rel(acc.cpu().numpy(), want) < TOL
+    norm = numpy.sqrt(part.sum().item())
+    assert abs(norm - numpy.linalg.norm(want)) < TOL * norm
+    y = torch.empty_like(x)
+    engine.apply_sector(d.get_fcigraph(), d.device_coeff(), op, y,
+                        alpha=0.5 - 2j, beta=1.5j, cin=d.device_coeff())
+    assert rel(y.cpu().numpy(), want + 1.5j * c) < TOL
+
+
+@pytest.mark.parametrize("kind,na,nb,norb", [
+    ("real", 5, 6, 12), ("real", 7, 6, 13), ("real", 7, 7, 14),
+    ("real", 2, 8, 15), ("real", 3, 10, 15), ("nonsymmetric", 4, 6, 13),
+    ("complex", 5, 5, 11), ("complex", 6, 7, 14), ("spin", 5, 4, 11),
+    ("spin_complex", 3, 4, 12)])
+def test_pull_matches_other_kernels(fqe, kind, na, nb, norb):
+    """Sectors too large for the oracle: the same operator on the slot-row
+    kernels (real symmetric) or the unfused ones."""
+    from fqe_amd import settings
+    print(f"pull {kind} {na} {nb} {norb}", flush=True)
+    d, c, g, rng = sector(fqe, na, nb, norb, 17 * norb + 3 * na + nb)
+    h = tensors(kind, norb, rng)
+    op = prepared(fqe, kind, h, norb)
+    assert takes_pull(d, op)
+    e = copy.deepcopy(d)
+    e.apply_inplace_scaled(h, op=op)
+    saved = settings.split_tile_fp64
+    settings.split_tile_fp64 = 0
+    try:
+        assert not takes_pull(d, op)
+        d.apply_inplace_scaled(h, op=op)
+    finally:
+        settings.split_tile_fp64 = saved
+    assert rel(e.coeff, d.coeff) < TOL
