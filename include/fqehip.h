@@ -189,9 +189,8 @@ typedef struct fqehip_sector {
    * FP64 row kernel over the live pair rows); NULL keeps the FP64 row
    * kernel that also scatters beta excitations. */
   const double* hbb_f64;
-  /* Digits of the same FP64 beta-beta block for the Ozaki-digit split apply
-   * (tile FQEHIP_TILE_OZAKI; fqehip_beta_block_digits): when set, the
-   * beta-beta GEMM also runs as digit products; NULL keeps it in FP64. */
+  /* Digits of the same FP64 beta-beta block (fqehip_beta_block_digits) for
+   * tile FQEHIP_TILE_OZAKI, see haa_oz. */
   const void* hbb_oz;
   /* Pull form of the complex128 two-body apply (real, complex or
    * spin-orbital operators): H C = Haa C + C Hbb^T + sum_q E^b_q (sum_p
@@ -203,8 +202,14 @@ typedef struct fqehip_sector {
   const double* pull_w;    /* [npull][npull] coupling, alpha pair p, beta pair q */
   const double* haa;       /* fqehip_spin_block of the alpha strings */
   const double* hbb;       /* fqehip_spin_block of the beta strings */
-  const uint32_t* pull_fwd; /* [npull][lenb] fqehip_pull_table of the beta strings */
+  const uint32_t* pull_fwd; /* fqehip_pull_table of the beta strings */
   int npull;               /* pairs of one spin: norb(norb+1)/2 or norb^2 */
+  /* Digits for tile FQEHIP_TILE_OZAKI (real operators): of W
+   * (fqehip_pull_digits), and of Haa (fqehip_beta_block_digits of haa;
+   * hbb_oz those of hbb).  Without w_oz the form runs in FP64; without
+   * haa_oz and hbb_oz its same-spin products do. */
+  const void* w_oz;
+  const void* haa_oz;
 } fqehip_sector;
 
 #define FQEHIP_TILE_ROWS4 4
@@ -217,17 +222,12 @@ typedef struct fqehip_sector {
  * Gather depth npair + 1: up to 128 for the column-owned and the digit
  * kernels (norb <= 15 compressed), up to 112 with this tile. */
 #define FQEHIP_TILE_SPLIT_F64_DTILE 32
-/* complex128 split path (hbb_f64 set): the alpha-row contraction as exact
- * products of 8-bit digits on the int8 matrix cores (Ozaki scheme: A' in
- * five balanced digits per pair row, D' as 48-bit integers per alpha
- * string, 20 digit pairs, int32 accumulation, FP64 assembly); complex128
- * storage and row accumulators, the slot rows in 48 bits per double (12
- * bytes per complex value, relative rounding at most 2^-37) within the
- * FP64 path's slot region, which fqehip_apply_slot_reduce reads back for
- * the same sector.  The workspace grows by the beta gather table and the
- * pair rows' digits, lena doubles (row maxima of |C|) and, with hbb_oz
- * set, by the C digit planes of the beta-beta GEMM (6 * 2 lena * ldk bytes
- * + lena doubles). */
+/* complex128, a pair-symmetric real operator: the pull form's products as
+ * exact products of 8-bit digits on the int8 matrix cores (Ozaki scheme:
+ * operator rows in five balanced digits, data as 48-bit integers, 20 digit
+ * pairs, int32 accumulation, FP64 assembly), for the parts whose digits are
+ * set (w_oz; haa_oz and hbb_oz); a sector without the pull form's tables
+ * runs the FP64 split path. */
 #define FQEHIP_TILE_OZAKI 64
 
 typedef struct fqehip_operator {
@@ -254,8 +254,9 @@ int fqehip_fused_tables(int norb, int nele, int64_t nstrings,
  *   fused_rows: slot rows and row accumulators into d_workspace;
  *   slot_reduce: out = alpha * (H C) + beta * cin with the epilogue of
  *   fqehip_scatter.
- * The slot rows' format follows the sector (FQEHIP_TILE_OZAKI with
- * hbb_f64: 48-bit), so both calls take the same sector. */
+ * On a sector of the pull form fused_rows writes H C into the row
+ * accumulators (at the start of the workspace) and slot_reduce applies the
+ * epilogue to them. */
 int fqehip_fused_supported(int precision, const fqehip_sector* s,
                            const fqehip_operator* op);
 
@@ -288,9 +289,14 @@ int fqehip_spin_block(int complex_op, int npair, int64_t len,
                       const int32_t* d_fwd, const double* d_v, int64_t lda,
                       const double* d_h, double* d_hcol, void* stream);
 /* Target words of the pull form's row kernel, from the forward table d_fwd
- * ([npair][len], sign*(tgt+1) or 0): 8 (tgt + 1) with the sign in bit 31. */
+ * ([npair][len], sign*(tgt+1) or 0): 8 (tgt + 1) with the sign in bit 31, npair
+ * rounded up to 16 rows of len, the last ones zero. */
 int fqehip_pull_table(int npair, int64_t len, const int32_t* d_fwd,
                       uint32_t* d_tab, void* stream);
+/* Tables of W for the digit rows: fqehip_pull_digits_bytes(npull) bytes at
+ * d_woz, npull <= 128, once per operator. */
+int64_t fqehip_pull_digits_bytes(int npull);
+int fqehip_pull_digits(int npull, const double* d_w, void* d_woz, void* stream);
 /* Whether fqehip_apply takes the pull form for this sector and operator. */
 int fqehip_pull_supported(int precision, const fqehip_sector* s,
                           const fqehip_operator* op);
@@ -300,9 +306,10 @@ int fqehip_pull_supported(int precision, const fqehip_sector* s,
  * (fqehip_beta_block_digits_bytes(lenb) bytes): int8 [5][lenb][ldk]
  * (ldk = lenb rounded up to 64; per column Ib' of the GEMM, i.e. row Ib'
  * of Hbb, scaled by 2^eh with |Hbb 2^eh| < 2^38 and rounded to integers z,
- * the five exact balanced digits of z, weights 2^32, 2^24, ..., 1), then
- * double [lenb] scales 2^-eh, then double [lenb] offset corrections of
- * the C digits (128 (1 + 2^8 + 2^16 + 2^24 + 2^32) sum of the column's z).
+ * the five exact balanced digits of z, weights 2^32, 2^24, ..., 1; the
+ * diagonal as zero), then double [lenb] scales 2^-eh, double [lenb] offset
+ * corrections of the C digits (128 (1 + 2^8 + 2^16 + 2^24 + 2^32) sum of the
+ * column's z), and double [lenb] the diagonal.
  * Once per operator and beta string count; lenb < 26214. */
 int64_t fqehip_beta_block_digits_bytes(int64_t lenb);
 int fqehip_beta_block_digits(int64_t lenb, const double* d_hcol, void* d_hoz,
@@ -348,7 +355,7 @@ int fqehip_apply_slot_reduce(int precision, const fqehip_sector* s,
 /* Bytes of workspace for one apply of a sector: the larger of the unfused
  * path (dvec + Y planes) and the fused path (slot rows + row
  * accumulators); with pull_w set and the sector within the pull form's
- * limits, its row accumulator alone. */
+ * limits, its row accumulators (and the digit kernels' maxima and planes). */
 int64_t fqehip_apply_workspace_bytes(int precision, const fqehip_sector* s);
 
 /* out = alpha * H C + beta * cin (see fqehip_scatter for acc/partials).

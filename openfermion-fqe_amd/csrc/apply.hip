@@ -609,22 +609,24 @@ int launch_fused(int precision, int norb, int npair, int64_t lena, int64_t lenb,
                  int nslot, const void* coeff, void* slots, void* rowacc,
                  bool split, int tile, hipStream_t st, const int32_t* done);
 // Defined in ozaki.hip.
-bool split_oz_supported(int norb, int npair, int64_t lena, int64_t lenb);
-int64_t split_oz_table_bytes(int64_t lenb);
-int launch_split_oz(int norb, int npair, int64_t lena, int64_t lenb,
-                    const double* a, const int32_t* pta, const int32_t* ptb,
-                    const int32_t* fwa, const int32_t* sla, int nslot,
-                    const double* coeff, const double* rowmax, void* btab,
-                    uint32_t* slots, double* rowacc, bool build_tables,
-                    hipStream_t st, const int32_t* done);
-int launch_row_absmax(int64_t lena, int64_t lenb, const double* coeff,
-                      double* rowmax, hipStream_t st, const int32_t* done);
+bool pull_oz_supported(const fqehip_sector* s);
+int launch_pull_rows_oz(const fqehip_sector* s, const double* coeff,
+                        const double* rowmax, double* rowacc, double ar,
+                        double ai, double br, double bi, const double* cin,
+                        double* out, double* acc, hipStream_t st,
+                        const int32_t* done);
+int launch_absmax(int64_t lena, int64_t lenb, const double* coeff,
+                  double* rowmax, double* colmax, hipStream_t st,
+                  const int32_t* done);
 bool beta_oz_shape_ok(int64_t lena, int64_t lenb);
 int64_t beta_oz_workspace_bytes(int64_t lena, int64_t lenb);
 int launch_beta_gemm_oz(int64_t lena, int64_t lenb, const void* hoz,
                         const double* coeff, const double* rowmax,
                         void* cwork, double* out, hipStream_t st,
                         const int32_t* done);
+int launch_alpha_gemm_oz(int64_t lena, int64_t lenb, const void* hoz,
+                         const double* coeff, const double* colmax, void* cwork,
+                         double* out, hipStream_t st, const int32_t* done);
 // Defined in beta_block.hip.
 bool beta_gemm_shape_ok(int64_t lena, int64_t lenb, int64_t ldh);
 int launch_beta_gemm(int64_t lena, int64_t lenb, int64_t ldh, const void* hhi,
@@ -634,8 +636,8 @@ bool beta_gemm_f64_shape_ok(int64_t lena, int64_t lenb);
 int launch_beta_gemm_f64(int64_t lena, int64_t lenb, const double* hcol,
                          const double* coeff, double* out, hipStream_t st,
                          const int32_t* done);
-int launch_slot_reduce(int precision, bool p48, int nslot, int64_t lena,
-                       int64_t lenb, const void* slots, const void* rowacc,
+int launch_slot_reduce(int precision, int nslot, int64_t lena, int64_t lenb,
+                       const void* slots, const void* rowacc,
                        double ar, double ai, double br, double bi,
                        const void* cin, void* out, double* acc,
                        double* partials, hipStream_t st, const int32_t* done);
@@ -839,32 +841,41 @@ size_t elem_size(int precision) {
   return precision == FQEHIP_C128 ? sizeof(double) : sizeof(float);
 }
 
-// The complex128 split apply with Ozaki-digit contractions.
-bool ozaki_split(int precision, const fqehip_sector* s) {
-  return precision == FQEHIP_C128 && s->hbb_f64 != nullptr &&
-         s->tile == FQEHIP_TILE_OZAKI;
-}
-
 // Whether two-body applies of the sector take the pull form: it carries the
 // form's tables and is within its limits.
 bool pull_sector(int precision, const fqehip_sector* s) {
   return precision == FQEHIP_C128 && s->pull_w != nullptr && pull_supported(s);
 }
 
-// Workspace of the fused / split paths: slot rows, row accumulators and,
-// for the Ozaki-digit split apply, the beta gather table (lenb x 128
-// words), the row maxima of |C| (lena doubles) and, with hbb_oz, the C
-// digit planes of the beta-beta GEMM.
-int64_t fused_workspace_bytes(int precision, const fqehip_sector* s) {
-  const int64_t n = s->lena * s->lenb;
-  int64_t b = static_cast<int64_t>(s->nslot + 1) * 2 * n *
-              static_cast<int64_t>(elem_size(precision));
-  if (ozaki_split(precision, s)) {
-    b += split_oz_table_bytes(s->lenb);
-    b += s->lena * static_cast<int64_t>(sizeof(double));  // row maxima
-    if (s->hbb_oz) b += beta_oz_workspace_bytes(s->lena, s->lenb);
+// Whether the pull form's opposite-spin rows (and, with the blocks' digits,
+// its same-spin products) are digit products.
+bool digit_rows(const fqehip_sector* s) {
+  return s->tile == FQEHIP_TILE_OZAKI && pull_oz_supported(s);
+}
+bool digit_blocks(const fqehip_sector* s) {
+  return digit_rows(s) && s->haa_oz && s->hbb_oz &&
+         beta_oz_shape_ok(s->lena, s->lenb) && beta_oz_shape_ok(s->lenb, s->lena);
+}
+
+// Workspace of the pull form: the row accumulators; for the digit kernels the
+// row maxima of |C|, and for the blocks its column maxima and the digit
+// planes of C (then of C^T).
+int64_t pull_workspace_bytes(const fqehip_sector* s) {
+  int64_t b = 16 * s->lena * s->lenb;
+  if (digit_rows(s)) b += 8 * s->lena;
+  if (digit_blocks(s)) {
+    const int64_t c = beta_oz_workspace_bytes(s->lena, s->lenb);
+    const int64_t ct = beta_oz_workspace_bytes(s->lenb, s->lena);
+    b += 8 * s->lenb + (c > ct ? c : ct);
   }
   return b;
+}
+
+// Workspace of the fused / split paths: slot rows and row accumulators.
+int64_t fused_workspace_bytes(int precision, const fqehip_sector* s) {
+  const int64_t n = s->lena * s->lenb;
+  return static_cast<int64_t>(s->nslot + 1) * 2 * n *
+         static_cast<int64_t>(elem_size(precision));
 }
 
 }  // namespace
@@ -879,10 +890,6 @@ extern "C" int fqehip_fused_supported(int precision, const fqehip_sector* s,
   if (!(s && op && op->a && !op->h1 && !op->complex_op && s->fwd_a &&
         s->fwd_b && s->slot_a))
     return 0;
-  if (ozaki_split(precision, s))
-    return split_oz_supported(s->norb, s->npair, s->lena, s->lenb) &&
-           (s->hbb_oz ? beta_oz_shape_ok(s->lena, s->lenb)
-                      : beta_gemm_f64_shape_ok(s->lena, s->lenb));
   if (precision == FQEHIP_C128 && s->hbb_f64)
     return split_f64_supported(s->npair, s->lena, s->lenb, s->tile) &&
            beta_gemm_f64_shape_ok(s->lena, s->lenb);
@@ -892,19 +899,49 @@ extern "C" int fqehip_fused_supported(int precision, const fqehip_sector* s,
 namespace fqehip {
 namespace {
 
-// fqehip_apply_fused_rows; reuse_tables: see apply_reusing_tables.
+// The pull form: rowacc (at the start of the workspace) = H C, or with out
+// set out = alpha (H C) + beta cin, acc += out, in the row kernel's epilogue.
+int pull_rows(const fqehip_sector* s, const fqehip_operator* op,
+              const double* c, void* d_workspace, double ar, double ai,
+              double br, double bi, const double* cin, double* out, double* acc,
+              const int32_t* done, hipStream_t st) {
+  double* rowacc = static_cast<double*>(d_workspace);
+  if (!digit_rows(s) || op->complex_op) {
+    int rc = launch_same_spin(s, op->complex_op, c, rowacc, st, done);
+    if (rc) return rc;
+    return launch_pull_rows(s, op->complex_op, c, rowacc, ar, ai, br, bi, cin,
+                            out, acc, st, done);
+  }
+  double* rowmax = rowacc + 2 * s->lena * s->lenb;
+  const bool blocks = digit_blocks(s);
+  double* colmax = blocks ? rowmax + s->lena : nullptr;
+  int rc = launch_absmax(s->lena, s->lenb, c, rowmax, colmax, st, done);
+  if (rc) return rc;
+  if (blocks) {
+    void* cwork = colmax + s->lenb;
+    rc = launch_beta_gemm_oz(s->lena, s->lenb, s->hbb_oz, c, rowmax, cwork,
+                             rowacc, st, done);
+    if (rc) return rc;
+    rc = launch_alpha_gemm_oz(s->lena, s->lenb, s->haa_oz, c, colmax, cwork,
+                              rowacc, st, done);
+  } else {
+    rc = launch_same_spin(s, 0, c, rowacc, st, done);
+  }
+  if (rc) return rc;
+  return launch_pull_rows_oz(s, c, rowmax, rowacc, ar, ai, br, bi, cin, out,
+                             acc, st, done);
+}
+
+// fqehip_apply_fused_rows.
 int fused_rows(int precision, const fqehip_sector* s, const fqehip_operator* op,
                const void* d_coeff, void* d_workspace, const int32_t* d_done,
-               void* stream, bool reuse_tables) {
+               void* stream) {
   if (int rc = check_sector_op(precision, s, op)) return rc;
   if (fqehip_pull_supported(precision, s, op)) {
     FQEHIP_CHECK_ARG(d_coeff && d_workspace, "NULL pointer");
-    const double* c = static_cast<const double*>(d_coeff);
-    double* rowacc = static_cast<double*>(d_workspace);
-    int rc = launch_same_spin(s, op->complex_op, c, rowacc, as_stream(stream), d_done);
-    if (rc) return rc;
-    return launch_pull_rows(s, op->complex_op, c, rowacc, 1.0, 0.0, 0.0, 0.0,
-                            nullptr, nullptr, nullptr, as_stream(stream), d_done);
+    return pull_rows(s, op, static_cast<const double*>(d_coeff), d_workspace,
+                     1.0, 0.0, 0.0, 0.0, nullptr, nullptr, nullptr, d_done,
+                     as_stream(stream));
   }
   FQEHIP_CHECK_ARG(fqehip_fused_supported(precision, s, op),
                    "the fused path does not support this sector/operator");
@@ -915,34 +952,6 @@ int fused_rows(int precision, const fqehip_sector* s, const fqehip_operator* op,
   char* ws = static_cast<char*>(d_workspace);
   void* rowacc = ws + static_cast<int64_t>(s->nslot) * 2 * n * elem_size(precision);
   hipStream_t st = as_stream(stream);
-  if (ozaki_split(precision, s)) {
-    // row maxima of |C| (digit scales), rowacc <- C Hbb^T (digit products
-    // when the operator's Hbb digits are set, else FP64), then the alpha
-    // rows (digit products)
-    void* btab = static_cast<double*>(rowacc) + 2 * n;
-    double* rowmax = reinterpret_cast<double*>(static_cast<char*>(btab) +
-                                               split_oz_table_bytes(s->lenb));
-    int rc = launch_row_absmax(s->lena, s->lenb,
-                               static_cast<const double*>(d_coeff), rowmax, st,
-                               d_done);
-    if (rc) return rc;
-    if (s->hbb_oz)
-      rc = launch_beta_gemm_oz(s->lena, s->lenb, s->hbb_oz,
-                               static_cast<const double*>(d_coeff), rowmax,
-                               rowmax + s->lena, static_cast<double*>(rowacc),
-                               st, d_done);
-    else
-      rc = launch_beta_gemm_f64(s->lena, s->lenb, s->hbb_f64,
-                                static_cast<const double*>(d_coeff),
-                                static_cast<double*>(rowacc), st, d_done);
-    if (rc) return rc;
-    return launch_split_oz(s->norb, s->npair, s->lena, s->lenb, op->a,
-                           s->ptab_a, s->ptab_b, s->fwd_a, s->slot_a, s->nslot,
-                           static_cast<const double*>(d_coeff), rowmax, btab,
-                           reinterpret_cast<uint32_t*>(ws),
-                           static_cast<double*>(rowacc), !reuse_tables, st,
-                           d_done);
-  }
   if (precision == FQEHIP_C128 && s->hbb_f64 != nullptr) {
     // rowacc <- C Hbb^T (FP64), then the live alpha rows add their part
     int rc = launch_beta_gemm_f64(s->lena, s->lenb, s->hbb_f64,
@@ -981,8 +990,7 @@ extern "C" int fqehip_apply_fused_rows(int precision, const fqehip_sector* s,
                                        const void* d_coeff, void* d_workspace,
                                        const int32_t* d_done, void* stream) {
   clear_error();
-  return fused_rows(precision, s, op, d_coeff, d_workspace, d_done, stream,
-                    false);
+  return fused_rows(precision, s, op, d_coeff, d_workspace, d_done, stream);
 }
 
 extern "C" int fqehip_apply_slot_reduce(int precision, const fqehip_sector* s,
@@ -1000,14 +1008,12 @@ extern "C" int fqehip_apply_slot_reduce(int precision, const fqehip_sector* s,
   const int64_t n = s->lena * s->lenb;
   const char* ws = static_cast<const char*>(d_workspace);
   if (pull_sector(precision, s))   // no slot rows: the accumulators are H C
-    return launch_slot_reduce(precision, false, 0, s->lena, s->lenb, ws, ws,
+    return launch_slot_reduce(precision, 0, s->lena, s->lenb, ws, ws,
                               alpha_re, alpha_im, beta_re, beta_im, d_cin,
                               d_out, d_acc, d_norm_partials, as_stream(stream),
                               d_done);
   const void* rowacc = ws + static_cast<int64_t>(s->nslot) * 2 * n * elem_size(precision);
-  // the Ozaki-digit row kernel writes the slot rows in 48 bits per double
-  return launch_slot_reduce(precision, ozaki_split(precision, s), s->nslot,
-                            s->lena, s->lenb, ws, rowacc,
+  return launch_slot_reduce(precision, s->nslot, s->lena, s->lenb, ws, rowacc,
                             alpha_re, alpha_im, beta_re, beta_im, d_cin, d_out,
                             d_acc, d_norm_partials, as_stream(stream), d_done);
 }
@@ -1016,24 +1022,21 @@ extern "C" int64_t fqehip_apply_workspace_bytes(int precision,
                                                const fqehip_sector* s) {
   if (!s) return -1;
   const int64_t n = s->lena * s->lenb;
-  if (pull_sector(precision, s)) return 2 * n * static_cast<int64_t>(sizeof(double));
+  if (pull_sector(precision, s)) return pull_workspace_bytes(s);
   const int64_t unfused = static_cast<int64_t>(2 * s->npair + 1) * 2 * n *
                           static_cast<int64_t>(elem_size(precision));
   const int64_t fused = fused_workspace_bytes(precision, s);
   return unfused > fused ? unfused : fused;
 }
 
-// fqehip_apply.  reuse_tables: the Ozaki-digit split apply takes the beta
-// gather table and the pair rows' digits from the workspace as an earlier
-// apply of the same sector and operator with the same workspace left them
-// (they depend on neither the coefficients nor alpha/beta), instead of
-// rebuilding them: the later terms of a Taylor series.
-int fqehip::apply_reusing_tables(
-    int precision, const fqehip_sector* s, const fqehip_operator* op,
-    const void* d_coeff, double alpha_re, double alpha_im, double beta_re,
-    double beta_im, const void* d_cin, void* d_out, double* d_acc,
-    double* d_norm_partials, const int32_t* d_done, void* d_workspace,
-    void* stream, bool reuse_tables) {
+extern "C" int fqehip_apply(int precision, const fqehip_sector* s,
+                            const fqehip_operator* op, const void* d_coeff,
+                            double alpha_re, double alpha_im, double beta_re,
+                            double beta_im, const void* d_cin, void* d_out,
+                            double* d_acc, double* d_norm_partials,
+                            const int32_t* d_done, void* d_workspace,
+                            void* stream) {
+  clear_error();
   if (int rc = check_sector_op(precision, s, op)) return rc;
   FQEHIP_CHECK_ARG(d_coeff && d_out, "NULL coefficient pointer");
   if (op->h1)
@@ -1049,26 +1052,20 @@ int fqehip::apply_reusing_tables(
                      "beta != 0 needs d_cin");
     // the epilogue in the row kernel, except in place (other rows still read
     // d_coeff) and for norm partials (one per 256 elements)
-    if (d_out == d_coeff || d_norm_partials) {
-      int rc = fused_rows(precision, s, op, d_coeff, d_workspace, d_done, stream,
-                          false);
-      if (rc) return rc;
-      return fqehip_apply_slot_reduce(precision, s, d_workspace, alpha_re,
-                                      alpha_im, beta_re, beta_im, d_cin, d_out,
-                                      d_acc, d_norm_partials, d_done, stream);
-    }
-    const double* c = static_cast<const double*>(d_coeff);
-    double* rowacc = static_cast<double*>(d_workspace);
-    hipStream_t st = as_stream(stream);
-    int rc = launch_same_spin(s, op->complex_op, c, rowacc, st, d_done);
+    if (d_out != d_coeff && !d_norm_partials)
+      return pull_rows(s, op, static_cast<const double*>(d_coeff), d_workspace,
+                       alpha_re, alpha_im, beta_re, beta_im,
+                       static_cast<const double*>(d_cin),
+                       static_cast<double*>(d_out), d_acc, d_done,
+                       as_stream(stream));
+    int rc = fused_rows(precision, s, op, d_coeff, d_workspace, d_done, stream);
     if (rc) return rc;
-    return launch_pull_rows(s, op->complex_op, c, rowacc, alpha_re, alpha_im,
-                            beta_re, beta_im, static_cast<const double*>(d_cin),
-                            static_cast<double*>(d_out), d_acc, st, d_done);
+    return fqehip_apply_slot_reduce(precision, s, d_workspace, alpha_re,
+                                    alpha_im, beta_re, beta_im, d_cin, d_out,
+                                    d_acc, d_norm_partials, d_done, stream);
   }
   if (fqehip_fused_supported(precision, s, op)) {
-    int rc = fused_rows(precision, s, op, d_coeff, d_workspace, d_done, stream,
-                        reuse_tables);
+    int rc = fused_rows(precision, s, op, d_coeff, d_workspace, d_done, stream);
     if (rc) return rc;
     return fqehip_apply_slot_reduce(precision, s, d_workspace, alpha_re,
                                     alpha_im, beta_re, beta_im, d_cin, d_out,
@@ -1090,20 +1087,6 @@ int fqehip::apply_reusing_tables(
   return fqehip_scatter(precision, s->npair, s->lena, s->lenb, s->ptab_a,
                         s->ptab_b, y, alpha_re, alpha_im, beta_re, beta_im,
                         d_cin, d_out, d_acc, d_norm_partials, d_done, stream);
-}
-
-extern "C" int fqehip_apply(int precision, const fqehip_sector* s,
-                            const fqehip_operator* op, const void* d_coeff,
-                            double alpha_re, double alpha_im, double beta_re,
-                            double beta_im, const void* d_cin, void* d_out,
-                            double* d_acc, double* d_norm_partials,
-                            const int32_t* d_done, void* d_workspace,
-                            void* stream) {
-  clear_error();
-  return apply_reusing_tables(precision, s, op, d_coeff, alpha_re, alpha_im,
-                              beta_re, beta_im, d_cin, d_out, d_acc,
-                              d_norm_partials, d_done, d_workspace, stream,
-                              false);
 }
 
 extern "C" int fqehip_taylor(int precision, const fqehip_sector* s,
@@ -1140,9 +1123,8 @@ extern "C" int fqehip_taylor(int precision, const fqehip_sector* s,
       cur = nxt;
       nxt = t;
     } else {
-      rc = apply_reusing_tables(precision, s, op, d_term, ar, ai, 0.0, 0.0,
-                                nullptr, d_term, d_result, d_partials, done,
-                                d_workspace, stream, order > 1);
+      rc = fqehip_apply(precision, s, op, d_term, ar, ai, 0.0, 0.0, nullptr,
+                        d_term, d_result, d_partials, done, d_workspace, stream);
     }
     if (rc) return rc;
     rc = fqehip_norm_finalize(d_partials, np, d_norm, accuracy, order, done,

@@ -1,39 +1,34 @@
-// Ozaki-digit variant of the complex128 split apply: the same operands,
-// layouts and scatter as the FP64 split path (complex128 C, FP64 row
-// accumulators; the slot rows in 48 bits per double, 12 bytes per complex
-// value, stream_store_p48), with the pair contraction Y = A' D' of the alpha
-// row kernel computed as exact integer products of 8-bit digits on the
-// matrix cores (v_mfma_i32_16x16x64_i8, int32 accumulation) instead of
-// FP64 matrix-core products.
+// Ozaki-digit variant of the pull form (pull.hip) for complex128 applies of
+// pair-symmetric real operators: the same operands and the same three parts
+// H C = Haa C + C Hbb^T + sum_q E^b_q (sum_p W[p][q] E^a_p C), with every
+// product formed exactly from 8-bit digits on the matrix cores
+// (v_mfma_i32_16x16x64_i8, int32 accumulation) instead of FP64 matrix-core
+// products, and assembled in FP64.
 //
-// Digits.  Per alpha string ia, A' (the live pair rows of the operator) is
-// scaled row by row by a power of two so that |A' 2^ea| < 2^38, rounded to
-// the integer z and split exactly into five balanced signed digits
-// a_0..a_4 in [-128, 127] of weights 2^32, 2^24, ..., 1 (from the low end:
-// d = ((z + 128) mod 256) - 128, z = (z - d) / 256).
-// D' (gathered from C) is scaled by one power of two per alpha string,
-// 2^ed with ed from a bound on |D'| (the largest row maximum of |C| over the
-// alpha sources of ia, plus twice the row maximum of row ia), so that
-// |D' 2^ed| < 2^46, and rounded to a 48-bit integer y.  The six bytes of y
-// (two's complement) are the digits d_0..d_5 of weights 1 .. 2^40.
-// d_0..d_4 are stored as unsigned bytes minus 128 (one XOR), d_5 as the
-// signed top byte, so no carry propagation is needed; the 128 offsets are
-// added back exactly, for every digit pair, through the row sums of the A'
-// integers.
+// Digits.  An operator row (of W: all alpha pairs p of one beta pair q; of
+// Haa, Hbb: all source strings of one target) is scaled by a power of two so
+// that |x 2^ea| < 2^38, rounded to the integer z and split exactly into five
+// balanced signed digits a_0..a_4 in [-128, 127] of weights 2^32, 2^24, ..., 1
+// (from the low end: d = ((z + 128) mod 256) - 128, z = (z - d) / 256).
+// Data (C) is scaled by one power of two per alpha string (rows and Hbb) or
+// beta string (Haa), from a bound on the magnitudes, so that |x 2^ed| < 2^46,
+// and rounded to a 48-bit integer y.  The six bytes of y (two's complement)
+// are the digits d_0..d_5 of weights 1 .. 2^40.  d_0..d_4 are stored as
+// unsigned bytes minus 128 (one XOR), d_5 as the signed top byte, so no carry
+// propagation is needed; the 128 offsets are added back exactly, for every
+// digit pair, through the sums of the operator integers.
 //
 // Products.  Of the 30 digit pairs, the 20 with i - t >= 0 (weight >= 2^32
 // of a maximum of 2^72) are formed, six int32 accumulators per output (one
 // per i - t); the dropped pairs weigh at most 2^-40 of the largest product
 // each, and since the offsets of all pairs are corrected, they enter as
 // sums of zero-mean terms: about 1e-11 of the result when the bound is a
-// few times the gathered values, and still below 1e-9 for vectors whose
-// weight sits on a few determinants.  Every int32 sum is exact (at most
-// 5 * 128 * 128 * 128 < 2^24 per accumulator).  The result is assembled in
-// FP64: Y = 2^-(ea+ed) (2^32 sum_m 2^(8m) acc_m + 128 (1 + 2^8 + 2^16 +
-// 2^24 + 2^32) sum_q z_q).
+// few times the values, and still below 1e-9 for vectors whose weight sits
+// on a few determinants.  Every int32 sum is exact.  A result is assembled in
+// FP64: 2^-(ea+ed) (2^32 sum_m 2^(8m) acc_m + 128 (1 + 2^8 + 2^16 + 2^24 +
+// 2^32) sum z).
 //
-// Reference: the opposite-spin and alpha same-spin terms of
-// lm_apply_array12_same_spin_opt / lm_apply_array12_diff_spin_opt
+// Reference: lm_apply_array12_same_spin_opt / lm_apply_array12_diff_spin_opt
 // (src/fqe/lib/fqe_data.c:668-720, :879-996), in complex128.
 #include "fqehip_common.h"
 #include "rows_common.h"
@@ -45,19 +40,25 @@ using namespace rows;
 
 typedef int int4v __attribute__((ext_vector_type(4)));
 
-constexpr int kOzKPad = 128;               // gathered rows (pairs + C), padded
-constexpr int kOzKSteps = kOzKPad / 64;    // k steps of the i8 MFMA
-constexpr int kOzADig = 5;                 // digits of A'
-constexpr int kOzDDig = 6;                 // digits 0..5 of the D' integers
-constexpr int kOzARow = kOzKPad + 16;      // bytes per LDS row of a digit plane
+constexpr int kOzK = 64;                   // live alpha pairs of a string, padded
+constexpr int kOzADig = 5;                 // digits of the operator
+constexpr int kOzDDig = 6;                 // digits 0..5 of the data integers
+constexpr int kOzARow = kOzK + 16;         // bytes per LDS row of a digit plane
+constexpr int kOzQ = 128;                  // beta pairs, padded (table pitch)
 constexpr double kMagic = 6755399441055744.0;  // 1.5 * 2^52: rint via one add
 
-// rowmax[I] = max over the row of max(|Re C[I][.]|, |Im C[I][.]|).
+// rowmax[I] = max over the row of max(|Re C[I][.]|, |Im C[I][.]|); zeroes
+// colmax (when not NULL) for k_col_absmax.
 __global__ void __launch_bounds__(256)
 k_row_absmax(int64_t lena, int64_t lenb, const double* __restrict__ coeff,
-             double* __restrict__ rowmax, const int32_t* __restrict__ done) {
+             double* __restrict__ rowmax, unsigned long long* __restrict__ colmax,
+             const int32_t* __restrict__ done) {
   __shared__ double red[4];
   if (done && *done) return;
+  if (colmax)
+    for (int64_t j = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; j < lenb;
+         j += static_cast<int64_t>(gridDim.x) * 256)
+      colmax[j] = 0;
   for (int64_t r = blockIdx.x; r < lena; r += gridDim.x) {
     const double* row = coeff + r * lenb * 2;
     double m = 0.0;
@@ -70,6 +71,27 @@ k_row_absmax(int64_t lena, int64_t lenb, const double* __restrict__ coeff,
       rowmax[r] = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
     __syncthreads();
   }
+}
+
+// colmax[j] = the same over column j (bits of a non-negative double, ordered
+// as the doubles are), 64 rows per workgroup.
+constexpr int kColRows = 64;
+__global__ void __launch_bounds__(256)
+k_col_absmax(int64_t lena, int64_t lenb, const double* __restrict__ coeff,
+             unsigned long long* __restrict__ colmax,
+             const int32_t* __restrict__ done) {
+  if (done && *done) return;
+  const int64_t j = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (j >= lenb) return;
+  const int64_t r0 = static_cast<int64_t>(blockIdx.y) * kColRows;
+  const int64_t r1 = r0 + kColRows < lena ? r0 + kColRows : lena;
+  double m = 0.0;
+#pragma unroll 8
+  for (int64_t r = r0; r < r1; ++r) {
+    const double2 v = reinterpret_cast<const double2*>(coeff)[r * lenb + j];
+    m = fmax(m, fmax(fabs(v.x), fabs(v.y)));
+  }
+  atomicMax(&colmax[j], static_cast<unsigned long long>(__double_as_longlong(m)));
 }
 
 // Digits 0..5 of four 48-bit integers y_j held as the (lo, hi) words of
@@ -111,595 +133,419 @@ __device__ __forceinline__ double as_double(uint32_t lo, uint32_t hi) {
 // every digit pair, 128 (1 + 2^8 + 2^16 + 2^24 + 2^32) per unit of the
 // operator integers' sum.
 constexpr double kOffsetUnit = 128.0 * 4311810305.0;
-// Invalid alpha gather offset, in 16-byte units: (kNoRow16 + column) * 16
-// lies past the end of C (lena * lenb * 16 <= 0x7ff00000 is a launch
-// requirement) and below 2^31 (lenb < 2^16).
+// Invalid row offset, in 16-byte units: (kNoRow16 + column) * 16 lies past the
+// end of C (lena * lenb * 16 <= 0x7ff00000 is a launch requirement) and below
+// 2^31 (lenb < 2^16).
 constexpr uint32_t kNoRow16 = 0x7ff0000u;
-// Beta gather table entry without an excitation (global-memory row): a
-// byte offset past the end of every row of C.
-constexpr uint32_t kNoCol = 0x7ffffff0u;
 
-// Beta gather table of the Ozaki row kernel, column-major and padded to
-// kOzKPad entries per column: tab[jb][q] = byte offset of the source column
-// of beta excitation q of column jb within its row (16 (|ptb| - 1)), with
-// the sign of the excitation in bit 31; `none` where there is none
-// (ptb == 0, or q >= npair).
-__global__ void __launch_bounds__(256)
-k_beta_table_oz(int npair, int64_t lenb, const int32_t* __restrict__ ptb,
-                uint32_t none, uint32_t* __restrict__ tab,
-                const int32_t* __restrict__ done) {
-  if (done && *done) return;
-  const int64_t total = lenb * kOzKPad;
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-       i < total; i += static_cast<int64_t>(gridDim.x) * 256) {
-    const int64_t jb = i / kOzKPad;
-    const int q = static_cast<int>(i % kOzKPad);
-    uint32_t w = none;
-    if (q < npair) {
-      const int32_t b = ptb[static_cast<int64_t>(q) * lenb + jb];
-      if (b)
-        w = (b < 0 ? 0x80000000u : 0u) |
-            (static_cast<uint32_t>(iabs(b) - 1) << 4);
+// Tables of W for the row kernel, once per operator: the digits of every
+// alpha pair's column, dig[p][t][q] bytes (t: digit of weight 2^(8(4 - t))),
+// the integers z[p][q] = rint(W 2^ea) as doubles, and ea, one for all of W:
+// |z| < 2^38, and sum_pq |z| < 2^49, so that a sum over any (p, q) of z times
+// 46-bit data, in units of 2^32, stays below 2^63.  One workgroup per pair p,
+// thread q; every workgroup forms the maximum and the sum anew, in one order.
+constexpr int64_t kWDigBytes = static_cast<int64_t>(kOzADig) * kOzQ;
+__global__ void __launch_bounds__(kOzQ)
+k_pull_digits(int npull, const double* __restrict__ w, uint8_t* __restrict__ dig,
+              double* __restrict__ z, int32_t* __restrict__ ea) {
+  __shared__ double red[2][kOzQ / 64];
+  const int p = blockIdx.x;
+  const int q = threadIdx.x;
+  double m = 0.0, t = 0.0;
+  if (q < npull) {
+#pragma unroll 8
+    for (int r = 0; r < npull; ++r) {
+      const double v = fabs(w[static_cast<int64_t>(r) * npull + q]);
+      m = fmax(m, v);
+      t += v;
     }
-    tab[i] = w;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    m = fmax(m, __shfl_xor(m, o));
+    t += __shfl_xor(t, o);
+  }
+  if ((q & 63) == 0) {
+    red[0][q >> 6] = m;
+    red[1][q >> 6] = t;
+  }
+  __syncthreads();
+  m = fmax(red[0][0], red[0][1]);
+  t = red[1][0] + red[1][1];
+  int e = 0;
+  if (m > 0.0) {
+    int em, et;
+    (void)frexp(m, &em);
+    (void)frexp(t, &et);
+    e = 38 - em < 49 - et ? 38 - em : 49 - et;
+  }
+  int64_t v = q < npull ? static_cast<int64_t>(rint(ldexp(w[static_cast<int64_t>(p) * npull + q], e))) : 0;
+  z[static_cast<int64_t>(p) * kOzQ + q] = static_cast<double>(v);
+  if (p == 0 && q == 0) *ea = e;
+#pragma unroll
+  for (int t5 = kOzADig - 1; t5 >= 0; --t5) {
+    const int64_t d = t5 ? ((v + 128) & 255) - 128 : v;
+    v = (v - d) >> 8;
+    dig[p * kWDigBytes + t5 * kOzQ + q] = static_cast<uint8_t>(d & 0xff);
   }
 }
 
-// Digits of one quarter row (32 consecutive k) of an operator row, by a
-// group of 4 consecutive lanes (one quarter each): the row's scale 2^ea with
-// |x 2^ea| < 2^38 from the group's maximum, the exact balanced digits of the
-// integers z = rint(x 2^ea) (from the low end, d = ((z + 128) mod 256) -
-// 128, z = (z - d) / 256; w[t] holds digit t, weight 2^(8(4 - t)), of k
-// 4x..4x+3 in word x), and the row sum of the z.
-__device__ __forceinline__ void quarter_row_digits(const double (&v)[32],
-                                                   uint32_t (&w)[kOzADig][8],
-                                                   int& ea, double& zsum) {
-  double amax = 0.0;
-#pragma unroll
-  for (int j = 0; j < 32; ++j) amax = fmax(amax, fabs(v[j]));
-  amax = fmax(amax, __shfl_xor(amax, 1));
-  amax = fmax(amax, __shfl_xor(amax, 2));
-  ea = 0;
-  if (amax > 0.0) {
-    int e;
-    (void)frexp(amax, &e);
-    ea = 38 - e;
-  }
-  zsum = 0.0;
-#pragma unroll
-  for (int t = 0; t < kOzADig; ++t)
-#pragma unroll
-    for (int x = 0; x < 8; ++x) w[t][x] = 0u;
-#pragma unroll
-  for (int j = 0; j < 32; ++j) {
-    int64_t z = static_cast<int64_t>(rint(ldexp(v[j], ea)));
-    zsum += static_cast<double>(z);
-#pragma unroll
-    for (int t = kOzADig - 1; t >= 0; --t) {
-      const int64_t d = t ? ((z + 128) & 255) - 128 : z;
-      z = (z - d) >> 8;
-      w[t][j >> 2] |= (static_cast<uint32_t>(d) & 0xffu) << (8 * (j & 3));
-    }
-  }
-  zsum += __shfl_xor(zsum, 1);
-  zsum += __shfl_xor(zsum, 2);
+// Opposite-spin rows, one alpha string ia per workgroup of 8 waves (see
+// k_pull_rows_f64 for the operands).  K is the de-excitation rows of ia as
+// they are, diagonal ones included: at most 64, one k step of the i8 MFMA.
+//
+// Set-up: row offsets, signs and the scale of the data; the digits of the
+// live columns of W transposed from dig[p][t][q] to [t][q][k] in LDS, four k
+// by four q at a time (v_perm_b32); and per q the offset correction from the
+// sum of the integers, split into the three int32 start values of the
+// accumulator classes 0, 2 and 4.
+//
+// Main loop: each wave owns 16 columns of a 128-column chunk, loads its C
+// values (lane l: column l%16, k = 16 (l/16) + j) two batches of four ahead,
+// forms the six digit operands in registers, and runs the 20 digit products
+// of every 16-row tile of W for the real and the imaginary part on the same
+// A operands.  i8 MFMA layouts: lane l holds A[row l%16][k 16 (l/16) + j] and
+// B[k 16 (l/16) + j][col l%16]; output item e is [row 4 (l/16) + e][col l%16].
+//
+// W has one scale and the data of ia one, so all of the row's Z have one
+// unit, 2^(32 - ea - ed): a value is the 64-bit integer sum_m 2^(8m) acc_m,
+// assembled with 32-bit integer operations, and is added to its target's
+// 64-bit accumulator in LDS as it is (ds_add_u64).  Integer addition has no
+// order, so the waves need no turns and every run gives the same bits, and
+// nothing is rounded after the digits were cut.  A negative sign of E^b_q is
+// one XOR (-v - 1, one unit off).  With per-row scales and FP64 assembly (four
+// v_cvt_f64_i32 per value) the kernel took 3.7 ms at norb 14 7a7b instead of
+// 3.4; without the products 2.4, without the additions 2.4, set-up alone 0.24
+// (the slot-row form of the same products: 4.0 + 1.3 for its reduction).  Two
+// waves per SIMD fit (256 registers), so products and additions overlap only
+// in part.
+struct OzRowsArgs {
+  int norb, compressed, nalpha, nq, nqt;
+  int64_t lena, lenb;
+  const uint8_t* dig;
+  const double* z;
+  const int32_t* ea;
+  const int32_t* dexc;
+  const uint32_t* fwd;
+  const double* coeff;
+  const double* rowmax;
+  double* rowacc;
+  double alpha_re, alpha_im, beta_re, beta_im;
+  const double* cin;
+  double* out;
+  double* acc;
+  const int32_t* done;
+};
+
+constexpr int kRowThreads = 512;
+constexpr int kRowCols = 128;              // columns per chunk of 8 waves
+constexpr int kOzPartBytes = 4 * kOzQ * 8;   // set-up scratch
+
+size_t oz_rows_lds_bytes(int64_t lenb, int nqt) {
+  const size_t acc = static_cast<size_t>(lenb) * 16;
+  return (acc > kOzPartBytes ? acc : kOzPartBytes) +
+         static_cast<size_t>(kOzADig) * 16 * nqt * kOzARow + 3 * kOzQ * 4 +
+         kOzK * (8 + 4 + 4) + 16;
 }
 
-// A' digits of every pair row p < npair (the same for every alpha string:
-// A[p][0..npair-1] and the h1' entry A[npair][p] at k = npair, zero beyond),
-// once per apply: pdig[p][t][k] bytes, pea[p] = ea, pzs[p] = sum of z.
-__global__ void __launch_bounds__(256)
-k_pair_digits_oz(int npair, const double* __restrict__ amat,
-                 uint8_t* __restrict__ pdig, int32_t* __restrict__ pea,
-                 double* __restrict__ pzs, const int32_t* __restrict__ done) {
-  if (done && *done) return;
-  const int p = blockIdx.x * 64 + (threadIdx.x >> 2);
-  const int k0 = (threadIdx.x & 3) * 32;
-  const int K = npair;
-  const bool ok = p < npair;
-  double v[32];
-#pragma unroll
-  for (int j = 0; j < 32; ++j) {
-    const int k = k0 + j;
-    double x = 0.0;
-    if (ok) {
-      if (k < K) x = amat[static_cast<int64_t>(p) * K + k];
-      else if (k == K) x = amat[static_cast<int64_t>(npair) * K + p];
-    }
-    v[j] = x;
-  }
-  uint32_t w[kOzADig][8];
-  int ea;
-  double zsum;
-  quarter_row_digits(v, w, ea, zsum);
-  if (!ok) return;
-#pragma unroll
-  for (int t = 0; t < kOzADig; ++t) {
-    uint4* dst = reinterpret_cast<uint4*>(pdig + (static_cast<int64_t>(p) * kOzADig + t) * kOzKPad + k0);
-    dst[0] = make_uint4(w[t][0], w[t][1], w[t][2], w[t][3]);
-    dst[1] = make_uint4(w[t][4], w[t][5], w[t][6], w[t][7]);
-  }
-  if ((threadIdx.x & 3) == 0) {
-    pea[p] = ea;
-    pzs[p] = zsum;
-  }
-}
-
-constexpr int kRowThreads = 512;           // 8 waves, 16 columns each
-constexpr int kRowCols = 128;              // columns per chunk
-constexpr int64_t kDstNone = -1;           // padding row: no store
-constexpr int64_t kDstRowacc = -2;         // folded row: into rowacc
-
-// Alpha rows of the split apply (see k_split_cols_f64 in fused.hip for the
-// operands), one alpha string per block at a time.  Set-up: the live pair
-// rows' A' digits go to LDS and, with ROW_LDS, row ia of C too (plus one
-// zero entry at index lenb, the target of absent beta excitations); then
-// each wave owns 16 columns of a 128-column chunk, gathers their D' values
-// (lane l: column l%16, k = 64 s + 16 (l/16) + j) four k values at a time
-// with the next four's loads in flight - the alpha part from global memory
-// (absent sources read out of range: no memory access), the beta part from
-// the LDS row (random 16-byte reads, which cost about a seventh of a
-// random global gather) or, without ROW_LDS, from global memory - forms
-// the six digit operands in registers and runs the 20 digit products
-// (weight classes m = i - t = 0..5) of each of the four 16-row tiles, the
-// real and imaginary parts on the same A' operands.  The next chunk's beta
-// table words load during the products.  i8 MFMA layouts: lane l holds
-// A[row l%16][k 16 (l/16) + j] and B[k 16 (l/16) + j][col l%16] (byte j of
-// its four words); output item e of lane l is [row 4 (l/16) + e][col l%16].
-// Work items: alpha strings 0 .. nwhole - 1 whole (in XCD order), then each
-// of the remaining strings as two items, its first and second half of the
-// column chunks (so a last, partial round of strings over the CUs takes
-// half as long).
-template <bool ROW_LDS>
-__global__ void __launch_bounds__(kRowThreads)
-k_split_rows_oz(int norb, int compressed, int npair, int64_t lena,
-                int64_t nwhole, int64_t lenb, const double* __restrict__ amat,
-                const int32_t* __restrict__ pta, const uint32_t* __restrict__ btab,
-                const uint8_t* __restrict__ pdig, const int32_t* __restrict__ pea,
-                const double* __restrict__ pzs,
-                const int32_t* __restrict__ fwa, const int32_t* __restrict__ sla,
-                int nslot, const double* __restrict__ coeff,
-                const double* __restrict__ rowmax, uint32_t* __restrict__ slots,
-                double* __restrict__ rowacc, const int32_t* __restrict__ done) {
+__global__ void __launch_bounds__(kRowThreads, 2) k_pull_rows_oz(OzRowsArgs p) {
   extern __shared__ __align__(16) char smem[];
-  if (done && *done) return;
+  if (p.done && *p.done) return;
   const int tid = threadIdx.x;
   const int wave = tid >> 6;
   const int lane = tid & 63;
-  const int K = npair;
-  const int Kg = K + 1;                     // gathered rows: pairs + C
-  uint8_t* adig = reinterpret_cast<uint8_t*>(smem);  // [5][kLiveRows][kOzARow]
-  double* gsa = reinterpret_cast<double*>(adig + kOzADig * kLiveRows * kOzARow);
-  uint32_t* goff = reinterpret_cast<uint32_t*>(gsa + kOzKPad);  // [kOzKPad]
-  double* drow = reinterpret_cast<double*>(goff + kOzKPad);     // [kOzKPad]
-  double* rscale = drow + kOzKPad;          // [kLiveRows] +-2^(32 - ea - ed)
-  double* corr = rscale + kLiveRows;        // [kLiveRows] offset correction
-  // [kLiveRows] destination of a live row: word offset of its slot row,
-  // kDstRowacc (the folded row) or kDstNone (padding)
-  int64_t* rdst = reinterpret_cast<int64_t*>(corr + kLiveRows);
-  double* red = reinterpret_cast<double*>(rdst + kLiveRows);  // [8] block scratch
-  RowTables rt;
-  rt.sbase = reinterpret_cast<int64_t*>(red + 8);
-  rt.aoff = reinterpret_cast<int32_t*>(rt.sbase + kRowTabs);
-  rt.asgn = rt.aoff + kRowTabs;
-  rt.ssgn = rt.asgn + kRowTabs;
-  int32_t* lpair = rt.ssgn + kRowTabs;      // [kLiveRows] pair of live row
-  uint8_t* crow = reinterpret_cast<uint8_t*>(lpair + kLiveRows);  // [lenb + 1] x 16 B
+  const int kq = lane >> 4;
+  const int cl = lane & 15;
+  const int lenb = static_cast<int>(p.lenb);
+  const int nqp = 16 * p.nqt;
+  const int64_t ia = xcd_order(blockIdx.x, p.lena);
+  const int accb = lenb * 16 > kOzPartBytes ? lenb * 16 : kOzPartBytes;
+  unsigned long long* accs = reinterpret_cast<unsigned long long*>(smem);  // [lenb][re, im]
+  double* part = reinterpret_cast<double*>(smem);       // set-up: [4][kOzQ]
+  uint8_t* adig = reinterpret_cast<uint8_t*>(smem + accb);   // [5][nqp][kOzARow]
+  int32_t* start = reinterpret_cast<int32_t*>(adig + kOzADig * nqp * kOzARow);  // [3][kOzQ]
+  double* gsa = reinterpret_cast<double*>(start + 3 * kOzQ);  // [kOzK] sign 2^ed
+  uint32_t* goff = reinterpret_cast<uint32_t*>(gsa + kOzK);
+  int32_t* lp = reinterpret_cast<int32_t*>(goff + kOzK);
+  int32_t* scale = lp + kOzK;                           // ed
+  const int nexc = p.nalpha * (p.norb - p.nalpha + 1);
 
-  const int nchunks = static_cast<int>((lenb + kRowCols - 1) / kRowCols);
-  const __amdgpu_buffer_rsrc_t rc = buffer_of(coeff, lena * lenb * 2 * sizeof(double));
-  const __amdgpu_buffer_rsrc_t rtb = buffer_of(btab, lenb * kOzKPad * 4);
-  const int kq = lane >> 4;                 // k group of the lane
-  const int cl = lane & 15;                 // column within the wave's 16
-
-  if (ROW_LDS && tid == 0)
-    *reinterpret_cast<u32x4*>(crow + 16 * lenb) = u32x4{0u, 0u, 0u, 0u};
-
-  // beta table words of the lane's 32 k values in a chunk:
-  // tw[s][v][u] for k = 64 s + 16 kq + 4 v + u
-  u32x4 tw[kOzKSteps][4];
-  auto load_table = [&](int chunk) {
-    const int64_t jb = static_cast<int64_t>(chunk) * kRowCols + wave * 16 + cl;
-    const int base = static_cast<int>(jb < lenb ? jb : 0) * (kOzKPad * 4) + 64 * kq;
+  if (wave == 0) {
+    int32_t src = 0, ij = 0, sg = 0;
+    double m = 0.0;
+    if (lane < nexc) {
+      const int32_t* e = p.dexc + (ia * nexc + lane) * 3;
+      src = e[0];
+      ij = e[1];
+      sg = e[2];
+      m = p.rowmax[src];
+    }
 #pragma unroll
-    for (int s = 0; s < kOzKSteps; ++s)
+    for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o));
+    int e = 0;
+    if (m > 0.0) {
+      (void)frexp(m, &e);
+      e = 46 - e;                           // |D 2^ed| < 2^46
+    }
+    const int i = ij / p.norb, j = ij % p.norb;
+    lp[lane] = lane < nexc ? (p.compressed ? comp_pair(i, j) : ij) : -1;
+    goff[lane] = lane < nexc ? static_cast<uint32_t>(src) * static_cast<uint32_t>(lenb) : kNoRow16;
+    gsa[lane] = static_cast<double>(sg) * ldexp(1.0, e);
+    if (lane == 0) *scale = e;
+  }
+  __syncthreads();
+  {
+    const int q = tid & (kOzQ - 1);
+    const int k0 = (tid >> 7) * 16;
+    double zs = 0.0;
 #pragma unroll
-      for (int v = 0; v < 4; ++v)
-        tw[s][v] = __builtin_amdgcn_raw_buffer_load_b128(rtb, base + 256 * s + 16 * v, 0, 0);
+    for (int k = k0; k < k0 + 16; ++k) zs += k < nexc ? p.z[lp[k] * kOzQ + q] : 0.0;
+    part[(tid >> 7) * kOzQ + q] = zs;
+  }
+  // W digits: block x = (t, four q, four k)
+  for (int x = tid; x < kOzADig * (nqp / 4) * (kOzK / 4); x += kRowThreads) {
+    const int k4 = x & 15;
+    const int tq = x >> 4;
+    const int t = tq / (nqp / 4);
+    const int q4 = tq - t * (nqp / 4);
+    uint32_t v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int pr = lp[4 * k4 + u];
+      v[u] = pr >= 0 ? *reinterpret_cast<const uint32_t*>(p.dig + pr * kWDigBytes + t * kOzQ + 4 * q4)
+                     : 0u;
+    }
+    // transpose: word y holds bytes (q 4 q4 + y) of k 4 k4 .. + 3
+    const uint32_t x01 = __builtin_amdgcn_perm(v[1], v[0], 0x05010400u);
+    const uint32_t y01 = __builtin_amdgcn_perm(v[1], v[0], 0x07030602u);
+    const uint32_t x23 = __builtin_amdgcn_perm(v[3], v[2], 0x05010400u);
+    const uint32_t y23 = __builtin_amdgcn_perm(v[3], v[2], 0x07030602u);
+    uint8_t* dst = adig + (t * nqp + 4 * q4) * kOzARow + 4 * k4;
+    *reinterpret_cast<uint32_t*>(dst) = __builtin_amdgcn_perm(x23, x01, 0x05040100u);
+    *reinterpret_cast<uint32_t*>(dst + kOzARow) = __builtin_amdgcn_perm(x23, x01, 0x07060302u);
+    *reinterpret_cast<uint32_t*>(dst + 2 * kOzARow) = __builtin_amdgcn_perm(y23, y01, 0x05040100u);
+    *reinterpret_cast<uint32_t*>(dst + 3 * kOzARow) = __builtin_amdgcn_perm(y23, y01, 0x07060302u);
+  }
+  __syncthreads();
+  if (tid < kOzQ) {
+    // 128 (1 + 2^8 + 2^16 + 2^24 + 2^32) sum z in units of 2^32
+    const double zs = part[tid] + part[kOzQ + tid] + part[2 * kOzQ + tid] + part[3 * kOzQ + tid];
+    const int64_t v = static_cast<int64_t>(rint(kOffsetUnit * 0x1p-32 * zs));
+    const int64_t v4 = (v + (int64_t(1) << 31)) >> 32;
+    const int64_t r4 = v - (v4 << 32);
+    const int64_t v2 = (r4 + (1 << 15)) >> 16;
+    start[tid] = static_cast<int32_t>(r4 - (v2 << 16));
+    start[kOzQ + tid] = static_cast<int32_t>(v2);
+    start[2 * kOzQ + tid] = static_cast<int32_t>(v4);
+  }
+  __syncthreads();
+  for (int x = tid; x < 2 * lenb; x += kRowThreads) accs[x] = 0;
+  __syncthreads();
+
+  const __amdgpu_buffer_rsrc_t rc = buffer_of(p.coeff, p.lena * p.lenb * 16);
+  const __amdgpu_buffer_rsrc_t rf = buffer_of(p.fwd, static_cast<int64_t>(nqp) * lenb * 4);
+  // the target words' offsets are those of element target + 1
+  char* accum = smem - 16;
+  const int nchunks = (lenb + kRowCols - 1) / kRowCols;
+  u32x4 la[3][4];
+  auto load = [&](int chunk, int b, u32x4 (&A)[4]) {
+    const int jb = chunk * kRowCols + wave * 16 + cl;
+    // columns past the row read column 0 and add nothing
+    const uint32_t ib = static_cast<uint32_t>(jb < lenb ? jb : 0);
+    const uint4 g = *reinterpret_cast<const uint4*>(goff + 16 * kq + 4 * b);
+    A[0] = __builtin_amdgcn_raw_buffer_load_b128(rc, static_cast<int>((g.x + ib) << 4), 0, 0);
+    A[1] = __builtin_amdgcn_raw_buffer_load_b128(rc, static_cast<int>((g.y + ib) << 4), 0, 0);
+    A[2] = __builtin_amdgcn_raw_buffer_load_b128(rc, static_cast<int>((g.z + ib) << 4), 0, 0);
+    A[3] = __builtin_amdgcn_raw_buffer_load_b128(rc, static_cast<int>((g.w + ib) << 4), 0, 0);
   };
-  const int64_t nitems = nwhole + 2 * (lena - nwhole);
-  const int hchunks = (nchunks + 1) / 2;    // chunks of a first half
-  auto first_chunk = [&](int64_t it) {
-    return (it >= nwhole && ((it - nwhole) & 1)) ? hchunks : 0;
-  };
-  load_table(first_chunk(blockIdx.x));
-
-  for (int64_t it = blockIdx.x; it < nitems; it += gridDim.x) {
-    const int64_t ia = it < nwhole ? xcd_order(it, nwhole) : nwhole + ((it - nwhole) >> 1);
-    const int c0 = first_chunk(it);
-    const int c1 = (it < nwhole || c0 > 0) ? nchunks : hchunks;
-    const int next_c0 = first_chunk(it + gridDim.x);
-    load_row_tables<double>(ia, K, lena, lenb, nslot, pta, fwa, sla, rt, tid,
-                            kRowThreads, K);
-    if (ROW_LDS) {
-      const double* src = coeff + ia * lenb * 2;
-      for (int64_t j = tid; j < lenb; j += kRowThreads)
-        *reinterpret_cast<double2*>(crow + 16 * j) =
-            *reinterpret_cast<const double2*>(src + 2 * j);
-    }
-    __syncthreads();
-    if (wave == 0) {
-      // compact the live rows: pairs exciting ia to another string, then
-      // the folded row npair
-      int base = 0;
-      for (int p0 = 0; p0 < K; p0 += 64) {
-        const int p = p0 + lane;
-        const bool live = p < K && rt.sbase[p] >= 0;
-        const uint64_t m = __ballot(live);
-        const int pos = base + __popcll(m & ((1ull << lane) - 1ull));
-        if (live && pos < kLiveRows) lpair[pos] = p;
-        base += __popcll(m);
-      }
-      if (lane >= base) lpair[lane] = lane == base ? npair : -1;
-    } else if (wave == 1) {
-      // bound on |D'|: alpha sources (sign 1) plus twice the beta part,
-      // which gathers within row ia
-      double m = 0.0;
-      for (int q = lane; q < Kg; q += 64) {
-        const int32_t off = rt.aoff[q];
-        if (off >= 0) m = fmax(m, rowmax[off / (2 * lenb)]);
-      }
+  load(0, 0, la[0]);
+  load(0, 1, la[1]);
+  for (int chunk = 0; chunk < nchunks; ++chunk) {
+    const int jb = chunk * kRowCols + wave * 16 + cl;
+    const bool colok = jb < lenb;
+    int4v dd[2][kOzDDig];                   // [re, im][digit]
 #pragma unroll
-      for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o));
-      if (lane == 0) red[0] = m + 2.0 * rowmax[ia];
-    } else if (tid >= 256 && tid < 256 + kOzKPad) {
-      const int k = tid - 256;
-      double v = 0.0;
-      if (k < Kg) {
-        for (int i = 0; i < norb; ++i) {
-          const int dp = compressed ? i + i * (i + 1) / 2 : i * (norb + 1);
-          if (rt.sbase[dp] == -2)
-            v += k < K ? amat[static_cast<int64_t>(dp) * K + k]
-                       : amat[static_cast<int64_t>(npair) * K + dp];
-        }
+    for (int b = 0; b < 4; ++b) {
+      if (b + 2 < 4) load(chunk, b + 2, la[(b + 2) % 3]);
+      uint32_t lre[4], hre[4], lim[4], him[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const u32x4 v = la[b % 3][u];
+        const double sa = gsa[16 * kq + 4 * b + u];
+        split_words(fma(sa, as_double(v[0], v[1]), kMagic), lre[u], hre[u]);
+        split_words(fma(sa, as_double(v[2], v[3]), kMagic), lim[u], him[u]);
       }
-      drow[k] = v;
-    }
-    __syncthreads();
-    int ed = 0;
-    {
-      const double bound = red[0];
-      if (bound > 0.0) {
-        int e;
-        (void)frexp(bound, &e);
-        ed = 46 - e;                        // |D' 2^ed| < 2^46
+      uint32_t ore[kOzDDig], oim[kOzDDig];
+      digits_of_four(lre, hre, ore);
+      digits_of_four(lim, him, oim);
+#pragma unroll
+      for (int i = 0; i < kOzDDig; ++i) {
+        // the digit words exist here, before the next batch's loads
+        asm volatile("" : "+v"(ore[i]), "+v"(oim[i]));
+        dd[0][i][b] = static_cast<int>(ore[i]);
+        dd[1][i][b] = static_cast<int>(oim[i]);
       }
     }
-    const double dsc = ldexp(1.0, ed);
-    if (tid >= 256 && tid < 256 + kOzKPad) {
-      const int q = tid - 256;
-      const int32_t off = q < Kg ? rt.aoff[q] : -1;
-      goff[q] = off >= 0 ? static_cast<uint32_t>(off) >> 1 : kNoRow16;
-      gsa[q] = off >= 0 ? static_cast<double>(rt.asgn[q]) * dsc : 0.0;
-    } else if (tid < 256) {
-      // live pair rows: A' digits of the apply's pair table (thread -> live
-      // row tid/4, k in [32 (tid%4), +32)); padding rows zero; the folded
-      // row is formed below
-      const int m = tid >> 2;
-      const int k0 = (tid & 3) * 32;
-      const int p = lpair[m];
-      if (p != npair) {
-        uint4 w[kOzADig][2];
+    // target words of every row tile, ahead of the next chunk's values: loads
+    // return in order, so none is waited for behind those
+    uint32_t fw[kOzQ / 16][4];
+    const int fo = colok ? (4 * kq * lenb + jb) * 4 : -1;
 #pragma unroll
-        for (int t = 0; t < kOzADig; ++t) {
-          if (p >= 0) {
-            const uint4* src = reinterpret_cast<const uint4*>(
-                pdig + (static_cast<int64_t>(p) * kOzADig + t) * kOzKPad + k0);
-            w[t][0] = src[0];
-            w[t][1] = src[1];
-          } else {
-            w[t][0] = w[t][1] = make_uint4(0u, 0u, 0u, 0u);
-          }
-        }
+    for (int r = 0; r < kOzQ / 16; ++r)
+      if (r < p.nqt)
 #pragma unroll
-        for (int t = 0; t < kOzADig; ++t) {
-          uint4* dst = reinterpret_cast<uint4*>(adig + (t * kLiveRows + m) * kOzARow + k0);
-          dst[0] = w[t][0];
-          dst[1] = w[t][1];
-        }
-        if ((tid & 3) == 0) {
-          // Y = 2^(32 - ea - ed) t + 2^-(ea + ed) corr (powers of two: exact),
-          // times the sign of the scatter to the slot row
-          const double sc = p >= 0 ? ldexp(1.0, -(pea[p] + ed)) * rt.ssgn[p] : 0.0;
-          corr[m] = p >= 0 ? kOffsetUnit * pzs[p] * sc : 0.0;
-          rscale[m] = 4294967296.0 * sc;
-          rdst[m] = p >= 0 ? 3 * (rt.sbase[p] >> 1) : kDstNone;
-        }
-      }
-    } else if (wave == 6) {
-      // the folded row (sum of the rows of ia's occupied diagonal pairs):
-      // lanes 4 g .. 4 g + 3 of group g < 4 take its quarters
-      const uint64_t fm = __ballot(lpair[lane] == npair);
-      const int m = fm ? __ffsll(static_cast<unsigned long long>(fm)) - 1 : -1;
-      if (m >= 0 && lane < 4) {
-        const int k0 = lane * 32;
-        double v[32];
-#pragma unroll
-        for (int j = 0; j < 32; ++j) v[j] = drow[k0 + j];
-        uint32_t w[kOzADig][8];
-        int ea;
-        double zsum;
-        quarter_row_digits(v, w, ea, zsum);
-#pragma unroll
-        for (int t = 0; t < kOzADig; ++t) {
-          uint4* dst = reinterpret_cast<uint4*>(adig + (t * kLiveRows + m) * kOzARow + k0);
-          dst[0] = make_uint4(w[t][0], w[t][1], w[t][2], w[t][3]);
-          dst[1] = make_uint4(w[t][4], w[t][5], w[t][6], w[t][7]);
-        }
-        if (lane == 0) {
-          const double sc = ldexp(1.0, -(ea + ed));
-          corr[m] = kOffsetUnit * zsum * sc;
-          rscale[m] = 4294967296.0 * sc;
-          rdst[m] = kDstRowacc;
-        }
-      }
+        for (int e = 0; e < 4; ++e)
+          fw[r][e] = __builtin_amdgcn_raw_buffer_load_b32(
+              rf, fo, (16 * r + e) * 4 * lenb, static_cast<int>(0x80000000u));
+    if (chunk + 1 < nchunks) {
+      load(chunk + 1, 0, la[0]);
+      load(chunk + 1, 1, la[1]);
     }
-    __syncthreads();
-    // row ia of C in global memory (beta gathers without ROW_LDS; offsets
-    // past the row read 0)
-    const __amdgpu_buffer_rsrc_t rrow = buffer_of(coeff + ia * lenb * 2, lenb * 16);
-    const double dsc2 = 2.0 * dsc;
-
-    for (int chunk = c0; chunk < c1; ++chunk) {
-      const int64_t jb = static_cast<int64_t>(chunk) * kRowCols + wave * 16 + cl;
-      const bool colok = jb < lenb;
-      // padding columns gather column 0 (valid memory) and store nothing
-      const uint32_t ib = static_cast<uint32_t>(colok ? jb : 0);
-      int4v dd[2][kOzDDig][kOzKSteps];      // [re, im][digit][k step]
-      // batch b: k = 64 (b / 4) + 16 kq + 4 (b % 4) + u, u = 0..3
-      // batch b: digits of D' for k = 64 (b / 4) + 16 kq + 4 (b % 4) + u
-      auto digits = [&](int b, const u32x4 (&A)[4], const u32x4 (&B)[4]) {
-        const int s = b >> 2, v = b & 3;
-        const int q0 = 64 * s + 16 * kq + 4 * v;
-        uint32_t lre[4], hre[4], lim[4], him[4];
+    // the products at a raised wave priority: the SIMD's other wave, loading
+    // and converting, issues in the gaps
+    __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const uint32_t sg = tw[s][v][u] & 0x80000000u;
-          const double sa = gsa[q0 + u];
-          const double vre = fma(sa, as_double(A[u][0], A[u][1]),
-                                 fma(dsc2, as_double(B[u][0], B[u][1] ^ sg), kMagic));
-          const double vim = fma(sa, as_double(A[u][2], A[u][3]),
-                                 fma(dsc2, as_double(B[u][2], B[u][3] ^ sg), kMagic));
-          split_words(vre, lre[u], hre[u]);
-          split_words(vim, lim[u], him[u]);
-        }
-        uint32_t ore[kOzDDig], oim[kOzDDig];
-        digits_of_four(lre, hre, ore);
-        digits_of_four(lim, him, oim);
+    for (int r = 0; r < kOzQ / 16; ++r) {
+      if (r >= p.nqt) break;
+      int4v a[kOzADig];
 #pragma unroll
-        for (int i = 0; i < kOzDDig; ++i) {
-          // the digit words exist here, before the next batch's loads
-          // (otherwise the conversions sink to the MFMAs and every
-          // batch's loaded values stay live at once)
-          asm volatile("" : "+v"(ore[i]), "+v"(oim[i]));
-          dd[0][i][s][v] = static_cast<int>(ore[i]);
-          dd[1][i][s][v] = static_cast<int>(oim[i]);
-        }
-        asm volatile("" ::: "memory");
-      };
-      auto alpha_load = [&](int b, u32x4 (&A)[4]) {
-        const int q0 = 64 * (b >> 2) + 16 * kq + 4 * (b & 3);
+      for (int t = 0; t < kOzADig; ++t)
+        a[t] = *reinterpret_cast<const int4v*>(adig + (t * nqp + 16 * r + cl) * kOzARow + 16 * kq);
+      int4v acc[2][6];
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-          A[u] = __builtin_amdgcn_raw_buffer_load_b128(
-              rc, static_cast<int>((goff[q0 + u] + ib) << 4), 0, 0);
-      };
-      if constexpr (ROW_LDS) {
-        // global alpha gathers two batches ahead; the beta gathers from
-        // the LDS row at use
-        u32x4 la[3][4];
-        alpha_load(0, la[0]);
-        alpha_load(1, la[1]);
+      for (int c = 0; c < 2; ++c)
 #pragma unroll
-        for (int b = 0; b < 4 * kOzKSteps; ++b) {
-          if (b + 2 < 4 * kOzKSteps) alpha_load(b + 2, la[(b + 2) % 3]);
-          const int s = b >> 2, v = b & 3;
-          u32x4 lb[4];
+        for (int m = 0; m < 6; ++m)
+          acc[c][m] = (m & 1) ? int4v{0, 0, 0, 0}
+                              : *reinterpret_cast<const int4v*>(start + (m >> 1) * kOzQ + 16 * r + 4 * kq);
+      // pairs (data digit i, operator digit t) with m = i - t >= 0
 #pragma unroll
-          for (int u = 0; u < 4; ++u)
-            lb[u] = *reinterpret_cast<const u32x4*>(crow + (tw[s][v][u] & 0x7fffffffu));
-          digits(b, la[b % 3], lb);
-        }
-      } else {
-        u32x4 la[2][4], lb[2][4];
-        auto issue = [&](int b) {
-          const int s = b >> 2, v = b & 3;
-          alpha_load(b, la[b & 1]);
+      for (int c = 0; c < 2; ++c)
 #pragma unroll
-          for (int u = 0; u < 4; ++u)
-            lb[b & 1][u] = __builtin_amdgcn_raw_buffer_load_b128(
-                rrow, static_cast<int>(tw[s][v][u] & 0x7fffffffu), 0, 0);
-        };
-        issue(0);
-#pragma unroll
-        for (int b = 0; b < 4 * kOzKSteps; ++b) {
-          if (b + 1 < 4 * kOzKSteps) issue(b + 1);
-          digits(b, la[b & 1], lb[b & 1]);
-        }
-      }
-      // the next chunk's table (the next item's first chunk after the last)
-      load_table(chunk + 1 < c1 ? chunk + 1 : next_c0);
-      // the products at a raised wave priority: the SIMD's other wave,
-      // gathering, issues in the gaps instead of competing for issue with
-      // the MFMA stream (measured: 4.21 -> 4.13 ms at norb 14; priority
-      // during the gather instead: no gain)
-      __builtin_amdgcn_s_setprio(1);
-#pragma unroll 1
-      for (int r = 0; r < kLiveRows / 16; ++r) {
-        int4v acc[2][6];
-#pragma unroll
-        for (int c = 0; c < 2; ++c)
-#pragma unroll
-          for (int m = 0; m < 6; ++m) acc[c][m] = int4v{0, 0, 0, 0};
-#pragma unroll
-        for (int s = 0; s < kOzKSteps; ++s) {
-          int4v a[kOzADig];
+        for (int i = 0; i < kOzDDig; ++i)
 #pragma unroll
           for (int t = 0; t < kOzADig; ++t)
-            a[t] = *reinterpret_cast<const int4v*>(
-                adig + (t * kLiveRows + 16 * r + cl) * kOzARow + 64 * s + 16 * kq);
-          // pairs (data digit i, operator digit t) with m = i - t >= 0
+            if (t <= i)
+              acc[c][i - t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
+                  a[t], dd[c][i], acc[c][i - t], 0, 0, 0);
 #pragma unroll
-          for (int c = 0; c < 2; ++c)
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t f = fw[r][e];
+        if (!f) continue;
+        unsigned long long* to = reinterpret_cast<unsigned long long*>(accum + (f << 1));
+        const uint32_t sg = static_cast<uint32_t>(static_cast<int32_t>(f) >> 31);
 #pragma unroll
-            for (int i = 0; i < kOzDDig; ++i)
-#pragma unroll
-              for (int t = 0; t < kOzADig; ++t)
-                if (t <= i)
-                  acc[c][i - t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
-                      a[t], dd[c][i][s], acc[c][i - t], 0, 0, 0);
-        }
-        if (colok) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int row = 16 * r + 4 * kq + e;
-            double y[2];
-#pragma unroll
-            for (int c = 0; c < 2; ++c) {
-              // classes 5 and 4, and 3 and 2, merged in int32: with K <= 128,
-              // |acc5| <= 65 * 64 * 128 < 2^19.1, |acc4| < 2^21.1,
-              // |acc3| < 2^22.1, |acc2| < 2^22.7, so both merges stay below
-              // 2^31
-              const int32_t m54 = acc[c][5][e] * 256 + acc[c][4][e];
-              const int32_t m32 = acc[c][3][e] * 256 + acc[c][2][e];
-              double t = static_cast<double>(m54);
-              t = fma(t, 65536.0, static_cast<double>(m32));
-              t = fma(t, 256.0, static_cast<double>(acc[c][1][e]));
-              t = fma(t, 256.0, static_cast<double>(acc[c][0][e]));
-              y[c] = fma(t, rscale[row], corr[row]);
-            }
-            const int64_t dst = rdst[row];
-            if (dst >= 0) {
-              stream_store_p48(slots + dst + 3 * jb, y[0], y[1]);
-            } else if (dst == kDstRowacc) {
-              double2* d = reinterpret_cast<double2*>(rowacc + ia * lenb * 2 + 2 * jb);
-              double2 o = *d;
-              o.x += y[0];
-              o.y += y[1];
-              *d = o;
-            }
-          }
+        for (int c = 0; c < 2; ++c) {
+          // classes merged in pairs in int32: with K <= 64 the odd classes
+          // are below 2^22.4 (at most five products of 64 x 2^14)
+          const int32_t m10 = acc[c][1][e] * 256 + acc[c][0][e];
+          const int32_t m32 = acc[c][3][e] * 256 + acc[c][2][e];
+          const int32_t m54 = acc[c][5][e] * 256 + acc[c][4][e];
+          const int64_t v = static_cast<int64_t>(m10) + (static_cast<int64_t>(m32) << 16);
+          const uint32_t lo = static_cast<uint32_t>(v) ^ sg;
+          const uint32_t hi = (static_cast<uint32_t>(v >> 32) + static_cast<uint32_t>(m54)) ^ sg;
+          __hip_atomic_fetch_add(to + c,
+                                 static_cast<unsigned long long>(lo) |
+                                     (static_cast<unsigned long long>(hi) << 32),
+                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         }
       }
-      __builtin_amdgcn_s_setprio(0);
     }
-    __syncthreads();
+    __builtin_amdgcn_s_setprio(0);
   }
-}
-
-size_t split_rows_oz_lds_bytes(bool row_lds, int64_t lenb) {
-  return static_cast<size_t>(kOzADig) * kLiveRows * kOzARow +
-         kOzKPad * (sizeof(double) + sizeof(uint32_t)) +
-         (kOzKPad + 3 * kLiveRows + 8) * sizeof(double) +
-         kRowTabs * (sizeof(int64_t) + 3 * sizeof(int32_t)) +
-         kLiveRows * sizeof(int32_t) +
-         (row_lds ? static_cast<size_t>(lenb + 1) * 16 : 0);
+  __syncthreads();
+  const double back = ldexp(1.0, 32 - *p.ea - *scale);
+  double2* racc = reinterpret_cast<double2*>(p.rowacc) + ia * p.lenb;
+  for (int x = tid; x < lenb; x += kRowThreads) {
+    const double2 r = racc[x];
+    const double re = r.x + back * static_cast<double>(static_cast<int64_t>(accs[2 * x]));
+    const double im = r.y + back * static_cast<double>(static_cast<int64_t>(accs[2 * x + 1]));
+    if (!p.out) {
+      racc[x] = make_double2(re, im);
+      continue;
+    }
+    const int64_t idx = ia * p.lenb + x;
+    double vr = p.alpha_re * re - p.alpha_im * im;
+    double vi = p.alpha_re * im + p.alpha_im * re;
+    if (p.beta_re != 0.0 || p.beta_im != 0.0) {
+      const double2 c = reinterpret_cast<const double2*>(p.cin)[idx];
+      vr += p.beta_re * c.x - p.beta_im * c.y;
+      vi += p.beta_re * c.y + p.beta_im * c.x;
+    }
+    reinterpret_cast<double2*>(p.out)[idx] = make_double2(vr, vi);
+    if (p.acc) {
+      p.acc[2 * idx] += vr;
+      p.acc[2 * idx + 1] += vi;
+    }
+  }
 }
 
 constexpr size_t kLdsLimit = 160 * 1024;
 
 }  // namespace
 
-// Alpha rows of the Ozaki-digit split apply (requirements as for the FP64
-// split kernel: npair + 1 <= 128, norb^2/4 + 1 <= 64 live rows, 32-bit byte
-// offsets); rowmax: the row maxima of |C| (launch_row_absmax first).
-bool split_oz_supported(int norb, int npair, int64_t lena, int64_t lenb) {
-  return npair + 1 <= kOzKPad && norb * norb / 4 + 1 <= kLiveRows &&
-         lenb < (1 << 16) &&
-         lena * lenb * 16 <= static_cast<int64_t>(kNoRow16) * 16;
+// Whether the digit kernels take a sector of the pull form: at most 64
+// de-excitation rows, 128 pairs, the accumulator row in LDS, 32-bit offsets.
+bool pull_oz_supported(const fqehip_sector* s) {
+  return s->w_oz && s->pull_fwd && s->dexc_a && s->npull <= kOzQ && s->npull > 0 &&
+         s->nalpha * (s->norb - s->nalpha + 1) <= kOzK && s->lenb < (1 << 16) &&
+         s->lena * s->lenb * 16 <= static_cast<int64_t>(kNoRow16) * 16 &&
+         kOzQ * s->lenb * 4 < (int64_t(1) << 31) &&
+         oz_rows_lds_bytes(s->lenb, (s->npull + 15) / 16) <= kLdsLimit;
 }
 
-// Bytes of the tables of launch_split_oz: the beta gather table (lenb x
-// 128 words), then the pair rows' A' digits (128 x 5 x 128 bytes), their
-// scale exponents (128 int32) and integer sums (128 doubles).
-constexpr int64_t kPairDigitBytes = kOzKPad * (kOzADig * kOzKPad + 4 + 8);
-int64_t split_oz_table_bytes(int64_t lenb) {
-  return lenb * kOzKPad * 4 + kPairDigitBytes;
-}
-
-// build_tables false: btab already holds the beta table and the pair rows'
-// digits of this sector and operator (an earlier call with the same btab).
-int launch_split_oz(int norb, int npair, int64_t lena, int64_t lenb,
-                    const double* a, const int32_t* pta, const int32_t* ptb,
-                    const int32_t* fwa, const int32_t* sla, int nslot,
-                    const double* coeff, const double* rowmax, void* btab,
-                    uint32_t* slots, double* rowacc, bool build_tables,
-                    hipStream_t st, const int32_t* done) {
-  if (lena == 0 || lenb == 0) return FQEHIP_OK;
-  if (!split_oz_supported(norb, npair, lena, lenb)) {
-    set_error("the Ozaki split apply needs npair + 1 <= %d, norb^2/4 + 1 <= %d, "
-              "lenb < 65536 and 16 lena lenb <= %lld",
-              kOzKPad, kLiveRows, static_cast<long long>(kNoRow16) * 16);
-    return FQEHIP_ERR_INVALID;
-  }
-  uint32_t* tab = static_cast<uint32_t*>(btab);
-  uint8_t* pdig = reinterpret_cast<uint8_t*>(tab + lenb * kOzKPad);
-  int32_t* pea = reinterpret_cast<int32_t*>(pdig + kOzKPad * kOzADig * kOzKPad);
-  double* pzs = reinterpret_cast<double*>(pea + kOzKPad);
-  const bool row_lds = split_rows_oz_lds_bytes(true, lenb) <= kLdsLimit;
-  if (build_tables) {
-    k_pair_digits_oz<<<(npair + 63) / 64, 256, 0, st>>>(npair, a, pdig, pea, pzs, done);
-    FQEHIP_CHECK_LAUNCH("k_pair_digits_oz");
-    const int64_t entries = lenb * kOzKPad;
-    const unsigned tgrid = static_cast<unsigned>(std::min<int64_t>((entries + 255) / 256, 4096));
-    // absent beta excitations: the zero entry after the LDS row, or past the
-    // end of the row in global memory
-    const uint32_t none = row_lds ? static_cast<uint32_t>(16 * lenb) : kNoCol;
-    k_beta_table_oz<<<tgrid, 256, 0, st>>>(npair, lenb, ptb, none, tab, done);
-    FQEHIP_CHECK_LAUNCH("k_beta_table_oz");
-  }
-  const int compressed = npair == norb * (norb + 1) / 2 ? 1 : 0;
-  // one workgroup per CU at a time: strings beyond the last full round over
-  // the CUs run as column halves when they fill at most half a round
-  int dev = 0, ncu = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
-    set_error("launch_split_oz: no device attributes");
-    return FQEHIP_ERR_HIP;
-  }
-  const int64_t rem = ncu > 0 ? lena % ncu : 0;
-  const int64_t nchunks = (lenb + kRowCols - 1) / kRowCols;
-  const int64_t nwhole = (nchunks >= 2 && 2 * rem <= ncu) ? lena - rem : lena;
-  const int64_t nitems = nwhole + 2 * (lena - nwhole);
-  const unsigned grid = static_cast<unsigned>(nitems < 65536 ? nitems : 65536);
-  const size_t lds = split_rows_oz_lds_bytes(row_lds, lenb);
-  if (row_lds)
-    k_split_rows_oz<true><<<grid, kRowThreads, lds, st>>>(
-        norb, compressed, npair, lena, nwhole, lenb, a, pta, tab, pdig, pea,
-        pzs, fwa, sla, nslot, coeff, rowmax, slots, rowacc, done);
-  else
-    k_split_rows_oz<false><<<grid, kRowThreads, lds, st>>>(
-        norb, compressed, npair, lena, nwhole, lenb, a, pta, tab, pdig, pea,
-        pzs, fwa, sla, nslot, coeff, rowmax, slots, rowacc, done);
-  FQEHIP_CHECK_LAUNCH("k_split_rows_oz");
+// The opposite-spin rows on top of rowacc (epilogue as launch_pull_rows).
+int launch_pull_rows_oz(const fqehip_sector* s, const double* coeff,
+                        const double* rowmax, double* rowacc, double ar,
+                        double ai, double br, double bi, const double* cin,
+                        double* out, double* acc, hipStream_t st,
+                        const int32_t* done) {
+  OzRowsArgs p{};
+  p.norb = s->norb;
+  p.compressed = s->npull == s->norb * (s->norb + 1) / 2 ? 1 : 0;
+  p.nalpha = s->nalpha;
+  p.nq = s->npull;
+  p.nqt = (s->npull + 15) / 16;
+  p.lena = s->lena;
+  p.lenb = s->lenb;
+  p.dig = static_cast<const uint8_t*>(s->w_oz);
+  p.z = reinterpret_cast<const double*>(p.dig + s->npull * kWDigBytes);
+  p.ea = reinterpret_cast<const int32_t*>(p.z + static_cast<int64_t>(s->npull) * kOzQ);
+  p.dexc = s->dexc_a;
+  p.fwd = s->pull_fwd;
+  p.coeff = coeff;
+  p.rowmax = rowmax;
+  p.rowacc = rowacc;
+  p.alpha_re = ar;
+  p.alpha_im = ai;
+  p.beta_re = br;
+  p.beta_im = bi;
+  p.cin = cin;
+  p.out = out;
+  p.acc = acc;
+  p.done = done;
+  k_pull_rows_oz<<<static_cast<unsigned>(s->lena), kRowThreads,
+                   oz_rows_lds_bytes(s->lenb, p.nqt), st>>>(p);
+  FQEHIP_CHECK_LAUNCH("k_pull_rows_oz");
   return FQEHIP_OK;
 }
 
 }  // namespace fqehip
 
 // ---------------------------------------------------------------------------
-// Beta-beta half of the Ozaki-digit split apply: rowacc[Ia][Ib'] =
-// sum_Ib C[Ia][Ib] Hbb[Ib'][Ib] as digit products on the int8 matrix cores.
+// Same-spin halves: C Hbb^T and Haa C = (C^T Haa^T)^T as digit products on the
+// int8 matrix cores, the second on the digits of C^T.
 //
-//   C: each row Ia scaled by 2^ec (|C 2^ec| < 2^46 from the row maximum,
+//   data: each row of the GEMM's left factor (row Ia of C; row Ib of C^T, i.e.
+//      column Ib of C) scaled by 2^ec (|C 2^ec| < 2^46 from its maximum,
 //      shared by the real and imaginary parts), rounded to 48-bit integers;
-//      digits 0..5 (bytes), 0..4 offset by -128 as in the alpha rows.
-//      M index of the GEMM = 2 Ia + (0 real | 1 imaginary).
-//   Hbb: each column Ib' scaled by 2^eh (|Hbb 2^eh| < 2^38), five balanced
+//      digits 0..5 (bytes), 0..4 offset by -128 as in the rows.
+//      M index of the GEMM = 2 row + (0 real | 1 imaginary).
+//   H: each target's row scaled by 2^eh (|H 2^eh| < 2^38), five balanced
 //      digits, built once per operator (fqehip_beta_block_digits) together
-//      with the column scales and the offset corrections.
+//      with the scales and the offset corrections.
 // Products with i - t >= 0 (20 pairs), six int32 accumulators per output
-// (exact for lenb < 26214: at most 5 * 128 * 128 * lenb < 2^31).
+// (exact for K < 26214: at most 5 * 128 * 128 * K < 2^31).
 // ---------------------------------------------------------------------------
 namespace fqehip {
 namespace {
@@ -773,25 +619,90 @@ k_c_digits(int64_t lena, int64_t lenb, int64_t ldk,
   }
 }
 
-// Hbb column maxima: colmax[Ib'] = max_Ib |Hbb[Ib'][Ib]| (hcol[Ib][Ib']).
+// C^T digits: planes of 2 lenb rows (2 Ib, 2 Ib + 1) of ldk bytes (K = Ia);
+// cscale[Ib] = 2^-ec.  A workgroup takes 64 alpha by 32 beta strings: rows of
+// C are read coalesced, four consecutive Ia of one column become one word per
+// digit, and the words go through LDS to be written 64 bytes per row.
+constexpr int kCtA = 64;
+constexpr int kCtB = 32;
+__global__ void __launch_bounds__(256)
+k_ct_digits(int64_t lena, int64_t lenb, int64_t ldk,
+            const double* __restrict__ coeff, const double* __restrict__ colmax,
+            uint32_t* __restrict__ cdig, double* __restrict__ cscale,
+            const int32_t* __restrict__ done) {
+  constexpr int kW = kCtA / 4;              // words per row of the tile
+  __shared__ uint32_t sm[6][2 * kCtB][kW + 1];
+  if (done && *done) return;
+  const int64_t b0 = static_cast<int64_t>(blockIdx.x) * kCtB;
+  const int64_t a0 = static_cast<int64_t>(blockIdx.y) * kCtA;
+  const int jl = threadIdx.x & (kCtB - 1);
+  const int64_t jb = b0 + jl;
+  int ec = 0;
+  const double mx = jb < lenb ? colmax[jb] : 0.0;
+  if (mx > 0.0) {
+    int e;
+    (void)frexp(mx, &e);
+    ec = 46 - e;
+  }
+  if (a0 == 0 && threadIdx.x < kCtB && jb < lenb) cscale[jb] = ldexp(1.0, -ec);
+  const double sc = ldexp(1.0, ec);
+  for (int g = threadIdx.x / kCtB; g < kW; g += 256 / kCtB) {
+    uint32_t lre[4], hre[4], lim[4], him[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int64_t ia = a0 + 4 * g + u;
+      double2 v = make_double2(0.0, 0.0);
+      if (ia < lena && jb < lenb) v = reinterpret_cast<const double2*>(coeff)[ia * lenb + jb];
+      split_words(fma(v.x, sc, kMagic), lre[u], hre[u]);
+      split_words(fma(v.y, sc, kMagic), lim[u], him[u]);
+    }
+    uint32_t ore[6], oim[6];
+    digits_of_four(lre, hre, ore);
+    digits_of_four(lim, him, oim);
+#pragma unroll
+    for (int i = 0; i < 6; ++i) {
+      sm[i][2 * jl][g] = ore[i];
+      sm[i][2 * jl + 1][g] = oim[i];
+    }
+  }
+  __syncthreads();
+  const int64_t groups = ldk / 4;
+  const int64_t rows = 2 * lenb;
+  for (int x = threadIdx.x; x < 6 * 2 * kCtB * kW; x += 256) {
+    const int wd = x & (kW - 1);
+    const int r = (x / kW) % (2 * kCtB);
+    const int i = x / (kW * 2 * kCtB);
+    const int64_t row = 2 * b0 + r;
+    const int64_t g = a0 / 4 + wd;
+    if (row < rows && g < groups) cdig[(i * rows + row) * groups + g] = sm[i][r][wd];
+  }
+}
+
+// Maxima of the rows of H off the diagonal: colmax[I'] = max_(I != I')
+// |H[I'][I]| (hcol[I][I']).
 __global__ void __launch_bounds__(256)
 k_hbb_colmax(int64_t lenb, const double* __restrict__ hcol,
              double* __restrict__ colmax) {
   const int64_t c = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   if (c >= lenb) return;
   double m = 0.0;
-  for (int64_t k = 0; k < lenb; ++k) m = fmax(m, fabs(hcol[k * lenb + c]));
+  for (int64_t k = 0; k < lenb; ++k)
+    if (k != c) m = fmax(m, fabs(hcol[k * lenb + c]));
   colmax[c] = m;
 }
 
 // Hbb digits: thread -> column Ib'; five exact balanced digits of every K
 // value's integer z (as for A' in the alpha rows), packed four K values per
 // word; then the column's scale 2^-eh and offset correction
-// 128 (1 + 2^8 + 2^16 + 2^24 + 2^32) sum_K z.
+// 128 (1 + 2^8 + 2^16 + 2^24 + 2^32) sum_K z.  The diagonal is taken out
+// (hdiag, added in FP64 by the GEMM): it is tens of times the other elements
+// of its row, and would set the scale they are rounded with (norb 14 7a7b:
+// 3.0e-11 normwise with it in the digits).
 __global__ void __launch_bounds__(256)
 k_hbb_digits(int64_t lenb, int64_t ldk, const double* __restrict__ hcol,
              const double* colmax, uint32_t* __restrict__ hdig,
-             double* __restrict__ hscale, double* hcorr) {
+             double* __restrict__ hscale, double* hcorr,
+             double* __restrict__ hdiag) {
   const int64_t c = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   if (c >= lenb) return;
   int eh = 0;
@@ -807,8 +718,8 @@ k_hbb_digits(int64_t lenb, int64_t ldk, const double* __restrict__ hcol,
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int64_t k = 4 * g + u;
-      int64_t z = k < lenb ? static_cast<int64_t>(rint(ldexp(hcol[k * lenb + c], eh)))
-                           : 0;
+      int64_t z = k < lenb && k != c
+                      ? static_cast<int64_t>(rint(ldexp(hcol[k * lenb + c], eh))) : 0;
       zsum += static_cast<double>(z);
 #pragma unroll
       for (int t = 4; t >= 0; --t) {
@@ -823,6 +734,7 @@ k_hbb_digits(int64_t lenb, int64_t ldk, const double* __restrict__ hcol,
   const double corr = kOffsetUnit * zsum;
   hscale[c] = ldexp(1.0, -eh);
   hcorr[c] = corr;
+  hdiag[c] = hcol[c * lenb + c];
 }
 
 // GEMM tile: 128 M rows (64 alpha strings, real and imaginary rows) x 64
@@ -854,13 +766,18 @@ __device__ __forceinline__ int bd_off(int row, int chunk) {
 
 typedef __attribute__((address_space(3))) void lds_void_t;
 
+// TRANS: the left factor is C^T (lena, lenb exchanged by the caller), and the
+// result is added to out at the transposed place.
+template <bool TRANS>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_beta_gemm_oz(int64_t lena, int64_t lenb, int64_t ldk,
                   const uint8_t* __restrict__ cdig,
                   const double* __restrict__ cscale,
                   const uint8_t* __restrict__ hdig,
                   const double* __restrict__ hscale,
-                  const double* __restrict__ hcorr, double* __restrict__ out,
+                  const double* __restrict__ hcorr,
+                  const double* __restrict__ hdiag,
+                  const double* __restrict__ coeff, double* __restrict__ out,
                   const int32_t* __restrict__ done, int tm, int tn,
                   int per_xcd) {
   // two buffers as two arrays: the compiler can tell the loads into one
@@ -983,6 +900,7 @@ k_beta_gemm_oz(int64_t lena, int64_t lenb, int64_t ldk,
       if (col >= lenb) continue;
       const double hs = hscale[col];
       const double hc = hcorr[col];
+      const double hd = hdiag[col];
 #pragma unroll
       for (int e = 0; e < 4; e += 2) {
         const int64_t row = m0 + wm + 16 * x + 4 * (lane >> 4) + e;
@@ -998,8 +916,13 @@ k_beta_gemm_oz(int64_t lena, int64_t lenb, int64_t ldk,
           v[c] = fma(t, 4294967296.0, hc) * hs;
         }
         const double cs = cscale[ia];
-        *reinterpret_cast<double2*>(out + (ia * lenb + col) * 2) =
-            make_double2(v[0] * cs, v[1] * cs);
+        const int64_t at = TRANS ? col * lena + ia : ia * lenb + col;
+        const double2 x0 = reinterpret_cast<const double2*>(coeff)[at];
+        double2* dst = reinterpret_cast<double2*>(out) + at;
+        double2 o = TRANS ? *dst : make_double2(0.0, 0.0);
+        o.x += fma(v[0], cs, hd * x0.x);
+        o.y += fma(v[1], cs, hd * x0.y);
+        *dst = o;
       }
     }
 }
@@ -1021,6 +944,26 @@ bool beta_oz_shape_ok(int64_t lena, int64_t lenb) {
          5 * lenb * beta_oz_ldk(lenb) < lim;
 }
 
+namespace {
+
+// The GEMM of the digits of len_m data rows with those of H (len_n x len_n).
+template <bool TRANS>
+void digit_gemm(int64_t len_m, int64_t len_n, const uint8_t* cdig,
+                const double* cscale, const void* hoz, const double* coeff,
+                double* out, hipStream_t st, const int32_t* done) {
+  const int64_t ldk = beta_oz_ldk(len_n);
+  const uint8_t* hdig = static_cast<const uint8_t*>(hoz);
+  const double* hscale = reinterpret_cast<const double*>(hdig + 5 * len_n * ldk);
+  const int tm = static_cast<int>((2 * len_m + kBgTM - 1) / kBgTM);
+  const int tn = static_cast<int>((len_n + kBgTN - 1) / kBgTN);
+  const int per_xcd = (tm * tn + kBgXcds - 1) / kBgXcds;
+  k_beta_gemm_oz<TRANS><<<static_cast<unsigned>(per_xcd * kBgXcds), 512, 0, st>>>(
+      len_m, len_n, ldk, cdig, cscale, hdig, hscale, hscale + len_n,
+      hscale + 2 * len_n, coeff, out, done, tm, tn, per_xcd);
+}
+
+}  // namespace
+
 int launch_beta_gemm_oz(int64_t lena, int64_t lenb, const void* hoz,
                         const double* coeff, const double* rowmax,
                         void* cwork, double* out, hipStream_t st,
@@ -1029,30 +972,48 @@ int launch_beta_gemm_oz(int64_t lena, int64_t lenb, const void* hoz,
   const int64_t ldk = beta_oz_ldk(lenb);
   uint8_t* cdig = static_cast<uint8_t*>(cwork);
   double* cscale = reinterpret_cast<double*>(cdig + 6 * 2 * lena * ldk);
-  const uint8_t* hdig = static_cast<const uint8_t*>(hoz);
-  const double* hscale = reinterpret_cast<const double*>(hdig + 5 * lenb * ldk);
-  const double* hcorr = hscale + lenb;
   const int64_t nthr = lena * (ldk / 4);
   k_c_digits<<<blocks_for(nthr, 256), 256, 0, st>>>(
       lena, lenb, ldk, coeff, rowmax, reinterpret_cast<uint32_t*>(cdig), cscale,
       done);
   FQEHIP_CHECK_LAUNCH("k_c_digits");
-  const int tm = static_cast<int>((2 * lena + kBgTM - 1) / kBgTM);
-  const int tn = static_cast<int>((lenb + kBgTN - 1) / kBgTN);
-  const int per_xcd = (tm * tn + kBgXcds - 1) / kBgXcds;
-  k_beta_gemm_oz<<<static_cast<unsigned>(per_xcd * kBgXcds), 512, 0, st>>>(
-      lena, lenb, ldk, cdig, cscale, hdig, hscale, hcorr, out, done, tm, tn,
-      per_xcd);
+  digit_gemm<false>(lena, lenb, cdig, cscale, hoz, coeff, out, st, done);
   FQEHIP_CHECK_LAUNCH("k_beta_gemm_oz");
   return FQEHIP_OK;
 }
 
-int launch_row_absmax(int64_t lena, int64_t lenb, const double* coeff,
-                      double* rowmax, hipStream_t st, const int32_t* done) {
+// out += Haa C, on the digits of C^T (in cwork, beta_oz_workspace_bytes(lenb,
+// lena) bytes); colmax: the column maxima of |C|.
+int launch_alpha_gemm_oz(int64_t lena, int64_t lenb, const void* hoz,
+                         const double* coeff, const double* colmax, void* cwork,
+                         double* out, hipStream_t st, const int32_t* done) {
+  if (lena == 0 || lenb == 0) return FQEHIP_OK;
+  const int64_t ldk = beta_oz_ldk(lena);
+  uint8_t* cdig = static_cast<uint8_t*>(cwork);
+  double* cscale = reinterpret_cast<double*>(cdig + 6 * 2 * lenb * ldk);
+  // every word of the ldk bytes of a row is written: the grid covers ldk / 64
+  const dim3 grid(blocks_for(lenb, kCtB), static_cast<unsigned>(ldk / kCtA));
+  k_ct_digits<<<grid, 256, 0, st>>>(lena, lenb, ldk, coeff, colmax,
+                                    reinterpret_cast<uint32_t*>(cdig), cscale, done);
+  FQEHIP_CHECK_LAUNCH("k_ct_digits");
+  digit_gemm<true>(lenb, lena, cdig, cscale, hoz, coeff, out, st, done);
+  FQEHIP_CHECK_LAUNCH("k_beta_gemm_oz");
+  return FQEHIP_OK;
+}
+
+// Row maxima of |C|, and with colmax its column maxima.
+int launch_absmax(int64_t lena, int64_t lenb, const double* coeff,
+                  double* rowmax, double* colmax, hipStream_t st,
+                  const int32_t* done) {
   if (lena == 0 || lenb == 0) return FQEHIP_OK;
   const unsigned grid = static_cast<unsigned>(lena < 65536 ? lena : 65536);
-  k_row_absmax<<<grid, 256, 0, st>>>(lena, lenb, coeff, rowmax, done);
+  unsigned long long* cm = reinterpret_cast<unsigned long long*>(colmax);
+  k_row_absmax<<<grid, 256, 0, st>>>(lena, lenb, coeff, rowmax, cm, done);
   FQEHIP_CHECK_LAUNCH("k_row_absmax");
+  if (!colmax) return FQEHIP_OK;
+  const dim3 cgrid(blocks_for(lenb, 256), blocks_for(lena, kColRows));
+  k_col_absmax<<<cgrid, 256, 0, st>>>(lena, lenb, coeff, cm, done);
+  FQEHIP_CHECK_LAUNCH("k_col_absmax");
   return FQEHIP_OK;
 }
 
@@ -1062,7 +1023,7 @@ using namespace fqehip;
 
 extern "C" int64_t fqehip_beta_block_digits_bytes(int64_t lenb) {
   if (lenb < 0) return -1;
-  return 5 * lenb * beta_oz_ldk(lenb) + 16 * lenb;
+  return 5 * lenb * beta_oz_ldk(lenb) + 24 * lenb;
 }
 
 extern "C" int fqehip_beta_block_digits(int64_t lenb, const double* d_hcol,
@@ -1082,7 +1043,8 @@ extern "C" int fqehip_beta_block_digits(int64_t lenb, const double* d_hcol,
   k_hbb_colmax<<<blocks_for(lenb, 256), 256, 0, st>>>(lenb, d_hcol, hcorr);
   FQEHIP_CHECK_LAUNCH("k_hbb_colmax");
   k_hbb_digits<<<blocks_for(lenb, 256), 256, 0, st>>>(lenb, ldk, d_hcol, hcorr,
-                                                      hdig, hscale, hcorr);
+                                                      hdig, hscale, hcorr,
+                                                      hcorr + lenb);
   FQEHIP_CHECK_LAUNCH("k_hbb_digits");
   return FQEHIP_OK;
 }
@@ -1098,11 +1060,30 @@ extern "C" int fqehip_beta_gemm_digits(int64_t lena, int64_t lenb,
   FQEHIP_CHECK_ARG(beta_oz_shape_ok(lena, lenb), "sector too large");
   hipStream_t st = as_stream(stream);
   double* rowmax = static_cast<double*>(d_work);
-  int rc = launch_row_absmax(lena, lenb, static_cast<const double*>(d_coeff),
-                             rowmax, st, d_done);
+  int rc = launch_absmax(lena, lenb, static_cast<const double*>(d_coeff),
+                         rowmax, nullptr, st, d_done);
   if (rc) return rc;
   return launch_beta_gemm_oz(lena, lenb, d_hoz,
                              static_cast<const double*>(d_coeff), rowmax,
                              rowmax + lena, static_cast<double*>(d_out), st,
                              d_done);
+}
+
+extern "C" int64_t fqehip_pull_digits_bytes(int npull) {
+  if (npull < 0) return -1;
+  return npull * (kWDigBytes + static_cast<int64_t>(kOzQ) * 8) + 8;
+}
+
+extern "C" int fqehip_pull_digits(int npull, const double* d_w, void* d_woz,
+                                  void* stream) {
+  clear_error();
+  FQEHIP_CHECK_ARG(npull >= 0 && npull <= kOzQ, "npull=%d outside 0..%d", npull, kOzQ);
+  if (npull == 0) return FQEHIP_OK;
+  FQEHIP_CHECK_ARG(d_w && d_woz, "NULL pointer");
+  uint8_t* dig = static_cast<uint8_t*>(d_woz);
+  double* z = reinterpret_cast<double*>(dig + npull * kWDigBytes);
+  int32_t* ea = reinterpret_cast<int32_t*>(z + static_cast<int64_t>(npull) * kOzQ);
+  k_pull_digits<<<npull, kOzQ, 0, as_stream(stream)>>>(npull, d_w, dig, z, ea);
+  FQEHIP_CHECK_LAUNCH("k_pull_digits");
+  return FQEHIP_OK;
 }

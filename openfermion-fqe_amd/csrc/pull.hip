@@ -237,7 +237,7 @@ struct PullArgs {
   int ks, pass, copies;                    // k steps, passes, accumulator rows
   const double* w;                         // [p][q] (complex: interleaved)
   const int32_t* dexc;                     // [lena][nexc][3]
-  const uint32_t* fwd;                     // [nq][lenb] (fqehip_pull_table)
+  const uint32_t* fwd;                     // fqehip_pull_table
   const double* coeff;
   double* rowacc;
   // out != NULL: out = alpha (rowacc + row) + beta cin, acc += that value;
@@ -341,7 +341,7 @@ __global__ void __launch_bounds__(512, 2) k_pull_rows_f64(PullArgs p) {
   __syncthreads();
 
   const __amdgpu_buffer_rsrc_t rc = buffer_of(p.coeff, p.lena * p.lenb * 16);
-  const __amdgpu_buffer_rsrc_t rf = buffer_of(p.fwd, static_cast<int64_t>(p.nq) * lenb * 4);
+  const __amdgpu_buffer_rsrc_t rf = buffer_of(p.fwd, static_cast<int64_t>((p.nq + 15) & ~15) * lenb * 4);
   const __amdgpu_buffer_rsrc_t rw =
       buffer_of(p.w, static_cast<int64_t>(p.nq) * p.nq * (CPLX ? 16 : 8));
   const int ntile = (lenb + 15) >> 4;
@@ -412,13 +412,13 @@ __global__ void __launch_bounds__(512, 2) k_pull_rows_f64(PullArgs p) {
       const uint32_t o = column(tile);
       // target words, volatile so that the loads stay ahead of the products
       uint32_t fv[G][4];
+      const int fo = jb < lenb ? (kq * lenb + jb) * 4 : -1;
 #pragma unroll
       for (int t = 0; t < G; ++t)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const int q = q0 + 16 * t + kq + 4 * e;
           fv[t][e] = __builtin_amdgcn_raw_buffer_load_b32(
-              rf, (q < p.nq && jb < lenb) ? (q * lenb + jb) * 4 : -1, 0, kVolatile);
+              rf, fo, (q0 + 16 * t + 4 * e) * 4 * lenb, kVolatile);
         }
       double4_t zr[G], zi[G];
 #pragma unroll
@@ -538,10 +538,11 @@ __global__ void __launch_bounds__(512, 2) k_pull_rows_f64(PullArgs p) {
 // the sign; 0 where the excitation vanishes.  (word << 1) is the byte offset
 // of accumulator target + 1.
 __global__ void __launch_bounds__(256)
-k_pull_table(int64_t n, const int32_t* __restrict__ fwd, uint32_t* __restrict__ tab) {
+k_pull_table(int64_t n, int64_t padded, const int32_t* __restrict__ fwd,
+             uint32_t* __restrict__ tab) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (i >= n) return;
-  const int32_t f = fwd[i];
+  if (i >= padded) return;
+  const int32_t f = i < n ? fwd[i] : 0;
   tab[i] = static_cast<uint32_t>(iabs(f)) << 3 | (f < 0 ? 0x80000000u : 0u);
 }
 
@@ -610,7 +611,7 @@ bool pull_supported(const fqehip_sector* s) {
          s->nalpha * (s->norb - s->nalpha + 1) <= 64 && noff < kPullMaxK &&
          s->lena * s->lenb * 16 < kOffLimit && s->lena * s->lena * 16 < kOffLimit &&
          s->lenb * s->lenb * 16 < kOffLimit &&
-         static_cast<int64_t>(s->npull) * s->lenb * 4 < kOffLimit &&
+         static_cast<int64_t>(s->npull + 15) * s->lenb * 4 < kOffLimit &&
          pull_plan(true, noff, s->lenb, s->npull, &pl);
 }
 
@@ -687,9 +688,11 @@ extern "C" int fqehip_pull_table(int npair, int64_t len, const int32_t* d_fwd,
   FQEHIP_CHECK_ARG(npair >= 0 && len >= 0 && len < (1 << 27), "npair=%d len=%lld",
                    npair, static_cast<long long>(len));
   const int64_t n = npair * len;
+  const int64_t padded = (npair + 15) / 16 * 16 * len;
   if (n == 0) return FQEHIP_OK;
   FQEHIP_CHECK_ARG(d_fwd && d_tab, "NULL pointer");
-  k_pull_table<<<blocks_for(n, 256), 256, 0, as_stream(stream)>>>(n, d_fwd, d_tab);
+  k_pull_table<<<blocks_for(padded, 256), 256, 0, as_stream(stream)>>>(n, padded, d_fwd,
+                                                                       d_tab);
   FQEHIP_CHECK_LAUNCH("k_pull_table");
   return FQEHIP_OK;
 }

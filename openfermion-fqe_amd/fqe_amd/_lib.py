@@ -44,7 +44,8 @@ class Sector(ctypes.Structure):
                 ("hbb_hi", c_void_p), ("hbb_lo", c_void_p), ("ldh", c_int64),
                 ("tile", c_int), ("hbb_f64", c_void_p), ("hbb_oz", c_void_p),
                 ("dexc_a", c_void_p), ("pull_w", c_void_p), ("haa", c_void_p),
-                ("hbb", c_void_p), ("pull_fwd", c_void_p), ("npull", c_int)]
+                ("hbb", c_void_p), ("pull_fwd", c_void_p), ("npull", c_int),
+                ("w_oz", c_void_p), ("haa_oz", c_void_p)]
 
 
 class Operator(ctypes.Structure):
@@ -104,6 +105,8 @@ _SIGNATURES = {
                                   c_int64, c_void_p, c_void_p, c_void_p]),
     "fqehip_pull_table": (c_int, [c_int, c_int64, c_void_p, c_void_p,
                                   c_void_p]),
+    "fqehip_pull_digits_bytes": (c_int64, [c_int]),
+    "fqehip_pull_digits": (c_int, [c_int, c_void_p, c_void_p, c_void_p]),
     "fqehip_pull_supported": (c_int, [c_int, POINTER(Sector),
                                       POINTER(Operator)]),
     "fqehip_batch_create": (c_int, [c_int, c_int, POINTER(BatchItem), c_double,

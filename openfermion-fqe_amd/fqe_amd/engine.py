@@ -48,7 +48,6 @@ class PreparedOperator:
         self.coupling: Optional[torch.Tensor] = None
         self._pull = {}
         self._hbb = {}
-        self._hoz = {}
 
     def beta_block(self, graph):
         """Beta-beta block of this operator on the beta strings of
@@ -75,23 +74,39 @@ class PreparedOperator:
             self._hbb[key] = (hhi, hlo, ldh, fwb, hcol)
         return self._hbb[key]
 
-    def beta_block_digits(self, graph):
-        """Ozaki digits of the FP64 beta-beta block (int8 digit planes,
-        column scales and offset corrections; fqehip_beta_block_digits),
-        cached per (nbeta, device); None when the block does not apply."""
-        blk = self.beta_block(graph)
-        if blk is None:
+    def pull_digits(self, graph):
+        """Digits of the pull form (W, Haa, Hbb; fqehip_pull_digits and
+        fqehip_beta_block_digits) on the sector of ``graph``, cached per
+        (electron count, device); None where the digit kernels do not
+        apply."""
+        tabs = self.pull_tables(graph)
+        if (tabs is None or self.complex_op or self.spin
+                or not self.pair_symmetric or self.coupling.shape[0] > 128
+                or max(graph.lena(), graph.lenb()) >= 26214):
             return None
-        key = (graph.nbeta(), self.a.device.index)
-        if key not in self._hoz:
-            lenb = graph.lenb()
-            nbytes = int(_lib.call("fqehip_beta_block_digits_bytes", lenb))
-            hoz = torch.empty(max(nbytes, 16), dtype=torch.uint8,
-                              device=self.a.device)
-            _lib.call("fqehip_beta_block_digits", lenb, _lib.ptr(blk[4]),
-                      _lib.ptr(hoz), _lib.stream_ptr())
-            self._hoz[key] = hoz
-        return self._hoz[key]
+        dev = self.a.device
+        if "w_oz" not in self._pull:
+            npull = self.coupling.shape[0]
+            woz = torch.empty(int(_lib.call("fqehip_pull_digits_bytes",
+                                            npull)),
+                              dtype=torch.uint8, device=dev)
+            _lib.call("fqehip_pull_digits", npull, _lib.ptr(self.coupling),
+                      _lib.ptr(woz), _lib.stream_ptr())
+            self._pull["w_oz"] = woz
+        out = [self._pull["w_oz"]]
+        for nele, block in ((graph.nalpha(), tabs[1]),
+                            (graph.nbeta(), tabs[2])):
+            key = ("digits", nele, dev.index)
+            if key not in self._pull:
+                n = block.shape[0]
+                nbytes = int(_lib.call("fqehip_beta_block_digits_bytes", n))
+                hoz = torch.empty(max(nbytes, 16), dtype=torch.uint8,
+                                  device=dev)
+                _lib.call("fqehip_beta_block_digits", n, _lib.ptr(block),
+                          _lib.ptr(hoz), _lib.stream_ptr())
+                self._pull[key] = hoz
+            out.append(self._pull[key])
+        return out
 
     def _spin_block(self, tables, alpha: bool) -> torch.Tensor:
         """Matrix of this two-body operator on the strings of one spin, by
@@ -331,8 +346,9 @@ def sector_struct(graph, op: PreparedOperator,
                    settings.split_tile_fp64 == _lib.TILE_SPLIT_F64_DTILE) else 128
     pull = None
     if (settings.fused and settings.split_fp64 and op.h1 is None
-            and settings.split_tile_fp64 is None and precision == _lib.C128
-            and settings.contraction == "fp64"):
+            and precision == _lib.C128
+            and (settings.split_tile_fp64 is None
+                 or settings.contraction == "ozaki")):
         pull = op.pull_tables(graph)
     if (fwa is not None and settings.split_fp64 and precision == _lib.C128
             and op.npair + 1 <= kmax and graph.norb() ** 2 // 4 + 1 <= 64):
@@ -355,11 +371,15 @@ def sector_struct(graph, op: PreparedOperator,
         s.hbb_f64 = _lib.ptr(hbb64)
         if settings.contraction == "ozaki":
             s.tile = _lib.TILE_OZAKI
-            if settings.ozaki_beta and graph.lenb() < 26214:
-                hoz = op.beta_block_digits(graph)
-                if hoz is not None:
-                    keep.append(hoz)
-                    s.hbb_oz = _lib.ptr(hoz)
+            digits = None
+            if s.lena * s.lenb >= settings.ozaki_min_determinants:
+                digits = op.pull_digits(graph)
+            if digits is not None:
+                keep += digits
+                s.w_oz = _lib.ptr(digits[0])
+                if settings.ozaki_beta:
+                    s.haa_oz = _lib.ptr(digits[1])
+                    s.hbb_oz = _lib.ptr(digits[2])
         elif settings.contraction == "fp64":
             s.tile = int(settings.split_tile_fp64 or 0)
         else:
@@ -381,15 +401,8 @@ def workspace(sector: _lib.Sector, precision: int,
     elem = 8 if precision == _lib.C128 else 4
     n = sector.lena * sector.lenb
     fused = (sector.nslot + 1) * 2 * n * elem
-    if sector.tile == _lib.TILE_OZAKI and sector.hbb_f64:
-        fused += 512 * sector.lenb        # beta gather table
-        fused += 128 * (5 * 128 + 12)     # pair rows' digits
-        fused += 8 * sector.lena          # row maxima of |C|
-        if sector.hbb_oz:                 # C digit planes and row scales
-            ldk = (sector.lenb + 63) // 64 * 64
-            fused += 6 * 2 * sector.lena * ldk + 8 * sector.lena
     need = max((2 * sector.npair + 1) * 2 * n * elem, fused)
-    if nbytes != need and not (sector.pull_w and nbytes == 16 * n):
+    if nbytes != need and not (sector.pull_w and nbytes >= 16 * n):
         raise _lib.FqeHipError(f"workspace size {nbytes} != {need}")
     nbytes = max(nbytes, 16 * sector.lena * sector.lenb, 16)
     return torch.empty(nbytes, dtype=torch.uint8, device=device)

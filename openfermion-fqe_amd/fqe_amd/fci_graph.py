@@ -89,12 +89,13 @@ class SpinTables:
         return self._ptab[key]
 
     def pull_table(self, compressed: bool) -> torch.Tensor:
-        """Target words of the pull form (fqehip_pull_table), int32
-        [npair][length]."""
+        """Target words of the pull form (fqehip_pull_table), int32 [npair
+        rounded up to 16][length]."""
         key = ("pull", bool(compressed))
         if key not in self._ptab:
             fwd, _ = self.fused_tables(compressed)
-            tab = torch.empty_like(fwd)
+            tab = torch.empty(((fwd.shape[0] + 15) // 16 * 16, self.length),
+                              dtype=torch.int32, device=self.device)
             if fwd.numel():
                 _lib.call("fqehip_pull_table", fwd.shape[0], self.length,
                           _lib.ptr(fwd), _lib.ptr(tab), _lib.stream_ptr())

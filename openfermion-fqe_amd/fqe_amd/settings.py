@@ -47,13 +47,20 @@ split_tile = 0
 # shared, double-buffered D tile, other operators on the unfused kernels.
 split_tile_fp64 = None
 
-# Arithmetic of the complex128 split row pass: "fp64" (FP64 matrix cores)
-# or "ozaki" (exact int8 digit products, FP64 assembly).
+# Arithmetic of complex128 applies of pair-symmetric real operators: "fp64"
+# (FP64 matrix cores) or "ozaki" (exact int8 digit products, FP64 assembly).
 contraction = "fp64"
 
-# With contraction = "ozaki": the beta-beta GEMM as digit products too
-# (else FP64 matrix cores for that half).
+# With contraction = "ozaki": the same-spin products as digit products too
+# (else FP64 matrix cores for those).
 ozaki_beta = True
+
+# With contraction = "ozaki": sectors below this many determinants run in
+# FP64, where the digit kernels' extra launches (maxima, digits) cost more
+# than the faster products save.  Measured, FP64 / digits: norb 11 5a6b
+# (213,444) 110 / 139 us, norb 12 4a6b (457,380) 207 / 202 us, norb 12 6a6b
+# (853,776) 383 / 314 us.
+ozaki_min_determinants = 400000
 
 # Largest apply workspace (bytes) allocated at once: a complex128 sector
 # whose unfused dvec + Y would need more runs the apply in panels of

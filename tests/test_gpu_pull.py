@@ -137,3 +137,44 @@ def test_pull_matches_other_kernels(fqe, kind, na, nb, norb):
     finally:
         settings.split_tile_fp64 = saved
     assert rel(e.coeff, d.coeff) < TOL
+
+
+@pytest.mark.parametrize("shape", ["synthetic", "constant"])
+@pytest.mark.parametrize("blocks", [True, False])
+@pytest.mark.parametrize("na,nb,norb", [(1, 1, 2), (1, 2, 3), (3, 2, 5),
+                                        (6, 1, 6), (4, 4, 8), (3, 7, 9),
+                                        (8, 5, 9), (6, 6, 11), (8, 2, 15)])
+def test_digit_rows_edges(fqe, na, nb, norb, blocks, shape):
+    """The digit kernels on every sector (ozaki_min_determinants = 0):
+    fewer than 64 columns or strings, ragged tiles, 3 to 120 pairs, 2 to 64
+    de-excitation rows; and the largest possible sums (every integral and
+    every coefficient equal).  Tolerance 3e-11 normwise: operator rounding
+    2^-39 and data rounding 2^-47 of the largest element, dropped digit
+    pairs below both, times the spread between the largest element and the
+    norm of a row (up to some hundreds here).  Integer sums: the same bits
+    on every run."""
+    from fqe_amd import settings
+    print(f"digit rows {na} {nb} {norb} {blocks} {shape}", flush=True)
+    d, c, g, rng = sector(fqe, na, nb, norb, 11 * norb + 5 * na + nb)
+    h = tensors("real", norb, rng)
+    if shape == "constant":
+        h = (numpy.full_like(h[0], 0.3), numpy.full_like(h[1], -0.3))
+        c = numpy.full_like(c, 1 + 1j) / numpy.sqrt(2.0 * c.size)
+        d.coeff = c
+    op = prepared(fqe, "real", h, norb)
+    saved = (settings.contraction, settings.ozaki_beta,
+             settings.ozaki_min_determinants)
+    settings.contraction, settings.ozaki_beta = "ozaki", blocks
+    settings.ozaki_min_determinants = 0
+    outs = []
+    try:
+        for _ in range(2):
+            e = copy.deepcopy(d)
+            e.apply_inplace_scaled(h, op=op)
+            outs.append(e.coeff)
+    finally:
+        (settings.contraction, settings.ozaki_beta,
+         settings.ozaki_min_determinants) = saved
+    d.apply_inplace_scaled(h, op=op)
+    assert rel(outs[0], d.coeff) < 3e-11
+    assert numpy.array_equal(outs[0], outs[1])
