@@ -575,7 +575,9 @@ typedef struct fqehip_batch fqehip_batch;
  * hbb_f64 NULL, tile not FQEHIP_TILE_OZAKI) run as one group: per Taylor
  * step one row launch and one reduction cover all of them (complex64: the
  * rows4 row body; complex128: the FP64 row body), instead of kernels per
- * sector; the other sectors keep their own kernels on the other branches. */
+ * sector, and so do the small real pull-form sectors (not counted by
+ * fqehip_batch_grouped) with two launches per step for each kernel shape;
+ * the other sectors keep their own kernels on the other branches. */
 int fqehip_batch_create(int precision, int nitems,
                         const fqehip_batch_item* items, double time,
                         int nterms, int nstreams, int group, void* stream,

@@ -5,8 +5,10 @@
 // (longest-processing-time order, each to the least-loaded stream) so the
 // graph has parallel branches: small sectors, which cannot fill the GPU
 // alone, run side by side.  Each sector keeps its own kernel variant (the
-// tile choice of its descriptor, picked by the host autotuner).
+// tile choice of its descriptor, picked by the host autotuner); the small
+// pull-form sectors of one kernel shape share their launches.
 #include "fqehip_common.h"
+#include "pull_common.h"
 
 #include <algorithm>
 #include <new>
@@ -19,6 +21,7 @@ struct fqehip_batch {
   std::vector<hipStream_t> streams;
   std::vector<hipEvent_t> events;
   fqehip::GroupSector* d_group = nullptr;   // grouped sectors (device)
+  std::vector<void*> d_pull;                // pull-form groups (device)
   int ngroup = 0;
   int nodes = 0;
 };
@@ -52,9 +55,66 @@ void release(fqehip_batch* b) {
   if (b->exec) (void)hipGraphExecDestroy(b->exec);
   if (b->graph) (void)hipGraphDestroy(b->graph);
   if (b->d_group) (void)hipFree(b->d_group);
+  for (void* d : b->d_pull) (void)hipFree(d);
   for (hipEvent_t e : b->events) (void)hipEventDestroy(e);
   for (hipStream_t s : b->streams) (void)hipStreamDestroy(s);
   delete b;
+}
+
+// A pull-form sector of its own (digit rows, large or complex sectors): the
+// terms alternate between d_term and the workspace's second buffer, starting
+// from d_coeff0, so the row kernel's epilogue does the whole step.
+int enqueue_pull_item(const fqehip_batch_item& it, double time, int nterms,
+                      hipStream_t st, int* nodes) {
+  void* sv = reinterpret_cast<void*>(st);
+  int rc = fqehip_convert_to_c128(FQEHIP_C128, it.sector.lena * it.sector.lenb,
+                                  it.d_coeff0, 1.0, 0.0, it.d_result, sv);
+  if (rc) return rc;
+  *nodes += 1;
+  if (it.d_apply_out) {
+    rc = fqehip_apply(FQEHIP_C128, &it.sector, &it.op, it.d_coeff0, 1.0, 0.0, 0.0,
+                      0.0, nullptr, it.d_apply_out, nullptr, nullptr, nullptr,
+                      it.d_workspace, sv);
+    if (rc) return rc;
+    *nodes += 2;
+  }
+  void* term[2] = {it.d_term,
+                   static_cast<char*>(it.d_workspace) + pull_spare_offset(&it.sector)};
+  const void* src = it.d_coeff0;
+  for (int k = 1; k <= nterms; ++k) {
+    void* dst = term[(k + 1) & 1];
+    rc = fqehip_apply(FQEHIP_C128, &it.sector, &it.op, src, 0.0,
+                      -time / static_cast<double>(k), 0.0, 0.0, nullptr, dst,
+                      it.d_result, nullptr, nullptr, it.d_workspace, sv);
+    if (rc) return rc;
+    *nodes += 2;
+    src = dst;
+  }
+  return FQEHIP_OK;
+}
+
+// A group of small pull-form sectors of one class on stream st: two launches
+// per step for all of them.
+int enqueue_pull_group(const fqehip_batch_item* items,
+                       const std::vector<int>& members,
+                       const PullGroupLaunch& g, const void* d_secs, double time,
+                       int nterms, hipStream_t st, int* nodes) {
+  if (nterms == 0)
+    for (int i : members) {
+      const fqehip_batch_item& it = items[i];
+      int rc = fqehip_convert_to_c128(FQEHIP_C128, it.sector.lena * it.sector.lenb,
+                                      it.d_coeff0, 1.0, 0.0, it.d_result,
+                                      reinterpret_cast<void*>(st));
+      if (rc) return rc;
+      *nodes += 1;
+    }
+  for (int step = g.any_apply ? 0 : 1; step <= nterms; ++step) {
+    int rc = launch_pull_group(g, d_secs, step, 0.0,
+                               step ? -time / static_cast<double>(step) : 0.0, st);
+    if (rc) return rc;
+    *nodes += 2;
+  }
+  return FQEHIP_OK;
 }
 
 // The work of one item on stream st (see the file comment).
@@ -63,6 +123,8 @@ int enqueue_item(int precision, const fqehip_batch_item& it, double time,
   const int64_t n = it.sector.lena * it.sector.lenb;
   if (n == 0) return FQEHIP_OK;
   void* sv = reinterpret_cast<void*>(st);
+  if (precision == FQEHIP_C128 && fqehip_pull_supported(precision, &it.sector, &it.op))
+    return enqueue_pull_item(it, time, nterms, st, nodes);
   if (hipMemcpyAsync(it.d_term, it.d_coeff0, n * esize(precision),
                      hipMemcpyDeviceToDevice, st) != hipSuccess) {
     set_error("batch: copy of the initial term failed");
@@ -185,8 +247,19 @@ extern "C" int fqehip_batch_create(int precision, int nitems,
   // complex128 k_fused_f64) run as one group: one row launch and one
   // reduction per step for all of them
   std::vector<int> grouped, single;
+  // small real pull-form sectors: one group per class
+  std::vector<std::vector<int>> pull(8);
   for (int i = 0; i < nitems; ++i) {
     const fqehip_batch_item& it = items[i];
+    if (group && it.sector.lena * it.sector.lenb > 0 && !it.op.complex_op &&
+        fqehip_pull_supported(precision, &it.sector, &it.op) &&
+        !digit_rows(&it.sector)) {
+      const int c = pull_group_class(&it.sector);
+      if (c > 0 && c < 8) {
+        pull[c].push_back(i);
+        continue;
+      }
+    }
     const bool g = group && it.sector.lena * it.sector.lenb > 0 &&
                    !it.sector.hbb_hi && !it.sector.hbb_f64 &&
                    it.sector.tile != FQEHIP_TILE_OZAKI &&
@@ -248,15 +321,52 @@ extern "C" int fqehip_batch_create(int precision, int nitems,
     }
     b->ngroup = static_cast<int>(grouped.size());
   }
+  std::vector<PullGroupLaunch> pgl(8);
+  std::vector<const void*> pgd(8, nullptr);
+  for (int c = 1; c < 8; ++c) {
+    if (pull[c].empty()) continue;
+    const int nsec = static_cast<int>(pull[c].size());
+    std::vector<char> host(pull_group_bytes(nsec));
+    std::vector<const fqehip_batch_item*> its;
+    std::vector<int64_t> spare;
+    for (int i : pull[c]) {
+      its.push_back(&items[i]);
+      spare.push_back(pull_spare_offset(&items[i].sector));
+    }
+    int rc = pull_group_fill(its.data(), spare.data(), nsec, host.data(), &pgl[c]);
+    void* d = nullptr;
+    if (rc == FQEHIP_OK && hipMalloc(&d, host.size()) != hipSuccess) {
+      set_error("batch: group descriptor allocation failed");
+      rc = FQEHIP_ERR_OOM;
+    }
+    if (d) b->d_pull.push_back(d);
+    if (rc == FQEHIP_OK && hipMemcpy(d, host.data(), host.size(),
+                                     hipMemcpyHostToDevice) != hipSuccess) {
+      set_error("batch: group descriptor upload failed");
+      rc = FQEHIP_ERR_HIP;
+    }
+    if (rc != FQEHIP_OK) {
+      release(b);
+      return rc;
+    }
+    pgd[c] = d;
+  }
   // longest processing time first, each to the least-loaded stream (the
-  // group occupies stream 0)
+  // group occupies stream 0, the pull groups the least-loaded ones after it)
   std::vector<int> order(single);
   std::sort(order.begin(), order.end(), [&](int x, int y) {
     return item_work(items[x]) > item_work(items[y]);
   });
   std::vector<double> load(nb, 0.0);
   load[0] = gwork;
-  std::vector<std::vector<int>> plan(nb);
+  std::vector<std::vector<int>> plan(nb), pplan(nb);
+  for (int c = 7; c >= 1; --c) {
+    if (pull[c].empty()) continue;
+    const int s = static_cast<int>(
+        std::min_element(load.begin(), load.end()) - load.begin());
+    pplan[s].push_back(c);
+    for (int i : pull[c]) load[s] += item_work(items[i]);
+  }
   for (int i : order) {
     const int s = static_cast<int>(
         std::min_element(load.begin(), load.end()) - load.begin());
@@ -278,6 +388,12 @@ extern "C" int fqehip_batch_create(int precision, int nitems,
     rc = enqueue_group(precision, items, grouped, b->d_group, grows, gblocks,
                        gmax_lenb, gapply, time, nterms, b->streams[0],
                        &b->nodes);
+  for (int s = 0; s < nb && rc == FQEHIP_OK; ++s)
+    for (int c : pplan[s]) {
+      rc = enqueue_pull_group(items, pull[c], pgl[c], pgd[c], time, nterms,
+                              b->streams[s], &b->nodes);
+      if (rc) break;
+    }
   for (int s = 0; s < nb && rc == FQEHIP_OK; ++s)
     for (int i : plan[s]) {
       rc = enqueue_item(precision, items[i], time, nterms, b->streams[s],

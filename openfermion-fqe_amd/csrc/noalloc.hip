@@ -15,6 +15,7 @@
 #include <mutex>
 
 #include "fqehip_common.h"
+#include "pull_common.h"
 
 namespace {
 
@@ -38,7 +39,7 @@ int64_t needed_bytes(int precision, const fqehip_sector* s,
     // what the pull form needs beyond its row accumulators (the digit
     // kernels' maxima and planes)
     if (fqehip_pull_supported(precision, s, op))
-      b += fqehip_apply_workspace_bytes(precision, s) - 2 * n * elem;
+      b += fqehip::pull_spare_offset(s) - 2 * n * elem;
     return b;
   }
   return static_cast<int64_t>(2 * s->npair + 1) * 2 * n * elem;

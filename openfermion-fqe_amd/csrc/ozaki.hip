@@ -31,6 +31,7 @@
 // Reference: lm_apply_array12_same_spin_opt / lm_apply_array12_diff_spin_opt
 // (src/fqe/lib/fqe_data.c:668-720, :879-996), in complex128.
 #include "fqehip_common.h"
+#include "pull_common.h"
 #include "rows_common.h"
 
 namespace fqehip {
@@ -234,6 +235,7 @@ struct OzRowsArgs {
   const double* cin;
   double* out;
   double* acc;
+  double* partials;
   const int32_t* done;
 };
 
@@ -456,6 +458,7 @@ __global__ void __launch_bounds__(kRowThreads, 2) k_pull_rows_oz(OzRowsArgs p) {
   __syncthreads();
   const double back = ldexp(1.0, 32 - *p.ea - *scale);
   double2* racc = reinterpret_cast<double2*>(p.rowacc) + ia * p.lenb;
+  double sq = 0.0;
   for (int x = tid; x < lenb; x += kRowThreads) {
     const double2 r = racc[x];
     const double re = r.x + back * static_cast<double>(static_cast<int64_t>(accs[2 * x]));
@@ -473,11 +476,13 @@ __global__ void __launch_bounds__(kRowThreads, 2) k_pull_rows_oz(OzRowsArgs p) {
       vi += p.beta_re * c.y + p.beta_im * c.x;
     }
     reinterpret_cast<double2*>(p.out)[idx] = make_double2(vr, vi);
+    sq += vr * vr + vi * vi;
     if (p.acc) {
       p.acc[2 * idx] += vr;
       p.acc[2 * idx + 1] += vi;
     }
   }
+  if (p.partials) row_norm(sq, p.partials + ia, smem);
 }
 
 constexpr size_t kLdsLimit = 160 * 1024;
@@ -496,9 +501,8 @@ bool pull_oz_supported(const fqehip_sector* s) {
 
 // The opposite-spin rows on top of rowacc (epilogue as launch_pull_rows).
 int launch_pull_rows_oz(const fqehip_sector* s, const double* coeff,
-                        const double* rowmax, double* rowacc, double ar,
-                        double ai, double br, double bi, const double* cin,
-                        double* out, double* acc, hipStream_t st,
+                        const double* rowmax, double* rowacc,
+                        const PullEpilogue& e, hipStream_t st,
                         const int32_t* done) {
   OzRowsArgs p{};
   p.norb = s->norb;
@@ -516,13 +520,14 @@ int launch_pull_rows_oz(const fqehip_sector* s, const double* coeff,
   p.coeff = coeff;
   p.rowmax = rowmax;
   p.rowacc = rowacc;
-  p.alpha_re = ar;
-  p.alpha_im = ai;
-  p.beta_re = br;
-  p.beta_im = bi;
-  p.cin = cin;
-  p.out = out;
-  p.acc = acc;
+  p.alpha_re = e.alpha_re;
+  p.alpha_im = e.alpha_im;
+  p.beta_re = e.beta_re;
+  p.beta_im = e.beta_im;
+  p.cin = e.cin;
+  p.out = e.out;
+  p.acc = e.acc;
+  p.partials = e.partials;
   p.done = done;
   k_pull_rows_oz<<<static_cast<unsigned>(s->lena), kRowThreads,
                    oz_rows_lds_bytes(s->lenb, p.nqt), st>>>(p);

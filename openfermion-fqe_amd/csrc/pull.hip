@@ -30,6 +30,7 @@
 #include <type_traits>
 
 #include "fqehip_common.h"
+#include "pull_common.h"
 #include "rows_common.h"
 
 namespace fqehip {
@@ -86,15 +87,12 @@ __device__ __forceinline__ double load_d(__amdgpu_buffer_rsrc_t r, int off) {
 }
 
 template <bool CPLX, int RA, int RB>
-__global__ void __launch_bounds__(256, RA * RB > 4 || CPLX ? 2 : 4)
-k_same_spin_f64(int64_t lena, int64_t lenb, const double* __restrict__ ha,
-                const double* __restrict__ hb, const double* __restrict__ coeff,
-                double* __restrict__ out, const int32_t* __restrict__ done,
-                int ta, int tb) {
+__device__ __forceinline__ void same_spin_tile(
+    int t, int64_t lena, int64_t lenb, const double* __restrict__ ha,
+    const double* __restrict__ hb, const double* __restrict__ coeff,
+    double* __restrict__ out, int ta, int tb) {
   constexpr int D = kSpinDepth;
   constexpr int kH = CPLX ? 16 : 8;               // bytes per H element
-  if (done && *done) return;
-  const int t = static_cast<int>(xcd_order(blockIdx.x, ta * tb));
   // groups of 8 tile rows, so neighbouring workgroups share C and H rows
   const int grp = t / (8 * tb);
   const int left = ta - grp * 8;
@@ -213,6 +211,17 @@ k_same_spin_f64(int64_t lena, int64_t lenb, const double* __restrict__ ha,
 }
 
 template <bool CPLX, int RA, int RB>
+__global__ void __launch_bounds__(256, RA * RB > 4 || CPLX ? 2 : 4)
+k_same_spin_f64(int64_t lena, int64_t lenb, const double* __restrict__ ha,
+                const double* __restrict__ hb, const double* __restrict__ coeff,
+                double* __restrict__ out, const int32_t* __restrict__ done,
+                int ta, int tb) {
+  if (done && *done) return;
+  same_spin_tile<CPLX, RA, RB>(static_cast<int>(xcd_order(blockIdx.x, ta * tb)),
+                               lena, lenb, ha, hb, coeff, out, ta, tb);
+}
+
+template <bool CPLX, int RA, int RB>
 void same_spin(int64_t lena, int64_t lenb, const double* ha, const double* hb,
                const double* coeff, double* out, hipStream_t st,
                const int32_t* done) {
@@ -246,6 +255,8 @@ struct PullArgs {
   const double* cin;
   double* out;
   double* acc;
+  const double* acc0;                      // not NULL: acc = acc0 + that value
+  double* partials;                        // not NULL: [ia] = |out row|^2
   const int32_t* done;
 };
 
@@ -282,10 +293,9 @@ size_t pull_lds_bytes(bool cplx, int ks, int64_t lenb, int tiles, int copies) {
 // additions, 5.1 without their order.  norb 12 6a6b: 0.24 against 0.47 + 0.09;
 // complex operator, norb 11 4a6b: 0.14 against 1.23 for the unfused kernels.
 template <bool CPLX, int G>
-__global__ void __launch_bounds__(512, 2) k_pull_rows_f64(PullArgs p) {
+__device__ __forceinline__ void pull_row(const PullArgs& p, int64_t ia,
+                                         char* smem) {
   constexpr int kF = CPLX ? 128 : 64;      // doubles per W fragment
-  extern __shared__ __align__(16) char smem[];
-  if (p.done && *p.done) return;
   const int tid = threadIdx.x;
   const int nt = blockDim.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -295,7 +305,6 @@ __global__ void __launch_bounds__(512, 2) k_pull_rows_f64(PullArgs p) {
   const int cl = lane & 15;
   const int lenb = static_cast<int>(p.lenb);
   const int ks = p.ks;
-  const int64_t ia = xcd_order(blockIdx.x, p.lena);
   double2* accs = reinterpret_cast<double2*>(smem);    // [copies][lenb]
   double* wf = reinterpret_cast<double*>(accs + p.copies * lenb);   // [ks][G][kF]
   double* lsg = wf + G * ks * kF;
@@ -506,6 +515,7 @@ __global__ void __launch_bounds__(512, 2) k_pull_rows_f64(PullArgs p) {
     __syncthreads();
   }
   double2* racc = reinterpret_cast<double2*>(p.rowacc) + ia * p.lenb;
+  double sq = 0.0;
   for (int x = tid; x < lenb; x += nt) {
     const double2 r = racc[x];
     double re = r.x, im = r.y;
@@ -527,11 +537,83 @@ __global__ void __launch_bounds__(512, 2) k_pull_rows_f64(PullArgs p) {
       vi += p.beta_re * c.y + p.beta_im * c.x;
     }
     reinterpret_cast<double2*>(p.out)[idx] = make_double2(vr, vi);
+    sq += vr * vr + vi * vi;
     if (p.acc) {
-      p.acc[2 * idx] += vr;
-      p.acc[2 * idx + 1] += vi;
+      double2* a = reinterpret_cast<double2*>(p.acc) + idx;
+      const double2 o = p.acc0 ? reinterpret_cast<const double2*>(p.acc0)[idx] : *a;
+      *a = make_double2(o.x + vr, o.y + vi);
     }
   }
+  if (p.partials) row_norm(sq, p.partials + ia, smem);
+}
+
+template <bool CPLX, int G>
+__global__ void __launch_bounds__(512, 2) k_pull_rows_f64(PullArgs p) {
+  extern __shared__ __align__(16) char smem[];
+  if (p.done && *p.done) return;
+  pull_row<CPLX, G>(p, xcd_order(blockIdx.x, p.lena), smem);
+}
+
+// One Taylor step of every sector of a batch group (sectors of G W tiles, real
+// operators, 4-wave workgroups).  Step 0 is apply_out = H C0; step k >= 1 is
+// term_k = alpha H term_(k-1), result += term_k (step 1: result = C0 + term_1),
+// with the terms alternating between two buffers, so no copy and no second
+// pass is needed.  Small sectors are bound by launches and idle CUs: a step of
+// one is 2 launches of ~10 us for a handful of workgroups.  30 random sectors
+// of 4 to 12 orbitals, one apply and 10 terms: 3602 us with each sector's own
+// launches (one in-place apply per term), 1229 us with the groups (2749 us
+// with the push-form row groups before the pull form).
+struct PullGroupSector {
+  PullArgs args;                           // coeff, out, acc per step
+  const double* ha;
+  const double* hb;
+  const double* coeff0;
+  double* apply_out;
+  double* term[2];
+  double* result;
+  int row0, tile0, ta, tb;                 // first workgroup of each kernel
+};
+
+__device__ __forceinline__ int group_find(const PullGroupSector* secs, int nsec,
+                                          int block, bool rows) {
+  int lo = 0, hi = nsec - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if ((rows ? secs[mid].row0 : secs[mid].tile0) <= block) lo = mid;
+    else hi = mid - 1;
+  }
+  return lo;
+}
+
+__device__ __forceinline__ const double* group_source(const PullGroupSector& s, int step) {
+  return step <= 1 ? s.coeff0 : s.term[step & 1];
+}
+
+__global__ void __launch_bounds__(256, 4)
+k_same_spin_group(const PullGroupSector* __restrict__ secs, int nsec, int step) {
+  const int i = group_find(secs, nsec, blockIdx.x, false);
+  const PullGroupSector& s = secs[i];
+  if (step == 0 && !s.apply_out) return;
+  same_spin_tile<false, 1, 1>(blockIdx.x - s.tile0, s.args.lena, s.args.lenb, s.ha,
+                              s.hb, group_source(s, step), s.args.rowacc, s.ta, s.tb);
+}
+
+template <int G>
+__global__ void __launch_bounds__(256, 2)
+k_pull_rows_group(const PullGroupSector* __restrict__ secs, int nsec, int step,
+                  double alpha_re, double alpha_im) {
+  extern __shared__ __align__(16) char smem[];
+  const int i = group_find(secs, nsec, blockIdx.x, true);
+  const PullGroupSector& s = secs[i];
+  PullArgs p = s.args;
+  p.coeff = group_source(s, step);
+  p.out = step == 0 ? s.apply_out : s.term[(step + 1) & 1];
+  if (!p.out) return;
+  p.alpha_re = step == 0 ? 1.0 : alpha_re;
+  p.alpha_im = step == 0 ? 0.0 : alpha_im;
+  p.acc = step == 0 ? nullptr : s.result;
+  p.acc0 = step == 1 ? s.coeff0 : nullptr;
+  pull_row<false, G>(p, blockIdx.x - s.row0, smem);
 }
 
 // Target words of the row kernel from a forward table: 8 (target + 1), bit 31
@@ -638,44 +720,130 @@ int launch_same_spin(const fqehip_sector* s, int complex_op,
   return FQEHIP_OK;
 }
 
-// The opposite-spin rows on top of rowacc; with out set also the epilogue
-// out = alpha (H C) + beta cin, acc += out (out must not alias coeff: other
-// workgroups still read it).
-int launch_pull_rows(const fqehip_sector* s, int complex_op,
-                     const double* coeff, double* rowacc, double ar, double ai,
-                     double br, double bi, const double* cin, double* out,
-                     double* acc, hipStream_t st, const int32_t* done) {
-  PullPlan pl;
+namespace {
+
+// The sector's part of the row kernel's arguments.
+bool pull_args(const fqehip_sector* s, int complex_op, PullArgs* p, PullPlan* pl) {
   if (!pull_plan(complex_op != 0, s->nalpha * (s->norb - s->nalpha), s->lenb,
-                 s->npull, &pl)) {
+                 s->npull, pl)) {
     set_error("k_pull_rows_f64: lenb=%lld does not fit in LDS",
               static_cast<long long>(s->lenb));
-    return FQEHIP_ERR_INVALID;
+    return false;
   }
-  PullArgs p{};
-  p.norb = s->norb;
-  p.compressed = s->npull == s->norb * (s->norb + 1) / 2 ? 1 : 0;
-  p.nele = s->nalpha;
-  p.nq = s->npull;
-  p.lena = s->lena;
-  p.lenb = s->lenb;
-  p.ks = pl.ks;
-  p.pass = pl.pass;
-  p.copies = pl.copies;
-  p.w = s->pull_w;
-  p.dexc = s->dexc_a;
-  p.fwd = s->pull_fwd;
+  *p = PullArgs{};
+  p->norb = s->norb;
+  p->compressed = s->npull == s->norb * (s->norb + 1) / 2 ? 1 : 0;
+  p->nele = s->nalpha;
+  p->nq = s->npull;
+  p->lena = s->lena;
+  p->lenb = s->lenb;
+  p->ks = pl->ks;
+  p->pass = pl->pass;
+  p->copies = pl->copies;
+  p->w = s->pull_w;
+  p->dexc = s->dexc_a;
+  p->fwd = s->pull_fwd;
+  return true;
+}
+
+}  // namespace
+
+// The opposite-spin rows on top of rowacc; with e.out set also the epilogue
+// out = alpha (H C) + beta cin, acc += out, partials[ia] = |out row|^2 (out must
+// not alias coeff: other workgroups still read it).
+int launch_pull_rows(const fqehip_sector* s, int complex_op,
+                     const double* coeff, double* rowacc,
+                     const PullEpilogue& e, hipStream_t st, const int32_t* done) {
+  PullPlan pl;
+  PullArgs p;
+  if (!pull_args(s, complex_op, &p, &pl)) return FQEHIP_ERR_INVALID;
   p.coeff = coeff;
   p.rowacc = rowacc;
-  p.alpha_re = ar;
-  p.alpha_im = ai;
-  p.beta_re = br;
-  p.beta_im = bi;
-  p.cin = cin;
-  p.out = out;
-  p.acc = acc;
+  p.alpha_re = e.alpha_re;
+  p.alpha_im = e.alpha_im;
+  p.beta_re = e.beta_re;
+  p.beta_im = e.beta_im;
+  p.cin = e.cin;
+  p.out = e.out;
+  p.acc = e.acc;
+  p.partials = e.partials;
   p.done = done;
   return complex_op ? launch_rows<true>(pl, p, st) : launch_rows<false>(pl, p, st);
+}
+
+// Batch groups.  The class of a sector is the W tile count its rows run with
+// (1..7); 0 for sectors that keep their own launches: 8-wave workgroups and
+// same-spin products past the smallest tile.
+int pull_group_class(const fqehip_sector* s) {
+  PullPlan pl;
+  if (!pull_plan(false, s->nalpha * (s->norb - s->nalpha), s->lenb, s->npull, &pl) ||
+      pl.threads != 256 || ((s->lena + 63) / 64) * ((s->lenb + 63) / 64) >= 100)
+    return 0;
+  return pl.tiles;
+}
+
+size_t pull_group_bytes(int nsec) { return nsec * sizeof(PullGroupSector); }
+
+// Fills host descriptors for the items of one class; rowacc and the second
+// term buffer from each item's workspace (spare: byte offset of the latter).
+int pull_group_fill(const fqehip_batch_item* const* items, const int64_t* spare,
+                    int nsec, void* host, PullGroupLaunch* g) {
+  PullGroupSector* secs = static_cast<PullGroupSector*>(host);
+  *g = PullGroupLaunch{};
+  g->nsec = nsec;
+  for (int i = 0; i < nsec; ++i) {
+    const fqehip_batch_item& it = *items[i];
+    const fqehip_sector& sc = it.sector;
+    PullGroupSector& o = secs[i];
+    o = PullGroupSector{};
+    PullPlan pl;
+    if (!pull_args(&sc, 0, &o.args, &pl)) return FQEHIP_ERR_INVALID;
+    o.args.rowacc = static_cast<double*>(it.d_workspace);
+    o.ha = sc.haa;
+    o.hb = sc.hbb;
+    o.coeff0 = static_cast<const double*>(it.d_coeff0);
+    o.apply_out = static_cast<double*>(it.d_apply_out);
+    o.term[0] = static_cast<double*>(it.d_term);
+    o.term[1] = reinterpret_cast<double*>(static_cast<char*>(it.d_workspace) + spare[i]);
+    o.result = it.d_result;
+    o.row0 = g->rows;
+    o.tile0 = g->tiles;
+    o.ta = static_cast<int>((sc.lena + 31) / 32);
+    o.tb = static_cast<int>((sc.lenb + 31) / 32);
+    g->rows += static_cast<int>(sc.lena);
+    g->tiles += o.ta * o.tb;
+    g->cls = pl.tiles;
+    g->lds = pl.lds > g->lds ? pl.lds : g->lds;
+    g->any_apply = g->any_apply || it.d_apply_out != nullptr;
+  }
+  return FQEHIP_OK;
+}
+
+// Step `step` of the group: the same-spin products, then the rows.
+int launch_pull_group(const PullGroupLaunch& g, const void* d_secs, int step,
+                      double ar, double ai, hipStream_t st) {
+  const PullGroupSector* secs = static_cast<const PullGroupSector*>(d_secs);
+  k_same_spin_group<<<g.tiles, 256, 0, st>>>(secs, g.nsec, step);
+  FQEHIP_CHECK_LAUNCH("k_same_spin_group");
+  switch (g.cls) {
+#define FQEHIP_PULL_CASE(N)                                                  \
+  case N:                                                                    \
+    k_pull_rows_group<N><<<g.rows, 256, g.lds, st>>>(secs, g.nsec, step, ar, ai); \
+    break;
+    FQEHIP_PULL_CASE(1)
+    FQEHIP_PULL_CASE(2)
+    FQEHIP_PULL_CASE(3)
+    FQEHIP_PULL_CASE(4)
+    FQEHIP_PULL_CASE(5)
+    FQEHIP_PULL_CASE(6)
+    FQEHIP_PULL_CASE(7)
+#undef FQEHIP_PULL_CASE
+    default:
+      set_error("k_pull_rows_group: class %d", g.cls);
+      return FQEHIP_ERR_INVALID;
+  }
+  FQEHIP_CHECK_LAUNCH("k_pull_rows_group");
+  return FQEHIP_OK;
 }
 
 }  // namespace fqehip

@@ -178,3 +178,55 @@ def test_digit_rows_edges(fqe, na, nb, norb, blocks, shape):
     d.apply_inplace_scaled(h, op=op)
     assert rel(outs[0], d.coeff) < 3e-11
     assert numpy.array_equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("nterms", [0, 1, 2, 5])
+@pytest.mark.parametrize("group", [True, False])
+def test_batch_terms(fqe, nterms, group):
+    """Pull-form sectors of a batch: alternating term buffers for every
+    parity of the last term, groups of one and several sectors of each W
+    tile count, sectors past the groups (8-wave workgroups), items without
+    the apply.  Against applies one by one; 1e-13 as the kernels are the
+    same and only the epilogue's order of additions differs."""
+    import ctypes
+    import torch
+    from fqe_amd import _lib, batched
+    rng = numpy.random.default_rng(5)
+    shapes = [(2, 1, 1), (3, 1, 2), (4, 2, 2), (4, 2, 0), (5, 5, 2), (6, 3, 3),
+              (7, 3, 4), (8, 4, 3), (9, 4, 4), (10, 5, 4), (6, 1, 3), (6, 3, 3)]
+    specs = []
+    for norb, na, nb in shapes:
+        h1, h2 = fo.synthetic_hamiltonian(norb, norb, rng)
+        g = fo.OracleGraph(na, nb, norb)
+        specs.append(batched.SectorSpec(
+            norb=norb, nalpha=na, nbeta=nb, h1=h1, h2=h2,
+            coeff=fo.synthetic_coeff(g.lena, g.lenb, rng)))
+    tiles = {f"{n},{a},{b}": "split" for n, a, b in shapes}
+    bt = batched.BatchedTaylor(specs, 0.1, nterms=nterms,
+                               dtype=torch.complex128, tiles=tiles, nstreams=3,
+                               group=group)
+    items = []
+    for i, p in enumerate(bt.sectors):
+        it = p.item()
+        if i % 3 == 2:
+            it.d_apply_out = None
+            p.apply_out.fill_(7.0)
+        items.append(it)
+    arr = (_lib.BatchItem * len(items))(*items)
+    handle = ctypes.c_void_p()
+    torch.cuda.synchronize()
+    _lib.call("fqehip_batch_create", bt.prec, len(items), arr, bt.time, nterms,
+              3, int(group), _lib.stream_ptr(), ctypes.byref(handle))
+    bt._batch = handle
+    for _ in range(2):
+        bt.launch()
+        got = bt.results()
+        torch.zeros(1000, device="cuda").sum().item()
+    bt.run_sequential()
+    for i, ((a0, e0), (a1, e1)) in enumerate(zip(got, bt.results())):
+        assert rel(e0, e1) < 1e-13, shapes[i]
+        if i % 3 == 2:
+            assert (a0 == 7.0).all(), shapes[i]
+        else:
+            assert rel(a0, a1) < 1e-13, shapes[i]
+    bt.close()
