@@ -8,7 +8,7 @@ one apply H|C> with C resident in HBM.
 
 The engine runs it three ways:
   * mixed precision at the metric's 1e-9 gate (``value``): complex128
-    storage, both contractions as exact products of 8-bit digits on the
+    storage, all contractions as exact products of 8-bit digits on the
     int8 matrix cores (Ozaki scheme, int32 accumulation, FP64 assembly);
   * FP64 (complex128 storage, FP64 matrix cores) beside it (``fp64``);
   * the BF16x3 engine (complex64 storage, BF16 hi/lo products with FP32
@@ -357,9 +357,14 @@ class EngineRun:
         self.n = self.c.numel()
         esz = 8 if self.prec == _lib.C128 else 4
         self.y_ptr = self.ws.data_ptr() + op.npair * 2 * self.n * esz
-        self.split = bool(self.s.hbb_hi) or bool(self.s.hbb_f64)
+        # complex128 two-body applies: the pull form, one call for the
+        # same-spin products and the opposite-spin rows
+        self.pull = bool(_lib.lib().fqehip_pull_supported(
+            self.prec, self.sref, self.oref))
+        self.split = bool(self.s.hbb_hi) and not self.pull
         self.rowacc_ptr = self.ws.data_ptr() + self.s.nslot * 2 * self.n * esz
-        self.names = (["fused_rows", "slot_reduce"] if self.fused else
+        self.names = (["pull_apply"] if self.pull else
+                      ["fused_rows", "slot_reduce"] if self.fused else
                       ["dvec_gather", "pair_gemm", "scatter"])
 
     def launch(self, events=None):
@@ -367,6 +372,13 @@ class EngineRun:
         st = L.stream_ptr()
         if events:
             events[0].record()
+        if self.pull:
+            L.call("fqehip_apply", self.prec, self.sref, self.oref,
+                   L.ptr(self.c), 1.0, 0.0, 0.0, 0.0, None, L.ptr(self.out),
+                   None, None, None, L.ptr(self.ws), st)
+            if events:
+                events[1].record()
+            return
         if self.fused:
             L.call("fqehip_apply_fused_rows", self.prec, self.sref, self.oref,
                    L.ptr(self.c), L.ptr(self.ws), None, st)
@@ -419,20 +431,10 @@ class EngineRun:
             L, s = self._lib, self.s
             ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
             ev[0].record()
-            work = self.rowacc_ptr + 2 * self.n * 8   # row maxima, digits
             for _ in range(steps):
-                if self.prec == L.C128 and s.hbb_oz:
-                    L.call("fqehip_beta_gemm_digits", s.lena, s.lenb,
-                           s.hbb_oz, L.ptr(self.c), work, self.rowacc_ptr,
-                           None, L.stream_ptr())
-                elif self.prec == L.C128:
-                    L.call("fqehip_beta_gemm_f64", s.lena, s.lenb, s.hbb_f64,
-                           L.ptr(self.c), self.rowacc_ptr, None,
-                           L.stream_ptr())
-                else:
-                    L.call("fqehip_beta_gemm", s.lena, s.lenb, s.hbb_hi,
-                           s.hbb_lo, s.ldh, L.ptr(self.c), self.rowacc_ptr,
-                           None, L.stream_ptr())
+                L.call("fqehip_beta_gemm", s.lena, s.lenb, s.hbb_hi,
+                       s.hbb_lo, s.ldh, L.ptr(self.c), self.rowacc_ptr,
+                       None, L.stream_ptr())
             ev[1].record()
             torch.cuda.synchronize()
             tb = ev[0].elapsed_time(ev[1]) / steps
@@ -458,14 +460,14 @@ def kernel_work(op, graph, n, esz, mixed, ozaki=False):
     all-rows kernel), by npair + 1 columns (extra h1' column); the
     beta-beta GEMM is lena x lenb x lenb complex times real (bfloat16
     hi/lo copies of Hbb for the mixed engine, FP64 columns for FP64).
-    The Ozaki-digit engine moves the FP64 engine's bytes except for the
-    slot rows, which it writes and the reduction reads in 48 bits per
-    double (12 bytes per complex value).  Its algorithmic int8 operations
-    ("ops") are the scheme's 20 digit products per product of the FP64
-    contraction: over the nslot + 1 live pair rows and npair + 1 gathered
-    rows per column (alpha rows) and 2 lena x lenb x lenb (beta-beta GEMM);
-    "executed_ops" are those of the padded tiles the kernels run (64 rows x
-    128 gathered rows; K = lenb rounded up to 64)."""
+    Pull form (every complex128 two-body apply): C is read and H C written
+    once, with the same-spin Hamiltonians, W and the excitation tables;
+    the operations are the products with Haa and Hbb (2 n (lena + lenb)
+    real columns) and, per alpha string, of W with the nalpha * (norb -
+    nalpha) excited rows and the string itself.  With digits ("ops") each
+    product counts the scheme's 20 digit products; "executed_ops" are those
+    of the padded tiles the kernels run (64 excited rows x 128 rows of W;
+    K rounded up to 64)."""
     from fqe_amd import settings
     p = op.npair
     nslot = graph.nalpha() * (graph.norb() - graph.nalpha())
@@ -476,20 +478,19 @@ def kernel_work(op, graph, n, esz, mixed, ozaki=False):
     lenb = graph.lenb()
     ldh = ((lenb + 127) // 128) * 128
     ldk = ((lenb + 63) // 64) * 64
+    lena = graph.lena()
+    lda = ((lena + 63) // 64) * 64
+    tables = 4 * (p * lenb + (nslot + 1) * lena)
+    pull = 2.0 * 2 * n * (lena + lenb + (nslot + 1) * p)
     if ozaki:
-        lena = graph.lena()
-        return {
-            "beta_gemm": {"bytes": 2 * 2 * n * esz + 5 * lenb * ldk,
-                          "ops": 20 * 2.0 * (2 * lena) * lenb * lenb,
-                          "executed_ops": 20 * 2.0 * (2 * lena) * ldk * lenb},
-            "alpha_rows": {"bytes": nslot * 12 * n + 3 * 2 * n * esz,
-                           "ops": 20 * 2.0 * (nslot + 1) * (p + 1) * 2 * n,
-                           "executed_ops": 20 * 2.0 * 64 * 128 * 2 * n},
-            "slot_reduce": {"bytes": nslot * 12 * n + 2 * 2 * n * esz},
-        }
+        return {"pull_apply": {
+            "bytes": 2 * 2 * n * esz + 5 * (lenb * ldk + lena * lda) + tables,
+            "ops": 20 * pull,
+            "executed_ops": 20 * 2.0 * 2 * n * (lda + ldk + 64 * 128)}}
     return {
-        "beta_gemm": {"bytes": 2 * 2 * n * esz + (2 * ldh * ldh * 2 if mixed
-                                                  else lenb * lenb * 8),
+        "pull_apply": {"bytes": 2 * 2 * n * esz + tables
+                       + esz * (lena * lena + lenb * lenb), "flops": pull},
+        "beta_gemm": {"bytes": 2 * 2 * n * esz + 2 * ldh * ldh * 2,
                       "flops": 2.0 * 2 * n * lenb},
         "alpha_rows": {"bytes": (nslot + 3) * 2 * n * esz,
                        "flops": 2.0 * rows * (p + 1) * 2 * n},
@@ -1066,6 +1067,7 @@ def main():
         wall, per = run.run(args.steps, args.warmup)
         outs[mode] = run.result()
         results[mode] = {"wall": wall, "per": per, "fused": run.fused,
+                         "pull": run.pull,
                          "tile": int(run.s.tile), "digits_beta":
                          bool(run.s.hbb_oz)}
         print(f"{mode}: {args.steps / wall:.2f} applies/s "
@@ -1128,8 +1130,8 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": ("c128 storage; int8 digit products on MFMA (Ozaki: A' 5 "
-                  "digits, D' and C 48-bit integers, 20 digit pairs), exact "
+        "dtype": ("c128 storage; int8 digit products on MFMA (Ozaki: H 5 "
+                  "digits, C 48-bit integers, 20 digit pairs), exact "
                   "int32 accumulation, FP64 assembly"),
         "data": "synthetic",
         "config": {"workload": (f"RestrictedHamiltonian apply, norb={norb} "
@@ -1137,7 +1139,8 @@ def main():
                                 f"{args.seed}, {norb} factors"),
                    "pair_basis": "compressed" if op.compressed else "ordered",
                    "npair": op.npair,
-                   "kernels": "split" if oz["fused"] else "unfused",
+                   "kernels": "pull" if oz["pull"] else
+                              "split" if oz["fused"] else "unfused",
                    "digit_beta_gemm": oz["digits_beta"]},
         "rel_err_mixed_vs_fp64_gpu": err_oz,
         "gate_1e-9_met": err_oz <= 1e-9,
