@@ -593,11 +593,15 @@ void fqehip_batch_destroy(fqehip_batch* batch);
  * d_out[p][q] = sum_i conj(a[p][i]) b[q][i] (complex128 [k][k]), FP64
  * matrix cores, fixed summation order.  The 2-RDM's dvec overlap
  * (src/fqe/fqe_data.py:1767-1782).  d_workspace:
- * fqehip_gram_workspace_bytes(n, k) bytes; k <= 4096.
+ * fqehip_gram_workspace_bytes(n, k) bytes; k <= 4096.  fqehip_gram takes
+ * interleaved rows, fqehip_gram_planar rows of n real then n imaginary
+ * parts; with d_a == d_b half of the products are computed.
  * ------------------------------------------------------------------- */
 int64_t fqehip_gram_workspace_bytes(int64_t n, int k);
 int fqehip_gram(int64_t n, int k, const double* d_a, const double* d_b,
                 double* d_out, double* d_workspace, void* stream);
+int fqehip_gram_planar(int64_t n, int k, const double* d_a, const double* d_b,
+                       double* d_out, double* d_workspace, void* stream);
 
 /* ---------------------------------------------------------------------
  * Spin-orbital apply on a full particle-number set (FqeDataSet): every

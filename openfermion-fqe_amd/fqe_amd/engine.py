@@ -523,3 +523,43 @@ def gram(a: torch.Tensor, b: torch.Tensor) -> numpy.ndarray:
               _lib.ptr(ws), _lib.stream_ptr())
     return out.cpu().numpy()
 
+
+def planar_rows(npair: int, vec: torch.Tensor) -> torch.Tensor:
+    """[npair + 1, 2, n] planes for the dvec of a vector, the vector itself
+    in the last row (real parts, then imaginary parts)."""
+    real = (torch.float64 if vec.dtype == torch.complex128
+            else torch.float32)
+    d = torch.empty((npair + 1, 2, vec.numel()), dtype=real,
+                    device=vec.device)
+    d[npair].copy_(torch.view_as_real(vec.reshape(-1)).T)
+    return d
+
+
+def gram_planar(a: torch.Tensor, b: torch.Tensor) -> numpy.ndarray:
+    """``gram`` of planar FP64 blocks [k, 2, n] (fqehip_gram_planar); half
+    of the products if a and b are the same block."""
+    k, _, n = a.shape
+    assert b.shape == (k, 2, n)
+    assert a.dtype == torch.float64 and b.dtype == torch.float64
+    assert a.is_contiguous() and b.is_contiguous()
+    ws = torch.empty(max(int(_lib.call("fqehip_gram_workspace_bytes", n, k)),
+                         16), dtype=torch.uint8, device=a.device)
+    out = torch.empty((k, k), dtype=torch.complex128, device=a.device)
+    _lib.call("fqehip_gram_planar", n, k, _lib.ptr(a), _lib.ptr(b),
+              _lib.ptr(out), _lib.ptr(ws), _lib.stream_ptr())
+    return out.cpu().numpy()
+
+
+def rdm12(d2: torch.Tensor, d: torch.Tensor, m: int
+          ) -> Tuple[numpy.ndarray, numpy.ndarray]:
+    """1- and 2-RDM in m orbitals from the planar rows of the bra's and the
+    ket's dvec (m^2 pairs, then the vector): rdm1[p, q] = <E_qp bra|ket> and
+    rdm2[j, k, i, l] = -<E_ij bra|E_kl ket> + delta_ki rdm1[j, l], both from
+    one Gram product."""
+    g = gram_planar(d2, d)
+    out1 = g[:-1, -1].reshape(m, m).T
+    out2 = -g[:-1, :-1].reshape((m,) * 4).transpose(1, 2, 0, 3)
+    for i in range(m):
+        out2[:, i, i, :] += out1
+    return out1.copy(), out2.copy()
+

@@ -221,17 +221,31 @@ class FqeData:
         real = torch.float64 if prec == _lib.C128 else torch.float32
         n = self.lena() * self.lenb()
         d = torch.empty((npair, 2, n), dtype=real, device=c.device)
-        ta = self._core.tables(True).pair_table(compressed)
-        tb = self._core.tables(False).pair_table(compressed)
-        _lib.call("fqehip_dvec_gather", prec, npair, self.lena(), self.lenb(),
-                  _lib.ptr(ta), _lib.ptr(tb), _lib.ptr(c), _lib.ptr(d),
-                  _lib.stream_ptr())
+        self._gather_dvec(c, d, npair, compressed)
         d = torch.complex(d[:, 0], d[:, 1])
         shape = ((npair,) if compressed else (norb, norb)) + (self.lena(),
                                                                self.lenb())
         return d.reshape(shape)
 
+    def _gather_dvec(self, c: torch.Tensor, d: torch.Tensor, npair: int,
+                     compressed: bool) -> None:
+        """Planar dvec of the contiguous coefficients into d."""
+        ta = self._core.tables(True).pair_table(compressed)
+        tb = self._core.tables(False).pair_table(compressed)
+        _lib.call("fqehip_dvec_gather", engine.precision_of(c.dtype), npair,
+                  self.lena(), self.lenb(), _lib.ptr(ta), _lib.ptr(tb),
+                  _lib.ptr(c), _lib.ptr(d), _lib.stream_ptr())
+
     # -- reduced density matrices ------------------------------------------
+    def _dvec_rows(self) -> torch.Tensor:
+        """[norb^2 + 1, 2, lena*lenb] FP64 planes: the dvec (ordered pairs),
+        then the coefficients."""
+        c = self.device_coeff()
+        n2 = self.norb() * self.norb()
+        d = engine.planar_rows(n2, c)
+        self._gather_dvec(c, d, n2, False)
+        return d.to(torch.float64)
+
     def _dvec128(self) -> torch.Tensor:
         """[norb^2, lena*lenb] complex128 device dvec (ordered pairs)."""
         d = self.calculate_dvec_spatial_device(compressed=False)
@@ -256,18 +270,11 @@ class FqeData:
         (``src/fqe/fqe_data.py:1767-1782``):
         rdm2[j, k, i, l] = -<E_ij bra|E_kl ket> + delta_ki rdm1[j, l].
         The norb^2 x norb^2 overlap matrix of the two dvecs is one FP64
-        matrix-core Gram product (fqehip_gram)."""
+        matrix-core Gram product (fqehip_gram_planar)."""
         bra = self if bradata is None else bradata
-        norb = self.norb()
-        n2 = norb * norb
-        d = self._dvec128()
-        d2 = d if bradata is None else bra._dvec128()
-        out1 = engine.block_dots(d2, self._coeff128()).reshape(norb, norb).T
-        m = engine.gram(d2, d)
-        out2 = -m.reshape((norb,) * 4).transpose(1, 2, 0, 3).copy()
-        for i in range(norb):
-            out2[:, i, i, :] += out1
-        return out1.copy(), out2
+        d = self._dvec_rows()
+        d2 = d if bradata is None else bra._dvec_rows()
+        return engine.rdm12(d2, d, self.norb())
 
     def ax_plus_y(self, sval: complex, other: 'FqeData') -> 'FqeData':
         assert hash(self) == hash(other)

@@ -113,14 +113,18 @@ class FqeDataSet:
 
     def _dvec(self, vec: torch.Tensor) -> torch.Tensor:
         """[(2 norb)^2, L] complex128 D[pq] = E_pq C."""
+        d = self._dvec_rows(vec)[:-1]
+        return torch.complex(d[:, 0], d[:, 1]).contiguous()
+
+    def _dvec_rows(self, vec: torch.Tensor) -> torch.Tensor:
+        """[(2 norb)^2 + 1, 2, L] planes of D[pq] = E_pq C, then C."""
         m = 2 * self._norb
-        # planar planes, then their complex128 copy
+        # planar planes and a complex128 copy
         _check_fits(2 * m * m * vec.numel() * 16, "the spin-orbital dvec")
-        d = torch.empty((m * m, 2, vec.numel()), dtype=torch.float64,
-                        device=vec.device)
+        d = engine.planar_rows(m * m, vec)
         _lib.call("fqehip_set_dvec", self._norb, self._nele, _lib.ptr(vec),
                   _lib.ptr(d), _lib.stream_ptr())
-        return torch.complex(d[:, 0], d[:, 1]).contiguous()
+        return d
 
     # -- apply -----------------------------------------------------------------
     def apply(self, array: Tuple[numpy.ndarray, ...]) -> 'FqeDataSet':
@@ -183,11 +187,6 @@ class FqeDataSet:
         (2 norb)^2 x (2 norb)^2 dvec overlap is one FP64 Gram product."""
         m = 2 * self._norb
         vec = self._vector()
-        d = self._dvec(vec)
-        d2 = d if bra is None else self._dvec(bra._vector())
-        out1 = engine.block_dots(d2, vec).reshape(m, m).T
-        g = engine.gram(d2, d)
-        out2 = -g.reshape((m,) * 4).transpose(1, 2, 0, 3).copy()
-        for i in range(m):
-            out2[:, i, i, :] += out1
-        return out1.copy(), out2
+        d = self._dvec_rows(vec)
+        d2 = d if bra is None else self._dvec_rows(bra._vector())
+        return engine.rdm12(d2, d, m)
