@@ -624,12 +624,18 @@ int fqehip_gram_planar(int64_t n, int k, const double* d_a, const double* d_b,
  * src/fqe/fqe_data_set.py:183-209); d_workspace holds
  * fqehip_set_workspace_bytes(norb, nele) bytes.  Spin-flip signs are the
  * reference's (src/fqe/fci_graph_set.py:137-150).  Gathers only: the same
- * bits on every run.  d_out must not alias d_coeff.
+ * bits on every run.  d_out must not alias d_coeff.  From 2 electrons on,
+ * unless its planes exceed the workspace, the two-body apply runs over
+ * pairs of annihilated orbitals and nele - 2 electrons instead of D and Y.
  * ------------------------------------------------------------------- */
 int64_t fqehip_set_length(int norb, int nele);
 int64_t fqehip_set_workspace_bytes(int norb, int nele);
 int fqehip_set_dvec(int norb, int nele, const double* d_coeff,
                     double* d_dvec, void* stream);
+/* The dvec-form tensors from the operator's: d_v = V of d_h2 ([M]^4 each)
+ * and d_h1 ([M]^2) turned into h1' in place. */
+int fqehip_set_tensors(int norb, double* d_h1, const double* d_h2,
+                       double* d_v, void* stream);
 int fqehip_set_apply(int norb, int nele, const double* d_h1,
                      const double* d_v, const double* d_coeff, double* d_out,
                      double* d_workspace, void* stream);

@@ -138,6 +138,8 @@ _SIGNATURES = {
     "fqehip_set_dvec": (c_int, [c_int, c_int, c_void_p, c_void_p, c_void_p]),
     "fqehip_set_contract": (c_int, [c_int, c_int, c_void_p, c_void_p,
                                     c_void_p]),
+    "fqehip_set_tensors": (c_int, [c_int, c_void_p, c_void_p, c_void_p,
+                                   c_void_p]),
     "fqehip_set_apply": (c_int, [c_int, c_int, c_void_p, c_void_p, c_void_p,
                                  c_void_p, c_void_p, c_void_p]),
     "fqehip_mlp_features": (c_int, [c_int, c_int64, c_int64, c_void_p,

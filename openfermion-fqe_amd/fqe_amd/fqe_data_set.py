@@ -45,6 +45,8 @@ def _check_fits(nbytes: int, what: str) -> None:
     every sector in HBM at once and has no chunking over pairs."""
     dev = _lib.device()
     free, _ = torch.cuda.mem_get_info(dev)
+    if nbytes <= free:             # torch's own figures take 100 us to get
+        return
     free += torch.cuda.memory_reserved(dev) - torch.cuda.memory_allocated(dev)
     if nbytes > free:
         raise MemoryError(
@@ -103,13 +105,11 @@ class FqeDataSet:
         return vec
 
     def _split_into(self, vec: torch.Tensor, out: 'FqeDataSet') -> None:
-        off = 0
-        for k in self._keys():
-            sec = out._data[k]
-            n = sec.lena() * sec.lenb()
-            sec.set_device_coeff(vec[off:off + n].reshape(sec.lena(),
-                                                          sec.lenb()))
-            off += n
+        secs = [out._data[k] for k in self._keys()]
+        shapes = [(sec.lena(), sec.lenb()) for sec in secs]
+        for sec, shape, part in zip(secs, shapes,
+                                    vec.split([a * b for a, b in shapes])):
+            sec.set_device_coeff(part.view(shape))
 
     def _dvec(self, vec: torch.Tensor) -> torch.Tensor:
         """[(2 norb)^2, L] complex128 D[pq] = E_pq C."""
@@ -135,6 +135,11 @@ class FqeDataSet:
 
     def apply_inplace(self, array: Tuple[numpy.ndarray, ...]) -> None:
         """reference ``src/fqe/fqe_data_set.py:118-128``"""
+        self.apply_inplace_scaled(array)
+
+    def apply_inplace_scaled(self, array: Tuple[numpy.ndarray, ...],
+                             beta: complex = 0.0) -> None:
+        """C <- H C + beta C over all sectors."""
         m = 2 * self._norb
         if len(array) not in (1, 2):
             raise NotImplementedError(
@@ -154,12 +159,11 @@ class FqeDataSet:
             h2 = numpy.asarray(array[1], dtype=numpy.complex128)
             if h2.shape != (m,) * 4:
                 raise ValueError(f"h2 must have shape {(m,) * 4}")
-            # dvec form (reference src/fqe/fqe_data_set.py:194-197)
-            v = -numpy.moveaxis(h2, 1, 2)
-            h1p = h1 - numpy.einsum("ikkj->ij", v)
-            th1 = torch.from_numpy(numpy.ascontiguousarray(h1p)).to(dev)
-            tv = torch.from_numpy(
-                numpy.ascontiguousarray(v.reshape(m * m, m * m))).to(dev)
+            th1, th2 = (torch.from_numpy(numpy.require(
+                x, requirements=["C", "W"])).to(dev) for x in (h1, h2))
+            tv = torch.empty_like(th2)
+            _lib.call("fqehip_set_tensors", self._norb, _lib.ptr(th1),
+                      _lib.ptr(th2), _lib.ptr(tv), _lib.stream_ptr())
             nbytes = int(_lib.call("fqehip_set_workspace_bytes", self._norb,
                                    self._nele))
             _check_fits(nbytes, "the spin-orbital two-body apply")
@@ -167,6 +171,8 @@ class FqeDataSet:
             _lib.call("fqehip_set_apply", self._norb, self._nele,
                       _lib.ptr(th1), _lib.ptr(tv), _lib.ptr(vec),
                       _lib.ptr(out), _lib.ptr(ws), _lib.stream_ptr())
+        if beta != 0.0:
+            out.add_(vec, alpha=beta)
         self._split_into(out, self)
 
     # -- reduced density matrices -----------------------------------------
