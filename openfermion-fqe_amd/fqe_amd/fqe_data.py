@@ -130,6 +130,13 @@ class FqeData:
             new._dev = None
         return new
 
+    def _shared_copy(self) -> 'FqeData':
+        """A copy that refers to the same coefficients: for a caller that
+        replaces them before it hands the copy out."""
+        new = FqeData.__new__(FqeData)
+        new.__dict__.update(self.__dict__)
+        return new
+
     def __hash__(self):
         return hash((self._nele, self._m_s))
 

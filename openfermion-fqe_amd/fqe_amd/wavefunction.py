@@ -130,6 +130,15 @@ class Wavefunction:
         new._civec = {k: copy.deepcopy(v) for k, v in self._civec.items()}
         return new
 
+    def _shared_copy(self) -> 'Wavefunction':
+        """A copy whose sectors refer to this one's coefficients, for an
+        apply that gives each sector new ones."""
+        new = Wavefunction.__new__(Wavefunction)
+        new.__dict__.update({k: copy.copy(v) for k, v in self.__dict__.items()
+                             if k != '_civec'})
+        new._civec = {k: v._shared_copy() for k, v in self._civec.items()}
+        return new
+
     # -- vector algebra --------------------------------------------------------
     def norm(self) -> float:
         total = 0.0
@@ -185,7 +194,7 @@ class Wavefunction:
         """out = H psi + e_0 psi (reference ``src/fqe/wavefunction.py:
         366-399``); the e_0 term is fused into the scatter epilogue."""
         op = _prepared(hamil, array, self._norb)
-        out = copy.deepcopy(self)
+        out = self._shared_copy()
         beta = e_0 if numpy.abs(e_0) > 1.e-15 else 0.0
         for sec in out._civec.values():
             sec.apply_inplace_scaled(array, alpha=1.0, beta=beta, op=op)
@@ -227,11 +236,10 @@ class Wavefunction:
                     "the GPU engine applies 1- and 1+2-body operators; 3- "
                     "and 4-body operators are outside its path")
             return self._apply_array(hamil.tensors(), hamil.e_0(), hamil)
-        out = copy.deepcopy(self)
+        out = self._shared_copy()
+        beta = hamil.e_0() if numpy.abs(hamil.e_0()) > 1.e-15 else 0.0
         for nsector in out._number_sectors().values():
-            nsector.apply_inplace(hamil.tensors())
-        if numpy.abs(hamil.e_0()) > 1.e-15:
-            out.ax_plus_y(hamil.e_0(), self)
+            nsector.apply_inplace_scaled(hamil.tensors(), beta)
         return out
 
     def expectationValue(self, ops, brawfn: 'Wavefunction' = None) -> complex:
