@@ -214,21 +214,22 @@ template <bool CPLX, int RA, int RB>
 __global__ void __launch_bounds__(256, RA * RB > 4 || CPLX ? 2 : 4)
 k_same_spin_f64(int64_t lena, int64_t lenb, const double* __restrict__ ha,
                 const double* __restrict__ hb, const double* __restrict__ coeff,
-                double* __restrict__ out, const int32_t* __restrict__ done,
+                double* __restrict__ out, const int32_t* done, PullSeries series,
                 int ta, int tb) {
   if (done && *done) return;
+  if (series.partials && series_done(series, static_cast<int>(lena))) return;
   same_spin_tile<CPLX, RA, RB>(static_cast<int>(xcd_order(blockIdx.x, ta * tb)),
                                lena, lenb, ha, hb, coeff, out, ta, tb);
 }
 
 template <bool CPLX, int RA, int RB>
 void same_spin(int64_t lena, int64_t lenb, const double* ha, const double* hb,
-               const double* coeff, double* out, hipStream_t st,
-               const int32_t* done) {
+               const double* coeff, double* out, const PullSeries& series,
+               hipStream_t st, const int32_t* done) {
   const int ta = static_cast<int>((lena + 32 * RA - 1) / (32 * RA));
   const int tb = static_cast<int>((lenb + 32 * RB - 1) / (32 * RB));
   k_same_spin_f64<CPLX, RA, RB><<<static_cast<unsigned>(ta * tb), 256, 0, st>>>(
-      lena, lenb, ha, hb, coeff, out, done, ta, tb);
+      lena, lenb, ha, hb, coeff, out, done, series, ta, tb);
 }
 
 // ---------------------------------------------------------------------------
@@ -239,6 +240,8 @@ constexpr int kPullTiles = 7;              // 16-row W tiles per pass
 constexpr int kPullDepth = 4;              // k steps of B in flight
 constexpr int kPullRows = kPullMaxK + 4 * kPullDepth;   // lrow entries
 constexpr uint32_t kPullNoRow = 0x80000000u;   // past the end of C
+
+constexpr int64_t kInRowMax = 12000;      // see pull_in_row
 
 struct PullArgs {
   int norb, compressed, nele, nq;          // nq: pairs of one spin
@@ -257,6 +260,9 @@ struct PullArgs {
   double* acc;
   const double* acc0;                      // not NULL: acc = acc0 + that value
   double* partials;                        // not NULL: [ia] = |out row|^2
+  const double* ha;                        // not NULL: the same-spin part is
+  const double* hb;                        // computed here, not read
+  PullSeries series;
   const int32_t* done;
 };
 
@@ -264,6 +270,85 @@ size_t pull_lds_bytes(bool cplx, int ks, int64_t lenb, int tiles, int copies) {
   return static_cast<size_t>(copies) * lenb * 16 +
          static_cast<size_t>(tiles) * ks * 64 * 8 * (cplx ? 2 : 1) +
          kPullMaxK * (8 + 4 + 4) + kPullRows * 4 + 8 * 4;
+}
+
+// Row ia of Haa C + C Hbb^T into accumulator row 0.  Eight lanes share a
+// column, each with every eighth term of both sums: the loads of a wave are
+// 128-byte pieces of eight rows of C and 64-byte pieces of eight rows of Hbb.
+// 32 terms of both make a step, and the next step's loads are in flight while
+// one is summed (latency bounds it: with the rows, 70 x 70 strings take 13.4 us,
+// 14.7 without the overlap, and 8 + 8 us as two kernels).
+template <bool CPLX>
+__device__ __forceinline__ void same_spin_row(const PullArgs& p, int64_t ia, int wave,
+                                              int nwave, int lane, double2* accs) {
+  constexpr int kH = CPLX ? 16 : 8;
+  const int lena = static_cast<int>(p.lena), lenb = static_cast<int>(p.lenb);
+  const int kp = lane & 7, xl = lane >> 3;
+  const __amdgpu_buffer_rsrc_t rc = buffer_of(p.coeff, p.lena * p.lenb * 16);
+  const __amdgpu_buffer_rsrc_t ra = buffer_of(p.ha, p.lena * p.lena * kH);
+  const __amdgpu_buffer_rsrc_t rb = buffer_of(p.hb, p.lenb * p.lenb * kH);
+  const int row = static_cast<int>(ia);
+  const int nj = ((lena > lenb ? lena : lenb) + 31) / 32;
+  struct Step {
+    double2 h[8], c[8];
+  };
+  auto load_h = [&](__amdgpu_buffer_rsrc_t r, int off) {
+    return CPLX ? bload_d2(r, off) : make_double2(load_d(r, off), 0.0);
+  };
+  // terms and columns past the last read zero
+  auto load = [&](Step& s, int x0, int jb) {
+    const int x = x0 + xl;
+    const bool ok = x < lenb;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int j = 32 * jb + 8 * u + kp;
+      const bool a = ok && j < lena, b = ok && j < lenb;
+      s.h[u] = load_h(ra, a ? (j * lena + row) * kH : -1);
+      s.c[u] = bload_d2(rc, a ? (j * lenb + x) * 16 : -1);
+      s.h[4 + u] = load_h(rb, b ? (j * lenb + x) * kH : -1);
+      s.c[4 + u] = bload_d2(rc, b ? (row * lenb + j) * 16 : -1);
+    }
+  };
+  double re = 0.0, im = 0.0;
+  int x0 = wave * 8, jb = 0;               // the step that is summed
+  auto sum = [&](const Step& s) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      re += s.h[u].x * s.c[u].x;
+      im += s.h[u].x * s.c[u].y;
+      if (CPLX) {
+        re -= s.h[u].y * s.c[u].y;
+        im += s.h[u].y * s.c[u].x;
+      }
+    }
+    if (++jb < nj) return;
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) {
+      re += __shfl_xor(re, o);
+      im += __shfl_xor(im, o);
+    }
+    if (kp == 0 && x0 + xl < lenb) accs[x0 + xl] = make_double2(re, im);
+    re = im = 0.0;
+    jb = 0;
+    x0 += nwave * 8;
+  };
+  int lx = x0, lj = 0;                     // the next step to load
+  auto next = [&](Step& s) {
+    load(s, lx, lj);
+    if (++lj == nj) {
+      lj = 0;
+      lx += nwave * 8;
+    }
+  };
+  Step s0, s1;
+  next(s0);
+  while (x0 < lenb) {
+    next(s1);
+    sum(s0);
+    if (x0 >= lenb) break;
+    next(s0);
+    sum(s1);
+  }
 }
 
 // One alpha string ia per workgroup; G 16-row tiles of W per pass.
@@ -292,6 +377,9 @@ size_t pull_lds_bytes(bool cplx, int ks, int64_t lenb, int tiles, int copies) {
 // 7.6 + 1.6 ms of the slot-row kernel and its reduction; 4.8 ms without the
 // additions, 5.1 without their order.  norb 12 6a6b: 0.24 against 0.47 + 0.09;
 // complex operator, norb 11 4a6b: 0.14 against 1.23 for the unfused kernels.
+//
+// Small sectors (pull_in_row) have no same-spin kernel before this one: see
+// same_spin_row.
 template <bool CPLX, int G>
 __device__ __forceinline__ void pull_row(const PullArgs& p, int64_t ia,
                                          char* smem) {
@@ -354,6 +442,9 @@ __device__ __forceinline__ void pull_row(const PullArgs& p, int64_t ia,
   const __amdgpu_buffer_rsrc_t rw =
       buffer_of(p.w, static_cast<int64_t>(p.nq) * p.nq * (CPLX ? 16 : 8));
   const int ntile = (lenb + 15) >> 4;
+
+  // ahead of the first addition: the barriers below are in between
+  if (p.ha) same_spin_row<CPLX>(p, ia, wave, nwave, lane, accs);
 
   for (int ps = 0; ps < p.pass; ++ps) {
     const int q0 = 16 * G * ps;
@@ -517,8 +608,12 @@ __device__ __forceinline__ void pull_row(const PullArgs& p, int64_t ia,
   double2* racc = reinterpret_cast<double2*>(p.rowacc) + ia * p.lenb;
   double sq = 0.0;
   for (int x = tid; x < lenb; x += nt) {
-    const double2 r = racc[x];
-    double re = r.x, im = r.y;
+    double re = 0.0, im = 0.0;
+    if (!p.ha) {
+      const double2 r = racc[x];
+      re = r.x;
+      im = r.y;
+    }
     for (int c = 0; c < p.copies; ++c) {
       const double2 v = accs[c * lenb + x];
       re += v.x;
@@ -551,6 +646,7 @@ template <bool CPLX, int G>
 __global__ void __launch_bounds__(512, 2) k_pull_rows_f64(PullArgs p) {
   extern __shared__ __align__(16) char smem[];
   if (p.done && *p.done) return;
+  if (p.series.partials && series_done(p.series, static_cast<int>(p.lena))) return;
   pull_row<CPLX, G>(p, xcd_order(blockIdx.x, p.lena), smem);
 }
 
@@ -628,6 +724,15 @@ k_pull_table(int64_t n, int64_t padded, const int32_t* __restrict__ fwd,
   tab[i] = static_cast<uint32_t>(iabs(f)) << 3 | (f < 0 ? 0x80000000u : 0u);
 }
 
+// Whether the rows compute their same-spin part themselves: it saves a launch,
+// but every row reads all of C and Hbb, in time about lenb max(lena, lenb).
+// Evolution of 28 terms in us, same-spin kernel / in the row: 20 x 15 strings
+// 434 / 340, 70 x 70 575 / 502, 126 x 84 610 / 547, 252 x 45 685 / 590;
+// 120 x 120 686 / 716, 45 x 252 840 / 1364, 252 x 252 1240 / 2114.
+bool pull_in_row(int64_t lena, int64_t lenb) {
+  return lenb * (lena > lenb ? lena : lenb) <= kInRowMax && lena <= 256;
+}
+
 // How a sector runs: W tiles per pass, waves, accumulator rows.
 struct PullPlan {
   int ks, tiles, pass, copies, threads;
@@ -697,9 +802,14 @@ bool pull_supported(const fqehip_sector* s) {
          pull_plan(true, noff, s->lenb, s->npull, &pl);
 }
 
+bool pull_one_launch(const fqehip_sector* s) {
+  return pull_in_row(s->lena, s->lenb);
+}
+
 // rowacc = Haa C + C Hbb^T (complex128, 16 lena lenb bytes).
 int launch_same_spin(const fqehip_sector* s, int complex_op,
-                     const double* coeff, double* rowacc, hipStream_t st,
+                     const double* coeff, double* rowacc,
+                     const PullSeries& series, hipStream_t st,
                      const int32_t* done) {
   // tiles of 64 x 128 (64 x 64 complex operators) once they give every CU two
   // workgroups; 32 x 64 from half a workgroup per CU on (norb 12 6a6b, 435 of
@@ -708,13 +818,13 @@ int launch_same_spin(const fqehip_sector* s, int complex_op,
   const bool large = (l + 63) / 64 * ((m + (complex_op ? 63 : 127)) / (complex_op ? 64 : 128)) >= 512;
   const bool mid = !large && (l + 63) / 64 * ((m + 63) / 64) >= 100;
   if (complex_op) {
-    if (large) same_spin<true, 2, 2>(l, m, s->haa, s->hbb, coeff, rowacc, st, done);
-    else if (mid) same_spin<true, 1, 2>(l, m, s->haa, s->hbb, coeff, rowacc, st, done);
-    else same_spin<true, 1, 1>(l, m, s->haa, s->hbb, coeff, rowacc, st, done);
+    if (large) same_spin<true, 2, 2>(l, m, s->haa, s->hbb, coeff, rowacc, series, st, done);
+    else if (mid) same_spin<true, 1, 2>(l, m, s->haa, s->hbb, coeff, rowacc, series, st, done);
+    else same_spin<true, 1, 1>(l, m, s->haa, s->hbb, coeff, rowacc, series, st, done);
   } else {
-    if (large) same_spin<false, 2, 4>(l, m, s->haa, s->hbb, coeff, rowacc, st, done);
-    else if (mid) same_spin<false, 1, 2>(l, m, s->haa, s->hbb, coeff, rowacc, st, done);
-    else same_spin<false, 1, 1>(l, m, s->haa, s->hbb, coeff, rowacc, st, done);
+    if (large) same_spin<false, 2, 4>(l, m, s->haa, s->hbb, coeff, rowacc, series, st, done);
+    else if (mid) same_spin<false, 1, 2>(l, m, s->haa, s->hbb, coeff, rowacc, series, st, done);
+    else same_spin<false, 1, 1>(l, m, s->haa, s->hbb, coeff, rowacc, series, st, done);
   }
   FQEHIP_CHECK_LAUNCH("k_same_spin_f64");
   return FQEHIP_OK;
@@ -743,6 +853,10 @@ bool pull_args(const fqehip_sector* s, int complex_op, PullArgs* p, PullPlan* pl
   p->w = s->pull_w;
   p->dexc = s->dexc_a;
   p->fwd = s->pull_fwd;
+  if (pull_in_row(s->lena, s->lenb)) {
+    p->ha = s->haa;
+    p->hb = s->hbb;
+  }
   return true;
 }
 
@@ -767,6 +881,7 @@ int launch_pull_rows(const fqehip_sector* s, int complex_op,
   p.out = e.out;
   p.acc = e.acc;
   p.partials = e.partials;
+  p.series = e.series;
   p.done = done;
   return complex_op ? launch_rows<true>(pl, p, st) : launch_rows<false>(pl, p, st);
 }
@@ -808,8 +923,10 @@ int pull_group_fill(const fqehip_batch_item* const* items, const int64_t* spare,
     o.result = it.d_result;
     o.row0 = g->rows;
     o.tile0 = g->tiles;
-    o.ta = static_cast<int>((sc.lena + 31) / 32);
-    o.tb = static_cast<int>((sc.lenb + 31) / 32);
+    if (!o.args.ha) {
+      o.ta = static_cast<int>((sc.lena + 31) / 32);
+      o.tb = static_cast<int>((sc.lenb + 31) / 32);
+    }
     g->rows += static_cast<int>(sc.lena);
     g->tiles += o.ta * o.tb;
     g->cls = pl.tiles;
@@ -823,8 +940,10 @@ int pull_group_fill(const fqehip_batch_item* const* items, const int64_t* spare,
 int launch_pull_group(const PullGroupLaunch& g, const void* d_secs, int step,
                       double ar, double ai, hipStream_t st) {
   const PullGroupSector* secs = static_cast<const PullGroupSector*>(d_secs);
-  k_same_spin_group<<<g.tiles, 256, 0, st>>>(secs, g.nsec, step);
-  FQEHIP_CHECK_LAUNCH("k_same_spin_group");
+  if (g.tiles > 0) {
+    k_same_spin_group<<<g.tiles, 256, 0, st>>>(secs, g.nsec, step);
+    FQEHIP_CHECK_LAUNCH("k_same_spin_group");
+  }
   switch (g.cls) {
 #define FQEHIP_PULL_CASE(N)                                                  \
   case N:                                                                    \

@@ -6,6 +6,18 @@
 
 namespace fqehip {
 
+// The convergence test of a Taylor series' last term, made by the next term's
+// row kernel (partials NULL: none).
+constexpr int64_t kSeriesRows = 1024;      // partials a wave reads at most
+struct PullSeries {
+  const double* partials = nullptr;        // |row|^2 of the last term
+  double accuracy = 0.0;
+  int term = 0;                            // its number
+  double* norm = nullptr;
+  int32_t* nterms = nullptr;
+  int32_t* done = nullptr;
+};
+
 // What a row kernel does with the finished row of H C: nothing (out NULL: the
 // row accumulators keep it), or out = alpha (H C) + beta cin, acc += out,
 // partials[ia] = |out row|^2.
@@ -15,6 +27,7 @@ struct PullEpilogue {
   double* out = nullptr;
   double* acc = nullptr;
   double* partials = nullptr;
+  PullSeries series;
 };
 
 // Launch shape of a batch group of pull-form sectors (one class).
@@ -25,8 +38,12 @@ struct PullGroupLaunch {
 };
 
 bool pull_supported(const fqehip_sector* s);
+// Whether an FP64 apply of the sector is the row kernel alone (which then also
+// takes the test of a series).
+bool pull_one_launch(const fqehip_sector* s);
 int launch_same_spin(const fqehip_sector* s, int complex_op,
-                     const double* coeff, double* rowacc, hipStream_t st,
+                     const double* coeff, double* rowacc,
+                     const PullSeries& series, hipStream_t st,
                      const int32_t* done);
 int launch_pull_rows(const fqehip_sector* s, int complex_op,
                      const double* coeff, double* rowacc,
@@ -64,6 +81,27 @@ __device__ __forceinline__ void row_norm(double v, double* partial, char* smem) 
     for (unsigned w = 0; w < blockDim.x / 64; ++w) t += red[w];
     *partial = t;
   }
+}
+
+// The test after a term of a Taylor series, by every wave for itself at the
+// start of the next term's first kernel (a kernel of its own costs as much as
+// the rows of a small sector): the norm of the last term from its row partials,
+// stored with the term count by the first workgroup.  A wave that already
+// finds the flag set by that workgroup returns as the test would tell it.
+__device__ __forceinline__ bool series_done(const PullSeries& q, int lena) {
+  const int lane = threadIdx.x & 63;
+  double s = 0.0;
+  for (int k = lane; k < lena; k += 64) s += q.partials[k];
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) s += __shfl_xor(s, o);
+  const double nrm = sqrt(s);
+  const bool done = nrm < q.accuracy;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    *q.norm = nrm;
+    *q.nterms = q.term;
+    if (done) *q.done = 1;
+  }
+  return done;
 }
 
 }  // namespace fqehip

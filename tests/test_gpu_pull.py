@@ -230,3 +230,40 @@ def test_batch_terms(fqe, nterms, group):
         else:
             assert rel(a0, a1) < 1e-13, shapes[i]
     bt.close()
+
+
+@pytest.mark.parametrize("na,nb,norb", [
+    (2, 2, 4), (3, 3, 7), (4, 3, 9), (5, 2, 10),       # one launch a term
+    (4, 4, 9), (2, 5, 10), (6, 1, 12),                 # same-spin kernel first
+    (6, 0, 13), (5, 1, 13)])                           # test in its own launch
+def test_series_terms(fqe, na, nb, norb):
+    """A Taylor series whose terms are tested for convergence at the start
+    of the next term's kernel: the sum against applies one by one, summed
+    in the same order and stopped at the same norm (1e-13: the kernels are
+    the same but for the epilogue), and no convergence where one term fewer
+    is allowed than it takes."""
+    rng = numpy.random.default_rng(50 * norb + na)
+    h1, h2 = fo.synthetic_hamiltonian(norb, norb, rng)
+    ham = fqe.get_restricted_hamiltonian((h1, h2))
+    d, c, g, rng = sector(fqe, na, nb, norb, 7)
+    key = (na + nb, na - nb)
+    wfn = fqe.Wavefunction([[na + nb, na - nb, norb]])
+    wfn.set_wfn("from_data", {key: c / numpy.linalg.norm(c)})
+    t = 0.01
+    term, acc, nterms = wfn, wfn.get_coeff(key).copy(), 0
+    for order in range(1, 30):
+        term = term.apply(ham)
+        term.scale(-1j * t / order)
+        acc = acc + term.get_coeff(key)
+        nterms = order
+        if term.norm() < 1e-12:
+            break
+    got = wfn.apply_generated_unitary(t, "taylor", ham, accuracy=1e-12,
+                                      expansion=nterms + 1)
+    assert rel(got.get_coeff(key), acc) < 1e-13
+    longer = wfn.apply_generated_unitary(t, "taylor", ham, accuracy=1e-12,
+                                         expansion=nterms + 6)
+    assert numpy.array_equal(longer.get_coeff(key), got.get_coeff(key))
+    with pytest.raises(RuntimeError):
+        wfn.apply_generated_unitary(t, "taylor", ham, accuracy=1e-12,
+                                    expansion=nterms)
