@@ -86,12 +86,18 @@ __device__ __forceinline__ double load_d(__amdgpu_buffer_rsrc_t r, int off) {
   return u2d(v[0], v[1]);
 }
 
-template <bool CPLX, int RA, int RB>
+//
+// SPLIT, for sectors whose tiles would leave most of the chip idle: the
+// workgroup owns the outputs of one wave and each wave takes a quarter of
+// both sums; the quarters are added in wave order (red: 4 x 256 RA RB values of
+// LDS).  It shortens the chain of k steps by four and brings four times as
+// many waves: 252 x 252 strings 20.6 -> 8.7 us, 330 x 462 30.8 -> 21.4.
+template <bool CPLX, int RA, int RB, bool SPLIT>
 __device__ __forceinline__ void same_spin_tile(
     int t, int64_t lena, int64_t lenb, const double* __restrict__ ha,
     const double* __restrict__ hb, const double* __restrict__ coeff,
-    double* __restrict__ out, int ta, int tb) {
-  constexpr int D = kSpinDepth;
+    double* __restrict__ out, int ta, int tb, double2* red) {
+  constexpr int D = SPLIT ? 2 * kSpinDepth : kSpinDepth;
   constexpr int kH = CPLX ? 16 : 8;               // bytes per H element
   // groups of 8 tile rows, so neighbouring workgroups share C and H rows
   const int grp = t / (8 * tb);
@@ -102,8 +108,9 @@ __device__ __forceinline__ void same_spin_tile(
   const int lane = threadIdx.x & 63;
   const int kq = lane >> 4;
   const int cl = lane & 15;
-  const int a0 = ((grp * 8 + w % rows) * 2 + (wave >> 1)) * 16 * RA;
-  const int b0 = ((w / rows) * 2 + (wave & 1)) * 16 * RB;
+  const int ti = grp * 8 + w % rows, tj = w / rows;
+  const int a0 = (SPLIT ? ti : ti * 2 + (wave >> 1)) * 16 * RA;
+  const int b0 = (SPLIT ? tj : tj * 2 + (wave & 1)) * 16 * RB;
   const int la = static_cast<int>(lena), lb = static_cast<int>(lenb);
   if (a0 >= la || b0 >= lb) return;
   const __amdgpu_buffer_rsrc_t rc = buffer_of(coeff, lena * lenb * 16);
@@ -118,6 +125,12 @@ __device__ __forceinline__ void same_spin_tile(
       are[i][j] = double4_t{0, 0, 0, 0};
       aim[i][j] = double4_t{0, 0, 0, 0};
     }
+  // the k steps of this wave: whole rings, so only the last ones can pass the end
+  auto first = [&](int ns) { return SPLIT ? wave * ((ns + 4 * D - 1) / (4 * D)) * D : 0; };
+  auto last = [&](int ns) {
+    const int e = SPLIT ? (wave + 1) * ((ns + 4 * D - 1) / (4 * D)) * D : ns;
+    return e < ns ? e : ns;
+  };
   // an operand value of a k step: real and imaginary part (H: real only
   // unless CPLX)
   auto load_h = [&](__amdgpu_buffer_rsrc_t r, int off, double& re, double& im) {
@@ -142,9 +155,9 @@ __device__ __forceinline__ void same_spin_tile(
         q[d][j] = bload_d2(rc, (k * lb + b0 + 16 * j + cl) * 16);
     };
 #pragma unroll
-    for (int d = 0; d < D; ++d) load(d, d);
-    const int ns = (la + 3) / 4;
-    for (int s0 = 0; s0 < ns; s0 += D) {
+    for (int d = 0; d < D; ++d) load(first((la + 3) / 4) + d, d);
+    const int end = last((la + 3) / 4);
+    for (int s0 = first((la + 3) / 4); s0 < end; s0 += D) {
 #pragma unroll
       for (int d = 0; d < D; ++d) {
 #pragma unroll
@@ -175,9 +188,9 @@ __device__ __forceinline__ void same_spin_tile(
         load_h(rhb, (k * lb + b0 + 16 * j + cl) * kH, qr[d][j], qi[d][j]);
     };
 #pragma unroll
-    for (int d = 0; d < D; ++d) load(d, d);
-    const int ns = (lb + 3) / 4;
-    for (int s0 = 0; s0 < ns; s0 += D) {
+    for (int d = 0; d < D; ++d) load(first((lb + 3) / 4) + d, d);
+    const int end = last((lb + 3) / 4);
+    for (int s0 = first((lb + 3) / 4); s0 < end; s0 += D) {
 #pragma unroll
       for (int d = 0; d < D; ++d) {
 #pragma unroll
@@ -196,6 +209,36 @@ __device__ __forceinline__ void same_spin_tile(
     }
   }
   // item e of lane l: row l/16 + 4 e, column l%16
+  if constexpr (SPLIT) {
+    constexpr int kOut = 256 * RA * RB;
+#pragma unroll
+    for (int i = 0; i < RA; ++i)
+#pragma unroll
+      for (int j = 0; j < RB; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          red[wave * kOut + ((i * RB + j) * 4 + e) * 64 + lane] =
+              make_double2(are[i][j][e], aim[i][j][e]);
+    __syncthreads();
+    // item (i, j, e) by wave e
+#pragma unroll
+    for (int i = 0; i < RA; ++i)
+#pragma unroll
+      for (int j = 0; j < RB; ++j) {
+        const double2* r = red + ((i * RB + j) * 4 + wave) * 64 + lane;
+        double2 v = r[0];
+#pragma unroll
+        for (int q = 1; q < 4; ++q) {
+          v.x += r[q * kOut].x;
+          v.y += r[q * kOut].y;
+        }
+        const int a = a0 + 16 * i + kq + 4 * wave;
+        const int b = b0 + 16 * j + cl;
+        if (a < la && b < lb)
+          *reinterpret_cast<double2*>(out + (static_cast<int64_t>(a) * lb + b) * 2) = v;
+      }
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < RA; ++i)
 #pragma unroll
@@ -210,25 +253,27 @@ __device__ __forceinline__ void same_spin_tile(
       }
 }
 
-template <bool CPLX, int RA, int RB>
+template <bool CPLX, int RA, int RB, bool SPLIT>
 __global__ void __launch_bounds__(256, RA * RB > 4 || CPLX ? 2 : 4)
 k_same_spin_f64(int64_t lena, int64_t lenb, const double* __restrict__ ha,
                 const double* __restrict__ hb, const double* __restrict__ coeff,
                 double* __restrict__ out, const int32_t* done, PullSeries series,
                 int ta, int tb) {
+  __shared__ double2 red[SPLIT ? 4 * 256 * RA * RB : 1];
   if (done && *done) return;
   if (series.partials && series_done(series, static_cast<int>(lena))) return;
-  same_spin_tile<CPLX, RA, RB>(static_cast<int>(xcd_order(blockIdx.x, ta * tb)),
-                               lena, lenb, ha, hb, coeff, out, ta, tb);
+  same_spin_tile<CPLX, RA, RB, SPLIT>(static_cast<int>(xcd_order(blockIdx.x, ta * tb)),
+                                      lena, lenb, ha, hb, coeff, out, ta, tb, red);
 }
 
-template <bool CPLX, int RA, int RB>
+template <bool CPLX, int RA, int RB, bool SPLIT = false>
 void same_spin(int64_t lena, int64_t lenb, const double* ha, const double* hb,
                const double* coeff, double* out, const PullSeries& series,
                hipStream_t st, const int32_t* done) {
-  const int ta = static_cast<int>((lena + 32 * RA - 1) / (32 * RA));
-  const int tb = static_cast<int>((lenb + 32 * RB - 1) / (32 * RB));
-  k_same_spin_f64<CPLX, RA, RB><<<static_cast<unsigned>(ta * tb), 256, 0, st>>>(
+  constexpr int kRows = (SPLIT ? 16 : 32) * RA, kCols = (SPLIT ? 16 : 32) * RB;
+  const int ta = static_cast<int>((lena + kRows - 1) / kRows);
+  const int tb = static_cast<int>((lenb + kCols - 1) / kCols);
+  k_same_spin_f64<CPLX, RA, RB, SPLIT><<<static_cast<unsigned>(ta * tb), 256, 0, st>>>(
       lena, lenb, ha, hb, coeff, out, done, series, ta, tb);
 }
 
@@ -241,7 +286,7 @@ constexpr int kPullDepth = 4;              // k steps of B in flight
 constexpr int kPullRows = kPullMaxK + 4 * kPullDepth;   // lrow entries
 constexpr uint32_t kPullNoRow = 0x80000000u;   // past the end of C
 
-constexpr int64_t kInRowMax = 12000;      // see pull_in_row
+constexpr int64_t kInRowMax = 5000;      // see pull_in_row
 
 struct PullArgs {
   int norb, compressed, nele, nq;          // nq: pairs of one spin
@@ -277,7 +322,7 @@ size_t pull_lds_bytes(bool cplx, int ks, int64_t lenb, int tiles, int copies) {
 // 128-byte pieces of eight rows of C and 64-byte pieces of eight rows of Hbb.
 // 32 terms of both make a step, and the next step's loads are in flight while
 // one is summed (latency bounds it: with the rows, 70 x 70 strings take 13.4 us,
-// 14.7 without the overlap, and 8 + 8 us as two kernels).
+// 14.7 without the overlap, and 8 + 5.5 us as two kernels).
 template <bool CPLX>
 __device__ __forceinline__ void same_spin_row(const PullArgs& p, int64_t ia, int wave,
                                               int nwave, int lane, double2* accs) {
@@ -687,11 +732,12 @@ __device__ __forceinline__ const double* group_source(const PullGroupSector& s, 
 
 __global__ void __launch_bounds__(256, 4)
 k_same_spin_group(const PullGroupSector* __restrict__ secs, int nsec, int step) {
+  __shared__ double2 red[4 * 256];
   const int i = group_find(secs, nsec, blockIdx.x, false);
   const PullGroupSector& s = secs[i];
   if (step == 0 && !s.apply_out) return;
-  same_spin_tile<false, 1, 1>(blockIdx.x - s.tile0, s.args.lena, s.args.lenb, s.ha,
-                              s.hb, group_source(s, step), s.args.rowacc, s.ta, s.tb);
+  same_spin_tile<false, 1, 1, true>(blockIdx.x - s.tile0, s.args.lena, s.args.lenb, s.ha,
+                              s.hb, group_source(s, step), s.args.rowacc, s.ta, s.tb, red);
 }
 
 template <int G>
@@ -724,11 +770,16 @@ k_pull_table(int64_t n, int64_t padded, const int32_t* __restrict__ fwd,
   tab[i] = static_cast<uint32_t>(iabs(f)) << 3 | (f < 0 ? 0x80000000u : 0u);
 }
 
+// Whether the same-spin product splits its sums (see launch_same_spin).
+bool split_same_spin(int64_t lena, int64_t lenb) {
+  return (lena + 63) / 64 * ((lenb + 63) / 64) < 180;
+}
+
 // Whether the rows compute their same-spin part themselves: it saves a launch,
 // but every row reads all of C and Hbb, in time about lenb max(lena, lenb).
-// Evolution of 28 terms in us, same-spin kernel / in the row: 20 x 15 strings
-// 434 / 340, 70 x 70 575 / 502, 126 x 84 610 / 547, 252 x 45 685 / 590;
-// 120 x 120 686 / 716, 45 x 252 840 / 1364, 252 x 252 1240 / 2114.
+// Evolution in us, same-spin kernel / in the row: 20 x 15 strings 449 / 339,
+// 35 x 35 420 / 346, 56 x 56 432 / 386, 70 x 70 505 / 500, 126 x 84 502 / 551,
+// 252 x 45 533 / 590.
 bool pull_in_row(int64_t lena, int64_t lenb) {
   return lenb * (lena > lenb ? lena : lenb) <= kInRowMax && lena <= 256;
 }
@@ -812,19 +863,21 @@ int launch_same_spin(const fqehip_sector* s, int complex_op,
                      const PullSeries& series, hipStream_t st,
                      const int32_t* done) {
   // tiles of 64 x 128 (64 x 64 complex operators) once they give every CU two
-  // workgroups; 32 x 64 from half a workgroup per CU on (norb 12 6a6b, 435 of
-  // them: 0.126 ms, 0.149 with 64 x 64, 0.164 with 32 x 32); else 32 x 32
+  // workgroups; 32 x 64 from 360 workgroups on (924 x 924 strings: 0.126 ms,
+  // 0.149 with 64 x 64); below, 16 x 16 with the sums split over the waves
+  // (924 x 924 0.164 ms; 715 x 715 0.083 against 0.099, 792 x 495 0.061 against
+  // 0.071 with 32 x 64; 16 x 32 split: 0.115, 0.082)
   const int64_t l = s->lena, m = s->lenb;
   const bool large = (l + 63) / 64 * ((m + (complex_op ? 63 : 127)) / (complex_op ? 64 : 128)) >= 512;
-  const bool mid = !large && (l + 63) / 64 * ((m + 63) / 64) >= 100;
+  const bool mid = !large && !split_same_spin(l, m);
   if (complex_op) {
     if (large) same_spin<true, 2, 2>(l, m, s->haa, s->hbb, coeff, rowacc, series, st, done);
     else if (mid) same_spin<true, 1, 2>(l, m, s->haa, s->hbb, coeff, rowacc, series, st, done);
-    else same_spin<true, 1, 1>(l, m, s->haa, s->hbb, coeff, rowacc, series, st, done);
+    else same_spin<true, 1, 1, true>(l, m, s->haa, s->hbb, coeff, rowacc, series, st, done);
   } else {
     if (large) same_spin<false, 2, 4>(l, m, s->haa, s->hbb, coeff, rowacc, series, st, done);
     else if (mid) same_spin<false, 1, 2>(l, m, s->haa, s->hbb, coeff, rowacc, series, st, done);
-    else same_spin<false, 1, 1>(l, m, s->haa, s->hbb, coeff, rowacc, series, st, done);
+    else same_spin<false, 1, 1, true>(l, m, s->haa, s->hbb, coeff, rowacc, series, st, done);
   }
   FQEHIP_CHECK_LAUNCH("k_same_spin_f64");
   return FQEHIP_OK;
@@ -888,11 +941,11 @@ int launch_pull_rows(const fqehip_sector* s, int complex_op,
 
 // Batch groups.  The class of a sector is the W tile count its rows run with
 // (1..7); 0 for sectors that keep their own launches: 8-wave workgroups and
-// same-spin products past the smallest tile.
+// same-spin products past the split tile.
 int pull_group_class(const fqehip_sector* s) {
   PullPlan pl;
   if (!pull_plan(false, s->nalpha * (s->norb - s->nalpha), s->lenb, s->npull, &pl) ||
-      pl.threads != 256 || ((s->lena + 63) / 64) * ((s->lenb + 63) / 64) >= 100)
+      pl.threads != 256 || !split_same_spin(s->lena, s->lenb))
     return 0;
   return pl.tiles;
 }
@@ -924,8 +977,8 @@ int pull_group_fill(const fqehip_batch_item* const* items, const int64_t* spare,
     o.row0 = g->rows;
     o.tile0 = g->tiles;
     if (!o.args.ha) {
-      o.ta = static_cast<int>((sc.lena + 31) / 32);
-      o.tb = static_cast<int>((sc.lenb + 31) / 32);
+      o.ta = static_cast<int>((sc.lena + 15) / 16);
+      o.tb = static_cast<int>((sc.lenb + 15) / 16);
     }
     g->rows += static_cast<int>(sc.lena);
     g->tiles += o.ta * o.tb;

@@ -120,9 +120,10 @@ class PreparedOperator:
         out = torch.empty((n, n), device=self.a.device,
                           dtype=torch.complex128 if self.complex_op else
                           torch.float64)
+        pairs = _lib.ptr(self.a) + 8 * first * (lda + 1)
+        one_body = _lib.ptr(self.a) + 8 * (w * self.npair * lda + first)
         _lib.call("fqehip_spin_block", int(self.complex_op), npull, n,
-                  _lib.ptr(fwd), _lib.ptr(self.a[first:, first:]), lda,
-                  _lib.ptr(self.a[w * self.npair:, first:]), _lib.ptr(out),
+                  _lib.ptr(fwd), pairs, lda, one_body, _lib.ptr(out),
                   _lib.stream_ptr())
         return out
 

@@ -117,7 +117,8 @@ def test_pull_matches_oracle(fqe, kind, na, nb, norb):
     ("real", 5, 6, 12), ("real", 7, 6, 13), ("real", 7, 7, 14),
     ("real", 2, 8, 15), ("real", 3, 10, 15), ("nonsymmetric", 4, 6, 13),
     ("complex", 5, 5, 11), ("complex", 6, 7, 14), ("spin", 5, 4, 11),
-    ("spin_complex", 3, 4, 12)])
+    ("spin_complex", 3, 4, 12), ("nonsymmetric", 5, 1, 12),
+    ("complex", 1, 6, 12), ("spin_complex", 4, 4, 9), ("real", 4, 4, 13)])
 def test_pull_matches_other_kernels(fqe, kind, na, nb, norb):
     """Sectors too large for the oracle: the same operator on the slot-row
     kernels (real symmetric) or the unfused ones."""
@@ -233,8 +234,8 @@ def test_batch_terms(fqe, nterms, group):
 
 
 @pytest.mark.parametrize("na,nb,norb", [
-    (2, 2, 4), (3, 3, 7), (4, 3, 9), (5, 2, 10),       # one launch a term
-    (4, 4, 9), (2, 5, 10), (6, 1, 12),                 # same-spin kernel first
+    (2, 2, 4), (3, 3, 7), (4, 4, 8),                   # one launch a term
+    (4, 3, 9), (5, 2, 10), (2, 5, 10), (6, 1, 12),     # same-spin kernel first
     (6, 0, 13), (5, 1, 13)])                           # test in its own launch
 def test_series_terms(fqe, na, nb, norb):
     """A Taylor series whose terms are tested for convergence at the start
