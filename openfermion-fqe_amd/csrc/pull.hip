@@ -772,7 +772,7 @@ k_pull_table(int64_t n, int64_t padded, const int32_t* __restrict__ fwd,
 
 // Whether the same-spin product splits its sums (see launch_same_spin).
 bool split_same_spin(int64_t lena, int64_t lenb) {
-  return (lena + 63) / 64 * ((lenb + 63) / 64) < 180;
+  return (lena + 63) / 64 * ((lenb + 63) / 64) < 150;
 }
 
 // Whether the rows compute their same-spin part themselves: it saves a launch,
@@ -863,10 +863,10 @@ int launch_same_spin(const fqehip_sector* s, int complex_op,
                      const PullSeries& series, hipStream_t st,
                      const int32_t* done) {
   // tiles of 64 x 128 (64 x 64 complex operators) once they give every CU two
-  // workgroups; 32 x 64 from 360 workgroups on (924 x 924 strings: 0.126 ms,
+  // workgroups; 32 x 64 from 300 workgroups on (924 x 924 strings: 0.126 ms,
   // 0.149 with 64 x 64); below, 16 x 16 with the sums split over the waves
-  // (924 x 924 0.164 ms; 715 x 715 0.083 against 0.099, 792 x 495 0.061 against
-  // 0.071 with 32 x 64; 16 x 32 split: 0.115, 0.082)
+  // (split / 32 x 64, ms: 924 x 924 0.164 / 0.128, 792 x 792 0.131 / 0.117, 715 x
+  // 715 0.083 / 0.099, 792 x 495 0.061 / 0.071)
   const int64_t l = s->lena, m = s->lenb;
   const bool large = (l + 63) / 64 * ((m + (complex_op ? 63 : 127)) / (complex_op ? 64 : 128)) >= 512;
   const bool mid = !large && !split_same_spin(l, m);

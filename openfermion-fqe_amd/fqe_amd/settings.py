@@ -58,8 +58,8 @@ ozaki_beta = True
 # With contraction = "ozaki": sectors below this many determinants run in
 # FP64, where the digit kernels' extra launches (maxima, digits) cost more
 # than the faster products save.  Measured, FP64 / digits: norb 11 5a6b
-# (213,444) 110 / 139 us, norb 12 4a6b (457,380) 207 / 202 us, norb 12 6a6b
-# (853,776) 383 / 314 us.
+# (213,444) 113 / 137 us, norb 12 4a5b (392,040) 186 / 181 us, norb 12 4a6b
+# (457,380) 207 / 198 us, norb 12 6a6b (853,776) 380 / 307 us.
 ozaki_min_determinants = 400000
 
 # Largest apply workspace (bytes) allocated at once: a complex128 sector
