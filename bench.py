@@ -503,19 +503,6 @@ def kernel_work(op, graph, n, esz, mixed, ozaki=False):
 
 
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "apply_norb14_pmc_traffic.md")
-SET_TRAFFIC_FILE = os.path.join(ROOT, "profiles",
-                                "set_apply_norb10_pmc_traffic.md")
-
-
-def _traffic_block(path):
-    if not os.path.exists(path):
-        return {}
-    text = open(path).read()
-    i = text.find("```json")
-    if i < 0:
-        return {}
-    j = text.find("```", i + 7)
-    return json.loads(text[i + 7:j])["traffic_bytes_per_launch"]
 
 
 def measured_traffic(norb, na, nb):
@@ -644,8 +631,8 @@ def host_boundary_rate(coeff, h1, h2, norb, na, nb, reps=3):
 
 def set_main(args):
     """FqeDataSet 1+2-body apply (complex128) through fqehip_set_apply, with
-    the three kernels timed on their own; the oracle's apply of the same
-    workload is the CPU baseline and the parity check."""
+    the apply timed on its own; the oracle's apply of the same workload is
+    the CPU baseline and the parity check."""
     import math
     import numpy
     import torch
@@ -705,15 +692,10 @@ def set_main(args):
     torch.cuda.synchronize()
     wall = time.perf_counter() - t0
     t_apply = timed(apply, args.steps)
-    t_dvec = timed(lambda: L.call("fqehip_set_dvec", norb, nele, L.ptr(tc),
-                                  d_ptr, st), args.steps)
-    t_vd = timed(lambda: L.call("fqehip_set_contract", norb, nele, L.ptr(tv),
-                                d_ptr, st), args.steps)
-    apply()
-    torch.cuda.synchronize()
     got = out.cpu().numpy()
-    flops_vd = 8.0 * m2 * m2 * n
-    achieved = flops_vd / (t_vd * 1e-3) / 1e12
+    pairs = m * (m - 1) // 2
+    nmid = math.comb(m, nele - 2)
+    achieved = 8.0 * pairs * pairs * nmid / (t_apply * 1e-3) / 1e12
     line = {
         "metric": "FqeDataSet 1+2-body applies/s (spin-orbital, complex128)",
         "value": round(args.steps / wall, 3), "unit": "applies/s",
@@ -724,18 +706,14 @@ def set_main(args):
         "config": {"workload": (f"FqeDataSet nele={nele} norb={norb}: every "
                                 f"sector, {n} determinants, random Hermitian "
                                 f"spin-mixing h1/h2, seed 5")},
-        "kernels_ms": {"k_set_dvec": round(t_dvec, 4),
-                       "contract (k_set_expand_v + k_set_gemm)": round(t_vd, 4),
-                       "k_set_out": round(t_apply - t_dvec - t_vd, 4),
-                       "apply": round(t_apply, 4)},
-        "roofline": {"kernel": "k_set_gemm", "bound": "mfma",
+        "kernels_ms": {"apply": round(t_apply, 4)},
+        "roofline": {"kernel": "apply", "bound": "mfma",
                      "achieved": round(achieved, 3), "peak": 78.6,
                      "unit": "TFLOP/s", "frac": round(achieved / 78.6, 4),
-                     "traffic": (_traffic_block(SET_TRAFFIC_FILE).get(
-                         "k_set_gemm") if norb == 10 else None),
-                     "note": ("8 M^4 L algorithmic FP64 flops per "
-                              "contraction (real block GEMM, m = k = 2 M^2, "
-                              "L columns); time includes the V expansion")},
+                     "traffic": None,
+                     "note": ("8 (M (M - 1) / 2)^2 C(M, nele - 2) FP64 flops "
+                              "of the contraction over annihilated pairs; "
+                              "time of the whole apply")},
     }
     if not args.no_cpu_baseline:
         from oracle import fqe_set_oracle as so

@@ -194,7 +194,10 @@ class Wavefunction:
         """out = H psi + e_0 psi (reference ``src/fqe/wavefunction.py:
         366-399``); the e_0 term is fused into the scatter epilogue."""
         op = _prepared(hamil, array, self._norb)
-        out = self._shared_copy()
+        # a sector without an array to apply keeps its coefficients
+        out = (self._shared_copy() if any(isinstance(x, numpy.ndarray)
+                                          for x in array)
+               else copy.deepcopy(self))
         beta = e_0 if numpy.abs(e_0) > 1.e-15 else 0.0
         for sec in out._civec.values():
             sec.apply_inplace_scaled(array, alpha=1.0, beta=beta, op=op)
