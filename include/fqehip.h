@@ -293,6 +293,10 @@ int fqehip_spin_block(int complex_op, int npair, int64_t len,
  * rounded up to 16 rows of len, the last ones zero. */
 int fqehip_pull_table(int npair, int64_t len, const int32_t* d_fwd,
                       uint32_t* d_tab, void* stream);
+/* Words at the start of that table of the beta strings that the row kernel
+ * reads for a sector (of its sizes norb, nalpha, lenb and npull; no pointer is
+ * used); -1 if the kernel does not take the sector. */
+int64_t fqehip_pull_table_count(const fqehip_sector* s, int complex_op);
 /* Tables of W for the digit rows: fqehip_pull_digits_bytes(npull) bytes at
  * d_woz, npull <= 128, once per operator. */
 int64_t fqehip_pull_digits_bytes(int npull);

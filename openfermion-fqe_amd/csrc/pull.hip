@@ -288,6 +288,15 @@ constexpr uint32_t kPullNoRow = 0x80000000u;   // past the end of C
 
 constexpr int64_t kInRowMax = 5000;      // see pull_in_row
 
+// The first beta pair of pass ps of G W tiles.  Passes are equal, so 9 tiles run
+// as 2 x 5; the last pass begins early enough to end with the table of target
+// words (the bounds check of its loads does not cover the row part of their
+// address), with zeros for the rows of W that an earlier pass had.
+__host__ __device__ __forceinline__ int pull_pass_start(int ps, int G, int nq) {
+  const int last = 16 * ((nq + 15) / 16 - G);
+  return 16 * G * ps < last ? 16 * G * ps : last;
+}
+
 struct PullArgs {
   int norb, compressed, nele, nq;          // nq: pairs of one spin
   int64_t lena, lenb;
@@ -492,14 +501,16 @@ __device__ __forceinline__ void pull_row(const PullArgs& p, int64_t ia,
   if (p.ha) same_spin_row<CPLX>(p, ia, wave, nwave, lane, accs);
 
   for (int ps = 0; ps < p.pass; ++ps) {
-    const int q0 = 16 * G * ps;
-    // elements of rows past the live ones, of pairs past the last and of the
-    // folded row (next loop) are out of range and read zero
+    const int q0 = pull_pass_start(ps, G, p.nq);
+    const int qnew = 16 * G * ps;          // pairs before it: an earlier pass
+    // elements of rows past the live ones, of pairs past the last or of an
+    // earlier pass and of the folded row (next loop) are out of range and read
+    // zero
 #pragma unroll 4
     for (int f = wave; f < G * ks; f += nwave) {
       const int q = q0 + 16 * (f % G) + cl;
       const int k = 4 * (f / G) + kq;
-      const int off = k < noff && q < p.nq ? (lp[k] * p.nq + q) * (CPLX ? 16 : 8) : -1;
+      const int off = k < noff && q >= qnew && q < p.nq ? (lp[k] * p.nq + q) * (CPLX ? 16 : 8) : -1;
       const double sg = k < noff ? lsg[k] : 0.0;
       if (CPLX) {
         const double2 v = bload_d2(rw, off);
@@ -514,7 +525,7 @@ __device__ __forceinline__ void pull_row(const PullArgs& p, int64_t ia,
       const int q = q0 + 16 * t + cl;
       double vr = 0.0, vi = 0.0;
       for (int d = kq; d < p.nele; d += 4) {
-        const int off = q < p.nq ? (ldiag[d] * p.nq + q) * (CPLX ? 16 : 8) : -1;
+        const int off = q >= qnew && q < p.nq ? (ldiag[d] * p.nq + q) * (CPLX ? 16 : 8) : -1;
         if (CPLX) {
           const double2 v = bload_d2(rw, off);
           vr += v.x;
@@ -1021,6 +1032,22 @@ int launch_pull_group(const PullGroupLaunch& g, const void* d_secs, int step,
 }  // namespace fqehip
 
 using namespace fqehip;
+
+extern "C" int64_t fqehip_pull_table_count(const fqehip_sector* s, int complex_op) {
+  PullPlan pl;
+  if (!s || s->npull <= 0 || s->lenb <= 0 ||
+      !pull_plan(complex_op != 0, s->nalpha * (s->norb - s->nalpha), s->lenb,
+                 s->npull, &pl))
+    return -1;
+  // as the row kernel walks them: 16 rows of every tile of every pass
+  int end = 0;
+  for (int ps = 0; ps < pl.pass; ++ps) {
+    const int q0 = pull_pass_start(ps, pl.tiles, s->npull);
+    if (q0 < 0 || q0 > end) return -1;
+    end = q0 + 16 * pl.tiles;
+  }
+  return static_cast<int64_t>(end) * s->lenb;
+}
 
 extern "C" int fqehip_pull_table(int npair, int64_t len, const int32_t* d_fwd,
                                  uint32_t* d_tab, void* stream) {
