@@ -367,7 +367,8 @@ int64_t fqehip_apply_workspace_bytes(int precision, const fqehip_sector* s);
  * (src/fqe/fqe_data.py:421-475, :582-710) and Wavefunction._apply_array
  * (src/fqe/wavefunction.py:366-399).  d_workspace holds
  * fqehip_apply_workspace_bytes(); d_coeff may alias d_out only if
- * beta == 0. */
+ * beta == 0.  A complex128 d_coeff may alias d_acc (two-body operators:
+ * d_coeff is read in full before d_acc is written). */
 int fqehip_apply(int precision, const fqehip_sector* s,
                  const fqehip_operator* op, const void* d_coeff,
                  double alpha_re, double alpha_im, double beta_re,

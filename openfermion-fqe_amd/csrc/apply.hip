@@ -923,6 +923,13 @@ int pull_rows(const fqehip_sector* s, const fqehip_operator* op,
   return launch_pull_rows_oz(s, c, rowmax, rowacc, e, st, done);
 }
 
+// Whether the n bytes at a and those at b have some in common (a may be NULL).
+bool overlap(const void* a, const void* b, int64_t n) {
+  const char* x = static_cast<const char*>(a);
+  const char* y = static_cast<const char*>(b);
+  return x && x < y + n && y < x + n;
+}
+
 // fqehip_apply_fused_rows.
 int fused_rows(int precision, const fqehip_sector* s, const fqehip_operator* op,
                const void* d_coeff, void* d_workspace, const int32_t* d_done,
@@ -1040,9 +1047,11 @@ extern "C" int fqehip_apply(int precision, const fqehip_sector* s,
   if (fqehip_pull_supported(precision, s, op)) {
     FQEHIP_CHECK_ARG((beta_re == 0.0 && beta_im == 0.0) || d_cin,
                      "beta != 0 needs d_cin");
-    // the epilogue in the row kernel, except in place (other rows still read
-    // d_coeff) and for norm partials (one per 256 elements)
-    if (d_out != d_coeff && !d_norm_partials) {
+    // the epilogue in the row kernel, except where it would write what other
+    // rows still read (d_out or d_acc on d_coeff) and for norm partials (one per
+    // 256 elements)
+    if (!overlap(d_out, d_coeff, 16 * n) && !overlap(d_acc, d_coeff, 16 * n) &&
+        !d_norm_partials) {
       PullEpilogue e;
       e.alpha_re = alpha_re;
       e.alpha_im = alpha_im;

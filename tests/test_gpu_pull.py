@@ -268,3 +268,39 @@ def test_series_terms(fqe, na, nb, norb):
     with pytest.raises(RuntimeError):
         wfn.apply_generated_unitary(t, "taylor", ham, accuracy=1e-12,
                                     expansion=nterms)
+
+
+@pytest.mark.parametrize("kind", ["real", "complex"])
+@pytest.mark.parametrize("na,nb,norb", [(3, 3, 6), (6, 1, 12), (5, 5, 11)])
+def test_accumulate_onto_the_input(fqe, kind, na, nb, norb):
+    """acc += alpha H C where acc is C (and where it overlaps C in part):
+    every row of C is read before any is written.  In the row kernel's
+    epilogue it would race with the rows that still read C.  Sectors whose
+    rows run in one wave of workgroups and in several.  1e-13: the same
+    kernels as the separate buffers', other epilogue."""
+    import torch
+    from fqe_amd import _lib, engine
+    print(f"acc on input {kind} {na} {nb} {norb}", flush=True)
+    d, c, g, rng = sector(fqe, na, nb, norb, 3 * norb + na)
+    op = prepared(fqe, kind, tensors(kind, norb, rng), norb)
+    assert takes_pull(d, op)
+    x = d.device_coeff()
+    n = x.numel()
+    want = torch.empty_like(x)
+    engine.apply_sector(d.get_fcigraph(), x, op, want, alpha=0.5 - 2j)
+    want = want.cpu().numpy()
+    for shift in (0, n // 2):
+        # C at the start of a longer buffer, acc `shift` elements after it
+        buf = torch.zeros(2 * n, dtype=x.dtype, device=x.device)
+        buf[:n] = x.reshape(-1)
+        before = buf.cpu().numpy()
+        out = torch.empty_like(x)
+        s, keep = engine.sector_struct(d.get_fcigraph(), op, _lib.C128)
+        ws = engine.workspace(s, _lib.C128, x.device)
+        _lib.call("fqehip_apply", _lib.C128, engine._as_ref(s),
+                  engine._as_ref(op.c_struct()), _lib.ptr(buf), 0.5, -2.0,
+                  0.0, 0.0, None, _lib.ptr(out), _lib.ptr(buf) + 16 * shift,
+                  None, None, _lib.ptr(ws), _lib.stream_ptr())
+        before[shift:shift + n] += want.reshape(-1)
+        assert rel(out.cpu().numpy(), want) < 1e-13
+        assert rel(buf.cpu().numpy(), before) < 1e-13
