@@ -234,8 +234,60 @@ def device() -> torch.device:
     return torch.device("cuda", torch.cuda.current_device())
 
 
+raw_stream = torch._C._cuda_getCurrentRawStream
+
+
 def stream_ptr() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return raw_stream(torch.cuda.current_device())
+
+
+class TableCache:
+    """Device tables that kernels on one stream fill once and calls on any
+    stream read.  A stream other than the building one waits for the event
+    recorded after the build until that event has passed, and the tensors
+    are recorded on it, so that their memory outlives its kernels.  Under
+    capture a table that is missing is built as part of the graph and not
+    kept (nothing runs before the replay), and none is waited for: what was
+    built before has to be complete when a capture begins."""
+
+    def __init__(self, device: torch.device) -> None:
+        self._index = device.index
+        self._items = {}     # key -> [value, event or None, streams in order]
+
+    def get(self, key, build, *args):
+        """The value of ``key``, made by build(*args) if it is missing."""
+        item = self._items.get(key)
+        if item is None:
+            return self._add(key, build(*args))
+        if raw_stream(self._index) not in item[2]:
+            self._admit(item)
+        return item[0]
+
+    def _add(self, key, value):
+        if not torch.cuda.is_current_stream_capturing():
+            event = torch.cuda.Event()
+            event.record()
+            self._items[key] = [value, event, {raw_stream(self._index)}]
+        return value
+
+    def _admit(self, item) -> None:
+        if torch.cuda.is_current_stream_capturing():
+            return
+        stream = torch.cuda.current_stream(self._index)
+        event = item[1]
+        if event is not None and event.query():
+            event = item[1] = None
+        if event is not None:
+            stream.wait_event(event)
+        else:
+            item[2].add(stream.cuda_stream)
+        value = item[0] if isinstance(item[0], (tuple, list)) else item[:1]
+        for t in value:
+            if isinstance(t, torch.Tensor):
+                t.record_stream(stream)
+
+    def __len__(self) -> int:
+        return len(self._items)
 
 
 def ptr(t) -> int:

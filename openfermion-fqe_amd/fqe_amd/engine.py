@@ -46,67 +46,65 @@ class PreparedOperator:
         # opposite-spin coupling W[p][q] = V[p][q] + V[q][p] (device, alpha
         # pair p, beta pair q) of a two-body operator: the pull form
         self.coupling: Optional[torch.Tensor] = None
-        self._pull = {}
-        self._hbb = {}
+        on = a if a is not None else h1
+        self._tables = _lib.TableCache(on.device)
 
     def beta_block(self, graph):
         """Beta-beta block of this operator on the beta strings of
         ``graph`` (fqehip_beta_block): (bfloat16 hi, bfloat16 lo, ldh, beta
-        forward table, FP64 columns), cached per (nbeta, device); None when
-        the split apply does not apply."""
+        forward table, FP64 columns, the GEMM matrix), cached per nbeta;
+        None when the split apply does not apply."""
         if not self.pair_symmetric or self.a is None or self.complex_op:
             return None
         lenb = graph.lenb()
         if (lenb + self.npair) * 8 > 160 * 1024:
             return None
-        key = (graph.nbeta(), self.a.device.index)
-        if key not in self._hbb:
-            fwb, _ = graph.tables(False).fused_tables(self.compressed)
-            ldh = int(_lib.call("fqehip_beta_block_ld", lenb))
-            hcol = torch.empty((lenb, lenb), dtype=torch.float64,
-                               device=self.a.device)
-            hhi = torch.empty((ldh, ldh), dtype=torch.int16,
-                              device=self.a.device)
-            hlo = torch.empty_like(hhi)
-            _lib.call("fqehip_beta_block", self.npair, lenb, _lib.ptr(fwb),
-                      _lib.ptr(self.a), _lib.ptr(hcol), _lib.ptr(hhi),
-                      _lib.ptr(hlo), ldh, _lib.stream_ptr())
-            self._hbb[key] = (hhi, hlo, ldh, fwb, hcol)
-        return self._hbb[key]
+        return self._tables.get(("hbb", graph.nbeta()), self._build_hbb,
+                                graph.tables(False))
+
+    def _build_hbb(self, tables):
+        lenb = tables.length
+        fwb, _ = tables.fused_tables(self.compressed)
+        ldh = int(_lib.call("fqehip_beta_block_ld", lenb))
+        hcol = torch.empty((lenb, lenb), dtype=torch.float64,
+                           device=self.a.device)
+        hhi = torch.empty((ldh, ldh), dtype=torch.int16, device=self.a.device)
+        hlo = torch.empty_like(hhi)
+        _lib.call("fqehip_beta_block", self.npair, lenb, _lib.ptr(fwb),
+                  _lib.ptr(self.a), _lib.ptr(hcol), _lib.ptr(hhi),
+                  _lib.ptr(hlo), ldh, _lib.stream_ptr())
+        return hhi, hlo, ldh, fwb, hcol, self.a
 
     def pull_digits(self, graph):
         """Digits of the pull form (W, Haa, Hbb; fqehip_pull_digits and
         fqehip_beta_block_digits) on the sector of ``graph``, cached per
-        (electron count, device); None where the digit kernels do not
-        apply."""
+        electron count; None where the digit kernels do not apply."""
         tabs = self.pull_tables(graph)
         if (tabs is None or self.complex_op or self.spin
                 or not self.pair_symmetric or self.coupling.shape[0] > 128
                 or max(graph.lena(), graph.lenb()) >= 26214):
             return None
-        dev = self.a.device
-        if "w_oz" not in self._pull:
-            npull = self.coupling.shape[0]
-            woz = torch.empty(int(_lib.call("fqehip_pull_digits_bytes",
-                                            npull)),
-                              dtype=torch.uint8, device=dev)
-            _lib.call("fqehip_pull_digits", npull, _lib.ptr(self.coupling),
-                      _lib.ptr(woz), _lib.stream_ptr())
-            self._pull["w_oz"] = woz
-        out = [self._pull["w_oz"]]
-        for nele, block in ((graph.nalpha(), tabs[1]),
-                            (graph.nbeta(), tabs[2])):
-            key = ("digits", nele, dev.index)
-            if key not in self._pull:
-                n = block.shape[0]
-                nbytes = int(_lib.call("fqehip_beta_block_digits_bytes", n))
-                hoz = torch.empty(max(nbytes, 16), dtype=torch.uint8,
-                                  device=dev)
-                _lib.call("fqehip_beta_block_digits", n, _lib.ptr(block),
-                          _lib.ptr(hoz), _lib.stream_ptr())
-                self._pull[key] = hoz
-            out.append(self._pull[key])
-        return out
+        return [self._tables.get("w_oz", self._build_coupling_digits)] + [
+            self._tables.get(("digits", nele), self._build_block_digits, block)
+            for nele, block in ((graph.nalpha(), tabs[1]),
+                                (graph.nbeta(), tabs[2]))]
+
+    def _build_coupling_digits(self) -> torch.Tensor:
+        npull = self.coupling.shape[0]
+        woz = torch.empty(int(_lib.call("fqehip_pull_digits_bytes", npull)),
+                          dtype=torch.uint8, device=self.a.device)
+        _lib.call("fqehip_pull_digits", npull, _lib.ptr(self.coupling),
+                  _lib.ptr(woz), _lib.stream_ptr())
+        return woz
+
+    def _build_block_digits(self, block: torch.Tensor) -> torch.Tensor:
+        n = block.shape[0]
+        nbytes = int(_lib.call("fqehip_beta_block_digits_bytes", n))
+        hoz = torch.empty(max(nbytes, 16), dtype=torch.uint8,
+                          device=self.a.device)
+        _lib.call("fqehip_beta_block_digits", n, _lib.ptr(block),
+                  _lib.ptr(hoz), _lib.stream_ptr())
+        return hoz
 
     def _spin_block(self, tables, alpha: bool) -> torch.Tensor:
         """Matrix of this two-body operator on the strings of one spin, by
@@ -129,8 +127,8 @@ class PreparedOperator:
 
     def pull_tables(self, graph):
         """(W, Haa, Hbb, beta target words, alpha de-excitation rows) of
-        the pull form on the sector of ``graph``, cached per (nalpha, nbeta,
-        device); None where the form does not apply (one-body operators,
+        the pull form on the sector of ``graph``, cached per (nalpha,
+        nbeta); None where the form does not apply (one-body operators,
         sectors past its limits)."""
         na, nb, norb = graph.nalpha(), graph.nbeta(), graph.norb()
         if (self.coupling is None or na * (norb - na + 1) > 64
@@ -140,20 +138,17 @@ class PreparedOperator:
         if ((max(graph.lena(), graph.lenb()) + self.coupling.shape[0]) * width
                 > 160 * 1024):
             return None
-        key = (na, nb, self.a.device.index)
-        if key not in self._pull:
-            ta, tb = graph.tables(True), graph.tables(False)
-            blocks = []
-            for nele, tab, alpha in ((na, ta, True), (nb, tb, False)):
-                # restricted operators: one matrix per electron count
-                side = ("side", alpha if self.spin else None, nele,
-                        self.a.device.index)
-                if side not in self._pull:
-                    self._pull[side] = self._spin_block(tab, alpha)
-                blocks.append(self._pull[side])
-            self._pull[key] = (self.coupling, blocks[0], blocks[1],
-                               tb.pull_table(self.compressed), ta.dexc)
-        return self._pull[key]
+        return self._tables.get((na, nb), self._build_pull, graph)
+
+    def _build_pull(self, graph):
+        ta, tb = graph.tables(True), graph.tables(False)
+        # restricted operators: one matrix per electron count
+        haa, hbb = (
+            self._tables.get(("side", alpha if self.spin else None, tab.nele),
+                             self._spin_block, tab, alpha)
+            for tab, alpha in ((ta, True), (tb, False)))
+        return (self.coupling, haa, hbb, tb.pull_table(self.compressed),
+                ta.dexc)
 
     def c_struct(self) -> _lib.Operator:
         return _lib.Operator(int(self.complex_op), _lib.ptr(self.a),

@@ -32,31 +32,43 @@ class SpinTables:
         self.length = comb(norb, nele)
         self.nexc = nele * (norb - nele + 1)
         self.device = device
-        self.strings = torch.empty(self.length, dtype=torch.int64,
-                                   device=device)
-        self.dexc = torch.empty((self.length, self.nexc, 3),
-                                dtype=torch.int32, device=device)
-        _lib.call("fqehip_string_tables", norb, nele, self.length,
-                  _lib.ptr(self.strings),
-                  _lib.ptr(self.dexc) if self.dexc.numel() else None,
-                  _lib.stream_ptr())
-        self._ptab = {}
+        self._tables = _lib.TableCache(device)
         self._maps = None
         self._map_offsets = None
+        self._base()
+
+    def _base(self) -> Tuple[torch.Tensor, torch.Tensor]:
+        """(strings, de-excitation rows)"""
+        return self._tables.get("base", self._build_base)
+
+    def _build_base(self) -> Tuple[torch.Tensor, torch.Tensor]:
+        strings = torch.empty(self.length, dtype=torch.int64,
+                              device=self.device)
+        dexc = torch.empty((self.length, self.nexc, 3), dtype=torch.int32,
+                           device=self.device)
+        _lib.call("fqehip_string_tables", self.norb, self.nele, self.length,
+                  _lib.ptr(strings), _lib.ptr(dexc) if dexc.numel() else None,
+                  _lib.stream_ptr())
+        return strings, dexc
+
+    strings = property(lambda self: self._base()[0])
+    dexc = property(lambda self: self._base()[1])
 
     def pair_table(self, compressed: bool) -> torch.Tensor:
         """int32 [npair][length]: sign*(source+1) or 0 (see fqehip.h)."""
-        key = bool(compressed)
-        if key not in self._ptab:
-            npair = (self.norb * (self.norb + 1) // 2 if compressed else
-                     self.norb * self.norb)
-            tab = torch.empty((npair, self.length), dtype=torch.int32,
-                              device=self.device)
-            _lib.call("fqehip_pair_table", self.norb, self.nele, self.length,
-                      _lib.ptr(self.dexc) if self.dexc.numel() else None,
-                      int(key), _lib.ptr(tab), _lib.stream_ptr())
-            self._ptab[key] = tab
-        return self._ptab[key]
+        return self._tables.get(bool(compressed), self._build_pairs,
+                                compressed)
+
+    def _build_pairs(self, compressed: bool) -> torch.Tensor:
+        npair = (self.norb * (self.norb + 1) // 2 if compressed else
+                 self.norb * self.norb)
+        dexc = self.dexc
+        tab = torch.empty((npair, self.length), dtype=torch.int32,
+                          device=self.device)
+        _lib.call("fqehip_pair_table", self.norb, self.nele, self.length,
+                  _lib.ptr(dexc) if dexc.numel() else None,
+                  int(bool(compressed)), _lib.ptr(tab), _lib.stream_ptr())
+        return tab
 
     def spin_pair_table(self, first: bool) -> torch.Tensor:
         """int32 [2 norb^2][length]: the full-basis pair table of this spin
@@ -64,43 +76,45 @@ class SpinTables:
         the other, so that pair p < norb^2 excites alpha strings only and
         p >= norb^2 beta strings only (spin-orbital operators on one
         sector)."""
-        key = ("spin", bool(first))
-        if key not in self._ptab:
-            pt = self.pair_table(False)
-            zero = torch.zeros_like(pt)
-            self._ptab[key] = torch.cat([pt, zero] if first else [zero, pt])
-        return self._ptab[key]
+        return self._tables.get(("spin", bool(first)), self._build_spin_pairs,
+                                first)
+
+    def _build_spin_pairs(self, first: bool) -> torch.Tensor:
+        pt = self.pair_table(False)
+        zero = torch.zeros_like(pt)
+        return torch.cat([pt, zero] if first else [zero, pt])
 
     def fused_tables(self, compressed: bool):
         """(forward table, slot table) of the fused apply, int32
         [npair][length] each (see fqehip_fused_tables)."""
-        key = ("fused", bool(compressed))
-        if key not in self._ptab:
-            pt = self.pair_table(compressed)
-            fwd = torch.empty_like(pt)
-            slot = torch.empty_like(pt)
-            if pt.numel():
-                _lib.call("fqehip_fused_tables", self.norb, self.nele,
-                          self.length,
-                          _lib.ptr(self.dexc) if self.dexc.numel() else None,
-                          int(bool(compressed)), _lib.ptr(pt), _lib.ptr(fwd),
-                          _lib.ptr(slot), _lib.stream_ptr())
-            self._ptab[key] = (fwd, slot)
-        return self._ptab[key]
+        return self._tables.get(("fused", bool(compressed)), self._build_fused,
+                                compressed)
+
+    def _build_fused(self, compressed: bool):
+        pt, dexc = self.pair_table(compressed), self.dexc
+        fwd = torch.empty_like(pt)
+        slot = torch.empty_like(pt)
+        if pt.numel():
+            _lib.call("fqehip_fused_tables", self.norb, self.nele, self.length,
+                      _lib.ptr(dexc) if dexc.numel() else None,
+                      int(bool(compressed)), _lib.ptr(pt), _lib.ptr(fwd),
+                      _lib.ptr(slot), _lib.stream_ptr())
+        return fwd, slot
 
     def pull_table(self, compressed: bool) -> torch.Tensor:
         """Target words of the pull form (fqehip_pull_table), int32 [npair
         rounded up to 16][length]."""
-        key = ("pull", bool(compressed))
-        if key not in self._ptab:
-            fwd, _ = self.fused_tables(compressed)
-            tab = torch.empty(((fwd.shape[0] + 15) // 16 * 16, self.length),
-                              dtype=torch.int32, device=self.device)
-            if fwd.numel():
-                _lib.call("fqehip_pull_table", fwd.shape[0], self.length,
-                          _lib.ptr(fwd), _lib.ptr(tab), _lib.stream_ptr())
-            self._ptab[key] = tab
-        return self._ptab[key]
+        return self._tables.get(("pull", bool(compressed)), self._build_pull,
+                                compressed)
+
+    def _build_pull(self, compressed: bool) -> torch.Tensor:
+        fwd, _ = self.fused_tables(compressed)
+        tab = torch.empty(((fwd.shape[0] + 15) // 16 * 16, self.length),
+                          dtype=torch.int32, device=self.device)
+        if fwd.numel():
+            _lib.call("fqehip_pull_table", fwd.shape[0], self.length,
+                      _lib.ptr(fwd), _lib.ptr(tab), _lib.stream_ptr())
+        return tab
 
     def map_lengths(self) -> numpy.ndarray:
         n, k = self.norb, self.nele
