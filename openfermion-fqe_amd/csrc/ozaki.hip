@@ -16,7 +16,9 @@
 // are the digits d_0..d_5 of weights 1 .. 2^40.  d_0..d_4 are stored as
 // unsigned bytes minus 128 (one XOR), d_5 as the signed top byte, so no carry
 // propagation is needed; the 128 offsets are added back exactly, for every
-// digit pair, through the sums of the operator integers.
+// digit pair, through the sums of the operator integers.  Data that are all zero
+// have no scale and get a zero factor on the way back: the offsets of the
+// digit pairs that are not formed (below) would be left in the result.
 //
 // Products.  Of the 30 digit pairs, the 20 with i - t >= 0 (weight >= 2^32
 // of a maximum of 2^72) are formed, six int32 accumulators per output (one
@@ -269,7 +271,7 @@ __global__ void __launch_bounds__(kRowThreads, 2) k_pull_rows_oz(OzRowsArgs p) {
   double* gsa = reinterpret_cast<double*>(start + 3 * kOzQ);  // [kOzK] sign 2^ed
   uint32_t* goff = reinterpret_cast<uint32_t*>(gsa + kOzK);
   int32_t* lp = reinterpret_cast<int32_t*>(goff + kOzK);
-  int32_t* scale = lp + kOzK;                           // ed
+  double* scale = reinterpret_cast<double*>(lp + kOzK);  // 2^-ed
   const int nexc = p.nalpha * (p.norb - p.nalpha + 1);
 
   if (wave == 0) {
@@ -293,7 +295,7 @@ __global__ void __launch_bounds__(kRowThreads, 2) k_pull_rows_oz(OzRowsArgs p) {
     lp[lane] = lane < nexc ? (p.compressed ? comp_pair(i, j) : ij) : -1;
     goff[lane] = lane < nexc ? static_cast<uint32_t>(src) * static_cast<uint32_t>(lenb) : kNoRow16;
     gsa[lane] = static_cast<double>(sg) * ldexp(1.0, e);
-    if (lane == 0) *scale = e;
+    if (lane == 0) *scale = m > 0.0 ? ldexp(1.0, -e) : 0.0;
   }
   __syncthreads();
   {
@@ -456,7 +458,7 @@ __global__ void __launch_bounds__(kRowThreads, 2) k_pull_rows_oz(OzRowsArgs p) {
     __builtin_amdgcn_s_setprio(0);
   }
   __syncthreads();
-  const double back = ldexp(1.0, 32 - *p.ea - *scale);
+  const double back = ldexp(*scale, 32 - *p.ea);
   double2* racc = reinterpret_cast<double2*>(p.rowacc) + ia * p.lenb;
   double sq = 0.0;
   for (int x = tid; x < lenb; x += kRowThreads) {
@@ -598,7 +600,7 @@ k_c_digits(int64_t lena, int64_t lenb, int64_t ldk,
     (void)frexp(mx, &e);
     ec = 46 - e;
   }
-  if (g == 0) cscale[ia] = ldexp(1.0, -ec);
+  if (g == 0) cscale[ia] = mx > 0.0 ? ldexp(1.0, -ec) : 0.0;
   const double sc = ldexp(1.0, ec);
   uint32_t lre[4], hre[4], lim[4], him[4];
 #pragma unroll
@@ -649,7 +651,8 @@ k_ct_digits(int64_t lena, int64_t lenb, int64_t ldk,
     (void)frexp(mx, &e);
     ec = 46 - e;
   }
-  if (a0 == 0 && threadIdx.x < kCtB && jb < lenb) cscale[jb] = ldexp(1.0, -ec);
+  if (a0 == 0 && threadIdx.x < kCtB && jb < lenb)
+    cscale[jb] = mx > 0.0 ? ldexp(1.0, -ec) : 0.0;
   const double sc = ldexp(1.0, ec);
   for (int g = threadIdx.x / kCtB; g < kW; g += 256 / kCtB) {
     uint32_t lre[4], hre[4], lim[4], him[4];

@@ -181,6 +181,45 @@ def test_digit_rows_edges(fqe, na, nb, norb, blocks, shape):
     assert numpy.array_equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("blocks", [True, False])
+@pytest.mark.parametrize("zero", ["alpha", "beta", "both", "all"])
+@pytest.mark.parametrize("na,nb,norb", [(4, 3, 8), (3, 5, 9), (5, 5, 10)])
+def test_digit_rows_with_empty_strings(fqe, na, nb, norb, zero, blocks):
+    """Alpha strings, beta strings, or both without any amplitude (every
+    string that occupies orbital 0), and a vector of zeros: a zero row or
+    column of C has no digit scale.  Tolerance as in test_digit_rows_edges;
+    of zeros, exactly zeros."""
+    from fqe_amd import settings
+    print(f"empty strings {na} {nb} {norb} {zero} {blocks}", flush=True)
+    d, c, g, rng = sector(fqe, na, nb, norb, 11 * norb + 5 * na + nb)
+    h = tensors("real", norb, rng)
+    c = c.copy()
+    core = d.get_fcigraph()
+    if zero in ("alpha", "both"):
+        c[core.string_alpha_all() & numpy.uint64(1) == 1, :] = 0.0
+    if zero in ("beta", "both"):
+        c[:, core.string_beta_all() & numpy.uint64(1) == 1] = 0.0
+    if zero == "all":
+        c[:] = 0.0
+    d.coeff = c
+    op = prepared(fqe, "real", h, norb)
+    saved = (settings.contraction, settings.ozaki_beta,
+             settings.ozaki_min_determinants)
+    settings.contraction, settings.ozaki_beta = "ozaki", blocks
+    settings.ozaki_min_determinants = 0
+    try:
+        e = copy.deepcopy(d)
+        e.apply_inplace_scaled(h, op=op)
+    finally:
+        (settings.contraction, settings.ozaki_beta,
+         settings.ozaki_min_determinants) = saved
+    d.apply_inplace_scaled(h, op=op)
+    if zero == "all":
+        assert not e.coeff.any()
+    else:
+        assert rel(e.coeff, d.coeff) < 3e-11
+
+
 @pytest.mark.parametrize("nterms", [0, 1, 2, 5])
 @pytest.mark.parametrize("group", [True, False])
 def test_batch_terms(fqe, nterms, group):
