@@ -298,7 +298,10 @@ int fqehip_pull_table(int npair, int64_t len, const int32_t* d_fwd,
  * used); -1 if the kernel does not take the sector. */
 int64_t fqehip_pull_table_count(const fqehip_sector* s, int complex_op);
 /* Tables of W for the digit rows: fqehip_pull_digits_bytes(npull) bytes at
- * d_woz, npull <= 128, once per operator. */
+ * d_woz, npull <= 128, once per operator.  Each row of W (all alpha pairs of
+ * one beta pair) is rounded to 2^-39 of its largest element; the products are
+ * summed as integers whose unit is finer than that for rows whose largest
+ * element is above 2^-23 sum |W|. */
 int64_t fqehip_pull_digits_bytes(int npull);
 int fqehip_pull_digits(int npull, const double* d_w, void* d_woz, void* stream);
 /* Whether fqehip_apply takes the pull form for this sector and operator. */

@@ -32,6 +32,8 @@
 //
 // Reference: lm_apply_array12_same_spin_opt / lm_apply_array12_diff_spin_opt
 // (src/fqe/lib/fqe_data.c:668-720, :879-996), in complex128.
+#include <type_traits>
+
 #include "fqehip_common.h"
 #include "pull_common.h"
 #include "rows_common.h"
@@ -143,15 +145,32 @@ constexpr uint32_t kNoRow16 = 0x7ff0000u;
 
 // Tables of W for the row kernel, once per operator: the digits of every
 // alpha pair's column, dig[p][t][q] bytes (t: digit of weight 2^(8(4 - t))),
-// the integers z[p][q] = rint(W 2^ea) as doubles, and ea, one for all of W:
-// |z| < 2^38, and sum_pq |z| < 2^49, so that a sum over any (p, q) of z times
-// 46-bit data, in units of 2^32, stays below 2^63.  One workgroup per pair p,
-// thread q; every workgroup forms the maximum and the sum anew, in one order.
+// the integers z[p][q] = rint(W 2^ea[q]) as doubles, |z| < 2^38, each row q with
+// the scale of its own largest element; the exponent e of the accumulators'
+// unit 2^(32 - e) (in units of the data), one for all of W: sum_pq |W| 2^e <
+// 2^49, so that a sum over any (p, q) of W 2^e times 46-bit data, in units of
+// 2^32, stays below 2^63; and what takes a row's products to that unit, shifts
+// to the right by ea[q] - e as bytes.  Without left shifts e is at most the
+// smallest ea, which is as fine as the digits of rows down to 2^-12 of the
+// largest one (the sums' rounding, a few units, is then 2^-49 of the largest
+// row, theirs 2^-38 of their own); beside a row that is smaller still, e is 12
+// below that row's ea, or at the limit of the sum, and the left_rows rows above
+// it shift to the left.
+// ea[q] is held to e + 31, where a whole row's digits are finer than the unit.  One
+// workgroup per pair p, thread q; every workgroup forms the maximum and the
+// sum anew, in one order.
+struct OzUnit {
+  int32_t e;
+  uint32_t left_rows;
+  uint8_t right[kOzQ], left[kOzQ];
+};
 constexpr int64_t kWDigBytes = static_cast<int64_t>(kOzADig) * kOzQ;
 __global__ void __launch_bounds__(kOzQ)
 k_pull_digits(int npull, const double* __restrict__ w, uint8_t* __restrict__ dig,
-              double* __restrict__ z, int32_t* __restrict__ ea) {
+              double* __restrict__ z, OzUnit* __restrict__ unit) {
   __shared__ double red[2][kOzQ / 64];
+  __shared__ uint32_t rows;
+  __shared__ int least[kOzQ / 64];
   const int p = blockIdx.x;
   const int q = threadIdx.x;
   double m = 0.0, t = 0.0;
@@ -163,28 +182,51 @@ k_pull_digits(int npull, const double* __restrict__ w, uint8_t* __restrict__ dig
       t += v;
     }
   }
+  const double mq = m;
+  int emin = 4096;                         // exponent of the smallest row
+  if (mq > 0.0) (void)frexp(mq, &emin);
+  if (q == 0) rows = 0;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     m = fmax(m, __shfl_xor(m, o));
     t += __shfl_xor(t, o);
+    const int x = __shfl_xor(emin, o);
+    emin = x < emin ? x : emin;
   }
   if ((q & 63) == 0) {
     red[0][q >> 6] = m;
     red[1][q >> 6] = t;
+    least[q >> 6] = emin;
   }
   __syncthreads();
+  emin = least[0] < least[1] ? least[0] : least[1];
   m = fmax(red[0][0], red[0][1]);
   t = red[1][0] + red[1][1];
-  int e = 0;
+  int e = 0, eq = 0;
   if (m > 0.0) {
     int em, et;
     (void)frexp(m, &em);
-    (void)frexp(t, &et);
-    e = 38 - em < 49 - et ? 38 - em : 49 - et;
+    (void)frexp(t * (1.0 + 0x1p-20), &et);   // the z are rounded
+    e = em - emin > 12 ? 26 - emin : 38 - em;
+    e = e < 49 - et ? e : 49 - et;
+    eq = e;
+    if (mq > 0.0) {
+      (void)frexp(mq, &em);
+      eq = 38 - em < e + 31 ? 38 - em : e + 31;
+    }
   }
-  int64_t v = q < npull ? static_cast<int64_t>(rint(ldexp(w[static_cast<int64_t>(p) * npull + q], e))) : 0;
+  int64_t v = q < npull ? static_cast<int64_t>(rint(ldexp(w[static_cast<int64_t>(p) * npull + q], eq))) : 0;
   z[static_cast<int64_t>(p) * kOzQ + q] = static_cast<double>(v);
-  if (p == 0 && q == 0) *ea = e;
+  if (p == 0) {
+    if (eq < e) atomicAdd(&rows, 1u);
+    unit->right[q] = static_cast<uint8_t>(eq > e ? eq - e : 0);
+    unit->left[q] = static_cast<uint8_t>(eq < e ? e - eq : 0);
+    __syncthreads();                       // p is the workgroup's
+    if (q == 0) {
+      unit->e = e;
+      unit->left_rows = rows;
+    }
+  }
 #pragma unroll
   for (int t5 = kOzADig - 1; t5 >= 0; --t5) {
     const int64_t d = t5 ? ((v + 128) & 255) - 128 : v;
@@ -210,25 +252,30 @@ k_pull_digits(int npull, const double* __restrict__ w, uint8_t* __restrict__ dig
 // A operands.  i8 MFMA layouts: lane l holds A[row l%16][k 16 (l/16) + j] and
 // B[k 16 (l/16) + j][col l%16]; output item e is [row 4 (l/16) + e][col l%16].
 //
-// W has one scale and the data of ia one, so all of the row's Z have one
-// unit, 2^(32 - ea - ed): a value is the 64-bit integer sum_m 2^(8m) acc_m,
-// assembled with 32-bit integer operations, and is added to its target's
-// 64-bit accumulator in LDS as it is (ds_add_u64).  Integer addition has no
-// order, so the waves need no turns and every run gives the same bits, and
-// nothing is rounded after the digits were cut.  A negative sign of E^b_q is
-// one XOR (-v - 1, one unit off).  With per-row scales and FP64 assembly (four
-// v_cvt_f64_i32 per value) the kernel took 3.7 ms at norb 14 7a7b instead of
-// 3.4; without the products 2.4, without the additions 2.4, set-up alone 0.24
-// (the slot-row form of the same products: 4.0 + 1.3 for its reduction).  Two
-// waves per SIMD fit (256 registers), so products and additions overlap only
-// in part.
+// A value is the 64-bit integer sum_m 2^(8m) acc_m in its row's unit
+// 2^(32 - ea[q] - ed), assembled with 32-bit integer operations and shifted
+// to the accumulators' unit 2^(32 - e - ed); it is added to its target's
+// 64-bit accumulator in LDS (ds_add_u64).  Integer addition has no order, so the
+// waves need no turns and every run gives the same bits.  The shift rounds down
+// and a negative sign of E^b_q is one XOR (-v - 1), half a unit low on average
+// each way, so the accumulators start at half a unit for each excitation that
+// reaches them; what is left is a few units.  The shift keeps the digits of a row
+// as fine as its own largest element allows (one scale for all of W would round
+// every row as the largest one, 0 to 3 bits for integrals of canonical orbitals,
+// and the whole ratio beside one large local integral).  norb 14 7a7b: 3.1 ms,
+// with the shift and, signed halves extended instead, without it; 3.7 with FP64
+// assembly (four v_cvt_f64_i32 per value);
+// without the products 2.4, without the additions 2.4, set-up alone 0.24 (the
+// slot-row form of the same products: 4.0 + 1.3 for its reduction).  Two waves
+// per SIMD fit (256 registers), so products and additions overlap only in part.
 struct OzRowsArgs {
   int norb, compressed, nalpha, nq, nqt;
   int64_t lena, lenb;
   const uint8_t* dig;
   const double* z;
-  const int32_t* ea;
+  const OzUnit* unit;
   const int32_t* dexc;
+  int half;                                // accumulators' start value
   const uint32_t* fwd;
   const double* coeff;
   const double* rowmax;
@@ -248,7 +295,7 @@ constexpr int kOzPartBytes = 4 * kOzQ * 8;   // set-up scratch
 size_t oz_rows_lds_bytes(int64_t lenb, int nqt) {
   const size_t acc = static_cast<size_t>(lenb) * 16;
   return (acc > kOzPartBytes ? acc : kOzPartBytes) +
-         static_cast<size_t>(kOzADig) * 16 * nqt * kOzARow + 3 * kOzQ * 4 +
+         static_cast<size_t>(kOzADig) * 16 * nqt * kOzARow + 3 * kOzQ * 4 + 2 * kOzQ +
          kOzK * (8 + 4 + 4) + 16;
 }
 
@@ -268,7 +315,8 @@ __global__ void __launch_bounds__(kRowThreads, 2) k_pull_rows_oz(OzRowsArgs p) {
   double* part = reinterpret_cast<double*>(smem);       // set-up: [4][kOzQ]
   uint8_t* adig = reinterpret_cast<uint8_t*>(smem + accb);   // [5][nqp][kOzARow]
   int32_t* start = reinterpret_cast<int32_t*>(adig + kOzADig * nqp * kOzARow);  // [3][kOzQ]
-  double* gsa = reinterpret_cast<double*>(start + 3 * kOzQ);  // [kOzK] sign 2^ed
+  uint32_t* shift = reinterpret_cast<uint32_t*>(start + 3 * kOzQ);   // right, left: bytes
+  double* gsa = reinterpret_cast<double*>(shift + kOzQ / 2);  // [kOzK] sign 2^ed
   uint32_t* goff = reinterpret_cast<uint32_t*>(gsa + kOzK);
   int32_t* lp = reinterpret_cast<int32_t*>(goff + kOzK);
   double* scale = reinterpret_cast<double*>(lp + kOzK);  // 2^-ed
@@ -338,12 +386,15 @@ __global__ void __launch_bounds__(kRowThreads, 2) k_pull_rows_oz(OzRowsArgs p) {
     const int64_t v4 = (v + (int64_t(1) << 31)) >> 32;
     const int64_t r4 = v - (v4 << 32);
     const int64_t v2 = (r4 + (1 << 15)) >> 16;
-    start[tid] = static_cast<int32_t>(r4 - (v2 << 16));
-    start[kOzQ + tid] = static_cast<int32_t>(v2);
-    start[2 * kOzQ + tid] = static_cast<int32_t>(v4);
+    // 2^31 + 2^16 (2^31 + 2^15) - 2^32 (2^15 + 1) = 0: so that the first two pairs
+    // of classes need no sign extension
+    start[tid] = static_cast<int32_t>(r4 - (v2 << 16) + (int64_t(1) << 31));
+    start[kOzQ + tid] = static_cast<int32_t>(v2 + (int64_t(1) << 31) + (1 << 15));
+    start[2 * kOzQ + tid] = static_cast<int32_t>(v4 - (1 << 15) - 1);
   }
+  if (tid < kOzQ / 2) shift[tid] = reinterpret_cast<const uint32_t*>(p.unit->right)[tid];
   __syncthreads();
-  for (int x = tid; x < 2 * lenb; x += kRowThreads) accs[x] = 0;
+  for (int x = tid; x < 2 * lenb; x += kRowThreads) accs[x] = p.half;
   __syncthreads();
 
   const __amdgpu_buffer_rsrc_t rc = buffer_of(p.coeff, p.lena * p.lenb * 16);
@@ -362,6 +413,9 @@ __global__ void __launch_bounds__(kRowThreads, 2) k_pull_rows_oz(OzRowsArgs p) {
     A[2] = __builtin_amdgcn_raw_buffer_load_b128(rc, static_cast<int>((g.z + ib) << 4), 0, 0);
     A[3] = __builtin_amdgcn_raw_buffer_load_b128(rc, static_cast<int>((g.w + ib) << 4), 0, 0);
   };
+  // LEFT: some rows shift to the left.  A whole second loop, so that the usual
+  // one has no more than its right shifts (as a condition per value 4% slower)
+  auto run = [&](auto LEFT) {
   load(0, 0, la[0]);
   load(0, 1, la[1]);
   for (int chunk = 0; chunk < nchunks; ++chunk) {
@@ -432,6 +486,8 @@ __global__ void __launch_bounds__(kRowThreads, 2) k_pull_rows_oz(OzRowsArgs p) {
             if (t <= i)
               acc[c][i - t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
                   a[t], dd[c][i], acc[c][i - t], 0, 0, 0);
+      const uint32_t right = shift[4 * r + kq];
+      const uint32_t left = LEFT ? shift[kOzQ / 4 + 4 * r + kq] : 0u;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const uint32_t f = fw[r][e];
@@ -440,25 +496,32 @@ __global__ void __launch_bounds__(kRowThreads, 2) k_pull_rows_oz(OzRowsArgs p) {
         const uint32_t sg = static_cast<uint32_t>(static_cast<int32_t>(f) >> 31);
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
-          // classes merged in pairs in int32: with K <= 64 the odd classes
-          // are below 2^22.4 (at most five products of 64 x 2^14)
-          const int32_t m10 = acc[c][1][e] * 256 + acc[c][0][e];
-          const int32_t m32 = acc[c][3][e] * 256 + acc[c][2][e];
-          const int32_t m54 = acc[c][5][e] * 256 + acc[c][4][e];
-          const int64_t v = static_cast<int64_t>(m10) + (static_cast<int64_t>(m32) << 16);
-          const uint32_t lo = static_cast<uint32_t>(v) ^ sg;
-          const uint32_t hi = (static_cast<uint32_t>(v >> 32) + static_cast<uint32_t>(m54)) ^ sg;
-          __hip_atomic_fetch_add(to + c,
-                                 static_cast<unsigned long long>(lo) |
-                                     (static_cast<unsigned long long>(hi) << 32),
+          // classes merged in pairs in 32 bits: with K <= 64 the odd classes
+          // are below 2^22.4 (at most five products of 64 x 2^14), and the
+          // first two pairs are positive (see start)
+          const uint32_t m10 = static_cast<uint32_t>(acc[c][1][e]) * 256u + acc[c][0][e];
+          const uint32_t m32 = static_cast<uint32_t>(acc[c][3][e]) * 256u + acc[c][2][e];
+          const uint32_t m54 = static_cast<uint32_t>(acc[c][5][e]) * 256u + acc[c][4][e];
+          uint32_t carry, none;
+          const uint32_t lo = __builtin_addc(m10, m32 << 16, 0u, &carry);
+          const uint32_t hi = __builtin_addc(m54, m32 >> 16, carry, &none);
+          int64_t v = static_cast<int64_t>(static_cast<uint64_t>(hi) << 32 | lo);
+          if (LEFT) v <<= (left >> (8 * e)) & 63;
+          v >>= (right >> (8 * e)) & 63;
+          const uint32_t vl = static_cast<uint32_t>(v) ^ sg;
+          const uint32_t vh = static_cast<uint32_t>(v >> 32) ^ sg;
+          __hip_atomic_fetch_add(to + c, static_cast<unsigned long long>(vh) << 32 | vl,
                                  __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         }
       }
     }
     __builtin_amdgcn_s_setprio(0);
   }
+  };
+  if (p.unit->left_rows) run(std::true_type{});
+  else run(std::false_type{});
   __syncthreads();
-  const double back = ldexp(*scale, 32 - *p.ea);
+  const double back = ldexp(*scale, 32 - p.unit->e);
   double2* racc = reinterpret_cast<double2*>(p.rowacc) + ia * p.lenb;
   double sq = 0.0;
   for (int x = tid; x < lenb; x += kRowThreads) {
@@ -516,7 +579,8 @@ int launch_pull_rows_oz(const fqehip_sector* s, const double* coeff,
   p.lenb = s->lenb;
   p.dig = static_cast<const uint8_t*>(s->w_oz);
   p.z = reinterpret_cast<const double*>(p.dig + s->npull * kWDigBytes);
-  p.ea = reinterpret_cast<const int32_t*>(p.z + static_cast<int64_t>(s->npull) * kOzQ);
+  p.unit = reinterpret_cast<const OzUnit*>(p.z + static_cast<int64_t>(s->npull) * kOzQ);
+  p.half = s->nbeta * (s->norb - s->nbeta + 1) / 2;
   p.dexc = s->dexc_a;
   p.fwd = s->pull_fwd;
   p.coeff = coeff;
@@ -1101,7 +1165,7 @@ extern "C" int fqehip_beta_gemm_digits(int64_t lena, int64_t lenb,
 
 extern "C" int64_t fqehip_pull_digits_bytes(int npull) {
   if (npull < 0) return -1;
-  return npull * (kWDigBytes + static_cast<int64_t>(kOzQ) * 8) + 8;
+  return npull * (kWDigBytes + static_cast<int64_t>(kOzQ) * 8) + sizeof(OzUnit);
 }
 
 extern "C" int fqehip_pull_digits(int npull, const double* d_w, void* d_woz,
@@ -1112,8 +1176,8 @@ extern "C" int fqehip_pull_digits(int npull, const double* d_w, void* d_woz,
   FQEHIP_CHECK_ARG(d_w && d_woz, "NULL pointer");
   uint8_t* dig = static_cast<uint8_t*>(d_woz);
   double* z = reinterpret_cast<double*>(dig + npull * kWDigBytes);
-  int32_t* ea = reinterpret_cast<int32_t*>(z + static_cast<int64_t>(npull) * kOzQ);
-  k_pull_digits<<<npull, kOzQ, 0, as_stream(stream)>>>(npull, d_w, dig, z, ea);
+  OzUnit* unit = reinterpret_cast<OzUnit*>(z + static_cast<int64_t>(npull) * kOzQ);
+  k_pull_digits<<<npull, kOzQ, 0, as_stream(stream)>>>(npull, d_w, dig, z, unit);
   FQEHIP_CHECK_LAUNCH("k_pull_digits");
   return FQEHIP_OK;
 }

@@ -46,6 +46,8 @@ class PreparedOperator:
         # opposite-spin coupling W[p][q] = V[p][q] + V[q][p] (device, alpha
         # pair p, beta pair q) of a two-body operator: the pull form
         self.coupling: Optional[torch.Tensor] = None
+        self.coupling_host: Optional[numpy.ndarray] = None
+        self._in_range: Optional[bool] = None
         on = a if a is not None else h1
         self._tables = _lib.TableCache(on.device)
 
@@ -82,12 +84,29 @@ class PreparedOperator:
         tabs = self.pull_tables(graph)
         if (tabs is None or self.complex_op or self.spin
                 or not self.pair_symmetric or self.coupling.shape[0] > 128
-                or max(graph.lena(), graph.lenb()) >= 26214):
+                or max(graph.lena(), graph.lenb()) >= 26214
+                or not self._digit_range()):
             return None
         return [self._tables.get("w_oz", self._build_coupling_digits)] + [
             self._tables.get(("digits", nele), self._build_block_digits, block)
             for nele, block in ((graph.nalpha(), tabs[1]),
                                 (graph.nbeta(), tabs[2]))]
+
+    def _digit_range(self) -> bool:
+        """Whether W's digits resolve its rows.  Their products are summed as
+        integers whose unit can be as fine as 2^-62 sum |W|: down to rows
+        whose largest element is 2^-23 sum |W| that is finer than the row's
+        own 38-bit digits (integrals of canonical orbitals: 2^-10 to 2^-14).
+        Beside one integral 10^7 times the others, as a penalty on an
+        orbital, the typical row is past that, and the sector runs in
+        FP64."""
+        if self._in_range is None:
+            w = numpy.abs(self.coupling_host)
+            rows = w.max(axis=0, initial=0.0)
+            rows = rows[rows > 0.0]
+            self._in_range = (rows.size == 0 or
+                              bool(w.sum() <= 2.0**23 * numpy.median(rows)))
+        return self._in_range
 
     def _build_coupling_digits(self) -> torch.Tensor:
         npull = self.coupling.shape[0]
@@ -203,9 +222,10 @@ def prepare_operator(tensors: Sequence[numpy.ndarray], norb: int,
     h1row = h1p.reshape(-1)[rows]
     full = numpy.vstack([vm, h1row[None, :]])  # (npair+1) x npair, complex
     a = _real_block_form(full, complex_op)
-    dev_a, coupling = _upload(a, vm + vm.T, complex_op, device)
+    w = vm + vm.T
+    dev_a, coupling = _upload(a, w, complex_op, device)
     prepared = PreparedOperator(norb, compressed, complex_op, dev_a, None)
-    prepared.coupling = coupling
+    prepared.coupling, prepared.coupling_host = coupling, w
     if not complex_op:
         sq = a[:-1, :]
         prepared.pair_symmetric = bool(numpy.array_equal(sq, sq.T))

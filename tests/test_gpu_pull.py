@@ -150,9 +150,9 @@ def test_digit_rows_edges(fqe, na, nb, norb, blocks, shape):
     fewer than 64 columns or strings, ragged tiles, 3 to 120 pairs, 2 to 64
     de-excitation rows; and the largest possible sums (every integral and
     every coefficient equal).  Tolerance 3e-11 normwise: operator rounding
-    2^-39 and data rounding 2^-47 of the largest element, dropped digit
-    pairs below both, times the spread between the largest element and the
-    norm of a row (up to some hundreds here).  Integer sums: the same bits
+    2^-39 of the row's largest element, data rounding 2^-47 of the largest
+    coefficient, dropped digit pairs below both, times the spread between
+    the largest element and the norm of a row (up to some hundreds here).  Integer sums: the same bits
     on every run."""
     from fqe_amd import settings
     print(f"digit rows {na} {nb} {norb} {blocks} {shape}", flush=True)
@@ -218,6 +218,43 @@ def test_digit_rows_with_empty_strings(fqe, na, nb, norb, zero, blocks):
         assert not e.coeff.any()
     else:
         assert rel(e.coeff, d.coeff) < 3e-11
+
+
+@pytest.mark.parametrize("large", [1e3, 1e5, 1e6, 1e9])
+@pytest.mark.parametrize("na,nb,norb", [(4, 3, 8), (3, 5, 9), (5, 5, 10)])
+def test_digit_rows_beside_a_large_integral(fqe, na, nb, norb, large):
+    """One local integral (00|00) far above the others, and no determinant of
+    the vector with orbital 0 occupied.  Only the row (00) of W is rounded as
+    coarsely as that integral asks; it reaches beta strings that occupy
+    orbital 0, and on the others the result keeps the tolerance of
+    test_digit_rows_edges.  Past the range of the digits the sector runs in
+    FP64."""
+    from fqe_amd import _lib, engine, settings
+    print(f"digit rows {na} {nb} {norb} large {large}", flush=True)
+    d, c, g, rng = sector(fqe, na, nb, norb, 11 * norb + 5 * na + nb)
+    h1, h2 = tensors("real", norb, rng)
+    h2 = h2.copy()
+    h2[0, 0, 0, 0] = -large * numpy.abs(h2).max()
+    c = c.copy()
+    core, bit = d.get_fcigraph(), numpy.uint64(1)
+    c[core.string_alpha_all() & bit == 1, :] = 0.0
+    beta = core.string_beta_all() & bit == 0
+    c[:, ~beta] = 0.0
+    d.coeff = c
+    op = prepared(fqe, "real", (h1, h2), norb)
+    saved = settings.contraction, settings.ozaki_min_determinants
+    settings.contraction, settings.ozaki_min_determinants = "ozaki", 0
+    try:
+        s, keep = engine.sector_struct(d.get_fcigraph(), op, _lib.C128)
+        assert bool(s.w_oz) == (large < 1e8)
+        e = copy.deepcopy(d)
+        e.apply_inplace_scaled((h1, h2), op=op)
+    finally:
+        settings.contraction, settings.ozaki_min_determinants = saved
+    d.apply_inplace_scaled((h1, h2), op=op)
+    assert rel(e.coeff[:, beta], d.coeff[:, beta]) < 3e-11
+    if large > 1e8:
+        assert numpy.array_equal(e.coeff, d.coeff)
 
 
 @pytest.mark.parametrize("nterms", [0, 1, 2, 5])
