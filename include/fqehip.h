@@ -304,6 +304,10 @@ int64_t fqehip_pull_table_count(const fqehip_sector* s, int complex_op);
  * element is above 2^-23 sum |W|. */
 int64_t fqehip_pull_digits_bytes(int npull);
 int fqehip_pull_digits(int npull, const double* d_w, void* d_woz, void* stream);
+/* Whether a sector of these sizes (norb, nalpha, lena, lenb, npull; no pointer
+ * is used) is within the limits of the pull form, before its tables are made:
+ * Haa alone can take 2 GB. */
+int fqehip_pull_fits_supported(const fqehip_sector* s, int complex_op);
 /* Whether fqehip_apply takes the pull form for this sector and operator. */
 int fqehip_pull_supported(int precision, const fqehip_sector* s,
                           const fqehip_operator* op);

@@ -852,8 +852,7 @@ int launch_rows(const PullPlan& pl, const PullArgs& p, hipStream_t st) {
 
 // The limits are those of a complex operator (the narrower ones), so that
 // the answer is the sector's alone.
-bool pull_supported(const fqehip_sector* s) {
-  if (!s->pull_w || !s->haa || !s->hbb || !s->dexc_a || !s->pull_fwd) return false;
+static bool pull_limits(const fqehip_sector* s) {
   const int noff = s->nalpha * (s->norb - s->nalpha);
   PullPlan pl;
   return s->npull > 0 && s->lena > 0 && s->lenb > 0 &&
@@ -862,6 +861,10 @@ bool pull_supported(const fqehip_sector* s) {
          s->lenb * s->lenb * 16 < kOffLimit &&
          static_cast<int64_t>(s->npull + 15) * s->lenb * 4 < kOffLimit &&
          pull_plan(true, noff, s->lenb, s->npull, &pl);
+}
+
+bool pull_supported(const fqehip_sector* s) {
+  return s->pull_w && s->haa && s->hbb && s->dexc_a && s->pull_fwd && pull_limits(s);
 }
 
 bool pull_one_launch(const fqehip_sector* s) {
@@ -1032,6 +1035,13 @@ int launch_pull_group(const PullGroupLaunch& g, const void* d_secs, int step,
 }  // namespace fqehip
 
 using namespace fqehip;
+
+extern "C" int fqehip_pull_fits_supported(const fqehip_sector* s, int complex_op) {
+  if (!s || s->norb <= 0 || !pull_limits(s)) return 0;
+  // the columns of Haa and Hbb in LDS (fqehip_spin_block)
+  const int64_t longest = s->lena > s->lenb ? s->lena : s->lenb;
+  return (longest + s->npull) * (complex_op ? 16 : 8) <= static_cast<int64_t>(kLdsLimit);
+}
 
 extern "C" int64_t fqehip_pull_table_count(const fqehip_sector* s, int complex_op) {
   PullPlan pl;

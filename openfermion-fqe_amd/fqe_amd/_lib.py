@@ -105,6 +105,7 @@ _SIGNATURES = {
                                   c_int64, c_void_p, c_void_p, c_void_p]),
     "fqehip_pull_table": (c_int, [c_int, c_int64, c_void_p, c_void_p,
                                   c_void_p]),
+    "fqehip_pull_fits_supported": (c_int, [POINTER(Sector), c_int]),
     "fqehip_pull_table_count": (c_int64, [POINTER(Sector), c_int]),
     "fqehip_pull_digits_bytes": (c_int64, [c_int]),
     "fqehip_pull_digits": (c_int, [c_int, c_void_p, c_void_p, c_void_p]),

@@ -149,17 +149,18 @@ class PreparedOperator:
         the pull form on the sector of ``graph``, cached per (nalpha,
         nbeta); None where the form does not apply (one-body operators,
         sectors past its limits)."""
-        na, nb, norb = graph.nalpha(), graph.nbeta(), graph.norb()
-        if (self.coupling is None or na * (norb - na + 1) > 64
-                or norb == 0):
+        if self.coupling is None:
             return None
-        width = 16 if self.complex_op else 8
-        if ((max(graph.lena(), graph.lenb()) + self.coupling.shape[0]) * width
-                > 160 * 1024):
-            return None
-        return self._tables.get((na, nb), self._build_pull, graph)
+        return self._tables.get((graph.nalpha(), graph.nbeta()),
+                                self._build_pull, graph)
 
     def _build_pull(self, graph):
+        limits = _lib.Sector(graph.norb(), graph.nalpha(), graph.nbeta(),
+                             self.npair, graph.lena(), graph.lenb())
+        limits.npull = self.coupling.shape[0]
+        if not _lib.call("fqehip_pull_fits_supported", _as_ref(limits),
+                         int(self.complex_op)):
+            return None
         ta, tb = graph.tables(True), graph.tables(False)
         # restricted operators: one matrix per electron count
         haa, hbb = (

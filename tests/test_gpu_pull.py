@@ -380,3 +380,25 @@ def test_accumulate_onto_the_input(fqe, kind, na, nb, norb):
         before[shift:shift + n] += want.reshape(-1)
         assert rel(out.cpu().numpy(), want) < 1e-13
         assert rel(buf.cpu().numpy(), before) < 1e-13
+
+
+@pytest.mark.parametrize("na,nb,norb", [(5, 8, 16), (8, 5, 16)])
+def test_no_blocks_past_the_limits(fqe, na, nb, norb):
+    """A sector that the pull form refuses (12870 strings of one spin) builds
+    none of its tables: Haa or Hbb would take 1.3 GB for nothing."""
+    import torch
+    from fqe_amd import _lib, engine, settings
+    from fqe_amd.fci_graph import FciGraph
+    graph = FciGraph(na, nb, norb)
+    op = prepared(fqe, "real", tensors("real", norb,
+                                       numpy.random.default_rng(1)), norb)
+    before = torch.cuda.memory_allocated()
+    assert op.pull_tables(graph) is None
+    s, keep = engine.sector_struct(graph, op, _lib.C128)
+    assert not s.pull_w and not s.haa and not s.hbb
+    # the string tables of the unfused path, npair rows each
+    tables = 3 * op.npair * 4 * (graph.lena() + graph.lenb())
+    assert torch.cuda.memory_allocated() - before <= tables + (1 << 20)
+    # within the limits again: one electron fewer
+    small = FciGraph(2, 2, norb)
+    assert op.pull_tables(small) is not None

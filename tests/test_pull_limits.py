@@ -51,3 +51,25 @@ def test_target_words_within_their_table(norb):
                 plans += 1
                 assert n == (npull + 15) // 16 * 16 * s.lenb, (na, nb, npull)
     assert plans
+
+
+def test_fits_is_what_the_sector_with_tables_gets():
+    """fqehip_pull_fits_supported without pointers answers as
+    fqehip_pull_supported does with them."""
+    import ctypes
+    from fqe_amd import _lib
+    lib = _lib.lib()
+    op = _lib.Operator()
+    op.a = 256
+    seen = set()
+    for norb in range(1, 25):
+        for na in range(norb + 1):
+            for nb in range(norb + 1):
+                s = sector(norb, na, nb, norb * (norb + 1) // 2)
+                fits = bool(lib.fqehip_pull_fits_supported(s, 0))
+                s.pull_w = s.haa = s.hbb = s.pull_fwd = s.dexc_a = 256
+                assert fits == bool(lib.fqehip_pull_supported(
+                    _lib.C128, ctypes.byref(s), ctypes.byref(op))), (norb, na,
+                                                                     nb)
+                seen.add(fits)
+    assert seen == {True, False}
