@@ -588,13 +588,15 @@ typedef struct fqehip_batch fqehip_batch;
  * step one row launch and one reduction cover all of them (complex64: the
  * rows4 row body; complex128: the FP64 row body), instead of kernels per
  * sector, and so do the small real pull-form sectors (not counted by
- * fqehip_batch_grouped) with two launches per step for each kernel shape;
+ * fqehip_batch_grouped) with one or two launches per step for each kernel
+ * shape (the same-spin products of the sectors that need them, the rows);
  * the other sectors keep their own kernels on the other branches. */
 int fqehip_batch_create(int precision, int nitems,
                         const fqehip_batch_item* items, double time,
                         int nterms, int nstreams, int group, void* stream,
                         fqehip_batch** out);
 int fqehip_batch_launch(fqehip_batch* batch, void* stream);
+/* Nodes of the recorded graph. */
 int fqehip_batch_nodes(const fqehip_batch* batch);
 /* Number of sectors the batch runs as one group. */
 int fqehip_batch_grouped(const fqehip_batch* batch);

@@ -65,18 +65,16 @@ void release(fqehip_batch* b) {
 // terms alternate between d_term and the workspace's second buffer, starting
 // from d_coeff0, so the row kernel's epilogue does the whole step.
 int enqueue_pull_item(const fqehip_batch_item& it, double time, int nterms,
-                      hipStream_t st, int* nodes) {
+                      hipStream_t st) {
   void* sv = reinterpret_cast<void*>(st);
   int rc = fqehip_convert_to_c128(FQEHIP_C128, it.sector.lena * it.sector.lenb,
                                   it.d_coeff0, 1.0, 0.0, it.d_result, sv);
   if (rc) return rc;
-  *nodes += 1;
   if (it.d_apply_out) {
     rc = fqehip_apply(FQEHIP_C128, &it.sector, &it.op, it.d_coeff0, 1.0, 0.0, 0.0,
                       0.0, nullptr, it.d_apply_out, nullptr, nullptr, nullptr,
                       it.d_workspace, sv);
     if (rc) return rc;
-    *nodes += 2;
   }
   void* term[2] = {it.d_term,
                    static_cast<char*>(it.d_workspace) + pull_spare_offset(&it.sector)};
@@ -87,7 +85,6 @@ int enqueue_pull_item(const fqehip_batch_item& it, double time, int nterms,
                       -time / static_cast<double>(k), 0.0, 0.0, nullptr, dst,
                       it.d_result, nullptr, nullptr, it.d_workspace, sv);
     if (rc) return rc;
-    *nodes += 2;
     src = dst;
   }
   return FQEHIP_OK;
@@ -98,7 +95,7 @@ int enqueue_pull_item(const fqehip_batch_item& it, double time, int nterms,
 int enqueue_pull_group(const fqehip_batch_item* items,
                        const std::vector<int>& members,
                        const PullGroupLaunch& g, const void* d_secs, double time,
-                       int nterms, hipStream_t st, int* nodes) {
+                       int nterms, hipStream_t st) {
   if (nterms == 0)
     for (int i : members) {
       const fqehip_batch_item& it = items[i];
@@ -106,25 +103,23 @@ int enqueue_pull_group(const fqehip_batch_item* items,
                                       it.d_coeff0, 1.0, 0.0, it.d_result,
                                       reinterpret_cast<void*>(st));
       if (rc) return rc;
-      *nodes += 1;
     }
   for (int step = g.any_apply ? 0 : 1; step <= nterms; ++step) {
     int rc = launch_pull_group(g, d_secs, step, 0.0,
                                step ? -time / static_cast<double>(step) : 0.0, st);
     if (rc) return rc;
-    *nodes += 2;
   }
   return FQEHIP_OK;
 }
 
 // The work of one item on stream st (see the file comment).
 int enqueue_item(int precision, const fqehip_batch_item& it, double time,
-                 int nterms, hipStream_t st, int* nodes) {
+                 int nterms, hipStream_t st) {
   const int64_t n = it.sector.lena * it.sector.lenb;
   if (n == 0) return FQEHIP_OK;
   void* sv = reinterpret_cast<void*>(st);
   if (precision == FQEHIP_C128 && fqehip_pull_supported(precision, &it.sector, &it.op))
-    return enqueue_pull_item(it, time, nterms, st, nodes);
+    return enqueue_pull_item(it, time, nterms, st);
   if (hipMemcpyAsync(it.d_term, it.d_coeff0, n * esize(precision),
                      hipMemcpyDeviceToDevice, st) != hipSuccess) {
     set_error("batch: copy of the initial term failed");
@@ -133,13 +128,11 @@ int enqueue_item(int precision, const fqehip_batch_item& it, double time,
   int rc = fqehip_convert_to_c128(precision, n, it.d_coeff0, 1.0, 0.0,
                                   it.d_result, sv);
   if (rc) return rc;
-  *nodes += 2;
   if (it.d_apply_out) {
     rc = fqehip_apply(precision, &it.sector, &it.op, it.d_coeff0, 1.0, 0.0,
                       0.0, 0.0, nullptr, it.d_apply_out, nullptr, nullptr,
                       nullptr, it.d_workspace, sv);
     if (rc) return rc;
-    *nodes += 3;
   }
   for (int k = 1; k <= nterms; ++k) {
     rc = fqehip_apply(precision, &it.sector, &it.op, it.d_term, 0.0,
@@ -147,7 +140,6 @@ int enqueue_item(int precision, const fqehip_batch_item& it, double time,
                       it.d_term, it.d_result, nullptr, nullptr, it.d_workspace,
                       sv);
     if (rc) return rc;
-    *nodes += 3;
   }
   return FQEHIP_OK;
 }
@@ -158,8 +150,7 @@ int enqueue_item(int precision, const fqehip_batch_item& it, double time,
 int enqueue_group(int precision, const fqehip_batch_item* items,
                   const std::vector<int>& grouped, const GroupSector* d_secs,
                   int64_t rows, int64_t blocks, int64_t max_lenb,
-                  bool any_apply, double time, int nterms, hipStream_t st,
-                  int* nodes) {
+                  bool any_apply, double time, int nterms, hipStream_t st) {
   void* sv = reinterpret_cast<void*>(st);
   for (int i : grouped) {
     const fqehip_batch_item& it = items[i];
@@ -172,7 +163,6 @@ int enqueue_group(int precision, const fqehip_batch_item* items,
     int rc = fqehip_convert_to_c128(precision, n, it.d_coeff0, 1.0, 0.0,
                                     it.d_result, sv);
     if (rc) return rc;
-    *nodes += 2;
   }
   const int nsec = static_cast<int>(grouped.size());
   for (int step = any_apply ? 0 : 1; step <= nterms; ++step) {
@@ -182,7 +172,6 @@ int enqueue_group(int precision, const fqehip_batch_item* items,
     rc = launch_group_reduce(precision, d_secs, nsec, blocks, step, 0.0,
                              step ? -time / static_cast<double>(step) : 0.0, st);
     if (rc) return rc;
-    *nodes += 2;
   }
   return FQEHIP_OK;
 }
@@ -386,18 +375,16 @@ extern "C" int fqehip_batch_create(int precision, int nitems,
       rc = FQEHIP_ERR_HIP;
   if (rc == FQEHIP_OK && !grouped.empty())
     rc = enqueue_group(precision, items, grouped, b->d_group, grows, gblocks,
-                       gmax_lenb, gapply, time, nterms, b->streams[0],
-                       &b->nodes);
+                       gmax_lenb, gapply, time, nterms, b->streams[0]);
   for (int s = 0; s < nb && rc == FQEHIP_OK; ++s)
     for (int c : pplan[s]) {
       rc = enqueue_pull_group(items, pull[c], pgl[c], pgd[c], time, nterms,
-                              b->streams[s], &b->nodes);
+                              b->streams[s]);
       if (rc) break;
     }
   for (int s = 0; s < nb && rc == FQEHIP_OK; ++s)
     for (int i : plan[s]) {
-      rc = enqueue_item(precision, items[i], time, nterms, b->streams[s],
-                        &b->nodes);
+      rc = enqueue_item(precision, items[i], time, nterms, b->streams[s]);
       if (rc) break;
     }
   for (int s = 0; s < nb && rc == FQEHIP_OK; ++s) {
@@ -417,6 +404,13 @@ extern "C" int fqehip_batch_create(int precision, int nitems,
     return rc;
   }
   b->graph = graph;
+  size_t nodes = 0;
+  if (hipGraphGetNodes(graph, nullptr, &nodes) != hipSuccess) {
+    release(b);
+    set_error("batch: the graph's nodes could not be counted");
+    return FQEHIP_ERR_HIP;
+  }
+  b->nodes = static_cast<int>(nodes);
   if (hipGraphInstantiate(&b->exec, graph, nullptr, nullptr, 0) != hipSuccess) {
     release(b);
     set_error("batch: graph instantiation failed");

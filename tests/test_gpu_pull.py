@@ -402,3 +402,37 @@ def test_no_blocks_past_the_limits(fqe, na, nb, norb):
     # within the limits again: one electron fewer
     small = FciGraph(2, 2, norb)
     assert op.pull_tables(small) is not None
+
+
+@pytest.mark.parametrize("nterms", [1, 4])
+@pytest.mark.parametrize("contraction,group,norb,na,nb,kernels,extra", [
+    ("fp64", True, 8, 4, 4, 1, 0),      # rows with their same-spin part
+    ("fp64", True, 9, 4, 4, 2, 0),      # same-spin products, rows
+    ("fp64", False, 8, 4, 4, 1, 1),     # on its own: the result's start value
+    ("fp64", False, 9, 4, 4, 2, 1),
+    # row maxima, column maxima, digits and product of C, of C^T, rows
+    ("ozaki", True, 9, 4, 4, 7, 1)])
+def test_batch_node_count(fqe, contraction, group, norb, na, nb, kernels,
+                          extra, nterms):
+    """fqehip_batch_nodes is the number of launches of the recorded graph:
+    `kernels` for the apply and each term, `extra` beside them."""
+    import torch
+    from fqe_amd import batched, settings
+    rng = numpy.random.default_rng(5)
+    h1, h2 = fo.synthetic_hamiltonian(norb, norb, rng)
+    g = fo.OracleGraph(na, nb, norb)
+    spec = batched.SectorSpec(norb=norb, nalpha=na, nbeta=nb, h1=h1, h2=h2,
+                              coeff=fo.synthetic_coeff(g.lena, g.lenb, rng))
+    saved = settings.ozaki_min_determinants
+    settings.ozaki_min_determinants = 0
+    try:
+        bt = batched.BatchedTaylor([spec], 0.1, nterms=nterms,
+                                   dtype=torch.complex128,
+                                   tiles={f"{norb},{na},{nb}": "split"},
+                                   nstreams=1, group=group,
+                                   contraction=contraction)
+    finally:
+        settings.ozaki_min_determinants = saved
+    bt.build()
+    assert bt.nodes() == kernels * (nterms + 1) + extra
+    bt.close()
