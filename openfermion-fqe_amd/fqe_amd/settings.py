@@ -72,3 +72,9 @@ max_workspace_bytes = 96 << 30
 # time_evolve; the graph and its buffers are cached on the operator for the
 # last (sector, time, accuracy, expansion) it ran.
 taylor_graph = False
+
+
+def kernel_choice():
+    """Every setting that picks an apply's kernels."""
+    return (fused, split, split_fp64, split_tile, split_tile_fp64, contraction,
+            ozaki_beta, ozaki_min_determinants)

@@ -558,9 +558,9 @@ def _taylor_single(out: Wavefunction, sec: FqeData,
     prec = engine.precision_of(c.dtype)
     if settings.taylor_graph:
         g = sec.get_fcigraph()
-        key = (g.nalpha(), g.nbeta(), g.norb(), c.dtype, settings.contraction,
-               settings.split_fp64, settings.split, float(time),
-               float(accuracy), int(expansion))
+        key = (g.nalpha(), g.nbeta(), g.norb(), c.dtype, float(time),
+               float(accuracy), int(expansion),
+               settings.kernel_choice())
         cached = getattr(op, "_taylor_graph", None)
         if cached is None or cached[0] != key:
             op._taylor_graph = None          # free the previous one first

@@ -83,3 +83,28 @@ def test_taylor_graph_not_converged_raises(fqe):
             wfn.apply_generated_unitary(1.0, "taylor", ham, expansion=4)
     finally:
         settings.taylor_graph = saved
+
+
+def test_taylor_graph_follows_the_settings(fqe):
+    """A graph recorded under one choice of kernels is not replayed under
+    another: the digit engine's threshold moved past the sector gives the
+    FP64 series' bits, as an operator that never used digits."""
+    from fqe_amd import settings
+    c, h1, h2 = fo.synthetic_workload(8, 4, 4, 3, 8)
+    saved = (settings.taylor_graph, settings.contraction,
+             settings.ozaki_min_determinants)
+    settings.taylor_graph, settings.contraction = True, "ozaki"
+    try:
+        outs = {}
+        for name, steps in (("digits then fp64", (0, 10**9)),
+                            ("fp64", (10**9,))):
+            wfn = fqe.Wavefunction([[8, 0, 8]])
+            wfn.set_wfn(strategy="from_data", raw_data={(8, 0): c})
+            ham = fqe.get_restricted_hamiltonian((h1, h2))
+            for least in steps:
+                settings.ozaki_min_determinants = least
+                outs[name] = wfn.time_evolve(0.1, ham).get_coeff((8, 0))
+    finally:
+        (settings.taylor_graph, settings.contraction,
+         settings.ozaki_min_determinants) = saved
+    assert numpy.array_equal(outs["digits then fp64"], outs["fp64"])
