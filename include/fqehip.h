@@ -197,7 +197,10 @@ typedef struct fqehip_sector {
    * W[p][q] E^a_p C).  When pull_w is set (with all the fields below) and
    * fqehip_pull_supported() holds, fqehip_apply takes it; its workspace is
    * then one complex128 row accumulator (16 lena lenb bytes).  For a complex
-   * operator (complex_op = 1) W, Haa and Hbb are complex128. */
+   * operator (complex_op = 1) W, Haa and Hbb are complex128.  Haa and Hbb are
+   * dense: an infinity or NaN in C reaches its whole row and column of H C,
+   * beside the determinants that H connects it with (with digits also every
+   * row that an alpha excitation takes it to). */
   const int32_t* dexc_a;   /* alpha de-excitation rows (fqehip_string_tables) */
   const double* pull_w;    /* [npull][npull] coupling, alpha pair p, beta pair q */
   const double* haa;       /* fqehip_spin_block of the alpha strings */

@@ -52,8 +52,19 @@ constexpr int kOzARow = kOzK + 16;         // bytes per LDS row of a digit plane
 constexpr int kOzQ = 128;                  // beta pairs, padded (table pitch)
 constexpr double kMagic = 6755399441055744.0;  // 1.5 * 2^52: rint via one add
 
-// rowmax[I] = max over the row of max(|Re C[I][.]|, |Im C[I][.]|); zeroes
-// colmax (when not NULL) for k_col_absmax.
+// max(m, |v|), infinity from a NaN on
+__device__ __forceinline__ double absmax(double m, double v) {
+  return v == v ? fmax(m, fabs(v)) : HUGE_VAL;
+}
+
+// 2^-e, the factor back of data with the maximum m scaled by 2^e: zero where all
+// are zero, and NaN where one is not finite and has no digits.
+__device__ __forceinline__ double factor_back(double m, int e) {
+  return m > 0.0 ? (m < HUGE_VAL ? ldexp(1.0, -e) : __longlong_as_double(0x7ff8000000000000ll)) : 0.0;
+}
+
+// rowmax[I] = max over the row of max(|Re C[I][.]|, |Im C[I][.]|), infinity where
+// one is not finite; zeroes colmax (when not NULL) for k_col_absmax.
 __global__ void __launch_bounds__(256)
 k_row_absmax(int64_t lena, int64_t lenb, const double* __restrict__ coeff,
              double* __restrict__ rowmax, unsigned long long* __restrict__ colmax,
@@ -67,7 +78,7 @@ k_row_absmax(int64_t lena, int64_t lenb, const double* __restrict__ coeff,
   for (int64_t r = blockIdx.x; r < lena; r += gridDim.x) {
     const double* row = coeff + r * lenb * 2;
     double m = 0.0;
-    for (int64_t k = threadIdx.x; k < 2 * lenb; k += 256) m = fmax(m, fabs(row[k]));
+    for (int64_t k = threadIdx.x; k < 2 * lenb; k += 256) m = absmax(m, row[k]);
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o));
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
@@ -94,7 +105,7 @@ k_col_absmax(int64_t lena, int64_t lenb, const double* __restrict__ coeff,
 #pragma unroll 8
   for (int64_t r = r0; r < r1; ++r) {
     const double2 v = reinterpret_cast<const double2*>(coeff)[r * lenb + j];
-    m = fmax(m, fmax(fabs(v.x), fabs(v.y)));
+    m = absmax(absmax(m, v.x), v.y);
   }
   atomicMax(&colmax[j], static_cast<unsigned long long>(__double_as_longlong(m)));
 }
@@ -343,7 +354,7 @@ __global__ void __launch_bounds__(kRowThreads, 2) k_pull_rows_oz(OzRowsArgs p) {
     lp[lane] = lane < nexc ? (p.compressed ? comp_pair(i, j) : ij) : -1;
     goff[lane] = lane < nexc ? static_cast<uint32_t>(src) * static_cast<uint32_t>(lenb) : kNoRow16;
     gsa[lane] = static_cast<double>(sg) * ldexp(1.0, e);
-    if (lane == 0) *scale = m > 0.0 ? ldexp(1.0, -e) : 0.0;
+    if (lane == 0) *scale = factor_back(m, e);
   }
   __syncthreads();
   {
@@ -664,7 +675,7 @@ k_c_digits(int64_t lena, int64_t lenb, int64_t ldk,
     (void)frexp(mx, &e);
     ec = 46 - e;
   }
-  if (g == 0) cscale[ia] = mx > 0.0 ? ldexp(1.0, -ec) : 0.0;
+  if (g == 0) cscale[ia] = factor_back(mx, ec);
   const double sc = ldexp(1.0, ec);
   uint32_t lre[4], hre[4], lim[4], him[4];
 #pragma unroll
@@ -715,8 +726,7 @@ k_ct_digits(int64_t lena, int64_t lenb, int64_t ldk,
     (void)frexp(mx, &e);
     ec = 46 - e;
   }
-  if (a0 == 0 && threadIdx.x < kCtB && jb < lenb)
-    cscale[jb] = mx > 0.0 ? ldexp(1.0, -ec) : 0.0;
+  if (a0 == 0 && threadIdx.x < kCtB && jb < lenb) cscale[jb] = factor_back(mx, ec);
   const double sc = ldexp(1.0, ec);
   for (int g = threadIdx.x / kCtB; g < kW; g += 256 / kCtB) {
     uint32_t lre[4], hre[4], lim[4], him[4];

@@ -436,3 +436,50 @@ def test_batch_node_count(fqe, contraction, group, norb, na, nb, kernels,
     bt.build()
     assert bt.nodes() == kernels * (nterms + 1) + extra
     bt.close()
+
+
+@pytest.mark.parametrize("value", [numpy.inf, numpy.nan])
+@pytest.mark.parametrize("kind,contraction,na,nb,norb", [
+    ("real", "fp64", 3, 3, 6), ("real", "fp64", 5, 4, 9),
+    ("complex", "fp64", 4, 4, 9), ("spin", "fp64", 4, 3, 8),
+    ("real", "ozaki", 4, 5, 9)])
+def test_coefficients_that_are_not_finite(fqe, kind, contraction, na, nb,
+                                          norb, value):
+    """One infinite or NaN coefficient: every determinant that H connects it
+    with is not finite, and outside its row and column of C (the digit
+    engine: and the rows that an alpha excitation reaches) the others keep
+    the values they have without it (1e-13: the same sums)."""
+    from fqe_amd import settings
+    print(f"not finite {kind} {contraction} {value}", flush=True)
+    d, c, g, rng = sector(fqe, na, nb, norb, 5 * norb + na)
+    h = tensors(kind, norb, rng)
+    op = prepared(fqe, kind, h, norb)
+    ia, ib = c.shape[0] // 3, c.shape[1] // 2
+
+    def apply(x):
+        e = copy.deepcopy(d)
+        e.coeff = x
+        e.apply_inplace_scaled(h, op=op)
+        return e.coeff
+    unit = numpy.zeros_like(c)
+    unit[ia, ib] = 1.0
+    connected = numpy.abs(apply(unit)) > 1e-12
+    bad = c.copy()
+    bad[ia, ib] = value
+    clean = c.copy()
+    clean[ia, ib] = 0.0
+    want = apply(clean)
+    saved = settings.contraction, settings.ozaki_min_determinants
+    settings.contraction, settings.ozaki_min_determinants = contraction, 0
+    try:
+        got = apply(bad)
+    finally:
+        settings.contraction, settings.ozaki_min_determinants = saved
+    assert not numpy.isfinite(got[connected]).any()
+    rest = ~connected
+    rest[ia, :] = rest[:, ib] = False
+    if contraction == "ozaki":
+        rest[connected.any(axis=1), :] = False
+    assert rest.any()
+    tol = 3e-11 if contraction == "ozaki" else 1e-13
+    assert rel(got[rest], want[rest]) < tol
