@@ -78,6 +78,7 @@ def big(fqe):
     return c, b, h1, h2
 
 
+@pytest.mark.skipif(not ref_lm.available(), reason="oracle/_ref not built")
 def test_norb14_fp64_vs_reference_c_and_mixed(fqe, big):
     print("norb=14 FP64 and mixed vs reference C", flush=True)
     c, _, h1, h2 = big
