@@ -127,7 +127,7 @@ def test_grouped_batch_complex128(fqe, contraction):
     split sectors: 1e-9), replays against each other, and the group
     against the per-sector kernels of run_sequential."""
     import torch
-    from fqe_amd import batched
+    from fqe_amd import batched, settings
     specs = batched.random_specs(24, seed=46, norb_range=(4, 9))
     cycle = ["rows4", "split", "rows4", "unfused"]
     tiles, want = {}, 0
@@ -136,9 +136,16 @@ def test_grouped_batch_complex128(fqe, contraction):
         if key not in tiles:
             tiles[key] = cycle[i % len(cycle)]
     print("variants", tiles, flush=True)
-    bt = batched.BatchedTaylor(specs, 0.1, nterms=10, dtype=torch.complex128,
-                               tiles=tiles, nstreams=4, group=True,
-                               contraction=contraction)
+    saved = settings.ozaki_min_determinants
+    settings.ozaki_min_determinants = 0
+    try:
+        bt = batched.BatchedTaylor(specs, 0.1, nterms=10,
+                                   dtype=torch.complex128, tiles=tiles,
+                                   nstreams=4, group=True,
+                                   contraction=contraction)
+    finally:
+        settings.ozaki_min_determinants = saved
+    assert any(p.s.w_oz for p in bt.sectors) == (contraction == "ozaki")
     bt.build()
     want = sum(1 for p in bt.sectors if p.variant == "rows4")
     assert bt.grouped() == want > 0

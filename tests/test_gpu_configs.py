@@ -90,13 +90,20 @@ def test_batched_256_sectors_seed3(fqe):
     print(f"  complex64 graph vs FP64: apply {ea:.2e}, Taylor {ee:.2e}",
           flush=True)
     assert ea < 1e-4 and ee < 1e-3
-    # the mixed engine at <= 1e-9: complex128 graph, every split-capable
-    # sector on the Ozaki-digit split kernels
-    from fqe_amd import _lib
+    # the mixed engine at <= 1e-9: complex128 graph, every sector that the
+    # digit kernels take on them
+    from fqe_amd import settings
     tiles = {f"{sp.norb},{sp.nalpha},{sp.nbeta}": "split" for sp in specs}
-    oz = batched.BatchedTaylor(specs, 0.1, nterms=10, dtype=torch.complex128,
-                               nstreams=8, tiles=tiles, contraction="ozaki")
-    ndigit = sum(1 for p in oz.sectors if p.s.tile == _lib.TILE_OZAKI)
+    saved = settings.ozaki_min_determinants
+    settings.ozaki_min_determinants = 0
+    try:
+        oz = batched.BatchedTaylor(specs, 0.1, nterms=10,
+                                   dtype=torch.complex128, nstreams=8,
+                                   tiles=tiles, contraction="ozaki")
+    finally:
+        settings.ozaki_min_determinants = saved
+    ndigit = sum(1 for p in oz.sectors
+                 if p.s.w_oz and p.s.haa_oz and p.s.hbb_oz)
     oz.build()
     oz.launch()
     ores = oz.results()

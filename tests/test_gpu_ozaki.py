@@ -36,17 +36,44 @@ def rel(a, b):
 
 
 class _contraction:
+    """Runs in this arithmetic, digits on sectors of every size."""
+
     def __init__(self, mode):
         self.mode = mode
 
     def __enter__(self):
         from fqe_amd import settings
-        self.saved = settings.contraction
-        settings.contraction = self.mode
+        self.saved = settings.contraction, settings.ozaki_min_determinants
+        settings.contraction, settings.ozaki_min_determinants = self.mode, 0
 
     def __exit__(self, *exc):
         from fqe_amd import settings
-        settings.contraction = self.saved
+        settings.contraction, settings.ozaki_min_determinants = self.saved
+
+
+def _digits(s):
+    """Whether the descriptor's sector runs on the digit kernels."""
+    return bool(s.pull_w and s.w_oz and s.haa_oz and s.hbb_oz)
+
+
+def test_ozaki_threshold(fqe):
+    """By default small sectors of the digit engine run in FP64 and large
+    ones on digits."""
+    from fqe_amd import _lib, engine, settings
+    from fqe_amd.fci_graph import FciGraph
+    saved = settings.contraction
+    settings.contraction = "ozaki"
+    try:
+        for norb, na, nb, digits in ((8, 4, 4, False), (10, 5, 5, False),
+                                     (12, 6, 6, True), (13, 6, 6, True)):
+            h = fo.synthetic_hamiltonian(norb, norb,
+                                         numpy.random.default_rng(norb))
+            op = engine.prepare_operator(h, norb, _lib.device())
+            s, keep = engine.sector_struct(FciGraph(na, nb, norb), op,
+                                           _lib.C128)
+            assert s.tile == _lib.TILE_OZAKI and _digits(s) == digits
+    finally:
+        settings.contraction = saved
 
 
 def _apply(fqe, c, h1, h2, na, nb, norb, mode, op=None):
@@ -75,7 +102,7 @@ def test_ozaki_apply_matches_fp64_and_oracle(fqe, na, nb, norb):
         d = fqe.FqeData(na, nb, norb, dtype=numpy.complex128)
         op = engine.prepare_operator((h1, h2), norb, _lib.device())
         s, keep = engine.sector_struct(d.get_fcigraph(), op, _lib.C128)
-        assert s.tile == _lib.TILE_OZAKI and s.hbb_f64
+        assert s.tile == _lib.TILE_OZAKI and s.hbb_f64 and _digits(s)
         assert _lib.lib().fqehip_fused_supported(
             _lib.C128, ctypes.byref(s), ctypes.byref(op.c_struct()))
         del keep
@@ -90,7 +117,7 @@ def test_ozaki_apply_matches_fp64_and_oracle(fqe, na, nb, norb):
 
 def test_ozaki_peaked_vector(fqe):
     """A vector dominated by one determinant (a ground-state-like shape):
-    the per-string D' scale must keep the small components accurate."""
+    the scale per string must keep the small components accurate."""
     norb, na, nb = 10, 5, 5
     rng = numpy.random.default_rng(77)
     h1, h2 = fo.synthetic_hamiltonian(norb, norb, rng)
@@ -140,13 +167,11 @@ def test_ozaki_norb14_vs_fp64_and_reference_c(fqe):
 
 
 def test_ozaki_norb15_global_beta_rows(fqe):
-    """norb=15 7a8b (41.4 M determinants), the largest sector the digit
-    split kernel takes (121 of its 128 pair rows): row ia (103 KB) no longer
-    fits in LDS beside the operator digits, so the beta gather reads it from
-    global memory.  Against the FP64 engine (the column-owned FP64 split
-    kernel at its widest gather, 121 of 128 rows) at the 1e-9 gate, and the
-    FP64 split result against the FP64 unfused path (its LDS-resident pair
-    GEMM, 8 row tiles) to 1e-12."""
+    """norb=15 7a8b (41.4 M determinants), the largest sector the digit rows
+    take (120 of 128 pairs, 64 de-excitation rows, a 103 KB accumulator row
+    beside the operator digits in LDS).  Against the FP64 engine (its pull
+    form with 8 W tiles in two passes) at the 1e-9 gate, and that against the
+    FP64 unfused path (its LDS-resident pair GEMM, 8 row tiles) to 1e-12."""
     import ctypes
     import torch
     from fqe_amd import _lib, engine
@@ -160,7 +185,7 @@ def test_ozaki_norb15_global_beta_rows(fqe):
         d = fqe.FqeData(na, nb, norb, dtype=numpy.complex128)
         op = engine.prepare_operator((h1, h2), norb, _lib.device())
         s, keep = engine.sector_struct(d.get_fcigraph(), op, _lib.C128)
-        assert s.tile == _lib.TILE_OZAKI and s.hbb_f64
+        assert s.tile == _lib.TILE_OZAKI and s.hbb_f64 and _digits(s)
         assert _lib.lib().fqehip_fused_supported(
             _lib.C128, ctypes.byref(s), ctypes.byref(op.c_struct()))
         del keep, d

@@ -483,3 +483,36 @@ def test_coefficients_that_are_not_finite(fqe, kind, contraction, na, nb,
     assert rest.any()
     tol = 3e-11 if contraction == "ozaki" else 1e-13
     assert rel(got[rest], want[rest]) < tol
+
+
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("na,nb,norb", [(4, 3, 8), (3, 5, 9), (6, 1, 12)])
+def test_series_in_digits(fqe, na, nb, norb, graph):
+    """A Taylor series on the digit kernels (norm test in its own launch,
+    second term buffer behind the digit planes) against the FP64 one: the
+    same number of terms, and 3e-11 as for one apply (each term's error is
+    that of its apply, and the terms after the first few are small)."""
+    from fqe_amd import settings
+    print(f"series in digits {na} {nb} {norb} {graph}", flush=True)
+    rng = numpy.random.default_rng(50 * norb + na)
+    h1, h2 = fo.synthetic_hamiltonian(norb, norb, rng)
+    ham = fqe.get_restricted_hamiltonian((h1, h2))
+    d, c, g, rng = sector(fqe, na, nb, norb, 7)
+    key = (na + nb, na - nb)
+    wfn = fqe.Wavefunction([[na + nb, na - nb, norb]])
+    wfn.set_wfn("from_data", {key: c / numpy.linalg.norm(c)})
+    want = wfn.time_evolve(0.05, ham)
+    saved = (settings.contraction, settings.ozaki_min_determinants,
+             settings.taylor_graph)
+    settings.contraction, settings.ozaki_min_determinants = "ozaki", 0
+    settings.taylor_graph = graph
+    try:
+        for _ in range(2):
+            got = wfn.time_evolve(0.05, ham)
+            assert got._taylor_terms == want._taylor_terms
+            assert rel(got.get_coeff(key), want.get_coeff(key)) < 3e-11
+            assert not numpy.array_equal(got.get_coeff(key),
+                                         want.get_coeff(key))
+    finally:
+        (settings.contraction, settings.ozaki_min_determinants,
+         settings.taylor_graph) = saved

@@ -27,8 +27,10 @@ def rel(a, b):
 
 def _evolve(fqe, c, h1, h2, na, nb, norb, t, graph, dtype, contraction):
     from fqe_amd import settings
-    saved = settings.taylor_graph, settings.contraction
+    saved = (settings.taylor_graph, settings.contraction,
+             settings.ozaki_min_determinants)
     settings.taylor_graph, settings.contraction = graph, contraction
+    settings.ozaki_min_determinants = 0
     try:
         key = (na + nb, na - nb)
         wfn = fqe.Wavefunction([[na + nb, na - nb, norb]], dtype=dtype)
@@ -42,7 +44,8 @@ def _evolve(fqe, c, h1, h2, na, nb, norb, t, graph, dtype, contraction):
             torch.zeros(1000, device="cuda").sum().item()
         return outs
     finally:
-        settings.taylor_graph, settings.contraction = saved
+        (settings.taylor_graph, settings.contraction,
+         settings.ozaki_min_determinants) = saved
 
 
 @pytest.mark.parametrize("na,nb,norb,dtype,contraction", [
