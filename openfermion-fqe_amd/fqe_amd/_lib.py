@@ -11,6 +11,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import threading
 from ctypes import POINTER, c_double, c_int, c_int32, c_int64, c_void_p
 
 import torch  # noqa: F401  (must precede the CDLL load, see module doc)
@@ -253,23 +254,40 @@ class TableCache:
 
     def __init__(self, device: torch.device) -> None:
         self._index = device.index
+        self._lock = threading.RLock()
+        self._fresh = None   # values made within the build under way
         self._items = {}     # key -> [value, event or None, streams in order]
 
     def get(self, key, build, *args):
         """The value of ``key``, made by build(*args) if it is missing."""
         item = self._items.get(key)
         if item is None:
-            return self._add(key, build(*args))
+            return self._build(key, build, args)
         if raw_stream(self._index) not in item[2]:
             self._admit(item)
         return item[0]
 
-    def _add(self, key, value):
-        if not torch.cuda.is_current_stream_capturing():
-            event = torch.cuda.Event()
-            event.record()
-            self._items[key] = [value, event, {raw_stream(self._index)}]
-        return value
+    def _build(self, key, build, args):
+        """One event for a build and the builds that it asks for."""
+        with self._lock:
+            if key in self._items:
+                return self.get(key, build, *args)
+            if self._fresh is not None:
+                if key not in self._fresh:
+                    self._fresh[key] = build(*args)
+                return self._fresh[key]
+            self._fresh = {}
+            try:
+                value = self._fresh[key] = build(*args)
+                if not torch.cuda.is_current_stream_capturing():
+                    event = torch.cuda.Event()
+                    event.record()
+                    stream = raw_stream(self._index)
+                    for k, v in self._fresh.items():
+                        self._items[k] = [v, event, {stream}]
+                return value
+            finally:
+                self._fresh = None
 
     def _admit(self, item) -> None:
         if torch.cuda.is_current_stream_capturing():
@@ -289,6 +307,10 @@ class TableCache:
 
     def __len__(self) -> int:
         return len(self._items)
+
+    def __reduce__(self):
+        """Copies and pickles build their tables anew."""
+        return TableCache, (torch.device("cuda", self._index),)
 
 
 def ptr(t) -> int:

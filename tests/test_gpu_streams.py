@@ -95,3 +95,20 @@ def test_tables_first_needed_under_capture(fqe, kind):
         torch.cuda.synchronize()
         assert numpy.array_equal(out.cpu().numpy(), want.cpu().numpy()), k
         x.mul_(0.5 - 1j)
+
+
+@pytest.mark.parametrize("how", ["deepcopy", "pickle"])
+def test_copies_of_an_applied_hamiltonian(fqe, how):
+    """A Hamiltonian that holds its device tables copies and pickles, and
+    the copy applies with the same bits."""
+    import copy
+    import pickle
+    rng = numpy.random.default_rng(3)
+    h = tensors("real", 7, rng)
+    wfn = fqe.Wavefunction([[7, 1, 7]])
+    wfn.set_wfn("random")
+    ham = fqe.get_restricted_hamiltonian(h)
+    want = wfn.apply(ham).get_coeff((7, 1))
+    other = (copy.deepcopy(ham) if how == "deepcopy" else
+             pickle.loads(pickle.dumps(ham)))
+    assert numpy.array_equal(wfn.apply(other).get_coeff((7, 1)), want)
