@@ -11,8 +11,8 @@
 // makes the same same-spin / opposite-spin split in its lm kernels
 // (src/fqe/lib/fqe_data.c:668-720 and :879-996).
 //
-//   k_spin_block:  Hbb column by column from the beta forward table
-//                  (one workgroup per source string, column in LDS);
+//   k_spin_block:  Hbb column by column, its non-zero elements found through
+//                  the beta forward table (one workgroup per source string);
 //   k_beta_split:  transpose and split into bfloat16 hi + lo, zero-padded
 //                  to ldh x ldh (ldh a multiple of 128);
 //   k_beta_gemm_bf16x3: out[Ia][Ib'] = sum_Ib C[Ia][Ib] Hbb[Ib'][Ib] on
@@ -43,15 +43,27 @@ __device__ __forceinline__ float from_bf16(__bf16 h) {
 
 __device__ __forceinline__ int32_t iabs(int32_t v) { return v < 0 ? -v : v; }
 
-// Column Ib of the block: LDS accumulator of lenb values, built in a fixed
-// order so that every run gives the same bits.  For each q in turn the
-// intermediate string s = E_q Ib is uniform over the workgroup; the
-// off-diagonal pairs p move one electron of s, so they reach distinct
-// targets t != s and are added by one thread each; the diagonal pairs
-// (t = s) and the one-body term of q are summed by wave 0 in a fixed lane
-// order (per-lane strided sums, then an xor butterfly) and added to s.
-// V[p][q] is amat[p * lda + q], the one-body term h1[q]; CPLX: both in the
-// real 2 x 2 block form (real part at [2p][2q], imaginary at [2p + 1][2q]).
+// Column s of the block, sum_pq V[p][q] E_p E_q + sum_q h[q] E_q between the
+// strings t and s, E_(ai) = a+_a a_i.  An element is non-zero for t = s and for
+// strings one or two excitations away, and each is computed as a whole by the
+// threads that own it (i, j occupied in s, a, b empty, i < j, a < b):
+//   i -> a, j -> b:  V[bj][ai] + V[ai][bj] - V[bi][aj] - V[aj][bi], times the sign
+//       of E_bj E_ai;
+//   i -> a:  h[ai] + V[ai][ii] + V[aa][ai] + sum over the other k of V[kk][ai] +
+//       V[ai][kk] - V[ki][ak] (k occupied) or V[ak][ki] (k empty), times the sign of
+//       E_ai: the ways over an intermediate string, in either order;
+//   t = s:  sum_k h[kk] + sum_kl V[kk][ll] + sum_ia V[ia][ai].
+// A compressed pair stands for both of its excitations, of which one applies.
+// V[p][q] is amat[p * lda + q], h[q] is h1[q]; CPLX: both in the real 2 x 2 block
+// form (real part at [2p][2q], imaginary at [2p + 1][2q]).
+//
+// One workgroup per source string; the column is assembled in LDS (targets are
+// scattered, 645 of 6435 at 15 orbitals) and written in one piece, so what
+// bounds it is that write and, below some hundreds of strings, two dependent
+// table lookups.  Every element has one order of additions: the same bits on
+// every run.  6435 strings of 15 orbitals: 137 us, 3432 of 14: 49, against 636
+// and 202 when the workgroup went through the pairs q one after the other with
+// two barriers each (V[p][q] E_p added to the column for all p at once).
 template <bool CPLX>
 struct BlockValue {
   double re, im;
@@ -61,67 +73,212 @@ struct BlockValue<false> {
   double re;
 };
 
+constexpr int kBlockOrb = 32;               // orbitals at most
+
+// Only the empty or the full shell, on one string: the excitations that do not
+// vanish are the occupation numbers, whatever the order of the pairs.
+template <bool CPLX>
+__global__ void __launch_bounds__(64)
+k_spin_block_one(int npair, const int32_t* __restrict__ fwd,
+                 const double* __restrict__ amat, int64_t lda,
+                 const double* __restrict__ h1, double* __restrict__ hcol) {
+  constexpr int kW = CPLX ? 2 : 1;
+  double re = 0.0, im = 0.0;
+  for (int q = threadIdx.x; q < npair; q += 64) {
+    if (!fwd[q]) continue;
+    re += h1[kW * q];
+    if (CPLX) im += h1[lda + kW * q];
+    for (int p = 0; p < npair; ++p) {
+      if (!fwd[p]) continue;
+      const double* e = amat + static_cast<int64_t>(kW) * p * lda + kW * q;
+      re += e[0];
+      if (CPLX) im += e[lda];
+    }
+  }
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) {
+    re += __shfl_xor(re, m);
+    im += __shfl_xor(im, m);
+  }
+  if (threadIdx.x == 0) {
+    hcol[0] = re;
+    if (CPLX) hcol[1] = im;
+  }
+}
+
+// LDS of a column: the values, then the lists of occupied and empty orbitals
+// and of their pairs (16 bits each).
+size_t spin_block_lds(int norb, int64_t len, bool cplx) {
+  // both shells' pairs: the most that any filling has
+  return static_cast<size_t>(len) * (cplx ? 16 : 8) +
+         (static_cast<size_t>(norb) * (norb - 1) / 2 + 2 * kBlockOrb) * 2;
+}
+
 template <bool CPLX>
 __global__ void __launch_bounds__(kBlockThreads)
-k_spin_block(int npair, int64_t lenb, const int32_t* __restrict__ fwd,
+k_spin_block(int norb, int compressed, int64_t len, const int32_t* __restrict__ fwd,
              const double* __restrict__ amat, int64_t lda,
              const double* __restrict__ h1, double* __restrict__ hcol) {
   typedef BlockValue<CPLX> V;
   constexpr int kW = CPLX ? 2 : 1;            // rows and columns per pair
   extern __shared__ __align__(16) char block_smem[];
   V* col = reinterpret_cast<V*>(block_smem);
-  V* diag = col + lenb;                       // [npair] diagonal terms of q
-  const int64_t ib = blockIdx.x;
+  uint16_t* occ = reinterpret_cast<uint16_t*>(col + len);
+  uint16_t* emp = occ + kBlockOrb;
+  uint16_t* pairs = emp + kBlockOrb;          // of occ, then of emp: low i, high j
+  const int64_t s = blockIdx.x;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  for (int64_t x = tid; x < lenb; x += kBlockThreads) col[x] = V{};
+  auto pair = [&](int i, int j) { return compressed ? comp_pair(i, j) : i * norb + j; };
+  auto jump = [&](int i, int j, int64_t from) { return fwd[pair(i, j) * len + from]; };
+  // every wave finds the occupied orbitals for itself
+  const uint32_t mask = static_cast<uint32_t>(
+      __ballot(lane < norb && jump(lane < norb ? lane : 0, lane < norb ? lane : 0, s) != 0));
+  const int no = __popc(mask), ne = norb - no;
+  const int npo = no * (no - 1) / 2, npe = ne * (ne - 1) / 2;
+  if (tid < norb) {
+    const uint32_t below = (1u << tid) - 1u;
+    if (mask >> tid & 1) occ[__popc(mask & below)] = static_cast<uint16_t>(tid);
+    else emp[__popc(~mask & below)] = static_cast<uint16_t>(tid);
+  }
+  for (int64_t x = tid; x < len; x += kBlockThreads) col[x] = V{};
   __syncthreads();
-  const int K = npair;
-  for (int q = 0; q < K; ++q) {
-    const int32_t f = fwd[static_cast<int64_t>(q) * lenb + ib];
-    if (!f) continue;                         // uniform over the workgroup
-    const int64_t s = iabs(f) - 1;
-    const double sf = f > 0 ? 1.0 : -1.0;
-    for (int p = tid; p < K; p += kBlockThreads) {
-      const int32_t g = fwd[static_cast<int64_t>(p) * lenb + s];
-      V v{};
-      if (g) {
-        const double sg = g > 0 ? sf : -sf;
-        const double* e = amat + static_cast<int64_t>(kW) * p * lda + kW * q;
-        V c{};
-        c.re = sg * e[0];
-        if constexpr (CPLX) c.im = sg * e[lda];
-        const int64_t t = iabs(g) - 1;
-        if (t == s) {
-          v = c;
+  for (int x = tid; x < no * no + ne * ne; x += kBlockThreads) {
+    const bool o = x < no * no;
+    const int n = o ? no : ne, y = o ? x : x - no * no;
+    const int i = y / n, j = y - i * n;
+    if (i >= j) continue;
+    const uint16_t* l = o ? occ : emp;
+    pairs[(o ? 0 : npo) + i * (2 * n - i - 1) / 2 + j - i - 1] =
+        static_cast<uint16_t>(l[i] | l[j] << 8);
+  }
+  __syncthreads();
+
+  auto add = [&](V& v, double f, int p, int q) {
+    const double* e = amat + static_cast<int64_t>(kW) * p * lda + kW * q;
+    v.re += f * e[0];
+    if constexpr (CPLX) v.im += f * e[lda];
+  };
+  auto add_h = [&](V& v, int q) {
+    v.re += h1[kW * q];
+    if constexpr (CPLX) v.im += h1[lda + kW * q];
+  };
+  auto put = [&](int32_t f, bool minus, V v) {    // at f's target with its sign
+    const double sg = (f < 0) != minus ? -1.0 : 1.0;
+    v.re *= sg;
+    if constexpr (CPLX) v.im *= sg;
+    col[iabs(f) - 1] = v;
+  };
+  for (int x = tid; x < npo * npe; x += kBlockThreads) {
+    const int y = x / npe;
+    const int ij = pairs[y], ab = pairs[npo + x - y * npe];
+    const int i = ij & 255, j = ij >> 8, a = ab & 255, b = ab >> 8;
+    const int32_t f1 = jump(a, i, s);
+    const int32_t f2 = jump(b, j, iabs(f1) - 1);
+    const int ai = pair(a, i), bj = pair(b, j), aj = pair(a, j), bi = pair(b, i);
+    V v{};
+    add(v, 1.0, bj, ai);
+    add(v, 1.0, ai, bj);
+    add(v, -1.0, bi, aj);
+    add(v, -1.0, aj, bi);
+    put(f2, f1 < 0, v);
+  }
+  // eight lanes to an element, every eighth k each
+  auto sum8 = [&](V& v) {
+#pragma unroll
+    for (int m = 1; m < 8; m <<= 1) {
+      v.re += __shfl_xor(v.re, m);
+      if constexpr (CPLX) v.im += __shfl_xor(v.im, m);
+    }
+  };
+  const int sub = tid & 7;
+  for (int x0 = 0; x0 < no * ne; x0 += kBlockThreads / 8) {
+    const int x = x0 + (tid >> 3);
+    const bool ok = x < no * ne;
+    const int i = ok ? occ[x / ne] : 0, a = ok ? emp[x % ne] : 0;
+    const int ai = pair(a, i);
+    V v{};
+    if (ok) {
+      if (sub == 0) add_h(v, ai);
+      for (int k = sub; k < norb; k += 8) {
+        const int kk = pair(k, k);
+        if (k == i) {
+          add(v, 1.0, ai, kk);
+        } else if (k == a) {
+          add(v, 1.0, kk, ai);
+        } else if (mask >> k & 1) {
+          add(v, 1.0, kk, ai);
+          add(v, 1.0, ai, kk);
+          add(v, -1.0, pair(k, i), pair(a, k));
         } else {
-          col[t].re += c.re;
-          if constexpr (CPLX) col[t].im += c.im;
+          add(v, 1.0, pair(a, k), pair(k, i));
         }
       }
-      diag[p] = v;
     }
-    __syncthreads();
-    if (tid < 64) {
-      V v{};
-      for (int p = lane; p < K; p += 64) {
-        v.re += diag[p].re;
-        if constexpr (CPLX) v.im += diag[p].im;
-      }
-#pragma unroll
-      for (int m = 32; m >= 1; m >>= 1) {
-        v.re += __shfl_xor(v.re, m);
-        if constexpr (CPLX) v.im += __shfl_xor(v.im, m);
-      }
-      if (lane == 0) {
-        col[s].re += v.re + sf * h1[kW * q];
-        if constexpr (CPLX) col[s].im += v.im + sf * h1[lda + kW * q];
-      }
-    }
-    __syncthreads();
+    sum8(v);
+    if (ok && sub == 0) put(jump(a, i, s), false, v);
   }
-  V* dst = reinterpret_cast<V*>(hcol) + ib * lenb;
-  for (int64_t x = tid; x < lenb; x += kBlockThreads) dst[x] = col[x];
+  if (tid < 64) {
+    V v{};
+    for (int x = lane; x < no * norb; x += 64) {
+      const int i = occ[x / norb], k = x % norb;
+      if (mask >> k & 1) add(v, 1.0, pair(i, i), pair(k, k));
+      else add(v, 1.0, pair(i, k), pair(k, i));
+      if (k == i) add_h(v, pair(i, i));
+    }
+    sum8(v);
+#pragma unroll
+    for (int m = 8; m < 64; m <<= 1) {
+      v.re += __shfl_xor(v.re, m);
+      if constexpr (CPLX) v.im += __shfl_xor(v.im, m);
+    }
+    if (lane == 0) col[s] = v;
+  }
+  __syncthreads();
+  V* dst = reinterpret_cast<V*>(hcol) + s * len;
+  for (int64_t x = tid; x < len; x += kBlockThreads) dst[x] = col[x];
+}
+
+// The orbitals behind npair pairs on len > 1 strings of one spin:
+// norb (norb + 1) / 2 compressed pairs or norb^2, and len a binomial of norb
+// (36 pairs are both, of 8 and of 6 orbitals, but no other number of strings
+// than one is).  False if there are none.
+bool spin_block_orbitals(int npair, int64_t len, int* norb, int* compressed) {
+  for (int n = 2; n <= kBlockOrb; ++n) {
+    const bool c = npair == n * (n + 1) / 2;
+    if (!c && npair != n * n) continue;
+    int64_t binom = n;
+    for (int k = 1; k < n; ++k) {
+      if (binom == len) {
+        *norb = n;
+        *compressed = c ? 1 : 0;
+        return true;
+      }
+      binom = binom * (n - k) / (k + 1);
+    }
+  }
+  return false;
+}
+
+template <bool CPLX>
+int spin_block(int npair, int64_t len, const int32_t* fwd, const double* amat,
+               int64_t lda, const double* h1, double* hcol, hipStream_t st) {
+  if (len == 1) {
+    k_spin_block_one<CPLX><<<1, 64, 0, st>>>(npair, fwd, amat, lda, h1, hcol);
+    FQEHIP_CHECK_LAUNCH("k_spin_block_one");
+    return FQEHIP_OK;
+  }
+  int norb = 0, compressed = 0;
+  if (!spin_block_orbitals(npair, len, &norb, &compressed)) {
+    set_error("k_spin_block: no orbitals have %d pairs and %lld strings", npair,
+              static_cast<long long>(len));
+    return FQEHIP_ERR_INVALID;
+  }
+  k_spin_block<CPLX><<<static_cast<unsigned>(len), kBlockThreads,
+                       spin_block_lds(norb, len, CPLX), st>>>(
+      norb, compressed, len, fwd, amat, lda, h1, hcol);
+  FQEHIP_CHECK_LAUNCH("k_spin_block");
+  return FQEHIP_OK;
 }
 
 // hhi/hlo[r][c] = split(Hbb[r][c]) = split(hcol[c][r]); zero outside lenb.
@@ -530,12 +687,9 @@ extern "C" int fqehip_beta_block(int npair, int64_t lenb, const int32_t* d_fwd_b
   FQEHIP_CHECK_ARG(d_a && d_hcol && d_hhi && d_hlo, "NULL pointer");
   FQEHIP_CHECK_ARG(npair == 0 || d_fwd_b, "NULL beta forward table");
   hipStream_t st = as_stream(stream);
-  // npair == 0 (no orbitals) leaves the LDS column zero: Hbb = 0
-  k_spin_block<false><<<static_cast<unsigned>(lenb), kBlockThreads,
-                        (lenb + npair) * sizeof(double), st>>>(
-      npair, lenb, d_fwd_b, d_a, npair,
-      d_a + static_cast<int64_t>(npair) * npair, d_hcol);
-  FQEHIP_CHECK_LAUNCH("k_spin_block");
+  int rc = spin_block<false>(npair, lenb, d_fwd_b, d_a, npair,
+                             d_a + static_cast<int64_t>(npair) * npair, d_hcol, st);
+  if (rc) return rc;
   dim3 grid(static_cast<unsigned>(ldh / 32), static_cast<unsigned>(ldh / 32));
   k_beta_split<<<grid, 256, 0, st>>>(lenb, ldh, d_hcol,
                                       reinterpret_cast<__bf16*>(d_hhi),
@@ -560,14 +714,8 @@ extern "C" int fqehip_spin_block(int complex_op, int npair, int64_t len,
   if (len == 0) return FQEHIP_OK;
   FQEHIP_CHECK_ARG(d_hcol && (npair == 0 || (d_fwd && d_v && d_h)), "NULL pointer");
   hipStream_t st = as_stream(stream);
-  if (complex_op)
-    k_spin_block<true><<<static_cast<unsigned>(len), kBlockThreads, lds, st>>>(
-        npair, len, d_fwd, d_v, lda, d_h, d_hcol);
-  else
-    k_spin_block<false><<<static_cast<unsigned>(len), kBlockThreads, lds, st>>>(
-        npair, len, d_fwd, d_v, lda, d_h, d_hcol);
-  FQEHIP_CHECK_LAUNCH("k_spin_block");
-  return FQEHIP_OK;
+  return complex_op ? spin_block<true>(npair, len, d_fwd, d_v, lda, d_h, d_hcol, st)
+                    : spin_block<false>(npair, len, d_fwd, d_v, lda, d_h, d_hcol, st);
 }
 
 extern "C" int fqehip_beta_gemm(int64_t lena, int64_t lenb,

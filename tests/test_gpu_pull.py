@@ -516,3 +516,36 @@ def test_series_in_digits(fqe, na, nb, norb, graph):
     finally:
         (settings.contraction, settings.ozaki_min_determinants,
          settings.taylor_graph) = saved
+
+
+@pytest.mark.parametrize("kind", ["real", "nonsymmetric", "complex"])
+@pytest.mark.parametrize("nele,norb", [
+    (0, 3), (1, 1), (1, 2), (2, 3), (3, 3), (0, 6), (6, 6), (0, 8), (8, 8),
+    (3, 6), (4, 8), (1, 8), (7, 8), (2, 9), (6, 9), (5, 10)])
+def test_spin_block_elements(fqe, kind, nele, norb):
+    """Every element of fqehip_spin_block against the same sum of dense
+    pair matrices, from the library's forward table, in numpy: no, one and
+    two excitations, empty and full shells, shells of one electron or one
+    hole, and 36 pairs as 8 compressed or 6 plain orbitals.  1e-13 of the
+    largest element (sums of at most norb^2 + 4 norb products)."""
+    from fqe_amd import engine
+    from fqe_amd.fci_graph import FciGraph
+    print(f"spin block {kind} {nele} {norb}", flush=True)
+    rng = numpy.random.default_rng(100 * norb + nele)
+    op = prepared(fqe, kind, tensors(kind, norb, rng), norb)
+    tab = FciGraph(nele, nele, norb).tables(True)
+    got = op._spin_block(tab, True).cpu().numpy().T       # by target, source
+    fwd = tab.fused_tables(op.compressed)[0].cpu().numpy()
+    a = op.a.cpu().numpy()
+    if op.complex_op:
+        a = a[::2, ::2] + 1j * a[1::2, ::2]
+    n = tab.length
+    pair = numpy.zeros((op.npair, n, n))
+    p, src = numpy.nonzero(fwd)
+    f = fwd[p, src]
+    pair[p, numpy.abs(f) - 1, src] = numpy.sign(f)
+    want = numpy.einsum("q,qij->ij", a[-1], pair)
+    for q in range(op.npair):
+        want = want + numpy.einsum("p,pij->ij", a[:-1, q], pair) @ pair[q]
+    scale = max(numpy.abs(want).max(), 1e-300)
+    assert numpy.abs(got - want).max() <= 1e-13 * scale
