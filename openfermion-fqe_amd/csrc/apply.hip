@@ -611,8 +611,8 @@ int launch_fused(int precision, int norb, int npair, int64_t lena, int64_t lenb,
                  bool split, int tile, hipStream_t st, const int32_t* done);
 // Defined in ozaki.hip.
 int launch_absmax(int64_t lena, int64_t lenb, const double* coeff,
-                  double* rowmax, double* colmax, hipStream_t st,
-                  const int32_t* done);
+                  double* rowmax, double* colmax, double* sums, int64_t nsum,
+                  hipStream_t st, const int32_t* done);
 bool beta_oz_shape_ok(int64_t lena, int64_t lenb);
 int64_t beta_oz_workspace_bytes(int64_t lena, int64_t lenb);
 int launch_beta_gemm_oz(int64_t lena, int64_t lenb, const void* hoz,
@@ -832,12 +832,18 @@ bool digit_blocks(const fqehip_sector* s) {
          beta_oz_shape_ok(s->lena, s->lenb) && beta_oz_shape_ok(s->lenb, s->lena);
 }
 
+// Sums of the digit rows in global memory (0: none).
+int64_t digit_sums(const fqehip_sector* s) {
+  return pull_oz_segments(s) > 1 ? 2 * s->lena * s->lenb : 0;
+}
+
 // Workspace of an apply in the pull form: the row accumulators; for the digit
-// kernels the row maxima of |C|, and for the blocks its column maxima and the
-// digit planes of C (then of C^T).
+// kernels the row maxima of |C| and, where rows are shared, their sums and
+// factors, and for the blocks its column maxima and the digit planes of C (then
+// of C^T).
 int64_t pull_apply_bytes(const fqehip_sector* s) {
   int64_t b = 16 * s->lena * s->lenb;
-  if (digit_rows(s)) b += 8 * s->lena;
+  if (digit_rows(s)) b += 8 * (2 * s->lena + digit_sums(s));
   if (digit_blocks(s)) {
     const int64_t c = beta_oz_workspace_bytes(s->lena, s->lenb);
     const int64_t ct = beta_oz_workspace_bytes(s->lenb, s->lena);
@@ -905,9 +911,11 @@ int pull_rows(const fqehip_sector* s, const fqehip_operator* op,
     return launch_pull_rows(s, op->complex_op, c, rowacc, rest, st, done);
   }
   double* rowmax = rowacc + 2 * s->lena * s->lenb;
+  double* sums = rowmax + s->lena;
+  const int64_t nsum = digit_sums(s);
   const bool blocks = digit_blocks(s);
-  double* colmax = blocks ? rowmax + s->lena : nullptr;
-  int rc = launch_absmax(s->lena, s->lenb, c, rowmax, colmax, st, done);
+  double* colmax = blocks ? sums + nsum + s->lena : nullptr;
+  int rc = launch_absmax(s->lena, s->lenb, c, rowmax, colmax, sums, nsum, st, done);
   if (rc) return rc;
   if (blocks) {
     void* cwork = colmax + s->lenb;
@@ -920,7 +928,7 @@ int pull_rows(const fqehip_sector* s, const fqehip_operator* op,
     rc = launch_same_spin(s, 0, c, rowacc, PullSeries{}, st, done);
   }
   if (rc) return rc;
-  return launch_pull_rows_oz(s, c, rowmax, rowacc, e, st, done);
+  return launch_pull_rows_oz(s, c, rowmax, rowacc, sums, e, st, done);
 }
 
 // Whether the n bytes at a and those at b have some in common (a may be NULL).

@@ -64,10 +64,12 @@ __device__ __forceinline__ double factor_back(double m, int e) {
 }
 
 // rowmax[I] = max over the row of max(|Re C[I][.]|, |Im C[I][.]|), infinity where
-// one is not finite; zeroes colmax (when not NULL) for k_col_absmax.
+// one is not finite; zeroes colmax (when not NULL) for k_col_absmax and the nsum
+// sums of k_pull_rows_oz.
 __global__ void __launch_bounds__(256)
 k_row_absmax(int64_t lena, int64_t lenb, const double* __restrict__ coeff,
              double* __restrict__ rowmax, unsigned long long* __restrict__ colmax,
+             unsigned long long* __restrict__ sums, int64_t nsum,
              const int32_t* __restrict__ done) {
   __shared__ double red[4];
   if (done && *done) return;
@@ -75,6 +77,9 @@ k_row_absmax(int64_t lena, int64_t lenb, const double* __restrict__ coeff,
     for (int64_t j = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; j < lenb;
          j += static_cast<int64_t>(gridDim.x) * 256)
       colmax[j] = 0;
+  for (int64_t j = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; j < nsum;
+       j += static_cast<int64_t>(gridDim.x) * 256)
+    sums[j] = 0;
   for (int64_t r = blockIdx.x; r < lena; r += gridDim.x) {
     const double* row = coeff + r * lenb * 2;
     double m = 0.0;
@@ -297,6 +302,9 @@ struct OzRowsArgs {
   double* acc;
   double* partials;
   const int32_t* done;
+  int nseg;                                // workgroups per alpha string
+  unsigned long long* sums;                // nseg > 1: [lena][lenb][re, im]
+  double* back;                            // and each row's factor
 };
 
 constexpr int kRowThreads = 512;
@@ -310,6 +318,38 @@ size_t oz_rows_lds_bytes(int64_t lenb, int nqt) {
          kOzK * (8 + 4 + 4) + 16;
 }
 
+// The finished row ia: rowacc + back * value(x), and the epilogue.
+template <typename F>
+__device__ __forceinline__ void oz_finish(const OzRowsArgs& p, int64_t ia, double back,
+                                          F value, char* smem) {
+  double2* racc = reinterpret_cast<double2*>(p.rowacc) + ia * p.lenb;
+  double sq = 0.0;
+  for (int x = threadIdx.x; x < static_cast<int>(p.lenb); x += kRowThreads) {
+    const double2 r = racc[x];
+    const double re = r.x + back * static_cast<double>(static_cast<int64_t>(value(2 * x)));
+    const double im = r.y + back * static_cast<double>(static_cast<int64_t>(value(2 * x + 1)));
+    if (!p.out) {
+      racc[x] = make_double2(re, im);
+      continue;
+    }
+    const int64_t idx = ia * p.lenb + x;
+    double vr = p.alpha_re * re - p.alpha_im * im;
+    double vi = p.alpha_re * im + p.alpha_im * re;
+    if (p.beta_re != 0.0 || p.beta_im != 0.0) {
+      const double2 c = reinterpret_cast<const double2*>(p.cin)[idx];
+      vr += p.beta_re * c.x - p.beta_im * c.y;
+      vi += p.beta_re * c.y + p.beta_im * c.x;
+    }
+    reinterpret_cast<double2*>(p.out)[idx] = make_double2(vr, vi);
+    sq += vr * vr + vi * vi;
+    if (p.acc) {
+      p.acc[2 * idx] += vr;
+      p.acc[2 * idx + 1] += vi;
+    }
+  }
+  if (p.partials) row_norm(sq, p.partials + ia, smem);
+}
+
 __global__ void __launch_bounds__(kRowThreads, 2) k_pull_rows_oz(OzRowsArgs p) {
   extern __shared__ __align__(16) char smem[];
   if (p.done && *p.done) return;
@@ -320,7 +360,9 @@ __global__ void __launch_bounds__(kRowThreads, 2) k_pull_rows_oz(OzRowsArgs p) {
   const int cl = lane & 15;
   const int lenb = static_cast<int>(p.lenb);
   const int nqp = 16 * p.nqt;
-  const int64_t ia = xcd_order(blockIdx.x, p.lena);
+  // nseg workgroups share a row, each with its part of the column chunks
+  const int64_t ia = p.nseg > 1 ? blockIdx.x / p.nseg : xcd_order(blockIdx.x, p.lena);
+  const int seg = p.nseg > 1 ? static_cast<int>(blockIdx.x) % p.nseg : 0;
   const int accb = lenb * 16 > kOzPartBytes ? lenb * 16 : kOzPartBytes;
   unsigned long long* accs = reinterpret_cast<unsigned long long*>(smem);  // [lenb][re, im]
   double* part = reinterpret_cast<double*>(smem);       // set-up: [4][kOzQ]
@@ -405,14 +447,16 @@ __global__ void __launch_bounds__(kRowThreads, 2) k_pull_rows_oz(OzRowsArgs p) {
   }
   if (tid < kOzQ / 2) shift[tid] = reinterpret_cast<const uint32_t*>(p.unit->right)[tid];
   __syncthreads();
-  for (int x = tid; x < 2 * lenb; x += kRowThreads) accs[x] = p.half;
+  for (int x = tid; x < 2 * lenb; x += kRowThreads) accs[x] = seg ? 0 : p.half;
   __syncthreads();
 
   const __amdgpu_buffer_rsrc_t rc = buffer_of(p.coeff, p.lena * p.lenb * 16);
   const __amdgpu_buffer_rsrc_t rf = buffer_of(p.fwd, static_cast<int64_t>(nqp) * lenb * 4);
   // the target words' offsets are those of element target + 1
   char* accum = smem - 16;
-  const int nchunks = (lenb + kRowCols - 1) / kRowCols;
+  const int chunks = (lenb + kRowCols - 1) / kRowCols;
+  const int first = chunks * seg / p.nseg;
+  const int nchunks = chunks * (seg + 1) / p.nseg;
   u32x4 la[3][4];
   auto load = [&](int chunk, int b, u32x4 (&A)[4]) {
     const int jb = chunk * kRowCols + wave * 16 + cl;
@@ -427,9 +471,9 @@ __global__ void __launch_bounds__(kRowThreads, 2) k_pull_rows_oz(OzRowsArgs p) {
   // LEFT: some rows shift to the left.  A whole second loop, so that the usual
   // one has no more than its right shifts (as a condition per value 4% slower)
   auto run = [&](auto LEFT) {
-  load(0, 0, la[0]);
-  load(0, 1, la[1]);
-  for (int chunk = 0; chunk < nchunks; ++chunk) {
+  load(first, 0, la[0]);
+  load(first, 1, la[1]);
+  for (int chunk = first; chunk < nchunks; ++chunk) {
     const int jb = chunk * kRowCols + wave * 16 + cl;
     const bool colok = jb < lenb;
     int4v dd[2][kOzDDig];                   // [re, im][digit]
@@ -533,32 +577,23 @@ __global__ void __launch_bounds__(kRowThreads, 2) k_pull_rows_oz(OzRowsArgs p) {
   else run(std::false_type{});
   __syncthreads();
   const double back = ldexp(*scale, 32 - p.unit->e);
-  double2* racc = reinterpret_cast<double2*>(p.rowacc) + ia * p.lenb;
-  double sq = 0.0;
-  for (int x = tid; x < lenb; x += kRowThreads) {
-    const double2 r = racc[x];
-    const double re = r.x + back * static_cast<double>(static_cast<int64_t>(accs[2 * x]));
-    const double im = r.y + back * static_cast<double>(static_cast<int64_t>(accs[2 * x + 1]));
-    if (!p.out) {
-      racc[x] = make_double2(re, im);
-      continue;
-    }
-    const int64_t idx = ia * p.lenb + x;
-    double vr = p.alpha_re * re - p.alpha_im * im;
-    double vi = p.alpha_re * im + p.alpha_im * re;
-    if (p.beta_re != 0.0 || p.beta_im != 0.0) {
-      const double2 c = reinterpret_cast<const double2*>(p.cin)[idx];
-      vr += p.beta_re * c.x - p.beta_im * c.y;
-      vi += p.beta_re * c.y + p.beta_im * c.x;
-    }
-    reinterpret_cast<double2*>(p.out)[idx] = make_double2(vr, vi);
-    sq += vr * vr + vi * vi;
-    if (p.acc) {
-      p.acc[2 * idx] += vr;
-      p.acc[2 * idx + 1] += vi;
-    }
+  if (p.nseg > 1) {
+    unsigned long long* sums = p.sums + ia * p.lenb * 2;
+    for (int x = tid; x < 2 * lenb; x += kRowThreads)
+      if (accs[x]) atomicAdd(sums + x, accs[x]);
+    if (seg == 0 && tid == 0) p.back[ia] = back;
+    return;
   }
-  if (p.partials) row_norm(sq, p.partials + ia, smem);
+  oz_finish(p, ia, back, [&](int x) { return accs[x]; }, smem);
+}
+
+// The rows that k_pull_rows_oz left as sums over its segments.
+__global__ void __launch_bounds__(kRowThreads) k_pull_sums_oz(OzRowsArgs p) {
+  __shared__ double red[kRowThreads / 64];
+  if (p.done && *p.done) return;
+  const int64_t ia = blockIdx.x;
+  const unsigned long long* sums = p.sums + ia * p.lenb * 2;
+  oz_finish(p, ia, p.back[ia], [&](int x) { return sums[x]; }, reinterpret_cast<char*>(red));
 }
 
 constexpr size_t kLdsLimit = 160 * 1024;
@@ -575,9 +610,23 @@ bool pull_oz_supported(const fqehip_sector* s) {
          oz_rows_lds_bytes(s->lenb, (s->npull + 15) / 16) <= kLdsLimit;
 }
 
-// The opposite-spin rows on top of rowacc (epilogue as launch_pull_rows).
+// Workgroups per alpha string of the digit rows.  A row is a workgroup until
+// there are too few for the chip; then its column chunks are shared out to as
+// many as fill it, which are summed in global memory (integers: in any order) at
+// the price of a launch and of a set-up each (some 18 us beside 6.5 per chunk).
+// Rows of 3432 columns, us with one workgroup / with segments and their sum: 14
+// rows 194 / 34, 91 rows 202 / 124; of 6435 columns: 105 rows 409 / 251.
+int pull_oz_segments(const fqehip_sector* s) {
+  const int64_t fill = 256 / (s->lena > 0 ? s->lena : 1);
+  const int64_t chunks = (s->lenb + kRowCols - 1) / kRowCols;
+  const int64_t n = fill < chunks ? fill : chunks;
+  return n > 1 ? static_cast<int>(n) : 1;
+}
+
+// The opposite-spin rows on top of rowacc (epilogue as launch_pull_rows); sums:
+// with segments, the zeroed 2 lena lenb integers, then lena doubles.
 int launch_pull_rows_oz(const fqehip_sector* s, const double* coeff,
-                        const double* rowmax, double* rowacc,
+                        const double* rowmax, double* rowacc, double* sums,
                         const PullEpilogue& e, hipStream_t st,
                         const int32_t* done) {
   OzRowsArgs p{};
@@ -606,9 +655,16 @@ int launch_pull_rows_oz(const fqehip_sector* s, const double* coeff,
   p.acc = e.acc;
   p.partials = e.partials;
   p.done = done;
-  k_pull_rows_oz<<<static_cast<unsigned>(s->lena), kRowThreads,
+  p.nseg = pull_oz_segments(s);
+  p.sums = reinterpret_cast<unsigned long long*>(sums);
+  p.back = sums + 2 * s->lena * s->lenb;
+  k_pull_rows_oz<<<static_cast<unsigned>(s->lena * p.nseg), kRowThreads,
                    oz_rows_lds_bytes(s->lenb, p.nqt), st>>>(p);
   FQEHIP_CHECK_LAUNCH("k_pull_rows_oz");
+  if (p.nseg > 1) {
+    k_pull_sums_oz<<<static_cast<unsigned>(s->lena), kRowThreads, 0, st>>>(p);
+    FQEHIP_CHECK_LAUNCH("k_pull_sums_oz");
+  }
   return FQEHIP_OK;
 }
 
@@ -1109,14 +1165,15 @@ int launch_alpha_gemm_oz(int64_t lena, int64_t lenb, const void* hoz,
   return FQEHIP_OK;
 }
 
-// Row maxima of |C|, and with colmax its column maxima.
+// Row maxima of |C|, with colmax its column maxima; zeroes nsum sums.
 int launch_absmax(int64_t lena, int64_t lenb, const double* coeff,
-                  double* rowmax, double* colmax, hipStream_t st,
-                  const int32_t* done) {
+                  double* rowmax, double* colmax, double* sums, int64_t nsum,
+                  hipStream_t st, const int32_t* done) {
   if (lena == 0 || lenb == 0) return FQEHIP_OK;
   const unsigned grid = static_cast<unsigned>(lena < 65536 ? lena : 65536);
   unsigned long long* cm = reinterpret_cast<unsigned long long*>(colmax);
-  k_row_absmax<<<grid, 256, 0, st>>>(lena, lenb, coeff, rowmax, cm, done);
+  k_row_absmax<<<grid, 256, 0, st>>>(lena, lenb, coeff, rowmax, cm,
+                                     reinterpret_cast<unsigned long long*>(sums), nsum, done);
   FQEHIP_CHECK_LAUNCH("k_row_absmax");
   if (!colmax) return FQEHIP_OK;
   const dim3 cgrid(blocks_for(lenb, 256), blocks_for(lena, kColRows));
@@ -1165,7 +1222,7 @@ extern "C" int fqehip_beta_gemm_digits(int64_t lena, int64_t lenb,
   hipStream_t st = as_stream(stream);
   double* rowmax = static_cast<double*>(d_work);
   int rc = launch_absmax(lena, lenb, static_cast<const double*>(d_coeff),
-                         rowmax, nullptr, st, d_done);
+                         rowmax, nullptr, nullptr, 0, st, d_done);
   if (rc) return rc;
   return launch_beta_gemm_oz(lena, lenb, d_hoz,
                              static_cast<const double*>(d_coeff), rowmax,

@@ -56,8 +56,9 @@ int launch_pull_group(const PullGroupLaunch& g, const void* d_secs, int step,
                       double ar, double ai, hipStream_t st);
 
 bool pull_oz_supported(const fqehip_sector* s);
+int pull_oz_segments(const fqehip_sector* s);
 int launch_pull_rows_oz(const fqehip_sector* s, const double* coeff,
-                        const double* rowmax, double* rowacc,
+                        const double* rowmax, double* rowacc, double* sums,
                         const PullEpilogue& e, hipStream_t st,
                         const int32_t* done);
 

@@ -549,3 +549,52 @@ def test_spin_block_elements(fqe, kind, nele, norb):
         want = want + numpy.einsum("p,pij->ij", a[:-1, q], pair) @ pair[q]
     scale = max(numpy.abs(want).max(), 1e-300)
     assert numpy.abs(got - want).max() <= 1e-13 * scale
+
+
+@pytest.mark.parametrize("na,nb,norb", [(1, 5, 10), (1, 6, 13), (2, 5, 11),
+                                        (2, 6, 12), (0, 5, 10), (10, 4, 10)])
+def test_digit_rows_in_segments(fqe, na, nb, norb):
+    """Few alpha strings and several 128-column chunks: a row's chunks are
+    shared among workgroups (two, all, uneven shares, and a single row), in
+    every form of the epilogue and in a Taylor series.  Tolerance and bits
+    as in test_digit_rows_edges and test_series_in_digits."""
+    import torch
+    from fqe_amd import _lib, engine, settings
+    print(f"digit segments {na} {nb} {norb}", flush=True)
+    d, c, g, rng = sector(fqe, na, nb, norb, 11 * norb + 5 * na + nb)
+    h = tensors("real", norb, rng)
+    op = prepared(fqe, "real", h, norb)
+    graph, x = d.get_fcigraph(), d.device_coeff()
+    key = (na + nb, na - nb)
+    wfn = fqe.Wavefunction([[na + nb, na - nb, norb]])
+    wfn.set_wfn("from_data", {key: c / numpy.linalg.norm(c)})
+    ham = fqe.get_restricted_hamiltonian(h)
+
+    def run():
+        out = torch.empty_like(x)
+        acc = torch.ones_like(x)
+        engine.apply_sector(graph, x, op, out, alpha=0.5 - 2j, beta=1.5j,
+                            cin=x, acc=torch.view_as_real(acc))
+        inplace = x.clone()
+        n = engine.norm_partials_count(x.numel())
+        part = torch.zeros(max(n, 1), dtype=torch.float64, device=x.device)
+        engine.apply_sector(graph, inplace, op, inplace, alpha=2.0,
+                            partials=part)
+        ev = wfn.time_evolve(0.05, ham)
+        return [t.cpu().numpy() for t in (out, acc, inplace)] + [
+            ev.get_coeff(key), numpy.sqrt(part.sum().item())], \
+            ev._taylor_terms
+    want, terms = run()
+    saved = settings.contraction, settings.ozaki_min_determinants
+    settings.contraction, settings.ozaki_min_determinants = "ozaki", 0
+    try:
+        s, keep = engine.sector_struct(graph, op, _lib.C128)
+        assert s.w_oz and s.haa_oz and s.hbb_oz
+        got, got_terms = run()
+        again, _ = run()
+    finally:
+        settings.contraction, settings.ozaki_min_determinants = saved
+    assert got_terms == terms
+    for a, b, w in zip(got, again, want):
+        assert rel(a, w) < 3e-11
+        assert numpy.array_equal(a, b)
