@@ -389,7 +389,7 @@ def sector_struct(graph, op: PreparedOperator,
         if settings.contraction == "ozaki":
             s.tile = _lib.TILE_OZAKI
             digits = None
-            if s.lena * s.lenb >= settings.ozaki_min_determinants:
+            if settings.runs_digits(s.lena, s.lenb):
                 digits = op.pull_digits(graph)
             if digits is not None:
                 keep += digits

@@ -57,10 +57,10 @@ ozaki_beta = True
 
 # With contraction = "ozaki": sectors below this many determinants run in
 # FP64, where the digit kernels' extra launches (maxima, digits) cost more
-# than the faster products save.  Measured, FP64 / digits: norb 11 5a6b
-# (213,444) 113 / 137 us, norb 12 4a5b (392,040) 186 / 181 us, norb 12 4a6b
-# (457,380) 207 / 198 us, norb 12 6a6b (853,776) 380 / 307 us.
-ozaki_min_determinants = 400000
+# than the faster products save; 0: digits wherever the kernels take them.
+# It is the size of a sector of as many alpha as beta strings; of others the
+# work of the same-spin products is compared with that one's (runs_digits).
+ozaki_min_determinants = 385000
 
 # Largest apply workspace (bytes) allocated at once: a complex128 sector
 # whose unfused dvec + Y would need more runs the apply in panels of
@@ -78,3 +78,24 @@ def kernel_choice():
     """Every setting that picks an apply's kernels."""
     return (fused, split, split_fp64, split_tile, split_tile_fp64, contraction,
             ozaki_beta, ozaki_min_determinants)
+
+
+def runs_digits(lena, lenb):
+    """Whether a sector runs on digits with contraction = "ozaki".
+    Measured, FP64 / digits in us (strings alpha x beta):
+    - by the work of the same-spin products: 462 x 462 91 / 132, 220 x 924
+      106 / 130, 495 x 792 180 / 175, 364 x 1001 231 / 217, 495 x 924 199 /
+      192, 792 x 792 316 / 266, 1001 x 1001 519 / 381;
+    - FP64 rows of few alpha strings leave the chip idle, digit rows are
+      shared out: 13 x 1716 120 / 92, 78 x 1716 163 / 136, 91 x 2002 245 /
+      170, 14 x 3432 356 / 152, but 66 x 924 80 / 93;
+    - a digit row costs its set-up, whatever its length: 6435 x 15 359 / 605,
+      3003 x 91 302 / 311, 3432 x 91 359 / 351 (first apply 803 / 1300),
+      6435 x 105 961 / 688."""
+    least = ozaki_min_determinants
+    if least == 0:
+        return True
+    if lena <= 128 and lenb * lenb >= 4 * least:
+        return True
+    work = lena * lenb * (lena + lenb) / (2 * least**1.5)
+    return work >= (1 if lenb >= 128 else 4)

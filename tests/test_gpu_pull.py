@@ -598,3 +598,14 @@ def test_digit_rows_in_segments(fqe, na, nb, norb):
     for a, b, w in zip(got, again, want):
         assert rel(a, w) < 3e-11
         assert numpy.array_equal(a, b)
+
+
+def test_which_sectors_run_on_digits(fqe):
+    """The rule at the sizes beside its measured crossings."""
+    from fqe_amd import settings
+    for lena, lenb, digits in (
+            (462, 462, False), (220, 924, False), (364, 1001, True),
+            (792, 792, True), (13, 1716, True), (66, 924, False),
+            (91, 2002, True), (3432, 14, False), (3432, 91, False),
+            (6435, 15, False), (6435, 105, True)):
+        assert settings.runs_digits(lena, lenb) == digits, (lena, lenb)
