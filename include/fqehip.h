@@ -584,7 +584,8 @@ typedef struct fqehip_batch fqehip_batch;
 
 /* Records the batch into a graph with up to nstreams parallel branches
  * (1..32), on capture streams of the batch's own (`stream` is not used
- * while recording).  Buffers are referenced, not copied: every launch on
+ * while recording).  With one branch, items may share d_term and d_workspace
+ * (pull-form sectors that do are not grouped); otherwise each needs its own.  Buffers are referenced, not copied: every launch on
  * a stream reads d_coeff0 and rewrites the outputs.  With group != 0 the
  * sectors that take the fused row kernel without the split (hbb_hi and
  * hbb_f64 NULL, tile not FQEHIP_TILE_OZAKI) run as one group: per Taylor

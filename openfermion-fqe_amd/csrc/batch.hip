@@ -181,6 +181,41 @@ int enqueue_group(int precision, const fqehip_batch_item* items,
 
 using namespace fqehip;
 
+namespace {
+
+// Items that write where another item reads or writes: on one stream items run
+// one after another and may share scratch, in a group's launches they do not.
+std::vector<bool> sharing_items(int precision, int nitems, const fqehip_batch_item* items) {
+  struct Range {
+    uintptr_t begin, end;
+    int item;
+    bool written;
+  };
+  std::vector<Range> r;
+  for (int i = 0; i < nitems; ++i) {
+    const fqehip_batch_item& it = items[i];
+    const int64_t n = it.sector.lena * it.sector.lenb;
+    auto add = [&](const void* p, int64_t bytes, bool written) {
+      const uintptr_t b = reinterpret_cast<uintptr_t>(p);
+      if (p && bytes > 0) r.push_back({b, b + static_cast<uintptr_t>(bytes), i, written});
+    };
+    add(it.d_coeff0, n * static_cast<int64_t>(esize(precision)), false);
+    add(it.d_apply_out, n * static_cast<int64_t>(esize(precision)), true);
+    add(it.d_term, n * static_cast<int64_t>(esize(precision)), true);
+    add(it.d_result, 16 * n, true);
+    add(it.d_workspace, fqehip_apply_workspace_bytes(precision, &it.sector), true);
+  }
+  std::sort(r.begin(), r.end(), [](const Range& a, const Range& b) { return a.begin < b.begin; });
+  std::vector<bool> shares(nitems, false);
+  for (size_t a = 0; a < r.size(); ++a)
+    for (size_t b = a + 1; b < r.size() && r[b].begin < r[a].end; ++b)
+      if (r[a].item != r[b].item && (r[a].written || r[b].written))
+        shares[r[a].item] = shares[r[b].item] = true;
+  return shares;
+}
+
+}  // namespace
+
 extern "C" int fqehip_batch_create(int precision, int nitems,
                                    const fqehip_batch_item* items,
                                    double time, int nterms, int nstreams,
@@ -238,11 +273,12 @@ extern "C" int fqehip_batch_create(int precision, int nitems,
   std::vector<int> grouped, single;
   // small real pull-form sectors: one group per class
   std::vector<std::vector<int>> pull(8);
+  const std::vector<bool> shares = sharing_items(precision, nitems, items);
   for (int i = 0; i < nitems; ++i) {
     const fqehip_batch_item& it = items[i];
     if (group && it.sector.lena * it.sector.lenb > 0 && !it.op.complex_op &&
         fqehip_pull_supported(precision, &it.sector, &it.op) &&
-        !digit_rows(&it.sector)) {
+        !digit_rows(&it.sector) && !shares[i]) {
       const int c = pull_group_class(&it.sector);
       if (c > 0 && c < 8) {
         pull[c].push_back(i);

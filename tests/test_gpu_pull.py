@@ -609,3 +609,47 @@ def test_which_sectors_run_on_digits(fqe):
             (91, 2002, True), (3432, 14, False), (3432, 91, False),
             (6435, 15, False), (6435, 105, True)):
         assert settings.runs_digits(lena, lenb) == digits, (lena, lenb)
+
+
+def test_batch_items_that_share_scratch(fqe):
+    """One branch runs its items one after another, so they may share the
+    term buffer and the workspace; a group's launches run them at once, so
+    those items stay out of it.  Against items with buffers of their own,
+    1e-13 as in test_batch_terms."""
+    import ctypes
+    import torch
+    from fqe_amd import _lib, batched
+    rng = numpy.random.default_rng(8)
+    shapes = [(8, 4, 4), (7, 3, 4), (9, 4, 4), (6, 3, 3), (8, 4, 3)]
+    specs = []
+    for norb, na, nb in shapes:
+        h1, h2 = fo.synthetic_hamiltonian(norb, norb, rng)
+        g = fo.OracleGraph(na, nb, norb)
+        specs.append(batched.SectorSpec(
+            norb=norb, nalpha=na, nbeta=nb, h1=h1, h2=h2,
+            coeff=fo.synthetic_coeff(g.lena, g.lenb, rng)))
+    tiles = {f"{n},{a},{b}": "split" for n, a, b in shapes}
+    own = batched.BatchedTaylor(specs, 0.1, nterms=4, dtype=torch.complex128,
+                                tiles=tiles, nstreams=2)
+    own.build()
+    own.launch()
+    want = own.results()
+    bt = batched.BatchedTaylor(specs, 0.1, nterms=4, dtype=torch.complex128,
+                               tiles=tiles, nstreams=1)
+    items = [p.item() for p in bt.sectors]
+    ws = max((p.ws for p in bt.sectors[:4]), key=lambda t: t.numel())
+    term = max((p.term for p in bt.sectors[:4]), key=lambda t: t.numel())
+    for it in items[:4]:                     # the last keeps its own
+        it.d_workspace, it.d_term = _lib.ptr(ws), _lib.ptr(term)
+    handle = ctypes.c_void_p()
+    torch.cuda.synchronize()
+    _lib.call("fqehip_batch_create", bt.prec, len(items),
+              (_lib.BatchItem * len(items))(*items), bt.time, 4, 1, 1,
+              _lib.stream_ptr(), ctypes.byref(handle))
+    bt._batch = handle
+    for _ in range(2):
+        bt.launch()
+        for (a0, e0), (a1, e1) in zip(bt.results(), want):
+            assert rel(a0, a1) < 1e-13 and rel(e0, e1) < 1e-13
+    own.close()
+    bt.close()
