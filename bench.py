@@ -230,10 +230,10 @@ def _time_graph(graph, steps, warmup):
 
 def batched_main(args):
     """Batched uneven sectors, one graph launch per batch: the autotuned
-    complex128 graph with Ozaki-digit split contractions (the mixed engine
-    at <= 1e-9; value), the autotuned complex128 FP64 graph, the complex64
-    BF16x3 graph (outside the gate), and the per-sector sequential FP64
-    path, on the same sectors."""
+    complex128 graph with Ozaki digit products where they pay (the mixed
+    engine at <= 1e-9; value), the autotuned complex128 FP64 graph, the
+    complex64 BF16x3 graph (outside the gate), and the per-sector sequential
+    FP64 path, on the same sectors."""
     import numpy
     import torch
     from fqe_amd import batched
@@ -275,7 +275,11 @@ def batched_main(args):
         counts = {}
         for v in tiles.values():
             counts[v] = counts.get(v, 0) + 1
+        digit = [p.n() for p in g.sectors if p.s.w_oz]
         runs[name] = {"wall": wall, "errs": errs(g.results()),
+                      "digits": f"{len(digit)} of {len(specs)} sectors, "
+                                f"{sum(digit)} of {g.determinants()} "
+                                "determinants",
                       "variants": counts, "grouped": g.grouped(),
                       "tune": t_tune, "build": t_build,
                       "ndet": g.determinants()}
@@ -293,8 +297,8 @@ def batched_main(args):
         "value": round(applies / oz["wall"], 1), "unit": "sector-applies/s",
         "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
         "ms_per_step": round(1e3 * oz["wall"], 3), "higher_is_better": True,
-        "dtype": ("c128 storage; split sectors with Ozaki int8 digit "
-                  "products, other sectors FP64"),
+        "dtype": ("c128 storage; Ozaki int8 digit products in "
+                  f"{oz['digits']}, FP64 in the others"),
         "data": "synthetic",
         "config": {"workload": f"{len(specs)} sectors, norb 6..12, nalpha and "
                                f"nbeta uniform in [1, norb-1], seed 3, "
@@ -936,8 +940,14 @@ def time_evolve_lines(with_cpu):
                                  "accuracy 1e-15, expansion 30"),
                     "timing": "median of 3 calls after one untimed call"}
             res = {}
-            for eng, graph in (("fp64", False), ("fp64", True),
-                               ("ozaki", False), ("ozaki", True)):
+            engines = ["fp64"]
+            if settings.runs_digits(*c.shape):
+                engines.append("ozaki")
+            else:
+                line["ozaki"] = ("runs in FP64: digits do not pay on a "
+                                 "sector of this size")
+            for eng, graph in ((e, g) for e in engines
+                               for g in (False, True)):
                 settings.contraction, settings.taylor_graph = eng, graph
                 try:
                     sec, ev = _timed_evolve(wfn, ham, t)
