@@ -393,9 +393,10 @@ int fqehip_apply(int precision, const fqehip_sector* s,
  * and tight serving loops.  The workspace is a library-owned device array
  * of FQEHIP_NOALLOC_SCRATCH_BYTES per GPU, held from library load until
  * the process ends; a sector whose apply needs more returns
- * FQEHIP_ERR_UNSUPPORTED (fqehip_apply_workspace_bytes bounds the need;
- * the fused path needs (nslot+1)*2*lena*lenb elements, e.g. norb=12
- * 6a6b complex64 fits, complex128 does not).  Arguments and results are
+ * FQEHIP_ERR_UNSUPPORTED.  A sector is measured by the fused path's
+ * (nslot+1)*2*lena*lenb elements, e.g. norb=12 6a6b complex64 fits,
+ * complex128 does not, or by the unfused path's planes, also where the pull
+ * form would need less.  Arguments and results are
  * those of fqehip_apply.  All calls on one GPU share its array: calls that
  * overlap on one GPU (other streams, other host threads) race. */
 #define FQEHIP_NOALLOC_SCRATCH_BYTES (256ll * 1024 * 1024)

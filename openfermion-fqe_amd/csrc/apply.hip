@@ -1128,7 +1128,7 @@ extern "C" int fqehip_taylor(int precision, const fqehip_sector* s,
   // wave can afford to read the partials, the test of a term is made at the
   // start of the next one's first kernel instead of in a launch of its own
   // (from the other of two sets of partials), and the smallest sectors' rows
-  // include the same-spin part: 586 -> 502 us at 8 orbitals half filled,
+  // include the same-spin part: 586 -> 480 us at 8 orbitals half filled,
   // 693 -> 663 us with 9 orbitals, 4 + 4 electrons (28 terms).
   void* cur = d_term;
   void* nxt = d_workspace;

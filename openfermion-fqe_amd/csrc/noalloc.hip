@@ -27,8 +27,10 @@ std::once_flag g_once[kMaxDevices];
 void* g_scratch[kMaxDevices];
 hipError_t g_status[kMaxDevices];
 
-// Workspace bytes of the path fqehip_apply takes for this sector and
-// operator (the one-body apply needs none).
+// What a sector is measured by against the fixed array: the slot rows of the
+// fused paths, or the dvec and Y planes (the one-body apply needs nothing).  The
+// pull form, which fqehip_apply takes where it can, needs less, but the sectors
+// that are taken and refused do not depend on the form.
 int64_t needed_bytes(int precision, const fqehip_sector* s,
                      const fqehip_operator* op) {
   if (op->h1) return 0;
@@ -37,7 +39,7 @@ int64_t needed_bytes(int precision, const fqehip_sector* s,
   if (fqehip_fused_supported(precision, s, op)) {
     int64_t b = static_cast<int64_t>(s->nslot + 1) * 2 * n * elem;
     // what the pull form needs beyond its row accumulators (the digit
-    // kernels' maxima and planes)
+    // kernels' maxima, sums and planes)
     if (fqehip_pull_supported(precision, s, op))
       b += fqehip::pull_spare_offset(s) - 2 * n * elem;
     return b;

@@ -790,7 +790,8 @@ bool split_same_spin(int64_t lena, int64_t lenb) {
 // but every row reads all of C and Hbb, in time about lenb max(lena, lenb).
 // Evolution in us, same-spin kernel / in the row: 20 x 15 strings 449 / 339,
 // 35 x 35 420 / 346, 56 x 56 432 / 386, 70 x 70 505 / 500, 126 x 84 502 / 551,
-// 252 x 45 533 / 590.
+// 252 x 45 533 / 590.  The line lies at the tie (4900); nothing between it and
+// 10584 was measured.
 bool pull_in_row(int64_t lena, int64_t lenb) {
   return lenb * (lena > lenb ? lena : lenb) <= kInRowMax && lena <= 256;
 }

@@ -119,7 +119,8 @@ class FqeDataSet:
     def _dvec_rows(self, vec: torch.Tensor) -> torch.Tensor:
         """[(2 norb)^2 + 1, 2, L] planes of D[pq] = E_pq C, then C."""
         m = 2 * self._norb
-        # planar planes and a complex128 copy
+        # planar planes and _dvec's complex128 copy, also asked of rdm12, which
+        # makes none, so that the sizes it takes stay the same
         _check_fits(2 * m * m * vec.numel() * 16, "the spin-orbital dvec")
         d = engine.planar_rows(m * m, vec)
         _lib.call("fqehip_set_dvec", self._norb, self._nele, _lib.ptr(vec),
