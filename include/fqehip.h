@@ -285,8 +285,9 @@ int fqehip_beta_block(int npair, int64_t lenb, const int32_t* d_fwd_b,
  * complex_op).  V[p][q] is element (p, q) of d_v with lda doubles per row and
  * h the row d_h (for complex_op both in the real 2 x 2 block form of
  * fqehip_operator, d_v and d_h at the real part of element (0, 0)); d_fwd the
- * forward table of the npair pairs.  fqehip_beta_block is the real case with
- * its bfloat16 split.  (len + npair) * 8 bytes (16 for complex_op) <= 160 KiB;
+ * forward table of the npair pairs, norb (norb + 1) / 2 or norb^2 with len a
+ * binomial of norb (norb <= 32).  fqehip_beta_block is the real case with its
+ * bfloat16 split.  (len + npair) * 8 bytes (16 for complex_op) <= 160 KiB;
  * the same bits on every run. */
 int fqehip_spin_block(int complex_op, int npair, int64_t len,
                       const int32_t* d_fwd, const double* d_v, int64_t lda,
